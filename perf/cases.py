@@ -299,3 +299,75 @@ def tolerance(case: dict):
     if case.get("dtype") == "fp32":
         return {"rel": 1e-5, "max": 4e-4}
     return {"rel": 4e-4, "max": 0.03}
+
+
+# ---------------------------------------------------------------- the same in 64 bits
+
+def _indices(packed: torch.Tensor, bits: int, n: int, k: int) -> torch.Tensor:
+    """The indices of a packed weight: one little-endian bit stream over the matrix in row-major order."""
+    shifts = torch.arange(8, device=packed.device, dtype=torch.uint8)
+    stream = ((packed.flatten()[:, None] >> shifts) & 1).flatten()[: n * k * bits].view(n * k, bits)
+    index = torch.zeros(n * k, dtype=torch.int64, device=packed.device)
+    for b in range(bits):
+        index += stream[:, b].to(torch.int64) << b
+    return index.view(n, k)
+
+
+def _weight64(layer, table: torch.Tensor) -> torch.Tensor:
+    """The matrix that a packed weight stands for, `table[index] * row norm`."""
+    index = _indices(layer.packed_weight_indices, layer.weight_bits, layer.out_features, layer.in_features)
+    return table.double()[index] * layer.row_norms.double()[:, None]
+
+
+def _quantized64(x: torch.Tensor, layer, table: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(codes, what they stand for, norms) of the tokens: unit norm, permute, sign, Hadamard blocks, nearest centroid."""
+    x = x.double()
+    norm = x.square().sum(-1, keepdim=True).sqrt()
+    y = (x / (norm + layer.activation_eps))[:, layer.rotation.permutation.to(x.device)] * layer.rotation.signs.to(x.device, torch.float64)
+    h = layer.rotation.block_size
+    y = y.reshape(-1, h)
+    distance = 1
+    while distance < h:
+        pairs = y.view(-1, h // (2 * distance), 2, distance)
+        y = torch.stack((pairs[:, :, 0] + pairs[:, :, 1], pairs[:, :, 0] - pairs[:, :, 1]), dim=2).view(-1, h)
+        distance *= 2
+    codes = torch.bucketize((y / math.sqrt(h)).view(x.shape), layer._activation_codebook_boundaries.double())
+    return codes, table.double()[codes] * norm, norm.squeeze(-1)
+
+
+def _linear64(x: torch.Tensor, layer) -> torch.Tensor:
+    y = _quantized64(x, layer, layer._activation_codebook_centroids)[1] @ _weight64(layer, layer._weight_codebook_centroids).T
+    return y if layer.bias is None else y + layer.bias.double()
+
+
+def _mlp64(x: torch.Tensor, up, down) -> torch.Tensor:
+    """The MLP; what one layer hands to the next has the tokens' type."""
+    h = torch.nn.functional.gelu(_linear64(x, up).to(x.dtype))
+    return _linear64(h, down)
+
+
+def exact(case: dict, seed: int):
+    """What `run` returns, in 64 bits, from the packed weights and codebooks that the layers hold."""
+    kind, s = case["kind"], prepare({**case, "graph": False}, seed)
+    if kind == "linear":
+        return _linear64(s["x"], s["layer"])
+    if kind == "mlp":
+        return _mlp64(s["x"], s["up"], s["down"])
+    if kind == "block":
+        linears = getattr(s["qkv"], "linears", None)
+        qkv = _linear64(s["attention_input"], s["qkv"]) if linears is None else tuple(_linear64(s["attention_input"], l) for l in linears)
+        return {"qkv": qkv, "out": _linear64(s["attention_output"], s["out"]), "mlp": _mlp64(s["mlp_input"], s["up"], s["down"])}
+    if kind == "adaln":
+        l = s["layer"]
+        padded = l.num_groups * l.group_size
+        w = (_indices(l.packed_weight, 4, l.out_features, padded) - 8).double() * l.scales.double().repeat_interleave(l.group_size, dim=1)
+        return s["x"].double() @ w[:, : l.in_features].T + l.bias.double()
+    if kind == "native":
+        table = s["codes"].double() * s["scale"]
+        _, values, norms = _quantized64(s["x"], s["layer"], table)
+        return {"packed": None, "norms": norms, "out": values @ _weight64(s["layer"], table).T}
+    if kind == "values":
+        l = s["layer"]
+        y = s["x"].double() @ _weight64(l, l._weight_codebook_centroids).T
+        return y if l.bias is None else y + l.bias.double()
+    return None   # (indices and a table lookup: compared bit for bit)
