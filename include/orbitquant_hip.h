@@ -181,7 +181,9 @@ int oq_debug_override(const char *name, const char *value);
  * workgroup), larger M the MFMA tile kernel.  A token row's result does not depend on the
  * rows computed with it as long as the call stays within 64 rows.  A problem with few output
  * tiles and many K-steps (some hundred tokens on a short-and-long matrix) is shared between
- * workgroups along K when the caller provides a workspace for the fp32 partial tiles:
+ * workgroups along K when the caller provides a workspace for the fp32 partial tiles, and a problem
+ * of some thousand tokens is decoded once into the workspace and multiplied from there (the same
+ * bits as without):
  *
  * workspace    NULL, or a device buffer of at least oq_packed_linear_workspace_bytes(...) bytes, 16-byte
  *              aligned, that this call may overwrite (calls on one stream are ordered and may share one).
@@ -215,6 +217,22 @@ int oq_packed_linear(const void *codes, int code_format, const float *token_norm
  * reference (its wrapper sizes its own temporaries).
  */
 uint64_t oq_packed_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits);
+
+/*
+ * oq_packed_linear for 4-bit codes (two per byte) on both sides whose codebooks are int8 tables, summed in
+ * int32 on the int8 matrix instructions:
+ *
+ *   out[m,n] = (sum_k act_table[code[m,k]] * w_table[idx[n,k]]) * (s[m] * scale) * r_w[n] + bias[n]
+ *
+ * (matmul_packed_w4a4_int8, torch_binding.cpp:39-46.)  For the shapes that
+ * oq_packed_linear_int8_workspace_bytes gives a size for, with a workspace of at least that size; OQ_ERR_UNSUPPORTED
+ * for the others (0), which oq_packed_linear is at least as fast on.
+ */
+int oq_packed_linear_int8(const void *codes, const float *token_norms, float scale, const int8_t *act_table,
+                          const uint8_t *packed_w, const uint16_t *row_norms, const int8_t *w_table, const void *bias,
+                          int bias_dtype, int64_t M, int64_t N, int64_t K, void *out, int out_dtype, void *workspace,
+                          uint64_t workspace_bytes, void *stream);
+uint64_t oq_packed_linear_int8_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /*
  * `count` packed linears on the SAME activation codes (the q, k and v projections of an attention

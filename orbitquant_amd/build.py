@@ -48,6 +48,8 @@ SOURCES = {
     "packed_gemm_staged.hip": PRELOAD,
     "packed_gemm_splitk.hip": [],
     "packed_gemm_av.hip": [],
+    "operand_order.hip": [],
+    "dense_gemm.hip": [],
     "packed_gemv.hip": PRELOAD,
     "packed_gemv_group.hip": [],
     "packed_gemv_rows.hip": [],

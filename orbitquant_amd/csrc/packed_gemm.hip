@@ -1,6 +1,7 @@
 // Tile GEMM, two-4-bit-codes-per-byte activations; tile choice and dispatch for both code formats.
 #include <stdlib.h>
 
+#include "dense_gemm.h"
 #include "packed_gemm_kernel.h"
 
 namespace oq {
@@ -101,30 +102,64 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits) {
   return best;
 }
 
+// Tile of the decode-first GEMM (dense_gemm.hip) for a launch that has the workspace for it, -1 for the others.  The
+// kernel above looks every operand value up once per tile that uses it; decoding each once costs two passes over
+// memory, 2 bytes written and read again per value, and leaves the matrix cores alone with the multiplication.
+// That pays from some thousand tokens on, sooner with one code per byte (eight lookups an operand instead of four):
+// 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072 (3-bit) 335 -> 304 us,
+// 4608 x 3072 x 3072 even (85 us), 1024 x 14336 x 4096 103 -> 124 us.  It has to promise 6 % over the best launch
+// without it.
+static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes) {
+  const double a_bytes = byte_codes ? 3.0 : 2.5, w_bytes = 2.0 + bits / 8.0;
+  double dense = 0.0, packed = 0.0;
+  const int tile = dense_choose_tile(M, N, K, MF_BF16, static_cast<double>(K) * (static_cast<double>(M) * a_bytes + static_cast<double>(N) * w_bytes), &dense);
+  if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
+  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
+  choose_tile_with_cost(M, N, K, bits, &packed, byte_codes);
+  return dense < 0.94 * packed ? tile : -1;
+}
+
+// The model's time in microseconds of the packed GEMM's best launch (nibble codes).
+double gemm_cost(int64_t M, int64_t N, int64_t K, int bits) {
+  double cost = 0.0;
+  choose_tile_with_cost(M, N, K, bits, &cost);
+  return cost;
+}
+
 bool gemm_supported(int64_t K, int bits) {
   return K % 64 == 0 && (bits == 2 || bits == 3 || bits == 4 || bits == 6 || bits == 8);
 }
 
-// a_mode: 0 nibble codes, 1 bf16 values, 2 fp16 values
-// Bytes of partial tiles a launch of this shape would like to have (0: it is a single launch anyway).
-uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits) {
+// Bytes of workspace a launch of this shape would like to have: both operands decoded into operand order (large
+// problems), or partial tiles (0: it is a launch that needs neither).
+uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes) {
+  if (gemm_choose_dense(M, N, K, bits, byte_codes) >= 0) return dense_workspace_bytes(M, N, K, MF_BF16);
   const int splits = gemm_choose_splits(M, N, K, bits);
   return splits > 1 ? static_cast<uint64_t>(M) * static_cast<uint64_t>(N) * 4u * static_cast<uint64_t>(splits) : 0u;
 }
 
+// a_mode: 0 nibble codes, 1 one code per byte.
 // `workspace` (the caller's; NULL or too small: the single launch, whatever the stream is doing) holds the
 // partial tiles of a launch that shares K between workgroups.
 int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float *act_cents, int a_levels,
                   const uint8_t *w, int bits, const uint16_t *row_norms, const float *w_cents,
                   const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
                   int out_dtype, const uint16_t *out_map, void *workspace, uint64_t workspace_bytes, hipStream_t stream) {
+  if (a_mode != A_NIBBLE && a_mode != A_U8) return fail(OQ_ERR_INVALID, "packed_gemm: a_mode %d", a_mode);
+  const int dense_tile = gemm_choose_dense(M, N, K, bits, a_mode == A_U8);
+  if (dense_tile >= 0 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
+      workspace_bytes >= dense_workspace_bytes(M, N, K, MF_BF16)) {
+    unsigned char *a_values = static_cast<unsigned char *>(workspace), *w_values = a_values + operand_order_bytes(M, K, 2);
+    if (int rc = decode_operands(static_cast<const uint8_t *>(a), a_mode == A_NIBBLE ? 4 : 8, act_cents, a_levels, M, K, false, a_values, stream)) return rc;
+    if (int rc = decode_operands(w, bits, w_cents, 1 << bits, N, K, false, w_values, stream)) return rc;
+    return dense_gemm(MF_BF16, a_values, w_values, row_scale, 1.0f, row_norms, bias, bias_dtype, M, N, K, out, out_dtype, out_map, dense_tile, stream);
+  }
   GemmArgs g{};
   g.a = static_cast<const uint8_t *>(a); g.row_scale = row_scale; g.act_cents = act_cents; g.a_levels = a_levels;
   g.w = w; g.row_norms = row_norms; g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype;
   g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
   g.out_map = OutMap{out_map, out_map != nullptr && out_dtype == OQ_BF16 ? kWideLoBf16 : -1};
   int tile = choose_tile_with_cost(M, N, K, bits, nullptr, a_mode == A_U8);
-  if (a_mode != A_NIBBLE && a_mode != A_U8) return fail(OQ_ERR_INVALID, "packed_gemm: a_mode %d", a_mode);
   g.k_splits = 1;
   if (const char *where = debug_env(ENV_GEMM_STAMPS)) g.stamps = reinterpret_cast<uint64_t *>(strtoull(where, nullptr, 0));  // builds with -DOQ_GEMM_STAMPS: a device buffer for the kernel's phase stamps
   const int splits = gemm_choose_splits(M, N, K, bits);

@@ -59,7 +59,10 @@ def _workspace(nbytes: int, like: torch.Tensor) -> tuple[int | None, int, torch.
     makes it safe to drop then."""
     if nbytes <= 0:
         return None, 0, None
-    buf = torch.empty(int(nbytes), dtype=torch.uint8, device=like.device)
+    try:
+        buf = torch.empty(int(nbytes), dtype=torch.uint8, device=like.device)
+    except torch.OutOfMemoryError:   # a workspace makes a call faster, none needs it
+        return None, 0, None
     return buf.data_ptr(), int(nbytes), buf
 
 

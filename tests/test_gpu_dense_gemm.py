@@ -1,0 +1,78 @@
+"""GPU tests of the GEMM that decodes both operands first (csrc/dense_gemm.hip, csrc/operand_order.hip): the same
+operand values summed in the same order as the packed GEMM's single launches, so the same bits, for every tile, at
+ragged sizes; and the rule that chooses it depends on the workspace the caller brings."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("needs an AMD GPU")
+    from orbitquant_amd import _lib
+
+    lib = _lib.load()
+    assert lib.oq_device_ok() == 0, lib.oq_last_error()
+    return torch.device("cuda:0")
+
+
+def operands(dev, m, k, n, wbits, abits, seed):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    codes = torch.randint(0, 1 << abits, (m, k), device=dev, generator=g, dtype=torch.uint8)
+    if abits <= 4:
+        codes = codes[:, ::2] | (codes[:, 1::2] << 4)
+    return dict(
+        codes=codes.contiguous(), norms=torch.rand(m, device=dev, generator=g) + 0.5,
+        acents=torch.randn(1 << abits, device=dev, generator=g) * 0.02, wcents=torch.randn(1 << wbits, device=dev, generator=g) * 0.02,
+        packed=torch.randint(0, 256, ((n * k * wbits + 7) // 8,), device=dev, generator=g, dtype=torch.uint8),
+        rn=(torch.rand(n, device=dev, generator=g) + 0.5).to(torch.bfloat16), bias=torch.randn(n, device=dev, generator=g))
+
+
+def multiply(o, m, k, n, wbits, abits, dtype, output_map=None):
+    from orbitquant_amd import ops
+
+    return ops.packed_linear(o["codes"], o["norms"], o["acents"], o["packed"], o["rn"], o["wcents"], code_format="nibble" if abits <= 4 else "u8",
+                             activation_bits=abits, weight_bits=wbits, out_features=n, in_features=k, bias=o["bias"], output_dtype=dtype,
+                             output_map=output_map)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("m,k,n,wbits,abits,dtype,mapped", [
+    (300, 64, 264, 4, 4, torch.bfloat16, False), (257, 192, 520, 3, 3, torch.float16, False), (512, 1024, 512, 2, 4, torch.bfloat16, True),
+    (129, 576, 1000, 6, 6, torch.float32, False), (65, 128, 72, 8, 8, torch.float16, True)])
+def test_same_bits_as_the_packed_gemm(dev, library_switch, tile, m, k, n, wbits, abits, dtype, mapped):
+    from orbitquant_amd import ops
+
+    o = operands(dev, m, k, n, wbits, abits, seed=m + n)
+    table = ops.activation_table(torch.nn.functional.gelu, dtype, dev) if mapped else None
+    library_switch("OQ_GEMM_TILE", 0)
+    library_switch("OQ_DENSE_GEMM", "never")
+    want = multiply(o, m, k, n, wbits, abits, dtype, table)
+    library_switch("OQ_DENSE_GEMM", tile)
+    assert torch.equal(multiply(o, m, k, n, wbits, abits, dtype, table), want)
+
+
+def test_chosen_for_large_problems_only_and_only_with_a_workspace(dev):
+    from orbitquant_amd import _lib, ops
+
+    lib = _lib.load()
+    m, k, n = 4104, 3072, 9216
+    want_bytes = lib.oq_packed_linear_workspace_bytes(m, n, k, 4, 0, 6)
+    assert want_bytes == (-(-m // 32) + n // 32) * (k // 64) * 4096
+    assert lib.oq_packed_linear_workspace_bytes(128, n, k, 4, 0, 6) < want_bytes // 8
+    o = operands(dev, m, k, n, 4, 6, seed=3)
+    with_workspace = multiply(o, m, k, n, 4, 6, torch.bfloat16)
+    out = torch.empty_like(with_workspace)
+    dt = ops._DTYPES
+    for workspace, size in ((None, 0), (torch.empty(4096, dtype=torch.uint8, device=dev), 4096)):   # none, too small
+        rc = lib.oq_packed_linear(o["codes"].data_ptr(), 0, o["norms"].data_ptr(), o["acents"].data_ptr(), 6, o["packed"].data_ptr(), 4,
+                                  o["rn"].data_ptr(), o["wcents"].data_ptr(), o["bias"].data_ptr(), dt[torch.float32], m, n, k, out.data_ptr(),
+                                  dt[torch.bfloat16], None if workspace is None else workspace.data_ptr(), size,
+                                  torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and torch.equal(out, with_workspace)
