@@ -313,6 +313,51 @@ def packed_linear(
     return out.reshape(*lead, out_features)
 
 
+def packed_linear_int8(
+    codes: torch.Tensor,
+    token_norms: torch.Tensor,
+    activation_table: torch.Tensor,
+    packed_weight_indices: torch.Tensor,
+    row_norms: torch.Tensor,
+    weight_table: torch.Tensor,
+    *,
+    scale: float,
+    out_features: int,
+    in_features: int,
+    bias: torch.Tensor | None = None,
+    output_dtype: torch.dtype = torch.bfloat16,
+) -> torch.Tensor | None:
+    """`packed_linear` of 4-bit codes on both sides through tables of sixteen int8 values, multiplied as integers
+    (`oq_packed_linear_int8`); None where that kernel does not pay, does not take the call or has no room for its
+    workspace (`packed_linear` takes it then)."""
+    lib = _lib.load()
+    width = in_features // 2
+    flat = codes.contiguous().reshape(-1, width)
+    m = flat.shape[0]
+    need = lib.oq_packed_linear_int8_workspace_bytes(m, int(out_features), int(in_features))
+    if need == 0 or flat.data_ptr() % 16 != 0 or packed_weight_indices.data_ptr() % 16 != 0:
+        return None
+    packed_weight_indices = _operand(packed_weight_indices, "packed_weight_indices", codes, dtype=torch.uint8,
+                                     min_numel=(out_features * in_features + 1) // 2)
+    row_norms = _operand(row_norms, "row_norms", codes, dtype=torch.bfloat16, numel=out_features)
+    activation_table = _operand(activation_table, "activation_table", codes, dtype=torch.int8, numel=16)
+    weight_table = _operand(weight_table, "weight_table", codes, dtype=torch.int8, numel=16)
+    bias = _operand(bias, "bias", codes, dtype=_FLOATS, numel=out_features)
+    norms = _operand(token_norms.reshape(-1), "token_norms", codes, dtype=torch.float32, numel=m)
+    out = torch.empty((m, out_features), dtype=output_dtype, device=codes.device)
+    ws_ptr, ws_bytes, ws = _workspace(need, codes)
+    if ws_ptr is None:
+        return None
+    with _OnDevice(codes):
+        rc = lib.oq_packed_linear_int8(
+            flat.data_ptr(), norms.data_ptr(), float(scale), activation_table.data_ptr(), packed_weight_indices.data_ptr(),
+            row_norms.data_ptr(), weight_table.data_ptr(), _ptr(bias), _dt(bias) if bias is not None else OQ_F32, m,
+            int(out_features), int(in_features), out.data_ptr(), _DTYPES[output_dtype], ws_ptr, ws_bytes, _stream(codes))
+    del ws
+    _lib.check(rc, "oq_packed_linear_int8")
+    return out.reshape(*codes.shape[:-1], out_features)
+
+
 def packed_linear_group(
     codes: torch.Tensor,
     token_norms: torch.Tensor,

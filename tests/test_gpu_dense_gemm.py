@@ -76,3 +76,23 @@ def test_chosen_for_large_problems_only_and_only_with_a_workspace(dev):
                                   dt[torch.bfloat16], None if workspace is None else workspace.data_ptr(), size,
                                   torch.cuda.current_stream().cuda_stream)
         assert rc == 0 and torch.equal(out, with_workspace)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("m,k,n", [(65, 64, 72), (300, 192, 264), (257, 1088, 520)])
+def test_int8_pair_sums_integers_exactly(dev, library_switch, tile, m, k, n):
+    import orbitquant_packed_matmul as package
+
+    o = operands(dev, m, k, n, 4, 4, seed=m)
+    library_switch("OQ_DENSE_GEMM", tile)
+    a_table = torch.tensor([-128, -79, -62, -48, -36, -25, -15, -5, 0, 15, 25, 36, 48, 62, 79, 127], dtype=torch.int8, device=dev)
+    w_table = a_table.flip(0).contiguous()
+    got = package.matmul_packed_w4a4_int8(o["codes"], o["packed"], o["norms"], o["rn"], a_table, w_table, activation_scale=0.005, weight_scale=0.004,
+                                          out_features=n, in_features=k, bias=o["bias"].half(), output_dtype=torch.float16)
+    value = lambda packed, rows, table: table.double()[torch.stack((packed & 15, packed >> 4), dim=-1).long()].view(rows, k)
+    sums = value(o["codes"], m, a_table) @ value(o["packed"].view(n, k // 2), n, w_table).T
+    exact = sums * (o["norms"].double() * (0.005 * 0.004))[:, None] * o["rn"].double() + o["bias"].half().double()
+    # one rounding of the sum, three of products, one of the addition (2^-24 each, of terms no larger than |exact| +
+    # |bias| in the addition), then half an ulp of fp16
+    bound = exact.abs() * 2.0 ** -11 + (exact.abs() + o["bias"].abs().double()) * 2.0 ** -20 + 2.0 ** -24
+    assert bool(((got.double() - exact).abs() <= bound).all())
