@@ -47,3 +47,25 @@ def test_dequantize_packed_weight(bits, N, K, dtype):
     want = torch.from_numpy(cents[idx] * norms.float().numpy()[:, None]).to(dtype)   # one fp32 product, one rounding
     assert got.shape == (N, K) and got.dtype == dtype
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("bits,N,K", [(2, 6, 8), (3, 4, 8), (4, 1, 8), (6, 2, 8), (8, 1, 8), (3, 2100, 2104), (4, 577, 7288), (6, 1090, 4104)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_dequantize_rows_of_whole_groups(bits, N, K, dtype):
+    """The smallest streams of whole dwords, and streams of more than one turn of the grid with odd row lengths."""
+    test_dequantize_packed_weight(bits, N, K, dtype)
+
+
+@pytest.mark.parametrize("bits", [3, 4])
+def test_dequantize_of_an_unaligned_stream(bits):
+    from orbitquant_amd import ops
+
+    N, K = 5, 64
+    rng = np.random.default_rng(bits)
+    idx = rng.integers(0, 1 << bits, size=(N, K), dtype=np.uint8)
+    buf = torch.empty(1 + N * K * bits // 8, dtype=torch.uint8, device="cuda:0")
+    buf[1:] = torch.from_numpy(o.pack_bits(idx.reshape(-1), bits)).to("cuda:0")
+    cents = torch.from_numpy(rng.standard_normal(1 << bits).astype(np.float32)).to("cuda:0")
+    got = ops.dequantize_packed_weight(buf[1:], torch.ones(N, dtype=torch.bfloat16, device="cuda:0"), cents, bits=bits, out_features=N,
+                                       in_features=K, dtype=torch.float32)
+    assert torch.equal(got.cpu(), cents.cpu()[torch.from_numpy(idx).long()])
