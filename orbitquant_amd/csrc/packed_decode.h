@@ -283,7 +283,8 @@ __device__ __forceinline__ void request_pair_seed(float (&lo_w)[4], float (&hi_w
   }
 }
 
-template <int BITS, bool HAS_A>
+// F16: the entries are fp16 values, for kernels that multiply in fp16.
+template <int BITS, bool HAS_A, bool F16 = false>
 __device__ __forceinline__ void write_pair_tables(uint32_t *lds, const float (&lo_w)[4], const float (&hi_w)[8],
                                                   const float (&lo_a_raw)[4], const float (&hi_a_raw)[4], int a_levels) {
   typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -310,7 +311,7 @@ __device__ __forceinline__ void write_pair_tables(uint32_t *lds, const float (&l
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const f32x2_t pair = {lo[i & 3], hi[i]};
-    const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2_t));
+    const uint32_t d = F16 ? pack16(lo[i & 3], hi[i], true) : __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2_t));
     *reinterpret_cast<uint4 *>(row0 + i * 1024) = make_uint4(d, d, d, d);
   }
 }

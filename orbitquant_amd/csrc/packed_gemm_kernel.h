@@ -50,7 +50,9 @@ namespace oq {
 // K-step pieces of its own FM*32 rows line by line (eight rows per load instruction), parks them in a slab of
 // LDS that belongs to it alone (row pitch 144 bytes), and reads its operands back with one 16-byte LDS read per
 // row tile and MFMA: no workgroup-wide staging, no barrier in the loop, no copy of the activations in memory.
-enum AMode { A_NIBBLE = 0, A_U8 = 1, A_TILED = 2, A_STAGED = 3 };
+// A_TILED_F16: A_TILED on fp16 values, weights looked up and multiplied in fp16.
+enum AMode { A_NIBBLE = 0, A_U8 = 1, A_TILED = 2, A_STAGED = 3, A_TILED_F16 = 4 };
+constexpr bool is_tiled(int a_mode) { return a_mode == A_TILED || a_mode == A_TILED_F16; }
 
 struct GemmArgs {
   const uint8_t *a;          // [M, K/2] nibble codes, [M, K] one code per byte, or the tiled 16-bit values
@@ -186,9 +188,9 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   const int64_t n_base = static_cast<int64_t>(pid_n) * TN + wn;
 
 
-  constexpr int kAStep = AM == A_NIBBLE ? 32 : AM == A_U8 ? 64 : AM == A_TILED ? 4096 : 128;  // bytes from one K-step of 64 to the next in a lane's activation stream
+  constexpr int kAStep = AM == A_NIBBLE ? 32 : AM == A_U8 ? 64 : is_tiled(AM) ? 4096 : 128;  // bytes from one K-step of 64 to the next in a lane's activation stream
   constexpr int kAVec = AM == A_NIBBLE ? 1 : AM == A_U8 ? 2 : 4;        // 16-byte loads per lane per K-step
-  constexpr int kAVecStride = AM == A_TILED ? 1024 : 16;
+  constexpr int kAVecStride = is_tiled(AM) ? 1024 : 16;
   // A_STAGED: load v of row tile e is row 32 e + 8 v + lane / 8, 16-byte chunk lane % 8 of the row's 128-byte K-step piece
   constexpr int kSlabPitch = 144, kSlabBytes = FM * 32 * kSlabPitch;
   __shared__ __attribute__((aligned(16))) unsigned char aslab[AM == A_STAGED ? 4 * kSlabBytes : 16];
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
 #pragma unroll
       for (int v = 0; v < 4; ++v)
         a_off32[i][v] = static_cast<uint32_t>(min(m_base + 32 * i + 8 * v + (lane >> 3), g.M - 1) * (g.K * 2) + (lane & 7) * 16);
-    } else if constexpr (AM == A_TILED) ap[i] = g.a + min(m_base / 32 + i, (g.M + 31) / 32 - 1) * (g.K / 64) * kAStep + lane * 16;
+    } else if constexpr (is_tiled(AM)) ap[i] = g.a + min(m_base / 32 + i, (g.M + 31) / 32 - 1) * (g.K / 64) * kAStep + lane * 16;
     else ap[i] = g.a + row_offset(min(m_base32 + 32 * i + r, M32 - 1), a_row_bytes32) + grp * (kAStep / 2);
   }
 #pragma unroll
@@ -304,9 +306,9 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   stamp_extra[2] = __builtin_amdgcn_s_memtime();  // centroids have arrived
 #endif
   if constexpr (kPairTables) {
-    write_pair_tables<BITS, kHasATable>(lds, seed_lo_w, seed_hi_w, seed_lo_a, seed_hi_a, g.a_levels);
+    write_pair_tables<BITS, kHasATable, AM == A_TILED_F16>(lds, seed_lo_w, seed_hi_w, seed_lo_a, seed_hi_a, g.a_levels);
   } else {
-    const uint32_t my_w = w_row_used ? pack16(w_c0, w_c1, false) : 0u;
+    const uint32_t my_w = w_row_used ? pack16(w_c0, w_c1, AM == A_TILED_F16) : 0u;
     const uint32_t my_a = pack16(a_ok0 ? a_c0 : 0.0f, a_ok1 ? a_c1 : 0.0f, false);
     write_row_tables(lds, my_w, my_a);
   }
@@ -406,7 +408,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   };
   // the activation operand of tile i out of `set`
   auto a_operand = [&](int set, int i) -> uint4 {
-    if constexpr (AM == A_TILED) {
+    if constexpr (is_tiled(AM)) {
       return make_uint4(0u, 0u, 0u, 0u);  // (the operand comes straight from the load registers, see phase)
     } else if constexpr (AM == A_STAGED) {
       return oa4[set][i];
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
     for (int m = 0; m < kGroups; ++m) {
       const int i = m / FN, j = m % FN;
       if (j == 0) {
-        if constexpr (AM == A_TILED) av = pa[decltype(mul_buf)::value][i][decltype(mul_q)::value];
+        if constexpr (is_tiled(AM)) av = pa[decltype(mul_buf)::value][i][decltype(mul_q)::value];
         else av = a_operand(set ^ 1, i);
       }
       const int lo = m * kLookups / kGroups, hi = (m + 1) * kLookups / kGroups, hi2 = (m + 2) * kLookups / kGroups;
@@ -449,8 +451,11 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
         __asm__ volatile("" ::"v"(bw.x), "v"(bw.y), "v"(bw.z), "v"(bw.w), "v"(av.x), "v"(av.y), "v"(av.z), "v"(av.w));  // the operands stay looked up
       }
 #else
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bw), __builtin_bit_cast(bf16x8, av),
-                                                          acc[i][j], 0, 0, 0);
+      if constexpr (AM == A_TILED_F16)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bw), __builtin_bit_cast(f16x8, av), acc[i][j], 0, 0, 0);
+      else
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bw), __builtin_bit_cast(bf16x8, av),
+                                                            acc[i][j], 0, 0, 0);
 #endif
 #pragma unroll
       for (int t = lo; t < hi; ++t) lookup_read(buf, q, set, t, addr[m & 1][t - lo]);

@@ -96,3 +96,28 @@ def test_int8_pair_sums_integers_exactly(dev, library_switch, tile, m, k, n):
     # |bias| in the addition), then half an ulp of fp16
     bound = exact.abs() * 2.0 ** -11 + (exact.abs() + o["bias"].abs().double()) * 2.0 ** -20 + 2.0 ** -24
     assert bool(((got.double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dense,tile", [("never", 0), ("never", 1), ("never", 3), ("never", 4), (0, None), (1, None), (2, None), (3, None)])
+@pytest.mark.parametrize("m,k,n,wbits", [(9, 64, 8, 2), (33, 256, 264, 3), (129, 192, 520, 4), (257, 1280, 200, 6), (65, 512, 72, 8)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_floating_activations_from_operand_order(dev, library_switch, dense, tile, m, k, n, wbits, dtype):
+    from orbitquant_amd import ops
+
+    library_switch("OQ_DENSE_GEMM", dense)
+    if tile is not None:
+        library_switch("OQ_GEMM_TILE", tile)
+    o = operands(dev, m, k, n, wbits, 4, seed=m + k)
+    g = torch.Generator(device=dev)
+    g.manual_seed(k)
+    x = torch.randn(m, k, device=dev, generator=g).to(dtype)
+    got = ops.matmul_packed_weight_values(x, o["packed"], o["rn"], o["wcents"], bits=wbits, out_features=n, in_features=k, bias=o["bias"],
+                                          token_scale=o["norms"])
+    index = ops.unpack_lowbit(o["packed"], wbits, n * k).view(n, k).long()
+    w = o["wcents"].to(dtype).double()[index]   # the tables hold values of the activations' type
+    factor = o["norms"].double()[:, None] * o["rn"].double()
+    exact = (x.double() @ w.T) * factor + o["bias"].double()
+    # K additions and three more operations in fp32, then half an ulp of the output type
+    magnitude = (x.double().abs() @ w.abs().T) * factor + o["bias"].double().abs()
+    bound = magnitude * (k + 4) * 2.0 ** -24 + exact.abs() * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) + 2.0 ** -25
+    assert bool(((got.double() - exact).abs() <= bound).all())
