@@ -61,6 +61,7 @@ def _adaln_fake(x, packed_weight, scales, bias, out_features, in_features, group
 
 _LIB.impl("adaln_int4_linear", _adaln_forward, "CUDA")
 torch.library.register_fake("orbitquant_amd::adaln_int4_linear", _adaln_fake, lib=_LIB)
+_adaln_int4_linear = torch.ops.orbitquant_amd.adaln_int4_linear.default
 
 
 class RTNInt4Linear(nn.Module):
@@ -130,8 +131,7 @@ class RTNInt4Linear(nn.Module):
         if x.device.type != "cuda":
             raise RuntimeError("RTNInt4Linear runs on AMD GPUs only (torch device 'cuda'); there is no CPU fallback")
         self.last_effective_runtime_mode = "hip_packed_adaln_int4"
-        return torch.ops.orbitquant_amd.adaln_int4_linear(x, self.packed_weight, self.scales, self.bias, self.out_features,
-                                                          self.in_features, self.group_size)
+        return _adaln_int4_linear(x, self.packed_weight, self.scales, self.bias, self.out_features, self.in_features, self.group_size)
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, int4 group {self.group_size}"

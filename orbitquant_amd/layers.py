@@ -83,6 +83,7 @@ def _quantized_linear_fake(
 
 _LIB.impl("quantized_linear", quantized_linear_forward, "CUDA")
 torch.library.register_fake("orbitquant_amd::quantized_linear", _quantized_linear_fake, lib=_LIB)
+_quantized_linear = torch.ops.orbitquant_amd.quantized_linear.default   # (the overload itself: no lookup per call)
 
 
 def packed_length(value_count: int, bits: int) -> int:
@@ -301,22 +302,23 @@ class OrbitLinear(nn.Module):
                 "OrbitLinear runs on AMD GPUs only (torch device 'cuda'); there is no CPU fallback")
         if x.dtype not in (torch.float32, torch.float16, torch.bfloat16):
             raise ValueError("x must be float32, float16 or bfloat16")
-        table = self._input_activation_table
+        table = self._buffers["_input_activation_table"]
         if table is not None and table.dtype != x.dtype:
             raise ValueError(f"the fused input activation was built for {table.dtype}, got {x.dtype}")
-        out_table = self._output_activation_table
+        out_table = self._buffers["_output_activation_table"]
         if out_table is not None and out_table.dtype != x.dtype:
             raise ValueError(f"the fused output activation was built for {out_table.dtype}, got {x.dtype}")
         self.last_effective_runtime_mode = "hip_packed"
         if self.share_input_quantization and not torch.compiler.is_compiling():
             return self._forward_shared(x, table, out_table)
         packed, weight_bits, weight_centroids = self._matmul_weight(x.numel() // self.in_features)
-        return torch.ops.orbitquant_amd.quantized_linear(
-            x, self._rotation_permutation, self._rotation_signs, self._activation_codebook_centroids,
-            self._activation_codebook_boundaries, packed, self.row_norms,
+        buffers = self._buffers   # (an attribute that is a buffer is found only after two failed lookups)
+        return _quantized_linear(
+            x, buffers["_rotation_permutation"], buffers["_rotation_signs"], buffers["_activation_codebook_centroids"],
+            buffers["_activation_codebook_boundaries"], packed, self.row_norms,
             weight_centroids, self.bias, self.rotation.block_size,
             self.activation_eps, self.rotation.normalization, self.activation_bits, weight_bits,
-            self.out_features, table, out_table, self._rotation_plan)
+            self.out_features, table, out_table, buffers["_rotation_plan"])
 
     def _forward_shared(self, x, table, out_table):
         """The forward as quantize + packed linear, with the codes of the most recent quantization kept

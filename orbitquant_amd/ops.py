@@ -49,7 +49,8 @@ _FLOATS = (torch.float32, torch.float16, torch.bfloat16)
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of `t`'s device as a raw handle (torch.cuda.current_stream makes an object for it)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _workspace(nbytes: int, like: torch.Tensor) -> tuple[int | None, int, torch.Tensor | None]:
@@ -66,6 +67,18 @@ def _workspace(nbytes: int, like: torch.Tensor) -> tuple[int | None, int, torch.
     return buf.data_ptr(), int(nbytes), buf
 
 
+def _scratch(sizes: tuple[int, ...], like: torch.Tensor) -> tuple[torch.Tensor, list[int]]:
+    """One allocation for the buffers that live between the launches of one call: (the tensor that owns them, their
+    addresses, each 256-byte aligned).  The caller keeps the tensor until its call has been issued."""
+    offsets, total = [], 0
+    for n in sizes:
+        offsets.append(total)
+        total += (n + 255) & -256
+    buf = torch.empty(total, dtype=torch.uint8, device=like.device)
+    base = buf.data_ptr()
+    return buf, [base + at for at in offsets]
+
+
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
@@ -76,8 +89,8 @@ class _OnDevice:
     __slots__ = ("_guard",)
 
     def __init__(self, t: torch.Tensor) -> None:
-        index = t.device.index
-        self._guard = None if index is None or index == torch.cuda.current_device() else torch.cuda.device(index)
+        index = t.device.index   # (a tensor on the GPU exists: torch's CUDA state is initialized)
+        self._guard = None if index is None or index == torch._C._cuda_getDevice() else torch.cuda.device(index)
 
     def __enter__(self):
         if self._guard is not None:
@@ -448,7 +461,7 @@ def quantized_linear(
     input before it is quantized / to the output before it is stored."""
     _require_gpu(x, "x")
     dim = x.shape[-1]
-    rows = x.contiguous().reshape(-1, dim)
+    rows = x if x.dim() == 2 and x.is_contiguous() else x.contiguous().reshape(-1, dim)
     m = rows.shape[0]
     permutation = _operand(permutation, "permutation", x, dtype=torch.int32, numel=dim)
     signs = _operand(signs, "signs", x, dtype=torch.int8, numel=dim)
@@ -469,8 +482,7 @@ def quantized_linear(
     bias = _operand(bias, "bias", x, dtype=_FLOATS, numel=out_features)
     plan = _plan_operand(plan, x, dim, block_size, 1 << activation_bits)
     nibble = activation_bits <= 4 and dim % 2 == 0
-    codes = torch.empty((m, dim // 2 if nibble else dim), dtype=torch.uint8, device=x.device)
-    norms = torch.empty(m, dtype=torch.float32, device=x.device)
+    scratch, (codes_ptr, norms_ptr) = _scratch((m * (dim // 2 if nibble else dim), 4 * m), x)
     out = torch.empty((m, out_features), dtype=x.dtype, device=x.device)
     lib = _lib.load()
     ws_ptr, ws_bytes, ws = _workspace(lib.oq_packed_linear_workspace_bytes(
@@ -481,10 +493,10 @@ def quantized_linear(
             boundaries.data_ptr(), act_centroids.data_ptr(), int(activation_bits), int(block_size), float(eps),
             float(inv_sqrt_block), _ptr(plan), packed_weight.data_ptr(), int(weight_bits), row_norms.data_ptr(),
             weight_centroids.data_ptr(), _ptr(bias), _dt(bias) if bias is not None else 0, out_features,
-            codes.data_ptr(), norms.data_ptr(), out.data_ptr(), _dt(out), _ptr(output_map), ws_ptr, ws_bytes, _stream(x))
-    del ws
+            codes_ptr, norms_ptr, out.data_ptr(), _dt(out), _ptr(output_map), ws_ptr, ws_bytes, _stream(x))
+    del ws, scratch
     _lib.check(rc, "oq_quantized_linear")
-    return out.reshape(*x.shape[:-1], out_features)
+    return out if x.dim() == 2 else out.reshape(*x.shape[:-1], out_features)
 
 
 def quantized_linear_group(
@@ -509,7 +521,7 @@ def quantized_linear_group(
 
     _require_gpu(x, "x")
     dim = x.shape[-1]
-    rows = x.contiguous().reshape(-1, dim)
+    rows = x if x.dim() == 2 and x.is_contiguous() else x.contiguous().reshape(-1, dim)
     m = rows.shape[0]
     weights = list(weights)
     if not 1 <= len(weights) <= 64:
@@ -537,8 +549,7 @@ def quantized_linear_group(
         keep.append((packed, row_norms, cents, int(bits), int(n), bias))
         outs.append(torch.empty((m, n), dtype=x.dtype, device=x.device))
     nibble = activation_bits <= 4 and dim % 2 == 0
-    codes = torch.empty((m, dim // 2 if nibble else dim), dtype=torch.uint8, device=x.device)
-    norms = torch.empty(m, dtype=torch.float32, device=x.device)
+    scratch, (codes_ptr, norms_ptr) = _scratch((m * (dim // 2 if nibble else dim), 4 * m), x)
     count = len(keep)
     ptrs = ctypes.c_void_p * count
     lib = _lib.load()
@@ -552,9 +563,9 @@ def quantized_linear_group(
             ptrs(*[k[0].data_ptr() for k in keep]), (ctypes.c_int * count)(*[k[3] for k in keep]),
             ptrs(*[k[1].data_ptr() for k in keep]), ptrs(*[k[2].data_ptr() for k in keep]),
             ptrs(*[_ptr(k[5]) for k in keep]), _DTYPES[bias_dtype] if bias_dtype is not None else OQ_F32,
-            (ctypes.c_int64 * count)(*[k[4] for k in keep]), codes.data_ptr(), norms.data_ptr(),
+            (ctypes.c_int64 * count)(*[k[4] for k in keep]), codes_ptr, norms_ptr,
             ptrs(*[o.data_ptr() for o in outs]), _dt(x), ws_ptr, ws_bytes, _stream(x))
-    del ws
+    del ws, scratch
     _lib.check(rc, "oq_quantized_linear_group")
     return [o.reshape(*x.shape[:-1], o.shape[-1]) for o in outs]
 
