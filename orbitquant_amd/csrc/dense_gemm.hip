@@ -54,6 +54,10 @@ __device__ __forceinline__ T mfma_piece(uint4 w, uint4 a, T c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, w), __builtin_bit_cast(i32x4, a), c, 0, 0, 0);
 }
 
+// s_waitcnt vmcnt(0): a copy into LDS counts as a memory load of the wavefront that issued it, and the others may read
+// its bytes only behind a barrier that comes after this wait.
+constexpr int kCopiesArrived = 0x0f70;
+
 template <int MF, int FM, int FN>
 __global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
   constexpr int kBlocks = 2 * (FM + FN), kStage = kBlocks * 4096;
@@ -133,6 +137,7 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
     else oa[set][t - FN] = *reinterpret_cast<const uint4 *>(stage + a_at + (t - FN) * 4096 + q * 1024);
   };
 
+  __builtin_amdgcn_s_waitcnt(kCopiesArrived);
   __syncthreads();
 #pragma unroll
   for (int t = 0; t < kOps; ++t) read_operand(stage0, 0, 0, t);
@@ -172,6 +177,7 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
     multiply(s1, s0, m_all, reads, cur, 2, p2, p_all, nxt, at1);
     multiply(s0, s0, m_all, reads, cur, 3, p0, p0, nxt, at1);
     multiply(s1, s0, m_ahead, no_reads, nxt, 0, p0, p0, nxt, at1);
+    __builtin_amdgcn_s_waitcnt(kCopiesArrived);
     __syncthreads();  // `nxt` has arrived, the last operands of `cur` are in registers
     multiply(s1, m_ahead, m_all, reads, nxt, 0, p0, p1, cur, at2);
   };
@@ -182,6 +188,7 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
   }
   if (ks < g.steps) step(stage0, stage1, ks);
 
+  __builtin_amdgcn_s_waitcnt(kCopiesArrived);
   __syncthreads();  // no copy is in flight, every wavefront is done with the stages
   EpiFactors<FM> epi;
   gemm_epilogue_factors<FM>(epi, epi_raw, TN, tid, g.row_scale != nullptr, g.bias != nullptr, g.bias_dtype);

@@ -343,8 +343,11 @@ def packed_linear_int8(
     """`packed_linear` of 4-bit codes on both sides through tables of sixteen int8 values, multiplied as integers
     (`oq_packed_linear_int8`); None where that kernel does not pay, does not take the call or has no room for its
     workspace (`packed_linear` takes it then)."""
-    lib = _lib.load()
+    _require_gpu(codes, "codes")
     width = in_features // 2
+    if codes.dtype != torch.uint8 or codes.shape[-1] != width:
+        raise ValueError(f"codes must be uint8 with last dimension {width}")
+    lib = _lib.load()
     flat = codes.contiguous().reshape(-1, width)
     m = flat.shape[0]
     need = lib.oq_packed_linear_int8_workspace_bytes(m, int(out_features), int(in_features))
