@@ -192,7 +192,8 @@ int quantize_weight_fast(const void *w, int w_dtype, int64_t N, int64_t K, const
   a.x = w; a.M = N; a.K = K; a.plan = static_cast<const unsigned char *>(plan);
   a.levels = levels; a.block = static_cast<int>(block); a.eps = eps;
   a.raw_bounds = boundaries; a.inv_sqrt_block = inv_sqrt_block; a.pack_bits = bits;
-  a.packed = packed_out; a.norms_bf16 = row_norms_out;
+  a.packed = packed_out; a.packed_aligned = (reinterpret_cast<uintptr_t>(packed_out) & 7u) == 0;
+  a.norms_bf16 = row_norms_out;
   return launch_fast(a, w_dtype, stream);
 }
 

@@ -133,3 +133,26 @@ def test_argument_checks(dev):
     assert call() == 0                      # a zero plan has the wrong magic: no indices are written, the row norms are NaN
     torch.cuda.synchronize()
     assert not packed.any() and bool(torch.isnan(norms.float()).all())
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize("k", [24, 1152, 4096])
+def test_rows_of_any_magnitude_and_any_start_of_the_stream(dev, bits, k):
+    """Rows that the fast quotient takes and rows that it leaves to the IEEE division (norms beyond 2^20 and below
+    eps, values below 2^-80 beside ordinary ones), in one stream and from starts that are not multiples of eight."""
+    n = 11
+    perm, signs, block, inv = o.rpbh_constants(k, 5, "paper")
+    bounds = np.linspace(-3, 3, 2 ** bits - 1).astype(np.float32) / np.float32(np.sqrt(k))
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(k + bits))
+    w[1] *= 2.0 ** 24
+    w[2] *= 2.0 ** -40
+    w[3] *= 2.0 ** -100
+    w[4] = 0
+    w[5, ::3] *= 2.0 ** -90
+    w[6, 1:] = 0
+    w[7] *= 2.0 ** 14
+    w[8] *= torch.linspace(-100, 0, k).exp2()
+    want_packed, want_norms, _ = o.quantize_weight(w.numpy(), perm, signs, bounds, block, 1e-10, bits, norm_order="sumsq_v1")
+    for row_tile in (None, 1):
+        packed, norms = gpu_quantize(dev, w, perm, signs, bounds, block, inv, bits, row_tile=row_tile)
+        assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
