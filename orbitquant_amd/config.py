@@ -22,7 +22,7 @@ class OrbitQuantConfig:
     block_size: int | str = "paper"
     codebook_version: int = 2
     activation_eps: float = 1e-10
-    weight_row_tile_size: int = 256
+    weight_row_tile_size: int = 256   # rows converted at a time on the host; a GPU weight is one launch
     runtime_mode: str = "hip_packed"
     adaln_group_size: int = 64
 

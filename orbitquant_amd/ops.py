@@ -144,7 +144,7 @@ def quantize_weight(weight: torch.Tensor, permutation: torch.Tensor, signs: torc
     packed = torch.empty((n * k * bits + 7) // 8, dtype=torch.uint8, device=w.device)
     norms = torch.empty(n, dtype=torch.bfloat16, device=w.device)
     lib = _lib.load()
-    step = n if not row_tile else max(1, int(row_tile))
+    step = max(1, int(row_tile) if row_tile else n)   # (a weight without rows launches nothing)
     with _OnDevice(w):
         for start in range(0, n, step):
             rows = min(step, n - start)

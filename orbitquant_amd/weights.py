@@ -47,7 +47,8 @@ def quantize_weight(
     row_tile: int = 4096,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """-> (packed uint8 [ceil(N*K*bits/8)], row_norms bfloat16 [N]), on the GPU for a GPU weight the
-    kernel takes, else on the CPU."""
+    kernel takes, else on the CPU.  `row_tile` bounds the rows whose fp32 copies the host path holds at a
+    time; the result does not depend on it, and a GPU weight is one launch without such copies."""
     if weight.ndim != 2:
         raise ValueError("weight must be a matrix")
     n, k = weight.shape
@@ -56,9 +57,8 @@ def quantize_weight(
         from . import ops
 
         device = weight.device
-        # (one launch for the matrix: `row_tile` bounds the fp32 copies of the host path, the kernel makes none, and at
-        # 256 rows a launch, one workgroup a CU, 14336 x 4096 took 56 launches of 16 us and some
-        # 200 us of Python; one launch 139 us)
+        # (one launch for the matrix: at 256 rows a launch, one workgroup a CU, 14336 x 4096 took 56 launches of 16 us
+        # and some 200 us of Python; one launch 139 us)
         return ops.quantize_weight(
             weight, rotation.permutation.to(torch.int32).to(device), rotation.signs.to(torch.int8).to(device),
             codebook.boundaries.to(device), bits=bits, block_size=rotation.block_size, eps=eps,

@@ -156,3 +156,14 @@ def test_rows_of_any_magnitude_and_any_start_of_the_stream(dev, bits, k):
     for row_tile in (None, 1):
         packed, norms = gpu_quantize(dev, w, perm, signs, bounds, block, inv, bits, row_tile=row_tile)
         assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
+
+
+def test_a_weight_without_rows(dev):
+    from orbitquant_amd import OrbitLinear, OrbitQuantConfig
+
+    perm, signs, block, inv = o.rpbh_constants(64, 5, "paper")
+    bounds = np.linspace(-0.3, 0.3, 15).astype(np.float32)
+    packed, norms = gpu_quantize(dev, torch.empty(0, 64), perm, signs, bounds, block, inv, 4)
+    assert packed.shape == (0,) and packed.dtype == torch.uint8 and norms.shape == (0,) and norms.dtype == torch.bfloat16
+    layer = OrbitLinear.from_weight(torch.empty(0, 64, device=dev), bias=None, config=OrbitQuantConfig())
+    assert layer.packed_weight_indices.numel() == 0 and layer.row_norms.shape == (0,)
