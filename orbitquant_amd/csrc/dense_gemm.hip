@@ -17,6 +17,8 @@
 // 1.5 GHz; the packed GEMM, whose table lookups cost energy too, 865 us at 1.3 GHz), so a tile is chosen for few LDS
 // bytes per product: 256 x 256 over four wavefronts, each 128 x 128.  Copies issued in a burst instead of between
 // matrix instructions cost 834 us.  In int8 406 us, 2.7 POP/s.
+#include <math.h>
+
 #include "dense_gemm.h"
 #include "gemm_epilogue.h"
 
@@ -226,32 +228,45 @@ int launch_dense_tile(const DenseArgs &g, int tile, hipStream_t stream) {
   return launch_dense<MF, 2, 2>(g, stream);
 }
 
+// 0 .. 1: how far the chip's clock has come down over a launch of that many operations (its power limit, reached
+// over some hundred microseconds): none at 2e10, all of it from 1e12 on.
+double launch_warmth(double operations) {
+  const double w = log(operations / 2.0e10) / log(50.0);
+  return w < 0.0 ? 0.0 : w < 1.0 ? w : 1.0;
+}
+
 }  // namespace
 
-// The best tile of this kernel for a problem and its cost in microseconds, the two passes into operand order
-// included (`pass_bytes`: what they read and write); -1 where the kernel cannot run.  A launch runs in rounds of 256
-// workgroups, each with a fixed prologue and epilogue and a time per K-step of 128 operand bytes, measured like the
-// constants of the packed GEMM's model: "busy" for launches of some 50 us and more (the matrix cores' power limit
-// then sets the clock: 8192 x 8192 x 8192 in 775 us bf16, 406 us int8), the other for shorter ones.  A pass is a
-// launch (3 us) at 5 TB/s (3-bit 12288 x 3072: 13.5 us).
+// The best tile of this kernel for a problem and its time in microseconds, the passes into operand order included
+// (`pass_bytes`: what they read and write); -1 where the kernel cannot run.  A launch runs in rounds of 256 workgroups,
+// one to a CU, each with a fixed prologue and epilogue and a time per K-step of 128 operand bytes that grows with the
+// length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16 at 2e10 operations, 1.14 us from 1e12 on) and
+// by up to a quarter where the operands outgrow the 256 MB last-level cache; on top come the passes, the output's
+// way to memory and the launches.  Fitted to 5000 timings of single calls, 256 to 16384 in each dimension, all tiles:
+// nine in ten within 15 %; the tile it picks is 1 % behind the best one on average.
 int dense_choose_tile(int64_t M, int64_t N, int64_t K, int mf, double pass_bytes, double *cost_out) {
   if (K % 64 != 0 || N % 8 != 0 || M > 0x7fff0000LL || N > 0x7fff0000LL || K > 0x0fffffffLL) return -1;
-  struct Shape { int tm, tn; double fixed, step_short, step_busy; };
-  static const Shape shapes[4] = {{256, 256, 7.0, 1.1, 1.45}, {256, 192, 6.0, 0.95, 1.2}, {256, 128, 5.5, 0.78, 0.92}, {128, 128, 5.0, 0.52, 0.6}};
-  const double steps = static_cast<double>(mf == MF_I8 ? (K + 127) / 128 : K / 64);
-  const bool busy = 2.0 * static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(K) > (mf == MF_I8 ? 1.0e11 : 5.0e10);
+  static const int sizes[4][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 128}};
+  struct Times { double fixed[4], step[4], warm, pass_mb, out_mb, launches; };
+  static const Times values16 = {{11.8, 9.5, 3.8, 2.0}, {0.96, 0.81, 0.665, 0.495}, 0.19, 0.19, 0.16, 12.0};
+  static const Times values8 = {{8.9, 7.5, 3.1, 2.0}, {0.96, 0.80, 0.70, 0.52}, 0.18, 0.22, 0.27, 8.5};
+  const bool i8 = mf == MF_I8;
+  const Times &t = i8 ? values8 : values16;
+  const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
+  const double steps = static_cast<double>(i8 ? (K + 127) / 128 : K / 64);
+  const double warm = launch_warmth((i8 ? 1.0 : 2.0) * m * n * k), spill = (i8 ? 1.0 : 2.0) * k * (m + n) / 256.0e6 - 1.0;
+  const double step_factor = (1.0 + t.warm * warm) * (1.0 + 1.3 * (spill < 0.0 ? 0.0 : spill < 0.2 ? spill : 0.2));
   int best = 0;
   double best_cost = 0.0;
-  for (int t = 0; t < 4; ++t) {
-    const Shape &sh = shapes[t];
-    const int64_t tiles = ((M + sh.tm - 1) / sh.tm) * ((N + sh.tn - 1) / sh.tn);
-    const double cost = static_cast<double>((tiles + 255) / 256) * (sh.fixed + steps * (busy ? sh.step_busy : sh.step_short));
-    if (t == 0 || cost < best_cost) {
-      best = t;
+  for (int tile = 0; tile < 4; ++tile) {
+    const int64_t tiles = ((M + sizes[tile][0] - 1) / sizes[tile][0]) * ((N + sizes[tile][1] - 1) / sizes[tile][1]);
+    const double cost = static_cast<double>((tiles + 255) / 256) * (t.fixed[tile] + steps * t.step[tile] * step_factor);
+    if (tile == 0 || cost < best_cost) {
+      best = tile;
       best_cost = cost;
     }
   }
-  if (cost_out != nullptr) *cost_out = best_cost + pass_bytes / 5.0e6 + 6.0;
+  if (cost_out != nullptr) *cost_out = best_cost + pass_bytes / 1.0e6 * t.pass_mb + 2.0 * m * n / 1.0e6 * t.out_mb + t.launches;
   if (const char *force = debug_env(ENV_DENSE_GEMM)) {  // "0" .. "3": that tile, always; anything else: never
     if (cost_out != nullptr) *cost_out = 0.0;
     return force[0] >= '0' && force[0] <= '3' ? force[0] - '0' : -1;

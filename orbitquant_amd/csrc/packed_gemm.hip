@@ -58,6 +58,30 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
   return best;
 }
 
+// What that launch takes, in microseconds, for the rules that weigh it against another kernel.  (The model above ranks
+// the tiles of one launch and so leaves out what they share; its short and busy constants are those of four-bit
+// weights on a few shapes.)  The same form with constants fitted to 3500 timings of single calls, 256 to 16384 in each
+// dimension: a time per K-step and tile for each form of the activations (two codes a byte, one code a byte, values
+// in operand order with the pass that puts them there), a factor for each weight width, the output's way to memory.
+// Nine in ten within 15 %.
+double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form) {
+  struct Times { double step[5], out_mb, launches, bits2, bits3, bits6, bits8; };
+  static const Times forms[3] = {{{0.81, 0.85, 1.39, 1.09, 1.12}, 0.20, 0.5, 1.09, 1.11, 1.69, 1.58},
+                                 {{1.12, 1.10, 1.72, 1.40, 1.40}, 0.18, 2.2, 1.06, 1.08, 1.56, 1.50},
+                                 {{0.94, 1.05, 2.03, 1.32, 1.35}, 0.19, 5.5, 0.95, 0.96, 1.88, 1.74}};
+  static const struct { int tm, tn, capacity; double fixed; } tiles[5] = {
+      {128, 128, 512, 4.5}, {128, 256, 256, 5.5}, {256, 256, 256, 7.0}, {256, 192, 256, 6.0}, {128, 96, 256, 7.5}};
+  const Times &f = forms[form];
+  const int tile = choose_tile_with_cost(M, N, K, bits, nullptr, form == PRICE_BYTES);
+  const auto &sh = tiles[tile];
+  const double width = bits == 2 ? f.bits2 : bits == 3 ? f.bits3 : bits == 6 ? f.bits6 : bits == 8 ? f.bits8 : 1.0;
+  const double steps = static_cast<double>(K / 64) / (tile == 4 ? 4.0 : 1.0), step = f.step[tile] * width;
+  const int64_t count = ((M + sh.tm - 1) / sh.tm) * ((N + sh.tn - 1) / sh.tn), rest = count % sh.capacity;
+  const double rest_step = tile == 0 && rest <= 256 ? 0.55 * step : step;  // (alone on its CU)
+  return static_cast<double>(count / sh.capacity) * (sh.fixed + steps * step) + (rest > 0 ? sh.fixed + steps * rest_step : 0.0) +
+         2.0 * static_cast<double>(M) * static_cast<double>(N) / 1.0e6 * f.out_mb + f.launches;
+}
+
 int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits) { return choose_tile_with_cost(M, N, K, bits, nullptr); }
 
 int gemm_splitk_reduce(const float *partials, int splits, int64_t M, int64_t N, const float *row_scale,
@@ -105,18 +129,20 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits) {
 // Tile of the decode-first GEMM (dense_gemm.hip) for a launch that has the workspace for it, -1 for the others.  The
 // kernel above looks every operand value up once per tile that uses it; decoding each once costs two passes over
 // memory, 2 bytes written and read again per value, and leaves the matrix cores alone with the multiplication.
-// That pays from some thousand tokens on, sooner with one code per byte (eight lookups an operand instead of four):
-// 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072 (3-bit) 335 -> 304 us,
-// 4608 x 3072 x 3072 even (85 us), 1024 x 14336 x 4096 103 -> 124 us.  It has to promise 6 % over the best launch
-// without it.
+// That pays on large problems, sooner with one code per byte (eight lookups an operand instead of four) and with
+// weights of six and eight bits:
+// 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072 (3-bit) 333 -> 300 us,
+// 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise 5 % over the best
+// launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
+// the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).
 static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes) {
-  const double a_bytes = byte_codes ? 3.0 : 2.5, w_bytes = 2.0 + bits / 8.0;
-  double dense = 0.0, packed = 0.0;
-  const int tile = dense_choose_tile(M, N, K, MF_BF16, static_cast<double>(K) * (static_cast<double>(M) * a_bytes + static_cast<double>(N) * w_bytes), &dense);
+  const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
+  double dense = 0.0;
+  const int tile = dense_choose_tile(M, N, K, MF_BF16, k * (m * (byte_codes ? 3.0 : 2.5) + n * (2.0 + bits / 8.0)), &dense);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
-  choose_tile_with_cost(M, N, K, bits, &packed, byte_codes);
-  return dense < 0.94 * packed ? tile : -1;
+  const double share = byte_codes || 2.0 * k * (m + n) <= 268435456.0 ? 0.95 : 0.8;
+  return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES) ? tile : -1;
 }
 
 // The model's time in microseconds of the packed GEMM's best launch (nibble codes).
