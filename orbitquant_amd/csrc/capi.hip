@@ -130,7 +130,7 @@ int generic_linear_codes(const void *codes, int code_format, const float *token_
                          hipStream_t stream);
 int unpack_dispatch(const uint8_t *packed, int bits, int64_t count, uint8_t *out, hipStream_t stream);
 bool gemm_supported(int64_t K, int bits);
-double gemm_cost(int64_t M, int64_t N, int64_t K, int bits);
+double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits);
 int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float *act_cents, int a_levels,
                   const uint8_t *w, int bits, const uint16_t *row_norms, const float *w_cents,
                   const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
@@ -307,14 +307,18 @@ int oq_packed_linear(const void *codes, int code_format, const float *token_norm
                             w_centroids, bias, bias_dtype, M, N, K, out, out_dtype, nullptr, workspace, workspace_bytes, stream);
 }
 
-// Tile of the int8 launch, -1 where oq_packed_linear is as fast or the only one.  The bf16 kernel it is compared with
-// multiplies the same integers at half the rate.  Measured against it: 4608 x 36864 x 4096 1141 -> 619 us,
-// 1024 x 14336 x 4096 103 -> 81 us, 2048 x 4096 x 4096 71 -> 58 us, 2048 x 4608 x 1152 34 -> 46 us.
+// Tile of the int8 launch, -1 where it does not run or oq_packed_linear, with the workspace that it asks for, is as
+// fast.  That one multiplies the same integers in bf16, at half the rate, without the two passes.  Measured against it:
+// 4608 x 36864 x 4096 1122 -> 616 us, 1024 x 14336 x 4096 100 -> 74 us, 2048 x 4096 x 4096 67 -> 52 us,
+// 2048 x 4608 x 1152 34 -> 46 us; where it shares K between workgroups 74 x 784 x 8000 18 -> 45 us, 300 x 2048 x 7488
+// 25 -> 50 us.  Asked for 10 %, the prices (dense_choose_tile, gemm_call_price) send 261 of 650 measured shapes here,
+// 5 of them to more than 3 % more time, all with rows of some hundred values.
 static int int8_choose_tile(int64_t M, int64_t N, int64_t K) {
   if (M <= 64 || N <= 0 || K <= 0 || K > 131071) return -1;  // (sums of K products of two int8 values stay below 2^31)
   double cost = 0.0;
   const int tile = dense_choose_tile(M, N, K, MF_I8, 1.5 * static_cast<double>(K) * static_cast<double>(M + N), &cost);
-  return tile >= 0 && cost < 0.94 * gemm_cost(M, N, K, 4) ? tile : -1;
+  if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
+  return cost < 0.9 * gemm_call_price(M, N, K, 4) ? tile : -1;
 }
 
 uint64_t oq_packed_linear_int8_workspace_bytes(int64_t M, int64_t N, int64_t K) {

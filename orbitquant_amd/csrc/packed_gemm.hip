@@ -97,7 +97,8 @@ int apply_value_map(void *out, int64_t count, const uint16_t *table, hipStream_t
 // read back, at 3 TB/s):
 // every part keeps at least sixteen K-steps, the partial tiles stay within 64 MB, and the split has to
 // promise 15 % over the best single launch.  OQ_GEMM_WG_SPLIT overrides (1 = never).
-int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits) {
+// `cost_out`: the time of the split launch, if it is one.
+int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_out = nullptr) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = K / 64;
   auto allowed = [&](int s) { return s >= 2 && s <= 8 && steps / s >= 16 && M * N * 4 * s <= (64ll << 20); };
   if (const char *force = debug_env(ENV_GEMM_WG_SPLIT)) {
@@ -123,6 +124,7 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits) {
       best_cost = cost;
     }
   }
+  if (cost_out != nullptr && best > 1) *cost_out = best_cost;
   return best;
 }
 
@@ -135,14 +137,24 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits) {
 // 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise 5 % over the best
 // launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
 // the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).
-static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes) {
+static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr) {
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   double dense = 0.0;
   const int tile = dense_choose_tile(M, N, K, MF_BF16, k * (m * (byte_codes ? 3.0 : 2.5) + n * (2.0 + bits / 8.0)), &dense);
+  if (cost_out != nullptr) *cost_out = dense;
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
   const double share = byte_codes || 2.0 * k * (m + n) <= 268435456.0 ? 0.95 : 0.8;
   return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES) ? tile : -1;
+}
+
+// What a call on two codes a byte takes with the workspace it asks for: decoded first, shared between workgroups
+// along K, or the single launch.
+double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits) {
+  double dense = 0.0, split = 0.0;
+  if (gemm_choose_dense(M, N, K, bits, false, &dense) >= 0) return dense;
+  const double single = gemm_price(M, N, K, bits, PRICE_NIBBLES);
+  return gemm_choose_splits(M, N, K, bits, &split) > 1 && split < single ? split : single;
 }
 
 // The model's time in microseconds of the packed GEMM's best launch (nibble codes).

@@ -40,3 +40,21 @@ def test_large_problems_are_decoded_first(lib, m, n, k, wbits, abits):
     (1024, 14336, 4096, 4, 4)])    # 95, 114
 def test_the_packed_kernel_keeps_what_it_is_faster_on(lib, m, n, k, wbits, abits):
     assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, _lib.OQ_CODES_NIBBLE, abits) == 0
+
+
+@pytest.mark.parametrize("m,n,k", [(4608, 36864, 4096), (1024, 14336, 4096), (2048, 4096, 4096), (4608, 3072, 12288)])
+def test_int8_tables_are_multiplied_as_integers_on_large_problems(lib, m, n, k):
+    assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) == operand_order(m, k, 1) + operand_order(n, k, 1)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (74, 784, 8000),               # K shared between workgroups 18 us, as integers 45
+    (128, 2048, 8128),             # 20, 53
+    (200, 1024, 4160),             # 17, 29
+    (300, 2048, 7488),             # 25, 50
+    (2237, 376, 15232),            # 39, 84
+    (1587, 10568, 512),            # one launch 30, as integers 43
+    (2048, 4608, 1152),            # 34, 46
+    (64, 36864, 4096), (4608, 36864, 131072), (4608, 36868, 4096), (4608, 36864, 4064), (0, 36864, 4096)])   # not taken at all
+def test_int8_tables_stay_with_the_launch_that_is_faster(lib, m, n, k):
+    assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) == 0
