@@ -98,6 +98,84 @@ def test_int8_pair_sums_integers_exactly(dev, library_switch, tile, m, k, n):
     assert bool(((got.double() - exact).abs() <= bound).all())
 
 
+A_TABLE = [-128, -79, -62, -48, -36, -25, -15, -5, 0, 15, 25, 36, 48, 62, 79, 127]
+
+
+def looked_up(packed, rows, k, table):
+    """The values of two 4-bit codes per byte, in 64 bits."""
+    return table.double()[torch.stack((packed & 15, packed >> 4), dim=-1).long()].view(rows, k)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+@pytest.mark.parametrize("m,k,n,table", [
+    (65, 64, 72, A_TABLE), (300, 192, 264, A_TABLE), (257, 16384, 520, list(range(112, 128))),   # sums beyond 2^24
+    (65, 131008, 8, [-128] * 15 + [-127])])                                                      # ... and near 2^31
+def test_int8_kernel_itself(dev, library_switch, tile, m, k, n, table):
+    """`ops.packed_linear_int8` and nothing in its place: the sums are the integers, rounded once to fp32.  The bf16
+    kernel rounds each partial sum, which from 2^24 on is another result."""
+    from orbitquant_amd import ops
+
+    o = operands(dev, m, k, n, 4, 4, seed=m + k)
+    library_switch("OQ_DENSE_GEMM", tile)
+    table = torch.tensor(table, dtype=torch.int8, device=dev)
+    ones, unit = torch.ones(m, device=dev), torch.ones(n, dtype=torch.bfloat16, device=dev)
+    got = ops.packed_linear_int8(o["codes"], ones, table, o["packed"], unit, table, scale=1.0, out_features=n, in_features=k,
+                                 output_dtype=torch.float32)
+    assert got is not None
+    want = (looked_up(o["codes"], m, k, table) @ looked_up(o["packed"], n, k, table).T).float()
+    assert torch.equal(got, want)
+    if k == 16384:
+        library_switch("OQ_DENSE_GEMM", "never")
+        in_bf16 = ops.packed_linear(o["codes"], ones, table.float(), o["packed"], unit, table.float(), code_format="nibble", activation_bits=4,
+                                    weight_bits=4, out_features=n, in_features=k, output_dtype=torch.float32)
+        assert not torch.equal(in_bf16, want)
+
+
+def test_int8_pair_takes_the_integer_kernel_by_itself(dev):
+    import orbitquant_packed_matmul as package
+    from orbitquant_amd import _lib, ops
+
+    m, k, n = 1024, 4096, 14336
+    o = operands(dev, m, k, n, 4, 4, seed=1)
+    table = torch.tensor(list(range(112, 128)), dtype=torch.int8, device=dev)
+    assert _lib.load().oq_packed_linear_int8_workspace_bytes(m, n, k) > 0
+    direct = ops.packed_linear_int8(o["codes"], o["norms"], table, o["packed"], o["rn"], table, scale=0.5, out_features=n, in_features=k,
+                                    output_dtype=torch.bfloat16)
+    assert direct is not None
+    got = package.matmul_packed_w4a4_int8(o["codes"], o["packed"], o["norms"], o["rn"], table, table, activation_scale=0.5, weight_scale=1.0,
+                                          out_features=n, in_features=k, output_dtype=torch.bfloat16)
+    assert torch.equal(got, direct)
+    rows = slice(1000, 1024)
+    sums = (looked_up(o["codes"][rows], 24, k, table) @ looked_up(o["packed"], n, k, table).T).float()
+    want = sums * (o["norms"][rows] * 0.5)[:, None] * o["rn"].float()   # the epilogue's fp32 products, in its order
+    assert torch.equal(got[rows], want.bfloat16())
+
+
+def test_int8_kernel_says_what_it_does_not_take(dev):
+    from orbitquant_amd import _lib, ops
+
+    lib = _lib.load()
+    m, k, n = 2048, 4096, 4096
+    need = lib.oq_packed_linear_int8_workspace_bytes(m, n, k)
+    assert need > 0
+    o = operands(dev, m, k, n, 4, 4, seed=2)
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    out, ws = torch.empty(m, n, device=dev), torch.empty(need, dtype=torch.uint8, device=dev)
+
+    def call(rows=m, workspace=ws.data_ptr(), size=need, codes=o["codes"].data_ptr(), activation_table=table.data_ptr()):
+        return lib.oq_packed_linear_int8(codes, o["norms"].data_ptr(), 1.0, activation_table, o["packed"].data_ptr(), o["rn"].data_ptr(),
+                                         table.data_ptr(), None, 0, rows, n, k, out.data_ptr(), _lib.OQ_F32, workspace, size,
+                                         torch.cuda.current_stream().cuda_stream)
+
+    assert call() == 0 and call(rows=0) == 0
+    invalid, unsupported = call(codes=None), call(rows=64)
+    assert invalid != 0 and unsupported not in (0, invalid)
+    assert call(activation_table=None) == invalid
+    assert call(workspace=None, size=0) == call(size=need - 1) == call(workspace=ws.data_ptr() + 8, size=need - 8) == invalid
+    assert call(codes=o["codes"].data_ptr() + 8) == unsupported
+    assert ops.packed_linear_int8(o["codes"][:64], o["norms"][:64], table, o["packed"], o["rn"], table, scale=1.0, out_features=n, in_features=k) is None
+
+
 @pytest.mark.parametrize("dense,tile", [("never", 0), ("never", 1), ("never", 3), ("never", 4), (0, None), (1, None), (2, None), (3, None)])
 @pytest.mark.parametrize("m,k,n,wbits", [(9, 64, 8, 2), (33, 256, 264, 3), (129, 192, 520, 4), (257, 1280, 200, 6), (65, 512, 72, 8)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
