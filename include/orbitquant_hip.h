@@ -363,9 +363,10 @@ int oq_quantized_linear_static(const void *x, int x_dtype, const uint16_t *input
  * workspace: NULL, or oq_matmul_packed_weight_workspace_bytes(...) bytes of device memory, 16-byte aligned,
  * that the call may overwrite.  With it, bf16 activations (from two tokens on; one token on large matrices)
  * and fp16 activations (from nine tokens on) are first rewritten into the matrix core's operand order
- * (2 * M * K bytes, rows padded to 32) and the tile kernel reads that copy; problems of many tokens decode the
- * weights into the workspace too.  Without it every wavefront stages its own rows through LDS (bf16: no buffer,
- * the same sums, 10-15 % slower on large problems) or the workgroup does (fp16).  The library allocates nothing.
+ * (2 * M * K bytes, rows padded to 32) and the tile kernel reads that copy; where it is faster (large problems,
+ * weights of six and eight bits) the weights are decoded into the workspace too.  Without it every wavefront stages
+ * its own rows through LDS (bf16: no buffer, the same sums, 10-15 % slower on large problems) or the workgroup does
+ * (fp16: sums in another order).  The library allocates nothing.
  */
 int oq_matmul_packed_weight(const void *x, int x_dtype, const float *token_scale,
                             const uint8_t *packed_w, int bits, const uint16_t *row_norms,

@@ -157,13 +157,6 @@ double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits) {
   return gemm_choose_splits(M, N, K, bits, &split) > 1 && split < single ? split : single;
 }
 
-// The model's time in microseconds of the packed GEMM's best launch (nibble codes).
-double gemm_cost(int64_t M, int64_t N, int64_t K, int bits) {
-  double cost = 0.0;
-  choose_tile_with_cost(M, N, K, bits, &cost);
-  return cost;
-}
-
 bool gemm_supported(int64_t K, int bits) {
   return K % 64 == 0 && (bits == 2 || bits == 3 || bits == 4 || bits == 6 || bits == 8);
 }

@@ -57,16 +57,19 @@ int launch_tiled_bits(const GemmArgs &g, int bits, int tile, hipStream_t stream)
 }  // namespace
 
 int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits);  // packed_gemm.hip
-double gemm_cost(int64_t M, int64_t N, int64_t K, int bits);
 
-// Tile of the decode-first GEMM, -1 where looking the weights up in every tile is as fast.  Both sides pay for the
-// activations' pass; the rule is that of the code path (packed_gemm.hip) with the weights' pass alone.
+// Tile of the decode-first GEMM, -1 where looking the weights up in every tile is as fast, or where that launch takes
+// the 128 x 96 tile: its four wavefronts share K and add up in another order, and this entry point gives the same sums
+// with and without a workspace.  Both sides pay for the activations' pass.  Asked for 10 %, the prices send 412 of 750
+// measured shapes to it, 12 of them to more than 3 % more time (rows of some hundred values); without the price of
+// values (gemm_price), 512 x 7488 with three bits took 73 us instead of 53 at 2 to 64 tokens.
 static int tiled_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool f16) {
   double dense = 0.0;
-  const int tile = dense_choose_tile(M, N, K, f16 ? MF_F16 : MF_BF16, static_cast<double>(K) * static_cast<double>(N) * (2.0 + bits / 8.0), &dense);
+  const double passes = static_cast<double>(K) * (static_cast<double>(N) * (2.0 + bits / 8.0) + static_cast<double>(M) * 4.0);
+  const int tile = dense_choose_tile(M, N, K, f16 ? MF_F16 : MF_BF16, passes, &dense);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
-  if (debug_env(ENV_GEMM_TILE) != nullptr) return -1;
-  return dense < 0.94 * gemm_cost(M, N, K, bits) ? tile : -1;
+  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_tile(M, N, K, bits) == 4) return -1;
+  return dense < 0.9 * gemm_price(M, N, K, bits, PRICE_VALUES) ? tile : -1;
 }
 
 // Bytes of workspace for [M, K] 16-bit activations: their operand-order copy (whole row tiles of 32), and the decoded

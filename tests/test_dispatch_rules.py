@@ -58,3 +58,17 @@ def test_int8_tables_are_multiplied_as_integers_on_large_problems(lib, m, n, k):
     (64, 36864, 4096), (4608, 36864, 131072), (4608, 36868, 4096), (4608, 36864, 4064), (0, 36864, 4096)])   # not taken at all
 def test_int8_tables_stay_with_the_launch_that_is_faster(lib, m, n, k):
     assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) == 0
+
+
+@pytest.mark.parametrize("m,n,k,wbits", [(4608, 14336, 4096, 3), (4608, 14336, 4096, 4), (2048, 4096, 4096, 6), (8, 512, 7488, 6)])
+def test_values_decode_the_weights_where_that_is_faster(lib, m, n, k, wbits):
+    # bf16: 559 -> 419, 510 -> 414, 136 -> 75, 115 -> 74 us
+    assert lib.oq_matmul_packed_weight_workspace_bytes(m, n, k, wbits, _lib.OQ_BF16) == operand_order(m, k) + operand_order(n, k)
+
+
+@pytest.mark.parametrize("m,n,k,wbits", [
+    (2, 512, 7488, 3), (64, 512, 7488, 3), (4608, 512, 7488, 3),        # 53, 59, 88 us packed; 74, 75, 93 decoded first
+    (2, 952, 15552, 2), (2701, 696, 8000, 2), (1445, 1000, 16320, 2),   # 107, 80, 143; 147, 93, 166
+    (3416, 2352, 3072, 2)])                                             # the packed launch shares K between wavefronts
+def test_values_leave_the_weights_packed_elsewhere(lib, m, n, k, wbits):
+    assert lib.oq_matmul_packed_weight_workspace_bytes(m, n, k, wbits, _lib.OQ_BF16) == operand_order(m, k)

@@ -199,3 +199,19 @@ def test_floating_activations_from_operand_order(dev, library_switch, dense, til
     magnitude = (x.double().abs() @ w.abs().T) * factor + o["bias"].double().abs()
     bound = magnitude * (k + 4) * 2.0 ** -24 + exact.abs() * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) + 2.0 ** -25
     assert bool(((got.double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,k,n,wbits", [(3416, 3072, 2352, 2), (2700, 3072, 2992, 8), (4608, 3072, 3072, 6), (1024, 4096, 4096, 3)])
+def test_bf16_values_sum_alike_with_and_without_a_workspace(dev, m, k, n, wbits):
+    """As the rules choose: beside packed launches that share K between wavefronts (the first two), decoded first (the
+    third), neither (the last)."""
+    from orbitquant_amd import _lib, ops
+
+    o = operands(dev, m, k, n, wbits, 4, seed=m)
+    x = torch.randn(m, k, device=dev, generator=torch.Generator(device=dev).manual_seed(n)).bfloat16()
+    with_workspace = ops.matmul_packed_weight_values(x, o["packed"], o["rn"], o["wcents"], bits=wbits, out_features=n, in_features=k, bias=o["bias"])
+    out = torch.empty_like(with_workspace)
+    rc = _lib.load().oq_matmul_packed_weight(x.data_ptr(), _lib.OQ_BF16, None, o["packed"].data_ptr(), wbits, o["rn"].data_ptr(), o["wcents"].data_ptr(),
+                                             o["bias"].data_ptr(), _lib.OQ_F32, m, n, k, out.data_ptr(), _lib.OQ_BF16, None, 0,
+                                             torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(out, with_workspace)
