@@ -181,9 +181,12 @@ int oq_debug_override(const char *name, const char *value);
  * workgroup), larger M the MFMA tile kernel.  A token row's result does not depend on the
  * rows computed with it as long as the call stays within 64 rows.  A problem with few output
  * tiles and many K-steps (some hundred tokens on a short-and-long matrix) is shared between
- * workgroups along K when the caller provides a workspace for the fp32 partial tiles, and a problem
- * of some thousand tokens is decoded once into the workspace and multiplied from there (the same
- * bits as without):
+ * workgroups along K when the caller provides a workspace for the fp32 partial tiles, and a large
+ * problem (some thousand tokens) is decoded once into the workspace and multiplied from there.  The
+ * workspace can change the order in which a sum's terms are added, and with it the last bits: a shared
+ * K is added in parts, and where the launch without a workspace shares K between the wavefronts of a
+ * workgroup (128 x 96 tiles), it is that launch that adds in parts and the decoded problem that does
+ * not.  Every other large problem gives the same bits with and without:
  *
  * workspace    NULL, or a device buffer of at least oq_packed_linear_workspace_bytes(...) bytes, 16-byte
  *              aligned, that this call may overwrite (calls on one stream are ordered and may share one).
@@ -329,9 +332,8 @@ int oq_quantized_linear_group(const void *x, int x_dtype, const uint16_t *input_
  * oq_quantized_linear for callers that cannot allocate device memory or bring a workspace:
  * code running under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  No counterpart in the reference.  Same arguments as oq_quantized_linear without
- * the two scratch pointers, and the same results (except where oq_quantized_linear shares K
- * between workgroups through a buffer of the library's own, see oq_packed_linear: this call
- * never does, and the two then differ by the order of the last additions): codes and norms pass through a buffer
+ * the two scratch pointers, and the results of oq_quantized_linear without a workspace (with one,
+ * the order of the additions can differ, see oq_packed_linear): codes and norms pass through a buffer
  * of OQ_STATIC_SCRATCH_BYTES that is part of the library's device image (every GPU the library
  * runs on holds its own copy until the process ends).  The call allocates and frees nothing.
  * Shapes whose codes ([M, K/2] bytes for a_bits <= 4 and even K, else [M, K], rounded up to
