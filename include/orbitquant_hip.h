@@ -222,6 +222,12 @@ int oq_packed_linear(const void *codes, int code_format, const float *token_norm
 uint64_t oq_packed_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits);
 
 /*
+ * What of it holds partial tiles of a K shared between workgroups: 0 for a problem that would be decoded into
+ * the workspace, and so the size to fall back on when that much memory is not there.
+ */
+uint64_t oq_packed_linear_least_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits);
+
+/*
  * oq_packed_linear for 4-bit codes (two per byte) on both sides whose codebooks are int8 tables, summed in
  * int32 on the int8 matrix instructions:
  *

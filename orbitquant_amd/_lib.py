@@ -22,7 +22,7 @@ EXPORTS = (
     "oq_device_ok", "oq_last_error", "oq_version", "oq_debug_override", "oq_rotate_quantize", "oq_rotate_plan_bytes", "oq_rotate_plan_build", "oq_quantize_weight", "oq_rotate_quantize_mapped",
     "oq_packed_linear", "oq_packed_linear_group", "oq_packed_linear_mapped", "oq_quantized_linear", "oq_quantized_linear_group", "oq_quantized_linear_static", "oq_matmul_packed_weight", "oq_matmul_packed_adaln_int4", "oq_quantize_adaln_weight", "oq_unpack_lowbit", "oq_pack_lowbit",
     "oq_dequantize_packed_weight", "oq_packed_linear_workspace_bytes", "oq_matmul_packed_weight_workspace_bytes",
-    "oq_packed_linear_int8", "oq_packed_linear_int8_workspace_bytes",
+    "oq_packed_linear_int8", "oq_packed_linear_int8_workspace_bytes", "oq_packed_linear_least_workspace_bytes",
 )
 
 _lib = None
@@ -66,6 +66,8 @@ def load() -> ctypes.CDLL:
                                      c_i64, c_i64, c_i64, vp, c_int, vp, c_u64, vp]
     lib.oq_packed_linear_workspace_bytes.restype = c_u64
     lib.oq_packed_linear_workspace_bytes.argtypes = [c_i64, c_i64, c_i64, c_int, c_int, c_int]
+    lib.oq_packed_linear_least_workspace_bytes.restype = c_u64
+    lib.oq_packed_linear_least_workspace_bytes.argtypes = [c_i64, c_i64, c_i64, c_int, c_int, c_int]
     lib.oq_matmul_packed_weight_workspace_bytes.restype = c_u64
     lib.oq_matmul_packed_weight_workspace_bytes.argtypes = [c_i64, c_i64, c_i64, c_int, c_int]
     lib.oq_packed_linear_int8.restype = c_int

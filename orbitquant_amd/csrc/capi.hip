@@ -101,7 +101,7 @@ int gemm_tiled_dispatch(bool f16, const void *x, const float *token_scale, const
                         const float *w_cents, const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
                         int out_dtype, void *workspace, uint64_t workspace_bytes, hipStream_t stream);
 uint64_t gemm_tiled_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool f16);
-uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes);
+uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, bool decoded);
 int gemm_staged_dispatch(const void *x, const float *token_scale, const uint8_t *w, int bits, const uint16_t *row_norms,
                          const float *w_cents, const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
                          int out_dtype, hipStream_t stream);
@@ -287,11 +287,19 @@ int oq_debug_override(const char *name, const char *value) {
   return debug_env_set(name, value);
 }
 
-uint64_t oq_packed_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits) {
+static uint64_t linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits, bool decoded) {
   if (M <= 0 || N <= 0 || K <= 0 || a_bits < 1 || a_bits > 8) return 0;
   if (gemv_supported(M, K, w_bits, code_format, 1 << a_bits)) return 0;  // the streaming kernel
   if (N % 8 != 0 || !gemm_supported(K, w_bits) || !(code_format == OQ_CODES_NIBBLE || M > 16)) return 0;
-  return gemm_workspace_bytes(M, N, K, w_bits, code_format == OQ_CODES_U8);
+  return gemm_workspace_bytes(M, N, K, w_bits, code_format == OQ_CODES_U8, decoded);
+}
+
+uint64_t oq_packed_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits) {
+  return linear_workspace_bytes(M, N, K, w_bits, code_format, a_bits, true);
+}
+
+uint64_t oq_packed_linear_least_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int code_format, int a_bits) {
+  return linear_workspace_bytes(M, N, K, w_bits, code_format, a_bits, false);
 }
 
 uint64_t oq_matmul_packed_weight_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_bits, int x_dtype) {

@@ -162,9 +162,9 @@ bool gemm_supported(int64_t K, int bits) {
 }
 
 // Bytes of workspace a launch of this shape would like to have: both operands decoded into operand order (large
-// problems), or partial tiles (0: it is a launch that needs neither).
-uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes) {
-  if (gemm_choose_dense(M, N, K, bits, byte_codes) >= 0) return dense_workspace_bytes(M, N, K, MF_BF16);
+// problems), or partial tiles (0: it is a launch that needs neither).  `decoded` false: without the decoded operands.
+uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, bool decoded) {
+  if (gemm_choose_dense(M, N, K, bits, byte_codes) >= 0) return decoded ? dense_workspace_bytes(M, N, K, MF_BF16) : 0u;
   const int splits = gemm_choose_splits(M, N, K, bits);
   return splits > 1 ? static_cast<uint64_t>(M) * static_cast<uint64_t>(N) * 4u * static_cast<uint64_t>(splits) : 0u;
 }

@@ -7,6 +7,8 @@ pass raw device pointers and the current HIP stream, and never synchronize.
 
 from __future__ import annotations
 
+import warnings
+
 import torch
 
 from . import _lib
@@ -53,18 +55,31 @@ def _stream(t: torch.Tensor) -> int:
     return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
-def _workspace(nbytes: int, like: torch.Tensor) -> tuple[int | None, int, torch.Tensor | None]:
+def _workspace(nbytes: int, like: torch.Tensor, smaller=lambda: ()) -> tuple[int | None, int, torch.Tensor | None]:
     """(address, size, tensor) of a workspace of `nbytes` for one call, from torch's caching allocator (the
     library allocates nothing: this wrapper owns allocation, as the reference's does).  The tensor is returned
     so that the caller keeps it alive until its call has been issued; stream-ordered reuse by the allocator
-    makes it safe to drop then."""
+    makes it safe to drop then.  `smaller()`: the sizes that the call can do with instead, in the order in which
+    they are tried when memory runs out (0: no workspace); where there are none, running out raises."""
     if nbytes <= 0:
         return None, 0, None
     try:
         buf = torch.empty(int(nbytes), dtype=torch.uint8, device=like.device)
-    except torch.OutOfMemoryError:   # a workspace makes a call faster, none needs it
-        return None, 0, None
+    except torch.OutOfMemoryError:
+        sizes = [n for n in smaller() if n < nbytes]
+        if not sizes:
+            raise
+        warnings.warn(f"no memory for a workspace of {nbytes} bytes: the call takes a slower kernel, which may add up "
+                      "in another order", RuntimeWarning, stacklevel=3)
+        return _workspace(sizes[0], like, lambda: sizes[1:])
     return buf.data_ptr(), int(nbytes), buf
+
+
+def _group_workspace(shapes: list[tuple], like: torch.Tensor) -> tuple[int | None, int, torch.Tensor | None]:
+    """`_workspace` for packed linears that run one after the other and share it."""
+    lib = _lib.load()
+    return _workspace(max(lib.oq_packed_linear_workspace_bytes(*shape) for shape in shapes), like,
+                      lambda: (max(lib.oq_packed_linear_least_workspace_bytes(*shape) for shape in shapes),))
 
 
 def _scratch(sizes: tuple[int, ...], like: torch.Tensor) -> tuple[torch.Tensor, list[int]]:
@@ -314,8 +329,8 @@ def packed_linear(
             row_norms.data_ptr(), weight_centroids.data_ptr(), _ptr(bias),
             _dt(bias) if bias is not None else OQ_F32, m, int(out_features), int(in_features),
             out.data_ptr(), _DTYPES[output_dtype])
-    ws_ptr, ws_bytes, ws = _workspace(lib.oq_packed_linear_workspace_bytes(m, int(out_features), int(in_features), int(weight_bits),
-                                                                            fmt, int(activation_bits)), codes)
+    shape = (m, int(out_features), int(in_features), int(weight_bits), fmt, int(activation_bits))
+    ws_ptr, ws_bytes, ws = _workspace(lib.oq_packed_linear_workspace_bytes(*shape), codes, lambda: (lib.oq_packed_linear_least_workspace_bytes(*shape),))
     with _OnDevice(codes):
         if output_map is None:
             rc = lib.oq_packed_linear(*args, ws_ptr, ws_bytes, _stream(codes))
@@ -361,7 +376,7 @@ def packed_linear_int8(
     bias = _operand(bias, "bias", codes, dtype=_FLOATS, numel=out_features)
     norms = _operand(token_norms.reshape(-1), "token_norms", codes, dtype=torch.float32, numel=m)
     out = torch.empty((m, out_features), dtype=output_dtype, device=codes.device)
-    ws_ptr, ws_bytes, ws = _workspace(need, codes)
+    ws_ptr, ws_bytes, ws = _workspace(need, codes, lambda: (0,))
     if ws_ptr is None:
         return None
     with _OnDevice(codes):
@@ -422,8 +437,7 @@ def packed_linear_group(
     ptrs = ctypes.c_void_p * count
     lib = _lib.load()
     fmt_code = {"u8": OQ_CODES_U8, "nibble": OQ_CODES_NIBBLE}[code_format]
-    ws_ptr, ws_bytes, ws = _workspace(max(lib.oq_packed_linear_workspace_bytes(m, k[4], int(in_features), k[3], fmt_code, int(activation_bits))
-                                          for k in keep), codes)   # members run one after the other and share it
+    ws_ptr, ws_bytes, ws = _group_workspace([(m, k[4], int(in_features), k[3], fmt_code, int(activation_bits)) for k in keep], codes)
     with _OnDevice(codes):
         rc = lib.oq_packed_linear_group(
             flat.data_ptr(), fmt, norms.data_ptr(), activation_centroids.data_ptr(), int(activation_bits), count,
@@ -488,8 +502,8 @@ def quantized_linear(
     scratch, (codes_ptr, norms_ptr) = _scratch((m * (dim // 2 if nibble else dim), 4 * m), x)
     out = torch.empty((m, out_features), dtype=x.dtype, device=x.device)
     lib = _lib.load()
-    ws_ptr, ws_bytes, ws = _workspace(lib.oq_packed_linear_workspace_bytes(
-        m, int(out_features), dim, int(weight_bits), OQ_CODES_NIBBLE if nibble else OQ_CODES_U8, int(activation_bits)), x)
+    shape = (m, int(out_features), dim, int(weight_bits), OQ_CODES_NIBBLE if nibble else OQ_CODES_U8, int(activation_bits))
+    ws_ptr, ws_bytes, ws = _workspace(lib.oq_packed_linear_workspace_bytes(*shape), x, lambda: (lib.oq_packed_linear_least_workspace_bytes(*shape),))
     with _OnDevice(x):
         rc = lib.oq_quantized_linear(
             rows.data_ptr(), _dt(rows), _ptr(input_map), m, dim, permutation.data_ptr(), signs.data_ptr(),
@@ -556,8 +570,8 @@ def quantized_linear_group(
     count = len(keep)
     ptrs = ctypes.c_void_p * count
     lib = _lib.load()
-    ws_ptr, ws_bytes, ws = _workspace(max(lib.oq_packed_linear_workspace_bytes(
-        m, k[4], dim, k[3], OQ_CODES_NIBBLE if nibble else OQ_CODES_U8, int(activation_bits)) for k in keep), x)
+    fmt_code = OQ_CODES_NIBBLE if nibble else OQ_CODES_U8
+    ws_ptr, ws_bytes, ws = _group_workspace([(m, k[4], dim, k[3], fmt_code, int(activation_bits)) for k in keep], x)
     with _OnDevice(x):
         rc = lib.oq_quantized_linear_group(
             rows.data_ptr(), _dt(rows), _ptr(input_map), m, dim, permutation.data_ptr(), signs.data_ptr(),
@@ -599,8 +613,9 @@ def matmul_packed_weight_values(
     token_scale = _operand(token_scale, "token_scale", x, dtype=torch.float32, numel=m)
     out = torch.empty((m, out_features), dtype=out_dtype, device=x.device)
     lib = _lib.load()
-    ws_ptr, ws_bytes, ws = _workspace(lib.oq_matmul_packed_weight_workspace_bytes(m, int(out_features), int(in_features), int(bits),
-                                                                                   _dt(x)), x)
+    copy = -(-m // 32) * 32 * int(in_features) * 2   # the activations alone: the weights stay packed, the same sums in bf16
+    ws_ptr, ws_bytes, ws = _workspace(lib.oq_matmul_packed_weight_workspace_bytes(m, int(out_features), int(in_features), int(bits), _dt(x)), x,
+                                      lambda: (copy, 0) if x.dtype == torch.float16 else (copy,))
     with _OnDevice(x):
         rc = lib.oq_matmul_packed_weight(
             flat.data_ptr(), _dt(flat), _ptr(token_scale), packed_weight_indices.data_ptr(), int(bits),

@@ -72,3 +72,15 @@ def test_values_decode_the_weights_where_that_is_faster(lib, m, n, k, wbits):
     (3416, 2352, 3072, 2)])                                             # the packed launch shares K between wavefronts
 def test_values_leave_the_weights_packed_elsewhere(lib, m, n, k, wbits):
     assert lib.oq_matmul_packed_weight_workspace_bytes(m, n, k, wbits, _lib.OQ_BF16) == operand_order(m, k)
+
+
+def test_the_least_workspace_holds_partial_tiles_only(lib):
+    sizes = lambda *shape: (lib.oq_packed_linear_workspace_bytes(*shape), lib.oq_packed_linear_least_workspace_bytes(*shape))
+    nibble, u8 = _lib.OQ_CODES_NIBBLE, _lib.OQ_CODES_U8
+    full, least = sizes(4608, 12288, 3072, 3, nibble, 3)
+    assert full > 0 and least == 0
+    full, least = sizes(32760, 13824, 5120, 4, u8, 6)
+    assert full > 0 and least == 0
+    full, least = sizes(128, 4096, 14336, 4, nibble, 4)     # K shared between workgroups
+    assert full == least > 0 and full % (128 * 4096 * 4) == 0
+    assert sizes(1, 4096, 4096, 4, nibble, 4) == sizes(1024, 14336, 4096, 4, nibble, 4) == (0, 0)

@@ -243,3 +243,55 @@ def test_bf16_values_sum_alike_with_and_without_a_workspace(dev, m, k, n, wbits)
                                              o["bias"].data_ptr(), _lib.OQ_F32, m, n, k, out.data_ptr(), _lib.OQ_BF16, None, 0,
                                              torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(out, with_workspace)
+
+
+@pytest.fixture
+def no_memory_from(monkeypatch):
+    """`no_memory_from(size)`: workspaces of that size and more cannot be allocated."""
+    from orbitquant_amd import ops
+
+    real = torch.empty
+
+    def limit_to(limit):
+        def empty(size, *args, **kwargs):
+            if isinstance(size, int) and size >= limit:
+                raise torch.OutOfMemoryError("no memory")
+            return real(size, *args, **kwargs)
+
+        monkeypatch.setattr(ops.torch, "empty", empty)
+
+    return limit_to
+
+
+def test_without_memory_for_the_decoded_operands(dev, no_memory_from):
+    """A warning, and the launch without them; memory that the call needed all along stays an error."""
+    import orbitquant_packed_matmul as package
+    from orbitquant_amd import ops
+
+    o = operands(dev, 4608, 3072, 12288, 3, 4, seed=1)
+    linear = lambda: multiply(o, 4608, 3072, 12288, 3, 4, torch.bfloat16)
+    x = {dtype: torch.randn(4608, 3072, device=dev).to(dtype) for dtype in (torch.bfloat16, torch.float16)}
+    v = operands(dev, 1, 3072, 3072, 6, 4, seed=2)
+    values = lambda dtype: ops.matmul_packed_weight_values(x[dtype], v["packed"], v["rn"], v["wcents"], bits=6, out_features=3072, in_features=3072)
+    t = operands(dev, 2048, 4096, 4096, 4, 4, seed=3)
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    pair = lambda: package.matmul_packed_w4a4_int8(t["codes"], t["packed"], t["norms"], t["rn"], table, table, activation_scale=0.05, weight_scale=0.04,
+                                                   out_features=4096, in_features=4096)
+    short = operands(dev, 128, 14336, 4096, 4, 4, seed=4)
+    want = [linear(), values(torch.bfloat16), values(torch.float16), pair()]
+    copy = 4608 * 3072 * 2
+    no_memory_from(copy + 1)
+    with pytest.warns(RuntimeWarning, match="workspace"):
+        assert torch.equal(linear(), want[0])
+    with pytest.warns(RuntimeWarning, match="workspace"):
+        assert torch.equal(values(torch.bfloat16), want[1])   # the activations' copy fits: the weights stay packed
+    no_memory_from(4 << 20)
+    with pytest.raises(torch.OutOfMemoryError):
+        values(torch.bfloat16)
+    with pytest.raises(torch.OutOfMemoryError):               # K shared between workgroups
+        multiply(short, 128, 14336, 4096, 4, 4, torch.bfloat16)
+    # the same operands in another order of additions: the results differ by roundings to the output type
+    with pytest.warns(RuntimeWarning, match="workspace"):
+        torch.testing.assert_close(values(torch.float16).float(), want[2].float(), rtol=2.0 ** -10, atol=1e-3)
+    with pytest.warns(RuntimeWarning, match="workspace"):
+        torch.testing.assert_close(pair().float(), want[3].float(), rtol=2.0 ** -7, atol=1e-3 * float(want[3].float().abs().max()))
