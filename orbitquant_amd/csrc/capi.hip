@@ -324,7 +324,7 @@ int oq_packed_linear(const void *codes, int code_format, const float *token_norm
 static int int8_choose_tile(int64_t M, int64_t N, int64_t K) {
   if (M <= 64 || N <= 0 || K <= 0 || K > 131071) return -1;  // (sums of K products of two int8 values stay below 2^31)
   double cost = 0.0;
-  const int tile = dense_choose_tile(M, N, K, MF_I8, 1.5 * static_cast<double>(K) * static_cast<double>(M + N), &cost);
+  const int tile = dense_choose_tile(M, N, K, dense_rows_at_a_time(M, K, MF_I8), MF_I8, 1.5 * static_cast<double>(K) * static_cast<double>(M + N), &cost);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   return cost < 0.9 * gemm_call_price(M, N, K, 4) ? tile : -1;
 }
@@ -340,16 +340,24 @@ int oq_packed_linear_int8(const void *codes, const float *token_norms, float sca
   if (int rc = check_matmul_common("packed_linear_int8", packed_w, 4, row_norms, reinterpret_cast<const float *>(w_table), bias, bias_dtype, M, N, K, out, out_dtype)) return rc;
   if (M == 0) return OQ_OK;
   if (codes == nullptr || act_table == nullptr) return fail(OQ_ERR_INVALID, "packed_linear_int8: null codes/table");
-  const uint64_t need = oq_packed_linear_int8_workspace_bytes(M, N, K);
+  const int tile = int8_choose_tile(M, N, K);
+  const uint64_t need = tile < 0 ? 0 : dense_workspace_bytes(M, N, K, MF_I8);
   if (need == 0 || !aligned16(codes) || !aligned16(packed_w) || !gemm_output_ok(N, out))
     return fail(OQ_ERR_UNSUPPORTED, "packed_linear_int8: M=%lld N=%lld K=%lld or an alignment (oq_packed_linear takes it)", (long long)M, (long long)N, (long long)K);
   if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)) return fail(OQ_ERR_INVALID, "packed_linear_int8: %llu bytes of workspace needed", (unsigned long long)need);
   hipStream_t s = as_stream(stream);
-  unsigned char *a_values = static_cast<unsigned char *>(workspace), *w_values = a_values + operand_order_bytes(M, K, 1);
-  if (int rc = decode_operands_int8(static_cast<const uint8_t *>(codes), act_table, M, K, a_values, s)) return rc;
-  if (int rc = decode_operands_int8(packed_w, w_table, N, K, w_values, s)) return rc;
-  return dense_gemm(MF_I8, a_values, w_values, token_norms, scale, row_norms, bias, bias_dtype, M, N, K, out, out_dtype, nullptr,
-                    int8_choose_tile(M, N, K), s);
+  const int64_t rows = dense_rows_at_a_time(M, K, MF_I8);
+  unsigned char *a_values = static_cast<unsigned char *>(workspace), *w_values = a_values + operand_order_bytes(rows, K, 1);
+  for (int64_t m = 0; m < M; m += rows) {
+    const int64_t count = M - m < rows ? M - m : rows;
+    if (int rc = decode_operands_int8(static_cast<const uint8_t *>(codes) + m * (K / 2), act_table, count, K, a_values, s)) return rc;
+    if (m == 0)
+      if (int rc = decode_operands_int8(packed_w, w_table, N, K, w_values, s)) return rc;
+    if (int rc = dense_gemm(MF_I8, a_values, w_values, token_norms != nullptr ? token_norms + m : nullptr, scale, row_norms, bias, bias_dtype, count, N, K,
+                            static_cast<unsigned char *>(out) + m * N * dtype_size(out_dtype), out_dtype, nullptr, tile, s))
+      return rc;
+  }
+  return OQ_OK;
 }
 
 int oq_packed_linear_group(const void *codes, int code_format, const float *token_norms, const float *act_centroids,

@@ -239,12 +239,12 @@ double launch_warmth(double operations) {
 
 // The best tile of this kernel for a problem and its time in microseconds, the passes into operand order included
 // (`pass_bytes`: what they read and write); -1 where the kernel cannot run.  A launch runs in rounds of 256 workgroups,
-// one to a CU, each with a fixed prologue and epilogue and a time per K-step of 128 operand bytes that grows with the
+// one to a CU (each part of the rows in rounds of its own), each with a fixed prologue and epilogue and a time per K-step of 128 operand bytes that grows with the
 // length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16 at 2e10 operations, 1.14 us from 1e12 on) and
 // by up to a quarter where the operands outgrow the 256 MB last-level cache; on top come the passes, the output's
 // way to memory and the launches.  Fitted to 5000 timings of single calls, 256 to 16384 in each dimension, all tiles:
 // nine in ten within 15 %; the tile it picks is 1 % behind the best one on average.
-int dense_choose_tile(int64_t M, int64_t N, int64_t K, int mf, double pass_bytes, double *cost_out) {
+int dense_choose_tile(int64_t M, int64_t N, int64_t K, int64_t rows_at_a_time, int mf, double pass_bytes, double *cost_out) {
   if (K % 64 != 0 || N % 8 != 0 || M > 0x7fff0000LL || N > 0x7fff0000LL || K > 0x0fffffffLL) return -1;
   static const int sizes[4][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 128}};
   struct Times { double fixed[4], step[4], warm, pass_mb, out_mb, launches; };
@@ -259,8 +259,8 @@ int dense_choose_tile(int64_t M, int64_t N, int64_t K, int mf, double pass_bytes
   int best = 0;
   double best_cost = 0.0;
   for (int tile = 0; tile < 4; ++tile) {
-    const int64_t tiles = ((M + sizes[tile][0] - 1) / sizes[tile][0]) * ((N + sizes[tile][1] - 1) / sizes[tile][1]);
-    const double cost = static_cast<double>((tiles + 255) / 256) * (t.fixed[tile] + steps * t.step[tile] * step_factor);
+    auto rounds = [&](int64_t rows) { return (((rows + sizes[tile][0] - 1) / sizes[tile][0]) * ((N + sizes[tile][1] - 1) / sizes[tile][1]) + 255) / 256; };
+    const double cost = static_cast<double>(M / rows_at_a_time * rounds(rows_at_a_time) + rounds(M % rows_at_a_time)) * (t.fixed[tile] + steps * t.step[tile] * step_factor);
     if (tile == 0 || cost < best_cost) {
       best = tile;
       best_cost = cost;

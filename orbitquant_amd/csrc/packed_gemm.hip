@@ -140,7 +140,7 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
 static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr) {
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   double dense = 0.0;
-  const int tile = dense_choose_tile(M, N, K, MF_BF16, k * (m * (byte_codes ? 3.0 : 2.5) + n * (2.0 + bits / 8.0)), &dense);
+  const int tile = dense_choose_tile(M, N, K, dense_rows_at_a_time(M, K, MF_BF16), MF_BF16, k * (m * (byte_codes ? 3.0 : 2.5) + n * (2.0 + bits / 8.0)), &dense);
   if (cost_out != nullptr) *cost_out = dense;
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
@@ -180,10 +180,18 @@ int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float
   const int dense_tile = gemm_choose_dense(M, N, K, bits, a_mode == A_U8);
   if (dense_tile >= 0 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
       workspace_bytes >= dense_workspace_bytes(M, N, K, MF_BF16)) {
-    unsigned char *a_values = static_cast<unsigned char *>(workspace), *w_values = a_values + operand_order_bytes(M, K, 2);
-    if (int rc = decode_operands(static_cast<const uint8_t *>(a), a_mode == A_NIBBLE ? 4 : 8, act_cents, a_levels, M, K, false, a_values, stream)) return rc;
-    if (int rc = decode_operands(w, bits, w_cents, 1 << bits, N, K, false, w_values, stream)) return rc;
-    return dense_gemm(MF_BF16, a_values, w_values, row_scale, 1.0f, row_norms, bias, bias_dtype, M, N, K, out, out_dtype, out_map, dense_tile, stream);
+    const int64_t rows = dense_rows_at_a_time(M, K, MF_BF16), row_bytes = a_mode == A_NIBBLE ? K / 2 : K;
+    unsigned char *a_values = static_cast<unsigned char *>(workspace), *w_values = a_values + operand_order_bytes(rows, K, 2);
+    for (int64_t m = 0; m < M; m += rows) {
+      const int64_t count = M - m < rows ? M - m : rows;
+      if (int rc = decode_operands(static_cast<const uint8_t *>(a) + m * row_bytes, a_mode == A_NIBBLE ? 4 : 8, act_cents, a_levels, count, K, false, a_values, stream)) return rc;
+      if (m == 0)  // (behind the activations, whose codes the caches still hold: in front of them 4608-token blocks lose 1.3 %)
+        if (int rc = decode_operands(w, bits, w_cents, 1 << bits, N, K, false, w_values, stream)) return rc;
+      if (int rc = dense_gemm(MF_BF16, a_values, w_values, row_scale != nullptr ? row_scale + m : nullptr, 1.0f, row_norms, bias, bias_dtype, count, N, K,
+                              static_cast<unsigned char *>(out) + m * N * dtype_size(out_dtype), out_dtype, out_map, dense_tile, stream))
+        return rc;
+    }
+    return OQ_OK;
   }
   GemmArgs g{};
   g.a = static_cast<const uint8_t *>(a); g.row_scale = row_scale; g.act_cents = act_cents; g.a_levels = a_levels;

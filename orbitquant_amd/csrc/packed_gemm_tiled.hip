@@ -66,7 +66,7 @@ int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits);  // packed_gemm
 static int tiled_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool f16) {
   double dense = 0.0;
   const double passes = static_cast<double>(K) * (static_cast<double>(N) * (2.0 + bits / 8.0) + static_cast<double>(M) * 4.0);
-  const int tile = dense_choose_tile(M, N, K, f16 ? MF_F16 : MF_BF16, passes, &dense);
+  const int tile = dense_choose_tile(M, N, K, M, f16 ? MF_F16 : MF_BF16, passes, &dense);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_tile(M, N, K, bits) == 4) return -1;
   return dense < 0.9 * gemm_price(M, N, K, bits, PRICE_VALUES) ? tile : -1;
@@ -77,7 +77,7 @@ static int tiled_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool f1
 uint64_t gemm_tiled_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool f16) {
   const int64_t row_tiles = (M + 31) / 32;
   if (row_tiles > 65535) return 0u;
-  return tiled_choose_dense(M, N, K, bits, f16) >= 0 ? dense_workspace_bytes(M, N, K, MF_BF16) : operand_order_bytes(M, K, 2);
+  return tiled_choose_dense(M, N, K, bits, f16) >= 0 ? operand_order_bytes(M, K, 2) + operand_order_bytes(N, K, 2) : operand_order_bytes(M, K, 2);
 }
 
 // x: bf16 (f16: fp16) [M, K], 16-byte aligned rows (K % 64 == 0).  `workspace`: the caller's buffer of
@@ -93,7 +93,7 @@ int gemm_tiled_dispatch(bool f16, const void *x, const float *token_scale, const
                      static_cast<const uint16_t *>(x), M, K, reinterpret_cast<uint4 *>(tiled));
   if (int rc = check_launch("tile_activations")) return rc;
   const int dense_tile = tiled_choose_dense(M, N, K, bits, f16);
-  if (dense_tile >= 0 && workspace_bytes >= dense_workspace_bytes(M, N, K, MF_BF16)) {
+  if (dense_tile >= 0 && workspace_bytes >= operand_order_bytes(M, K, 2) + operand_order_bytes(N, K, 2)) {
     unsigned char *w_values = tiled + operand_order_bytes(M, K, 2);
     if (int rc = decode_operands(w, bits, w_cents, 1 << bits, N, K, f16, w_values, stream)) return rc;
     return dense_gemm(f16 ? MF_F16 : MF_BF16, tiled, w_values, token_scale, 1.0f, row_norms, bias, bias_dtype, M, N, K, out, out_dtype, nullptr,

@@ -84,3 +84,13 @@ def test_the_least_workspace_holds_partial_tiles_only(lib):
     full, least = sizes(128, 4096, 14336, 4, nibble, 4)     # K shared between workgroups
     assert full == least > 0 and full % (128 * 4096 * 4) == 0
     assert sizes(1, 4096, 4096, 4, nibble, 4) == sizes(1024, 14336, 4096, 4, nibble, 4) == (0, 0)
+
+
+@pytest.mark.parametrize("m,n,k", [(32760, 5120, 13824), (131072, 3072, 12288), (2000000, 4096, 4096)])
+def test_the_decoded_activations_are_bounded(lib, m, n, k):
+    # 512 MB of them and one more row of tiles for every part, whatever the token count; the weights are decoded whole
+    part = (512 << 20) + 256 * k * 2
+    size = lib.oq_packed_linear_workspace_bytes(m, n, k, 6, _lib.OQ_CODES_U8, 6)
+    assert operand_order(n, k) < size <= part + operand_order(n, k) and size < operand_order(m, k) + operand_order(n, k)
+    size = lib.oq_packed_linear_int8_workspace_bytes(4 * m, n, k)
+    assert operand_order(n, k, 1) < size <= part + operand_order(n, k, 1)

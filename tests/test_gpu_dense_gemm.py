@@ -42,6 +42,14 @@ def multiply(o, m, k, n, wbits, abits, dtype, output_map=None):
                              output_map=output_map)
 
 
+A_TABLE = [-128, -79, -62, -48, -36, -25, -15, -5, 0, 15, 25, 36, 48, 62, 79, 127]
+
+
+def looked_up(packed, rows, k, table):
+    """The values of two 4-bit codes per byte, in 64 bits."""
+    return table.double()[torch.stack((packed & 15, packed >> 4), dim=-1).long()].view(rows, k)
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2, 3])
 @pytest.mark.parametrize("m,k,n,wbits,abits,dtype,mapped", [
     (300, 64, 264, 4, 4, torch.bfloat16, False), (257, 192, 520, 3, 3, torch.float16, False), (512, 1024, 512, 2, 4, torch.bfloat16, True),
@@ -76,6 +84,42 @@ def test_chosen_for_large_problems_only_and_only_with_a_workspace(dev):
                                   dt[torch.bfloat16], None if workspace is None else workspace.data_ptr(), size,
                                   torch.cuda.current_stream().cuda_stream)
         assert rc == 0 and torch.equal(out, with_workspace)
+
+
+@pytest.mark.parametrize("tile", [0, 3])
+@pytest.mark.parametrize("wbits,abits,mapped", [(3, 4, False), (6, 6, True)])
+def test_activations_decoded_in_parts(dev, library_switch, tile, wbits, abits, mapped):
+    """More rows than are decoded at a time: two parts, the second one ragged."""
+    from orbitquant_amd import _lib, ops
+
+    m, k, n = 16640 + 33, 16384, 264
+    fmt = _lib.OQ_CODES_U8 if abits > 4 else _lib.OQ_CODES_NIBBLE
+    o = operands(dev, m, k, n, wbits, abits, seed=abits)
+    table = ops.activation_table(torch.nn.functional.gelu, torch.bfloat16, dev) if mapped else None
+    library_switch("OQ_GEMM_TILE", 0)
+    library_switch("OQ_DENSE_GEMM", "never")
+    want = multiply(o, m, k, n, wbits, abits, torch.bfloat16, table)
+    library_switch("OQ_DENSE_GEMM", tile)
+    size = _lib.load().oq_packed_linear_workspace_bytes(m, n, k, wbits, fmt, abits)
+    assert size < (-(-m // 32) + -(-n // 32)) * (k // 64) * 4096
+    assert torch.equal(multiply(o, m, k, n, wbits, abits, torch.bfloat16, table), want)
+
+
+def test_int8_activations_decoded_in_parts(dev, library_switch):
+    from orbitquant_amd import _lib, ops
+
+    m, k, n = 32768 + 97, 16448, 72
+    o = operands(dev, m, k, n, 4, 4, seed=9)
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    library_switch("OQ_DENSE_GEMM", 1)
+    assert _lib.load().oq_packed_linear_int8_workspace_bytes(m, n, k) < (-(-m // 32) + -(-n // 32)) * -(-k // 128) * 4096
+    got = ops.packed_linear_int8(o["codes"], o["norms"], table, o["packed"], o["rn"], table, scale=0.01, out_features=n, in_features=k,
+                                 output_dtype=torch.float32)
+    w = looked_up(o["packed"], n, k, table)
+    for start in (0, 16000, 32000):   # around the seam, and the ends
+        rows = slice(start, start + 1000)
+        sums = (looked_up(o["codes"][rows], len(got[rows]), k, table) @ w.T).float()
+        assert torch.equal(got[rows], sums * (o["norms"][rows] * 0.01)[:, None] * o["rn"].float())
 
 
 @pytest.mark.parametrize("m,k,n,wbits,abits,shares_k", [
@@ -124,14 +168,6 @@ def test_int8_pair_sums_integers_exactly(dev, library_switch, tile, m, k, n):
     # |bias| in the addition), then half an ulp of fp16
     bound = exact.abs() * 2.0 ** -11 + (exact.abs() + o["bias"].abs().double()) * 2.0 ** -20 + 2.0 ** -24
     assert bool(((got.double() - exact).abs() <= bound).all())
-
-
-A_TABLE = [-128, -79, -62, -48, -36, -25, -15, -5, 0, 15, 25, 36, 48, 62, 79, 127]
-
-
-def looked_up(packed, rows, k, table):
-    """The values of two 4-bit codes per byte, in 64 bits."""
-    return table.double()[torch.stack((packed & 15, packed >> 4), dim=-1).long()].view(rows, k)
 
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3])
