@@ -235,3 +235,19 @@ def test_activation_table_on_the_cpu():
         ops.activation_table(gelu, torch.float32, "cpu")
     with pytest.raises(ValueError):
         ops.activation_table(lambda t: t.float(), torch.bfloat16, "cpu")
+
+
+def test_the_wrappers_do_without_private_names_of_torch(monkeypatch):
+    import importlib.util
+
+    from orbitquant_amd import ops
+
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        if hasattr(torch._C, name):
+            monkeypatch.delattr(torch._C, name)
+    spec = importlib.util.spec_from_file_location("orbitquant_amd.ops_without", ops.__file__)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    assert module._current_device is torch.cuda.current_device
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda index: type("Stream", (), {"cuda_stream": 100 + index})())
+    assert module._stream(type("Tensor", (), {"device": torch.device("cuda", 3)})()) == 103
