@@ -331,3 +331,55 @@ def test_without_memory_for_the_decoded_operands(dev, no_memory_from):
         torch.testing.assert_close(values(torch.float16).float(), want[2].float(), rtol=2.0 ** -10, atol=1e-3)
     with pytest.warns(RuntimeWarning, match="workspace"):
         torch.testing.assert_close(pair().float(), want[3].float(), rtol=2.0 ** -7, atol=1e-3 * float(want[3].float().abs().max()))
+
+
+def same_bits(a, b):
+    """Equal, NaN where the other is NaN."""
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_infinities_and_nan_in_values_stay_in_their_rows(dev, library_switch, tile, dtype):
+    from orbitquant_amd import ops
+
+    m, k, n = 263, 192, 264
+    o = operands(dev, m, k, n, 4, 4, seed=21)
+    x = torch.randn(m, k, device=dev, generator=torch.Generator(device=dev).manual_seed(3)).to(dtype)
+    x[1, 5], x[64, 0], x[200, 191], x[262, 100] = float("nan"), float("inf"), -float("inf"), float("nan")   # (the last row is repeated as padding)
+    call = lambda: ops.matmul_packed_weight_values(x, o["packed"], o["rn"], o["wcents"], bits=4, out_features=n, in_features=k, bias=o["bias"],
+                                                   token_scale=o["norms"])
+    library_switch("OQ_GEMM_TILE", 0)
+    library_switch("OQ_DENSE_GEMM", "never")
+    want = call()
+    library_switch("OQ_DENSE_GEMM", tile)
+    got = call()
+    touched = torch.zeros(m, dtype=torch.bool, device=dev)
+    touched[[1, 64, 200, 262]] = True
+    assert torch.equal((~got.isfinite()).any(dim=1), touched) and bool(got[[1, 262]].isnan().all())
+    assert same_bits(got, want)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
+def test_infinities_and_nan_in_token_norms_and_bias(dev, library_switch, tile):
+    from orbitquant_amd import ops
+
+    m, k, n = 263, 192, 264
+    o = operands(dev, m, k, n, 4, 4, seed=22)
+    o["norms"][[0, 130, 262]] = torch.tensor([float("nan"), float("inf"), 0.0], device=dev)
+    o["bias"][[7, 263]] = torch.tensor([float("inf"), float("nan")], device=dev)
+    library_switch("OQ_GEMM_TILE", 0)
+    library_switch("OQ_DENSE_GEMM", "never")
+    want = multiply(o, m, k, n, 4, 4, torch.float32)
+    library_switch("OQ_DENSE_GEMM", tile)
+    got = multiply(o, m, k, n, 4, 4, torch.float32)
+    assert same_bits(got, want) and bool(got[0].isnan().all()) and bool(got[:, 263].isnan().all())
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    integers = ops.packed_linear_int8(o["codes"], o["norms"], table, o["packed"], o["rn"], table, scale=0.5, out_features=n, in_features=k,
+                                      bias=o["bias"], output_dtype=torch.float32)
+    sums = (looked_up(o["codes"], m, k, table) @ looked_up(o["packed"], n, k, table).T).float()
+    exact = (sums * (o["norms"] * 0.5)[:, None] * o["rn"].float()).double() + o["bias"].double()
+    assert torch.equal(integers.isfinite(), exact.float().isfinite()) and torch.equal(integers.isnan(), exact.isnan())
+    finite = exact.isfinite()   # (the last product and the addition round once or twice)
+    magnitude = (exact.abs() + 2 * o["bias"].double().abs())[finite]
+    assert bool(((integers.double() - exact).abs()[finite] <= magnitude * 2.0 ** -23).all())

@@ -69,3 +69,20 @@ def test_dequantize_of_an_unaligned_stream(bits):
     got = ops.dequantize_packed_weight(buf[1:], torch.ones(N, dtype=torch.bfloat16, device="cuda:0"), cents, bits=bits, out_features=N,
                                        in_features=K, dtype=torch.float32)
     assert torch.equal(got.cpu(), cents.cpu()[torch.from_numpy(idx).long()])
+
+
+@pytest.mark.parametrize("K", [64, 60])   # whole groups, and the form for any K
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_dequantize_infinities_and_nan(K, dtype):
+    from orbitquant_amd import ops
+
+    N = 6
+    rng = np.random.default_rng(K)
+    idx = rng.integers(0, 16, size=(N, K), dtype=np.uint8)
+    cents = torch.from_numpy(rng.standard_normal(16).astype(np.float32))
+    cents[3], cents[7], cents[9] = float("inf"), float("nan"), 0.0
+    norms = torch.tensor([1.0, float("inf"), float("nan"), 0.0, -2.0, 3e38]).to(torch.bfloat16)
+    got = ops.dequantize_packed_weight(torch.from_numpy(o.pack_bits(idx.reshape(-1), 4)).to("cuda:0"), norms.to("cuda:0"), cents.to("cuda:0"), bits=4,
+                                       out_features=N, in_features=K, dtype=dtype).cpu()
+    want = (cents[torch.from_numpy(idx).long()] * norms.float()[:, None]).to(dtype)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))

@@ -167,3 +167,25 @@ def test_a_weight_without_rows(dev):
     assert packed.shape == (0,) and packed.dtype == torch.uint8 and norms.shape == (0,) and norms.dtype == torch.bfloat16
     layer = OrbitLinear.from_weight(torch.empty(0, 64, device=dev), bias=None, config=OrbitQuantConfig())
     assert layer.packed_weight_indices.numel() == 0 and layer.row_norms.shape == (0,)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_rows_with_infinities_and_nan(dev, dtype):
+    """Their norms are not finite, so they take the IEEE division: a NaN has no boundary below it (the oracle's search
+    sorts it last), a finite value over an infinite norm is zero.  The rows beside them are what they are alone."""
+    k, bits = 1152, 4
+    perm, signs, block, inv = o.rpbh_constants(k, 5, "paper")
+    bounds = np.linspace(-3, 3, 2 ** bits - 1).astype(np.float32) / np.float32(np.sqrt(k))
+    w = torch.randn(7, k, generator=torch.Generator().manual_seed(9)).to(dtype)
+    w[1, 3], w[3, 1000], w[5, 0], w[5, 1] = float("nan"), float("inf"), -float("inf"), float("inf")
+    packed, norms = gpu_quantize(dev, w, perm, signs, bounds, block, inv, bits)
+    want_packed, want_norms, _ = o.quantize_weight(w.float().numpy(), perm, signs, bounds, block, 1e-10, bits, norm_order="sumsq_v1")
+    assert torch.equal(norms.cpu().isnan(), want_norms.isnan()) and torch.equal(norms.cpu().nan_to_num(0.0), want_norms.nan_to_num(0.0))
+    got, want = packed.cpu().numpy().reshape(7, -1), want_packed.reshape(7, -1)
+    codes = lambda rows: np.stack((rows & 15, rows >> 4), axis=-1)
+    for row in (1, 3, 5):
+        assert np.array_equal(codes(got[row]), np.where(codes(want[row]) == 15, 0, codes(want[row])))
+    for row in (0, 2, 4, 6):
+        assert np.array_equal(got[row], want[row])
+        alone, _ = gpu_quantize(dev, w[row : row + 1], perm, signs, bounds, block, inv, bits)
+        assert torch.equal(alone, packed.view(7, -1)[row])
