@@ -383,3 +383,37 @@ def test_infinities_and_nan_in_token_norms_and_bias(dev, library_switch, tile):
     finite = exact.isfinite()   # (the last product and the addition round once or twice)
     magnitude = (exact.abs() + 2 * o["bias"].double().abs())[finite]
     assert bool(((integers.double() - exact).abs()[finite] <= magnitude * 2.0 ** -23).all())
+
+
+@pytest.mark.parametrize("integers", [False, True])
+def test_a_captured_large_problem_computes_what_the_eager_call_does(dev, integers):
+    import orbitquant_packed_matmul as package
+    from orbitquant_amd import _lib
+
+    lib = _lib.load()
+    m, k, n = 2040, 4096, 4096
+    o = operands(dev, m, k, n, 4 if integers else 6, 4 if integers else 6, seed=5)
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    if integers:
+        assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) > 0
+        call = lambda: package.matmul_packed_w4a4_int8(o["codes"], o["packed"], o["norms"], o["rn"], table, table, activation_scale=0.05, weight_scale=0.04,
+                                                       out_features=n, in_features=k)
+    else:
+        assert lib.oq_packed_linear_workspace_bytes(m, n, k, 6, _lib.OQ_CODES_U8, 6) > lib.oq_packed_linear_least_workspace_bytes(m, n, k, 6, _lib.OQ_CODES_U8, 6)
+        call = lambda: multiply(o, m, k, n, 6, 6, torch.bfloat16)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for seed in range(4):
+        fresh = operands(dev, m, k, n, 4 if integers else 6, 4 if integers else 6, seed=10 + seed)
+        for name in ("codes", "norms"):
+            o[name].copy_(fresh[name])
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        assert torch.equal(replayed, call())
