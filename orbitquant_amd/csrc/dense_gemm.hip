@@ -13,10 +13,11 @@
 // operands are in registers: behind it the next stage has arrived (its copies were issued a quarter to a whole
 // K-step earlier) and this one is free for the copies of the K-step after.
 //
-// What bounds it: in bf16 the card's power (8192 x 8192 x 8192 in 775 us, 1.42 PFLOP/s, with the clock held near
-// 1.5 GHz; the packed GEMM, whose table lookups cost energy too, 865 us at 1.3 GHz), so a tile is chosen for few LDS
-// bytes per product: 256 x 256 over four wavefronts, each 128 x 128.  Copies issued in a burst instead of between
-// matrix instructions cost 834 us.  In int8 406 us, 2.7 POP/s.
+// What bounds it: at 8192 x 8192 x 8192 in bf16 (775 - 803 us, 1.37 - 1.42 PFLOP/s) the matrix cores are busy 85 % of
+// the launch's cycles and the clock, nominally 2.4 GHz, stands at 1.53; the packed GEMM (845 - 865 us) has them as busy
+// at 1.46 GHz, with four times the LDS instructions.  So a tile is chosen for few LDS bytes per product: 256 x 256 over
+// four wavefronts, each 128 x 128.  Copies issued in a burst instead of between matrix instructions cost 834 us.  In int8
+// 402 - 406 us, 2.7 POP/s, busy 82 % at 1.60 GHz.
 #include <math.h>
 
 #include "dense_gemm.h"
@@ -228,8 +229,8 @@ int launch_dense_tile(const DenseArgs &g, int tile, hipStream_t stream) {
   return launch_dense<MF, 2, 2>(g, stream);
 }
 
-// 0 .. 1: how far the chip's clock has come down over a launch of that many operations (its power limit, reached
-// over some hundred microseconds): none at 2e10, all of it from 1e12 on.
+// 0 .. 1: how far the chip's clock has come down over a launch of that many operations: none at 2e10, all of it from
+// 1e12 on (1.8 GHz at 3e11, 1.5 at 1e12, of nominally 2.4).
 double launch_warmth(double operations) {
   const double w = log(operations / 2.0e10) / log(50.0);
   return w < 0.0 ? 0.0 : w < 1.0 ? w : 1.0;
@@ -239,11 +240,11 @@ double launch_warmth(double operations) {
 
 // The best tile of this kernel for a problem and its time in microseconds, the passes into operand order included
 // (`pass_bytes`: what they read and write); -1 where the kernel cannot run.  A launch runs in rounds of 256 workgroups,
-// one to a CU (each part of the rows in rounds of its own), each with a fixed prologue and epilogue and a time per K-step of 128 operand bytes that grows with the
-// length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16 at 2e10 operations, 1.14 us from 1e12 on) and
-// by up to a quarter where the operands outgrow the 256 MB last-level cache; on top come the passes, the output's
-// way to memory and the launches.  Fitted to 5000 timings of single calls, 256 to 16384 in each dimension, all tiles:
-// nine in ten within 15 %; the tile it picks is 1 % behind the best one on average.
+// one to a CU (each part of the rows in rounds of its own), each with a fixed prologue and epilogue and a time per
+// K-step of 128 operand bytes that grows with the length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16
+// at 2e10 operations, 1.14 us from 1e12 on) and by up to a quarter where the operands outgrow the 256 MB last-level
+// cache; on top come the passes, the output's way to memory and the launches.  Fitted to 5000 timings of single calls, 256 to 16384 in each dimension, all tiles
+// (rms error 9 %); the tile it picks is 1 % behind the best one on average.
 int dense_choose_tile(int64_t M, int64_t N, int64_t K, int64_t rows_at_a_time, int mf, double pass_bytes, double *cost_out) {
   if (K % 64 != 0 || N % 8 != 0 || M > 0x7fff0000LL || N > 0x7fff0000LL || K > 0x0fffffffLL) return -1;
   static const int sizes[4][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 128}};
