@@ -182,11 +182,9 @@ int oq_debug_override(const char *name, const char *value);
  * rows computed with it as long as the call stays within 64 rows.  A problem with few output
  * tiles and many K-steps (some hundred tokens on a short-and-long matrix) is shared between
  * workgroups along K when the caller provides a workspace for the fp32 partial tiles, and a large
- * problem (some thousand tokens) is decoded once into the workspace and multiplied from there.  The
- * workspace can change the order in which a sum's terms are added, and with it the last bits: a shared
- * K is added in parts, and where the launch without a workspace shares K between the wavefronts of a
- * workgroup (128 x 96 tiles), it is that launch that adds in parts and the decoded problem that does
- * not.  Every other large problem gives the same bits with and without:
+ * problem (some thousand tokens) is decoded once into the workspace and multiplied from there.  A
+ * shared K is added in parts, so the last bits of such a result depend on the workspace; a decoded
+ * problem gives the same bits as without:
  *
  * workspace    NULL, or a device buffer of at least oq_packed_linear_workspace_bytes(...) bytes, 16-byte
  *              aligned, that this call may overwrite (calls on one stream are ordered and may share one).
@@ -233,9 +231,9 @@ uint64_t oq_packed_linear_least_workspace_bytes(int64_t M, int64_t N, int64_t K,
  *
  *   out[m,n] = (sum_k act_table[code[m,k]] * w_table[idx[n,k]]) * (s[m] * scale) * r_w[n] + bias[n]
  *
- * (matmul_packed_w4a4_int8, torch_binding.cpp:39-46.)  For the shapes that
+ * (matmul_packed_w4a4_int8, torch_binding.cpp:39-46.)  act_table and w_table: int8 [16].  For the shapes that
  * oq_packed_linear_int8_workspace_bytes gives a size for, with a workspace of at least that size; OQ_ERR_UNSUPPORTED
- * for the others (0), which oq_packed_linear is at least as fast on.
+ * for the others (0), which oq_packed_linear, with its workspace, is about as fast or faster on.
  */
 int oq_packed_linear_int8(const void *codes, const float *token_norms, float scale, const int8_t *act_table,
                           const uint8_t *packed_w, const uint16_t *row_norms, const int8_t *w_table, const void *bias,

@@ -136,7 +136,10 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
 // 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072 (3-bit) 333 -> 300 us,
 // 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise 5 % over the best
 // launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
-// the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).
+// the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).  Where that launch takes the
+// 128 x 96 tile it keeps the problem: four wavefronts that share K and add four partial sums leave a smaller error than
+// one running sum (2048 x 4096 x 14336 in fp32: 7.3e-8 of the result against 2.3e-7), and a workspace does not change
+// the bits of a result.
 static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr) {
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   double dense = 0.0;
@@ -144,6 +147,7 @@ static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byt
   if (cost_out != nullptr) *cost_out = dense;
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
+  if (choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes) == 4) return -1;
   const double share = byte_codes || 2.0 * k * (m + n) <= 268435456.0 ? 0.95 : 0.8;
   return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES) ? tile : -1;
 }

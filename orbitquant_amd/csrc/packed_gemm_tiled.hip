@@ -59,8 +59,8 @@ int launch_tiled_bits(const GemmArgs &g, int bits, int tile, hipStream_t stream)
 int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits);  // packed_gemm.hip
 
 // Tile of the decode-first GEMM, -1 where looking the weights up in every tile is as fast, or where that launch takes
-// the 128 x 96 tile: its four wavefronts share K and add up in another order, and this entry point gives the same sums
-// with and without a workspace.  Both sides pay for the activations' pass.  Asked for 10 %, the prices send 412 of 750
+// the 128 x 96 tile, for the reasons given at gemm_choose_dense: its sums are more exact, and the same with and without
+// a workspace.  Both sides pay for the activations' pass.  Asked for 10 %, the prices send 412 of 750
 // measured shapes to it, 12 of them to more than 3 % more time (rows of some hundred values); without the price of
 // values (gemm_price), 512 x 7488 with three bits took 73 us instead of 53 at 2 to 64 tokens.
 static int tiled_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool f16) {

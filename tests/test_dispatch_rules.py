@@ -37,7 +37,9 @@ def test_large_problems_are_decoded_first(lib, m, n, k, wbits, abits):
     (4971, 3704, 1088, 2, 4),      # 54, 77
     (2048, 3072, 12288, 3, 4),     # 155, 175
     (4608, 3072, 3072, 3, 3),      # 85, 86
-    (1024, 14336, 4096, 4, 4)])    # 95, 114
+    (1024, 14336, 4096, 4, 4),     # 95, 114
+    # its wavefronts share K, and leave a third of the error
+    (2048, 4096, 14336, 3, 4), (2048, 9216, 3072, 3, 4), (4608, 4096, 8192, 2, 4), (1341, 5248, 9216, 2, 4)])
 def test_the_packed_kernel_keeps_what_it_is_faster_on(lib, m, n, k, wbits, abits):
     assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, _lib.OQ_CODES_NIBBLE, abits) == 0
 

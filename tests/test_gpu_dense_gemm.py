@@ -122,32 +122,35 @@ def test_int8_activations_decoded_in_parts(dev, library_switch):
         assert torch.equal(got[rows], sums * (o["norms"][rows] * 0.01)[:, None] * o["rn"].float())
 
 
-@pytest.mark.parametrize("m,k,n,wbits,abits,shares_k", [
-    (2040, 4096, 4096, 6, 6, False), (4608, 3072, 12288, 3, 4, False),
-    (6564, 2560, 520, 8, 6, True), (1415, 2560, 2728, 8, 4, True)])   # without a workspace: 128 x 96 tiles, K shared inside
-def test_with_and_without_a_workspace_as_the_rules_choose(dev, m, k, n, wbits, abits, shares_k):
+@pytest.mark.parametrize("m,k,n,wbits,abits,decoded", [
+    (2040, 4096, 4096, 6, 6, True), (4608, 3072, 12288, 3, 4, True),
+    (6564, 2560, 520, 8, 6, False), (2048, 14336, 4096, 3, 4, False)])   # packed: 128 x 96 tiles, K shared inside
+def test_with_and_without_a_workspace_as_the_rules_choose(dev, m, k, n, wbits, abits, decoded):
     from orbitquant_amd import _lib, ops
 
     lib = _lib.load()
     o = operands(dev, m, k, n, wbits, abits, seed=m)
     fmt = _lib.OQ_CODES_U8 if abits > 4 else _lib.OQ_CODES_NIBBLE
-    assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, fmt, abits) == (-(-m // 32) + -(-n // 32)) * (k // 64) * 4096
-    with_workspace = multiply(o, m, k, n, wbits, abits, torch.float32)
+    asked = (-(-m // 32) + -(-n // 32)) * (k // 64) * 4096
+    assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, fmt, abits) == (asked if decoded else 0)
+    with_workspace, room = torch.empty(m, n, device=dev), torch.empty(asked, dtype=torch.uint8, device=dev)
     without = torch.empty_like(with_workspace)
-    rc = lib.oq_packed_linear(o["codes"].data_ptr(), fmt, o["norms"].data_ptr(), o["acents"].data_ptr(), abits, o["packed"].data_ptr(), wbits,
-                              o["rn"].data_ptr(), o["wcents"].data_ptr(), o["bias"].data_ptr(), _lib.OQ_F32, m, n, k, without.data_ptr(), _lib.OQ_F32,
-                              None, 0, torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    assert torch.equal(without, with_workspace) != shares_k
+    for out, workspace, size in ((with_workspace, room.data_ptr(), asked), (without, None, 0)):
+        rc = lib.oq_packed_linear(o["codes"].data_ptr(), fmt, o["norms"].data_ptr(), o["acents"].data_ptr(), abits, o["packed"].data_ptr(), wbits,
+                                  o["rn"].data_ptr(), o["wcents"].data_ptr(), o["bias"].data_ptr(), _lib.OQ_F32, m, n, k, out.data_ptr(), _lib.OQ_F32,
+                                  workspace, size, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+    assert torch.equal(without, with_workspace)
     index = ops.unpack_lowbit(o["packed"], wbits, n * k).view(n, k).long()
     codes = o["codes"].long() if abits > 4 else torch.stack((o["codes"] & 15, o["codes"] >> 4), dim=-1).view(m, k).long()
     a, w = o["acents"].bfloat16().double()[codes], o["wcents"].bfloat16().double()[index]   # the tables hold bf16
     factor = o["norms"].double()[:, None] * o["rn"].double()
     exact = (a @ w.T) * factor + o["bias"].double()
-    # K additions and four more operations in fp32, whatever their order
-    bound = ((a.abs() @ w.abs().T) * factor + o["bias"].double().abs()) * (k + 4) * 2.0 ** -24
-    for got in (with_workspace, without):
-        assert bool(((got.double() - exact).abs() <= bound).all())
+    # K additions and four more operations in fp32; a quarter of the additions where four wavefronts share K
+    bound = ((a.abs() @ w.abs().T) * factor + o["bias"].double().abs()) * ((k if decoded else k // 4 + 4) + 4) * 2.0 ** -24
+    assert bool(((with_workspace.double() - exact).abs() <= bound).all())
+    if not decoded:   # what the decode-first kernel would leave instead
+        assert float((with_workspace.double() - exact).norm() / exact.norm()) < 1e-7
 
 
 @pytest.mark.parametrize("tile", [0, 1, 2, 3])
