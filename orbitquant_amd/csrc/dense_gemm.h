@@ -20,7 +20,7 @@ int dense_gemm(int mf, const void *a, const void *w, const float *row_scale, flo
 // Rows of activation codes decoded at a time: all of them up to 512 MB of decoded values, above that parts of about
 // equal size, whole tiles each, multiplied one after the other with the weights decoded once.  (The second linear of a
 // video DiT's FFN, 32760 x 5120 x 13824, then asks for 0.6 GB instead of 1.05, in the same time: two parts of five full
-// rounds of workgroups.  At a quarter of the bound its parts would not fill their rounds.)
+// rounds of workgroups.  At half the bound it would be four parts of two and a half rounds, twelve instead of ten.)
 constexpr uint64_t kDecodedActivationBytes = 512ull << 20;
 
 inline int64_t dense_rows_at_a_time(int64_t M, int64_t K, int mf) {

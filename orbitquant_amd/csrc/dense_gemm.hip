@@ -243,8 +243,8 @@ double launch_warmth(double operations) {
 // one to a CU (each part of the rows in rounds of its own), each with a fixed prologue and epilogue and a time per
 // K-step of 128 operand bytes that grows with the length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16
 // at 2e10 operations, 1.14 us from 1e12 on) and by up to a quarter where the operands outgrow the 256 MB last-level
-// cache; on top come the passes, the output's way to memory and the launches.  Fitted to 5000 timings of single calls, 256 to 16384 in each dimension, all tiles
-// (rms error 9 %); the tile it picks is 1 % behind the best one on average.
+// cache; on top come the passes, the output's way to memory and the launches.  Fitted to 5000 timings of single calls,
+// 256 to 16384 in each dimension, all tiles (rms error 9 %); the tile it picks is 1 % behind the best one on average.
 int dense_choose_tile(int64_t M, int64_t N, int64_t K, int64_t rows_at_a_time, int mf, double pass_bytes, double *cost_out) {
   if (K % 64 != 0 || N % 8 != 0 || M > 0x7fff0000LL || N > 0x7fff0000LL || K > 0x0fffffffLL) return -1;
   static const int sizes[4][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 128}};

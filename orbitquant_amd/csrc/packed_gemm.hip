@@ -132,10 +132,9 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
 // kernel above looks every operand value up once per tile that uses it; decoding each once costs two passes over
 // memory, 2 bytes written and read again per value, and leaves the matrix cores alone with the multiplication.
 // That pays on large problems, sooner with one code per byte (eight lookups an operand instead of four) and with
-// weights of six and eight bits:
-// 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072 (3-bit) 333 -> 300 us,
-// 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise 5 % over the best
-// launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
+// weights of six and eight bits: 32760 x 13824 x 5120 with 6-bit activations 4368 -> 3419 us, 4608 x 12288 x 3072
+// (3-bit) 333 -> 300 us, 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise
+// 5 % over the best launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
 // the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).  Where that launch takes the
 // 128 x 96 tile it keeps the problem: four wavefronts that share K and add four partial sums leave a smaller error than
 // one running sum (2048 x 4096 x 14336 in fp32: 7.3e-8 of the result against 2.3e-7), and a workspace does not change
@@ -153,7 +152,7 @@ static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byt
 }
 
 // What a call on two codes a byte takes with the workspace it asks for: decoded first, shared between workgroups
-// along K, or the single launch.
+// along K (where the two prices differ, the lower one), or the single launch.
 double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits) {
   double dense = 0.0, split = 0.0;
   if (gemm_choose_dense(M, N, K, bits, false, &dense) >= 0) return dense;
