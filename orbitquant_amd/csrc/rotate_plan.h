@@ -7,16 +7,19 @@
 //     (b < RN(y * c)) == (t < y) for every y.  The kernel compares y with t and skips the multiply.
 //   * cells: the one-read bucketize table over the thresholds (256 uniform cells; cell c holds
 //     the number of thresholds in lower cells and the single threshold inside it).
-//   * gather entries: permutation and sign of every rotated slot merged into the LDS byte
-//     address the kernel reads its input from (16-bit inputs are staged twice, as x and as -x,
-//     so a slot with a negative sign simply points into the second copy; fp32 inputs are staged
-//     once and carry the sign in bit 31 of the entry).
+//   * gather entries: the permutation as the LDS byte address at which the kernel finds a rotated
+//     slot's input when it stages the row in 16-bit values (fp32 rows: twice as far from the start of
+//     the staging area).  The signs are applied while the row is staged, so they are kept by the
+//     position of the input, not of the slot: sign of slot i at position perm[i].  That needs a
+//     permutation that takes every position once; for one that does not (bijective == 0) the kernel
+//     stages the row as it is and applies the signs by slot, after the gather.
 // Layout of the blob (all offsets in bytes, the blob 16-byte aligned):
 //   0     PlanHeader (64 bytes)
 //   64    thresholds  float[256]   (+inf beyond levels - 1)
 //   1088  cells       uint2[256]   (x: threshold bits or +inf, y: count below)
-//   3136  gather16    uint32[K]
-//   3136 + 4K  gather32  uint32[K]
+//   3136  gather      uint32[K]
+//   3136 + 4K  signs by input position  uint16[K]   (0x8000: negative)
+//   3136 + 6K  signs by slot            uint16[K]
 #pragma once
 
 #include "oq_common.h"
@@ -40,7 +43,8 @@ struct PlanHeader {
   float cell_scale;      // cell(v) = sat_u8(v * cell_scale + cell_offset)
   float cell_offset;
   float inv_sqrt_block;  // the factor folded into the thresholds
-  uint32_t reserved[8];
+  uint32_t bijective;    // the permutation takes every position once
+  uint32_t reserved[7];
 };
 static_assert(sizeof(PlanHeader) == 64, "the header is 64 bytes");
 

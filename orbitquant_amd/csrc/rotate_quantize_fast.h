@@ -11,6 +11,7 @@
 //     lower / upper lanes of a pair by their bank masks (distances 4 and 8 lanes), an exclusive-or
 //     plus a DPP add inside quads, lane-group swaps of register pairs for 16 and 32 lanes;
 //   * permutation, sign, the 1/sqrt(block) factor and the bucketize table come from the plan;
+//     the signs are applied to the row as it is staged, four exclusive-ors for eight 16-bit values;
 //   * x / (s + eps) is four instructions: q = fma(x, rh, x * rl) with rh + rl = 1 / (s + eps) to
 //     twice the working precision is a faithful quotient, and one residual correction
 //     fma(fma(-q, d, x), rh, q) with rh the correctly rounded reciprocal rounds it correctly
@@ -68,10 +69,13 @@ struct FastArgs {
 // LDS: cells (2048) | thresholds (1024) | centroids (1024) | reduction slots (64) | staging
 constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then one flag per wavefront
 
-// staging: 4 bytes per value (fp32 once, 16-bit twice)
-__host__ __device__ inline size_t fast_lds_bytes(int64_t K) { return static_cast<size_t>(kStageAt) + 4u * static_cast<size_t>(K); }
-// ... and behind it, for a launch with an input map, the map's 16 KB window (value_map.h)
-inline size_t fast_lds_bytes_mapped(int64_t K) { return fast_lds_bytes(K) + static_cast<size_t>(kWideBytes); }
+// The row is staged once, in its own type; behind it, for a launch with an input map, the map's 16 KB window
+// (value_map.h).  Long rows are bound by how many wavefronts a CU holds, and that by LDS and registers: with a second,
+// negated copy of 16-bit rows and 177 registers for blocks of 4096, 4608 x 12288 took 108 us and 32760 x 13824 609 us;
+// with one copy and 122 registers 72 and 457 us.
+__host__ __device__ inline size_t fast_lds_bytes(int64_t K, int dtype) {
+  return static_cast<size_t>(kStageAt) + (dtype == OQ_F32 ? 4u : 2u) * static_cast<size_t>(K);
+}
 
 // ---- lane-exchange butterflies, eight values per call -------------------------------------------
 // y'[lane] = (lane & J) ? y[lane ^ J] - y[lane] : y[lane] + y[lane ^ J]
@@ -187,7 +191,7 @@ __device__ __forceinline__ void count_below(const uint2 (&ent)[kChunk], const fl
 // little-endian stream; the norm is stored as bf16.
 enum EmitMode { EMIT_NIBBLE = 0, EMIT_U8 = 1, EMIT_ANY = 2, EMIT_WEIGHT = 3 };
 
-// One row.  `smem`: fast_lds_bytes(K) bytes, 16-byte aligned.  All 64 * waves threads of the
+// One row.  `smem`: fast_lds_bytes(K, DT) bytes (and kWideBytes more if MAPPED), 16-byte aligned.  All 64 * waves threads of the
 // workgroup make the call.
 template <int DT, int LOG_H, int EMIT, bool MAPPED = false>
 __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsigned char *smem, const int64_t row,
@@ -203,7 +207,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   float *cent = reinterpret_cast<float *>(smem + kCentAt);
   float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..11] per-wavefront flags
   unsigned char *stage = smem + kStageAt;
-  const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset) + (DT == OQ_F32 ? K : 0);
+  const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset);
+  const uint16_t *signs_by_position = reinterpret_cast<const uint16_t *>(gather + K), *signs_by_slot = signs_by_position + K;
 
   // A plan built for another shape must not be walked.  No codes are written then, and the row's norm
   // is stored as NaN, so that the mismatch cannot pass for a result: every output computed from it is NaN.
@@ -217,6 +222,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     return;
   }
   const float cell_scale = hdr->cell_scale, cell_offset = hdr->cell_offset;
+  const bool bijective = hdr->bijective != 0u;  // (uniform: the signs go on while the row is staged)
 
   // tables: entry tid is requested now and stored to LDS after the row has been requested (loads
   // return in order); workgroups of fewer than 256 threads fetch the rest when they store.
@@ -231,13 +237,13 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // an input map's window goes to LDS first (every wavefront looks values up in it as it reads the row)
   const uint16_t *hot = nullptr;
   if constexpr (MAPPED) {
-    uint16_t *window = reinterpret_cast<uint16_t *>(smem + fast_lds_bytes(K));
+    uint16_t *window = reinterpret_cast<uint16_t *>(smem + fast_lds_bytes(K, DT));
     fill_map_window<kWideLog2>(window, a.map, kWideLoBf16, tid, waves * 64);
     hot = window;
     __syncthreads();
   }
 
-  // ---- phase A: stage the row (16-bit inputs as x and as -x), sum of squares -----------------
+  // ---- phase A: stage the row with its signs, sum of squares ----------------------------------
   // Virtual lane t of the documented [passes][256 lanes][8] order is lane t % 64 of group t / 64;
   // wavefront w owns the groups w, w + waves, ... with all their passes, and keeps four passes of
   // a group requested ahead of the one it is summing.  (Adding a lane's first pass to +0 is exact.)
@@ -248,16 +254,18 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   bool tiny32 = false;               // fp32: a nonzero value below 2^-80 was seen
   const uint32_t kMadMul = 0xfffefffeu, kMadAdd = 0x2eff2effu;
   const int lane_first = lane * kChunk;
-  constexpr int kBatch = 4;
+  constexpr int kBatch = DT == OQ_F32 ? 2 : 4;
 #pragma nounroll
   for (int grp = wave; grp < 4; grp += waves) {  // uniform over the wavefront
     float q = 0.0f;
-    uint4 raw_lo[kBatch], raw_hi[kBatch];  // a ring of requested chunks (fp32: both halves; 16-bit: raw_lo only)
+    uint4 raw_lo[kBatch], raw_hi[kBatch], raw_signs[kBatch];  // a ring of requested chunks (fp32: both halves; 16-bit: raw_lo only) and their signs
     auto request = [&](int b, int p) {
       const int i0 = p * kPass + grp * kLaneSpan + lane_first;  // chunks past the row: i0 >= Ki
       raw_lo[b] = make_uint4(0u, 0u, 0u, 0u);
       raw_hi[b] = raw_lo[b];
+      raw_signs[b] = raw_lo[b];
       if (i0 < Ki) {
+        raw_signs[b] = *reinterpret_cast<const uint4 *>(signs_by_position + static_cast<uint32_t>(i0));
         const uint4 *src = reinterpret_cast<const uint4 *>(xrow + static_cast<uint32_t>(i0) * kElem);
         raw_lo[b] = src[0];
         if constexpr (DT == OQ_F32) raw_hi[b] = src[1];
@@ -275,9 +283,15 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
           float f[kChunk];
           if constexpr (DT == OQ_F32) {
             if (i0 < Ki) {
+              uint4 lo = raw_lo[b], hi = raw_hi[b];
+              if (bijective) {
+                const uint4 sg = raw_signs[b];
+                lo.x ^= sg.x << 16; lo.y ^= sg.x & 0x80000000u; lo.z ^= sg.y << 16; lo.w ^= sg.y & 0x80000000u;
+                hi.x ^= sg.z << 16; hi.y ^= sg.z & 0x80000000u; hi.z ^= sg.w << 16; hi.w ^= sg.w & 0x80000000u;
+              }
               uint4 *dst = reinterpret_cast<uint4 *>(stage + 4 * i0);
-              dst[0] = raw_lo[b];
-              dst[1] = raw_hi[b];
+              dst[0] = lo;
+              dst[1] = hi;
             }
             const uint32_t w[kChunk] = {raw_lo[b].x, raw_lo[b].y, raw_lo[b].z, raw_lo[b].w,
                                         raw_hi[b].x, raw_hi[b].y, raw_hi[b].z, raw_hi[b].w};
@@ -298,9 +312,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
             }
             const uint32_t w[4] = {in.x, in.y, in.z, in.w};
             if (i0 < Ki) {
-              *reinterpret_cast<uint4 *>(stage + 2 * i0) = in;
-              *reinterpret_cast<uint4 *>(stage + 2 * (Ki + i0)) =
-                  make_uint4(w[0] ^ 0x80008000u, w[1] ^ 0x80008000u, w[2] ^ 0x80008000u, w[3] ^ 0x80008000u);
+              const uint4 sg = raw_signs[b];
+              *reinterpret_cast<uint4 *>(stage + 2 * i0) = bijective ? make_uint4(w[0] ^ sg.x, w[1] ^ sg.y, w[2] ^ sg.z, w[3] ^ sg.w) : in;
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -379,7 +392,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // The two rare modes (IEEE division for this row, binary search instead of the cell table) pass
   // through an empty asm statement inside the loop on purpose: as loop invariants the compiler
   // clones the whole loop per combination.
-  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (hdr->cells != 0 ? 0u : 2u));
+  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (hdr->cells != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
   const uint32_t neg1 = (lane & 1) ? 0x80000000u : 0u, neg2 = (lane & 2) ? 0x80000000u : 0u;
   // The gather entries of a step are requested one step ahead (past the last step: the row's
@@ -401,7 +414,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     const int unit_base = u * (G * kLaneSpan);
     uint32_t modes_now = row_modes;
     asm volatile("" : "+s"(modes_now));
-    const bool plain = (modes_now & 1u) != 0u, searched = (modes_now & 2u) != 0u;
+    const bool plain = (modes_now & 1u) != 0u, searched = (modes_now & 2u) != 0u, signs_left = (modes_now & 4u) != 0u;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
       // Lanes past the end of the row (last unit of a row with H < 512 only) walk the row's last
@@ -425,12 +438,17 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
 #pragma unroll
         for (int e = 0; e < kChunk; ++e) {  // the entries are LDS addresses (the workgroup's LDS starts at 0)
           if constexpr (DT == OQ_F32) {
-            const uint32_t raw = lds_read_u32(ent[e] & 0x7fffffffu);
-            xv[e] = __uint_as_float(raw ^ (ent[e] & 0x80000000u));
+            xv[e] = __uint_as_float(lds_read_u32(2u * ent[e] - plan::kStageAddress));
           } else {
             xv[e] = f16_bits_to_f32(lds_read_u16(ent[e]));
           }
         }
+      }
+      if (signs_left) {
+        const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(unit_base + j * kLaneSpan + lane_first, Ki - kChunk));
+        const uint32_t w[4] = {sg.x, sg.y, sg.z, sg.w};
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) xv[e] = __uint_as_float(__float_as_uint(xv[e]) ^ (((e & 1) != 0 ? w[e / 2] : w[e / 2] << 16) & 0x80000000u));
       }
       if constexpr (EMIT == EMIT_WEIGHT) {
 #pragma unroll
@@ -450,19 +468,25 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       if constexpr (H > 128) rq::swap_stage<16>(y[j]);
       if constexpr (H > 256) rq::swap_stage<32>(y[j]);
     }
-    // distances 512 and up: between the steps of the unit, in registers
+    // distances 512 and up: between the steps of the unit, in registers, one slot of every step at a time
+    if constexpr (G > 1) {
 #pragma unroll
-    for (int dist = 1; dist < G; dist <<= 1) {
+      for (int e = 0; e < kChunk; ++e) {
 #pragma unroll
-      for (int j = 0; j < G; ++j) {
-        if ((j & dist) == 0) {
+        for (int dist = 1; dist < G; dist <<= 1) {
 #pragma unroll
-          for (int e = 0; e < kChunk; ++e) {
-            const float l = y[j][e], r = y[j + dist][e];
-            y[j][e] = l + r;
-            y[j + dist][e] = l - r;
+          for (int j = 0; j < G; ++j) {
+            if ((j & dist) == 0) {
+              const float l = y[j][e], r = y[j + dist][e];
+              y[j][e] = l + r;
+              y[j + dist][e] = l - r;
+            }
           }
         }
+        // (as if used here: the compiler otherwise sinks the last butterflies to where a step's codes are made, and
+        // keeps both of their operands until then)
+#pragma unroll
+        for (int j = 0; j < G; ++j) asm volatile("" : "+v"(y[j][e]));
       }
     }
     // bucketize against the folded thresholds and emit

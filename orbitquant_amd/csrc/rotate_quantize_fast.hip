@@ -8,8 +8,9 @@ namespace {
 using namespace rqf;
 
 // ---- plan construction: once per layer, twice per converted weight ----------
-// Workgroup 0 makes the header and the tables, the others 256 gather entries each (all in one workgroup they were a
-// chain of K / 256 memory round trips: 10.2 -> 4.9 us for rows of some thousand values).
+// Workgroup 0 makes the header and the tables, the last one checks that the permutation is one, the others write 256
+// gather entries and signs each (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
+// for rows of some thousand values).
 // Floats in an order-preserving integer code, so that "the largest float t with RN(t * c) <= b" can
 // be found by bisection over all of them.
 __device__ __forceinline__ uint32_t float_to_ordered(float f) {
@@ -26,15 +27,38 @@ __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *p
   __shared__ float thr[256];
   __shared__ int bad;
   const int tid = threadIdx.x;
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ uint32_t taken[16384 / 32];  // (K is at most 16384)
+    for (int i = tid; i < 16384 / 32; i += 256) taken[i] = 0u;
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    bool twice = false;
+    for (int base = tid; base < K; base += 16 * 256) {
+      uint32_t p[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) p[j] = static_cast<uint32_t>(perm[min(base + j * 256, K - 1)]);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        if (base + j * 256 >= K) continue;
+        if (p[j] >= static_cast<uint32_t>(K)) twice = true;
+        else twice = (atomicOr(&taken[p[j] >> 5], 1u << (p[j] & 31u)) >> (p[j] & 31u) & 1u) != 0u || twice;
+      }
+    }
+    if (twice) bad = 1;
+    __syncthreads();
+    if (tid == 0) reinterpret_cast<plan::PlanHeader *>(out)->bijective = bad == 0 ? 1u : 0u;
+    return;
+  }
   if (blockIdx.x > 0) {
-    uint32_t *g16 = reinterpret_cast<uint32_t *>(out + plan::kGatherOffset);
-    uint32_t *g32 = g16 + K;
+    uint32_t *gather = reinterpret_cast<uint32_t *>(out + plan::kGatherOffset);
+    uint16_t *by_position = reinterpret_cast<uint16_t *>(gather + K), *by_slot = by_position + K;
     const int i = (static_cast<int>(blockIdx.x) - 1) * 256 + tid;
     if (i < K) {
       const uint32_t p = static_cast<uint32_t>(perm[i]);
-      const bool negative = signs[i] < 0;
-      g16[i] = plan::kStageAddress + 2u * p + (negative ? 2u * static_cast<uint32_t>(K) : 0u);
-      g32[i] = (plan::kStageAddress + 4u * p) | (negative ? 0x80000000u : 0u);
+      const uint16_t sign = signs[i] < 0 ? 0x8000u : 0u;
+      gather[i] = plan::kStageAddress + 2u * p;
+      by_slot[i] = sign;
+      if (p < static_cast<uint32_t>(K)) by_position[p] = sign;
     }
     return;
   }
@@ -86,22 +110,25 @@ __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *p
   }
   __syncthreads();
   if (tid == 0) {
-    plan::PlanHeader h{};
-    h.magic = plan::kMagic;
-    h.K = static_cast<uint32_t>(K);
-    h.block = static_cast<uint32_t>(block);
-    h.levels = static_cast<uint32_t>(levels);
-    h.cells = (usable && bad == 0) ? plan::kCells : 0;
-    h.cell_scale = scale;
-    h.cell_offset = offset;
-    h.inv_sqrt_block = c;
-    *reinterpret_cast<plan::PlanHeader *>(out) = h;
+    plan::PlanHeader *h = reinterpret_cast<plan::PlanHeader *>(out);  // (`bijective` is the last workgroup's to write)
+    h->magic = plan::kMagic;
+    h->K = static_cast<uint32_t>(K);
+    h->block = static_cast<uint32_t>(block);
+    h->levels = static_cast<uint32_t>(levels);
+    h->cells = (usable && bad == 0) ? plan::kCells : 0;
+    h->cell_scale = scale;
+    h->cell_offset = offset;
+    h->inv_sqrt_block = c;
+    for (uint32_t &r : h->reserved) r = 0u;
   }
 }
 
 // ---- the kernel ------------------------------------------------------------------------------------
+// Wavefronts per SIMD that the registers leave room for (an input map's lookups take more of them).
+constexpr int waves_per_simd(int log_h, bool mapped) { return log_h <= 9 ? (mapped ? 6 : 8) : log_h == 10 ? (mapped ? 6 : 7) : log_h == 11 ? 5 : 4; }
+
 template <int DT, int LOG_H, int EMIT, bool MAPPED>
-__global__ __launch_bounds__(512) void rotate_quantize_fast_kernel(FastArgs a) {
+__global__ __launch_bounds__(512, waves_per_simd(LOG_H, MAPPED)) void rotate_quantize_fast_kernel(FastArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   rotate_quantize_row_fast<DT, LOG_H, EMIT, MAPPED>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6);
 }
@@ -164,7 +191,7 @@ int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *bou
   if (!(inv_sqrt_block > 0.0f) || !(inv_sqrt_block < 3.0e38f))
     return fail(OQ_ERR_INVALID, "rotate_plan_build: inv_sqrt_block must be positive and finite");
   if ((reinterpret_cast<uintptr_t>(plan_out) & 15u) != 0) return fail(OQ_ERR_INVALID, "rotate_plan_build: the plan must be 16-byte aligned");
-  hipLaunchKernelGGL(rotate_plan_build_kernel, dim3(static_cast<unsigned>(1 + (K + 255) / 256)), dim3(256), 0, stream, perm, signs, boundaries, levels,
+  hipLaunchKernelGGL(rotate_plan_build_kernel, dim3(static_cast<unsigned>(2 + (K + 255) / 256)), dim3(256), 0, stream, perm, signs, boundaries, levels,
                      static_cast<int>(K), static_cast<int>(block), inv_sqrt_block, static_cast<unsigned char *>(plan_out));
   return check_launch("rotate_plan_build");
 }
@@ -230,15 +257,15 @@ static int launch_fast(FastArgs &a, int x_dtype, hipStream_t stream) {
   const int64_t unit = block > kLaneSpan ? block : kLaneSpan;
   a.units = static_cast<int>((K + unit - 1) / unit);
   // Wavefronts per row (each owns whole units): four, which is also what staging the row uses,
-  // eight for rows of sixteen units and more (measured: 5120 values in 5 units of 1024, 210 us on four
-  // against 237 us on five; 13824 values in 27 units of 512, 608 us on eight against 655 us on four).
+  // eight for rows of sixteen units and more (measured on 32760 rows: 5120 values in 5 units of 1024, 165 us on four
+  // against 201 us on five; 13824 values in 27 units of 512, 458 us on eight, 454 on four, and few rows are sooner done on eight).
   int waves = a.units >= 16 ? 8 : (a.units < 4 ? a.units : 4);
   if (a.M <= 16) waves = a.units < 8 ? a.units : 8;  // few rows: every unit its own wavefront
   if (const char *forced = debug_env(ENV_RQ_WAVES)) {
     const int w = atoi(forced);
     if (w >= 1 && w <= 8) waves = w < a.units ? w : a.units;
   }
-  const size_t smem = a.map != nullptr ? fast_lds_bytes_mapped(K) : fast_lds_bytes(K);
+  const size_t smem = fast_lds_bytes(K, x_dtype) + (a.map != nullptr ? kWideBytes : 0);
   if (smem > 160 * 1024) return -1;
   switch (x_dtype) {
     case OQ_F32: return launch_dtype<OQ_F32>(a, log_h, waves, smem, stream);

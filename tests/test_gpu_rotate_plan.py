@@ -105,6 +105,24 @@ def test_ragged_rows(dev, k, h):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,h", [(1536, 512), (6144, 2048)])
+def test_gather_that_repeats_positions(dev, dtype, k, h):
+    """A gather that is no permutation has no sign per input position: the kernel applies the signs by slot."""
+    from oracle import oracle_c
+
+    perm, signs, hh, inv, cents, bounds, t = constants(dev, k, h, 4)
+    perm = perm.copy()
+    perm[1::3] = perm[0::3][: len(perm[1::3])]
+    t["perm"] = torch.from_numpy(perm.astype(np.int32)).to(dev)
+    x = make_rows(21, k, dtype, seed=h)
+    (codes, _, norms), (codes_plain, _, _) = both_kernels(x.to(dev), t, h, inv, code_format="u8")
+    want_codes, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, signs, bounds, h, 1e-10, inv)
+    assert np.array_equal(codes.cpu().numpy(), want_codes)
+    assert np.array_equal(norms.cpu().numpy().view(np.int32), want_norms.view(np.int32))
+    assert torch.equal(codes, codes_plain)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_rows_that_take_the_ieee_division(dev, dtype):
     """Tiny values, tiny and huge norms, infinities and NaNs: the row-level test must send these
     rows to the plain division, and the result must still be the specification's."""
