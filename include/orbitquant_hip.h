@@ -265,7 +265,7 @@ int oq_packed_linear_group(const void *codes, int code_format, const float *toke
  * oq_packed_linear followed by an elementwise function of the 16-bit outputs given as a
  * table (output_map[bits of y] = bits of f(y), 65536 entries of the output dtype, 16-byte
  * aligned, on the device): out = f(linear) bit for bit, f(...) applied before the store
- * (tile kernels: in the epilogue; other kernels: by a small elementwise launch).  out_dtype
+ * (tile and streaming kernels: where they store; other kernels: by a small elementwise launch).  out_dtype
  * must be OQ_F16 or OQ_BF16.  No counterpart in the reference, like oq_rotate_quantize_mapped:
  * it is the activation that follows a linear, without its kernel.
  */
@@ -297,8 +297,8 @@ int oq_packed_linear_mapped(const void *codes, int code_format, const float *tok
  * `output_map` (NULL for none) is a table like `input_map`, of the OUTPUT dtype (16-bit
  * only), applied to every output value before it is stored: out = f(linear(x)) bit for bit
  * what f applied to the stored result of the plain call gives.  The tile kernels look the
- * values up in their epilogue; the small-M and shape-agnostic kernels are followed by a tiny
- * elementwise launch.  It is the cheaper place for the activation between two linears (a
+ * values up in their epilogue, the small-M kernels where they store; the shape-agnostic kernels are
+ * followed by a tiny elementwise launch.  It is the cheaper place for the activation between two linears (a
  * lookup per output value in a kernel that is waiting for its stores, instead of a lookup
  * per input value in the quantizer, which has no such slack).
  */

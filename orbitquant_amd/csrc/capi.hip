@@ -118,7 +118,7 @@ int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map,
                           const int8_t *signs, const float *boundaries, const float *act_cents, int levels,
                           int64_t block, float eps, float inv_sqrt_block, const uint8_t *packed_w, int bits,
                           const uint16_t *row_norms, const float *w_cents, const void *bias, int bias_dtype,
-                          int64_t N, void *out, int out_dtype, hipStream_t stream, bool *launched);
+                          int64_t N, void *out, int out_dtype, const uint16_t *out_map, hipStream_t stream, bool *launched);
 int generic_matmul_float(const void *x, int x_dtype, const float *token_scale, const uint8_t *packed_w,
                          int bits, const uint16_t *row_norms, const float *w_cents, const void *bias,
                          int bias_dtype, int64_t M, int64_t N, int64_t K, void *out, int out_dtype,
@@ -145,7 +145,7 @@ bool gemv_supported(int64_t M, int64_t K, int bits, int code_format, int a_level
 int gemv_dispatch(const void *codes, int code_format, const float *row_scale, const float *act_cents, int a_levels,
                   const uint8_t *w, int bits, const uint16_t *row_norms, const float *w_cents,
                   const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
-                  int out_dtype, hipStream_t stream);
+                  int out_dtype, const uint16_t *out_map, hipStream_t stream);
 int gemv_group_dispatch(const void *codes, int code_format, const float *row_scale, const float *act_cents, int a_levels,
                         int count, const uint8_t *const *w, const int *bits, const uint16_t *const *row_norms,
                         const float *const *w_cents, const void *const *bias, int bias_dtype, int64_t M,
@@ -246,7 +246,7 @@ int oq_quantize_weight(const void *w, int w_dtype, int64_t N, int64_t K, const v
   return rc < 0 ? fail(OQ_ERR_UNSUPPORTED, "quantize_weight: no kernel for block %lld", (long long)block) : rc;
 }
 
-// oq_packed_linear with an optional output map (applied by the tile kernels' epilogue, by a
+// oq_packed_linear with an optional output map (applied where the tile and the streaming kernels store, by a
 // small elementwise launch after the other kernels).
 static int packed_linear_impl(const void *codes, int code_format, const float *token_norms,
                               const float *act_centroids, int a_bits, const uint8_t *packed_w, int w_bits,
@@ -269,8 +269,8 @@ static int packed_linear_impl(const void *codes, int code_format, const float *t
   const bool tiled_out = gemm_output_ok(N, out);  // the tiled kernels store 16-byte row segments
   int rc;
   if (fast_ptrs && gemv_supported(M, K, w_bits, code_format, a_levels)) {
-    rc = gemv_dispatch(codes, code_format, token_norms, act_centroids, a_levels, packed_w, w_bits, row_norms, w_centroids,
-                       bias, bias_dtype, M, N, K, out, out_dtype, s);
+    return gemv_dispatch(codes, code_format, token_norms, act_centroids, a_levels, packed_w, w_bits, row_norms, w_centroids,
+                         bias, bias_dtype, M, N, K, out, out_dtype, out_map, s);
   } else if (fast_ptrs && tiled_out && gemm_supported(K, w_bits) && (code_format == OQ_CODES_NIBBLE || M > 16)) {
     return gemm_dispatch(code_format == OQ_CODES_NIBBLE ? 0 : 1, codes, token_norms, act_centroids, a_levels, packed_w, w_bits, row_norms, w_centroids,
                          bias, bias_dtype, M, N, K, out, out_dtype, out_map, workspace, workspace_bytes, s);
@@ -419,9 +419,8 @@ int oq_quantized_linear(const void *x, int x_dtype, const uint16_t *input_map, i
     bool launched = false;
     const int rc = token_linear_dispatch(x, x_dtype, input_map, K, perm, signs, boundaries, act_centroids, levels, block,
                                          eps, inv_sqrt_block, packed_w, w_bits, row_norms, w_centroids, bias,
-                                         bias_dtype, N, out, out_dtype, s, &launched);
-    if (rc != OQ_OK) return rc;
-    if (launched) return output_map == nullptr ? OQ_OK : apply_value_map(out, N, output_map, s);
+                                         bias_dtype, N, out, out_dtype, output_map, s, &launched);
+    if (rc != OQ_OK || launched) return rc;
   }
   if (codes_scratch == nullptr || norms_scratch == nullptr)
     return fail(OQ_ERR_INVALID, "quantized_linear: this shape takes two launches and needs the scratch buffers");

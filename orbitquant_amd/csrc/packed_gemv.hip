@@ -18,11 +18,11 @@ __global__ __launch_bounds__(64 * WAVES) void packed_gemv_kernel(const uint8_t *
                                                                  const float *act_cents, int64_t K, int64_t N,
                                                                  const uint16_t *row_norms, int M, int a_levels,
                                                                  const float *row_scale, const void *bias, int bias_dtype,
-                                                                 void *out, int out_dtype) {
+                                                                 void *out, int out_dtype, const uint16_t *out_map) {
   OQ_GEMV_TABLE_BLOCK(lds);
   GemvArgs g;
   g.a = a; g.row_scale = row_scale; g.act_cents = act_cents; g.a_levels = a_levels; g.w = w; g.row_norms = row_norms;
-  g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype; g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
+  g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype; g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype; g.out_map = out_map;
   packed_gemv_body<BYTES, BITS, R, WAVES, false, ASTAGE>(g, lds, blockIdx.x, [](auto) {});
 }
 
@@ -37,7 +37,7 @@ int launch(const GemvArgs &g, hipStream_t stream) {
     if (gemv_stages_activations(g.M, g.K)) kern = packed_gemv_kernel<BYTES, BITS, R, WAVES, true>;
   }
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), 0, stream, g.w, g.a, g.w_cents, g.act_cents, g.K,
-                     g.N, g.row_norms, g.M, g.a_levels, g.row_scale, g.bias, g.bias_dtype, g.out, g.out_dtype);
+                     g.N, g.row_norms, g.M, g.a_levels, g.row_scale, g.bias, g.bias_dtype, g.out, g.out_dtype, g.out_map);
   return check_launch("packed_gemv");
 }
 
@@ -83,11 +83,11 @@ bool gemv_supported(int64_t M, int64_t K, int bits, int code_format, int a_level
 int gemv_dispatch(const void *codes, int code_format, const float *row_scale, const float *act_cents, int a_levels,
                   const uint8_t *w, int bits, const uint16_t *row_norms, const float *w_cents,
                   const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
-                  int out_dtype, hipStream_t stream) {
+                  int out_dtype, const uint16_t *out_map, hipStream_t stream) {
   GemvArgs g{};
   g.a = static_cast<const uint8_t *>(codes); g.row_scale = row_scale; g.act_cents = act_cents; g.a_levels = a_levels;
   g.w = w; g.row_norms = row_norms; g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype;
-  g.M = static_cast<int>(M); g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
+  g.M = static_cast<int>(M); g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype; g.out_map = out_map;
   if (M > 16) return gemv_rows_dispatch(g, bits, code_format != OQ_CODES_NIBBLE, stream);
 #define OQ_GEMV_BITS(BYTES)                                                   \
   switch (bits) {                                                             \

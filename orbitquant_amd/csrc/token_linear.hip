@@ -31,7 +31,7 @@ int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map,
                           const int8_t *signs, const float *boundaries, const float *act_cents, int levels,
                           int64_t block, float eps, float inv_sqrt_block, const uint8_t *packed_w, int bits,
                           const uint16_t *row_norms, const float *w_cents, const void *bias, int bias_dtype,
-                          int64_t N, void *out, int out_dtype, hipStream_t stream, bool *launched) {
+                          int64_t N, void *out, int out_dtype, const uint16_t *out_map, hipStream_t stream, bool *launched) {
   *launched = false;
   rq::RqArgs q;
   bool vec = false;
@@ -48,7 +48,7 @@ int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map,
   if (static_cast<size_t>(gemv::kGemvTableBytes) + dynamic > kLdsPerWorkgroup) return OQ_OK;  // the caller takes two launches
   gemv::GemvArgs g{};
   g.act_cents = act_cents; g.a_levels = levels; g.w = packed_w; g.row_norms = row_norms; g.w_cents = w_cents;
-  g.bias = bias; g.bias_dtype = bias_dtype; g.M = 1; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
+  g.bias = bias; g.bias_dtype = bias_dtype; g.M = 1; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype; g.out_map = out_map;
   *launched = true;
   switch (bits) {
     case 2: return token_linear_launch_w2(q, g, x_dtype, rq_bytes, stream);
