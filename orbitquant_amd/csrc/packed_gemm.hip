@@ -9,7 +9,7 @@ namespace oq {
 int gemm_launch_bytes(const GemmArgs &g, int bits, int tile, hipStream_t stream);  // packed_gemm_bytes.hip
 
 // Tile choice by a small cost model.  A launch runs in rounds of as many workgroups as fit on
-// the chip at once (256; 512 for the 128x128 tile, which fits two to a CU) plus one partial
+// the chip at once (256; 512 for the 128x128 and 64x64 tiles, which fit two to a CU) plus one partial
 // round; a workgroup costs a fixed prologue + epilogue and a time per K-step of 64.  The
 // constants are microseconds measured on an MI355X: the "busy" set for launches long enough
 // to run at sustained clocks with every CU occupied, the other for short launches; weight
@@ -21,6 +21,7 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
   const char *force = debug_env(ENV_GEMM_TILE);
   if (force != nullptr && force[0] >= '0' && force[0] <= '3') return force[0] - '0';
   if (force != nullptr && force[0] == '4' && can_split) return 4;
+  if (force != nullptr && force[0] == '5' && K >= 256) return 5;
   struct Shape { int tm, tn; double fixed, step_short, step_busy, other_bits, bytes; };
   static const Shape shapes[4] = {{128, 128, 4.5, 0.8, 1.19, 1.28, 1.20}, {128, 256, 5.5, 1.0, 1.0, 1.34, 1.07},
                                   {256, 256, 7.0, 1.5, 1.68, 1.13, 1.10}, {256, 192, 6.0, 1.15, 1.24, 1.30, 1.23}};
@@ -54,6 +55,20 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
       best_cost = cost;
     }
   }
+  if (K >= 256 && bits <= 4) {  // (a quarter of the K-steps, more or less one, for each wavefront)
+    // 64x64 tiles, shared along K the same way: few tokens or few rows, which leave the chip empty on larger tiles.  Twice
+    // the lookups per product, so only where the tiles fit about one round: 256 x 1152 x 1152 12.4 -> 7.0 us, 128 x 4096 x
+    // 4096 19.3 -> 13.1 us, 77 x 8192 x 8192 25.9 -> 23.5 us, but 333 x 14336 x 4096 54 us on 128x96 and 65 on these.  Of
+    // 510 random shapes (9 to 4096 tokens; both code formats and fp16 values) 290 take it; over all of them the choice
+    // is 0.4 % behind the best tile on average, the geometric mean of time against the other tiles 0.85, 0.84 and 0.71.
+    const int64_t small = ((M + 63) / 64) * ((N + 63) / 64), full = small / 512, rest = small % 512;
+    const double width = (bits == 4 ? 1.0 : 1.2) * (byte_codes ? 1.2 : 1.0), quarter = static_cast<double>((K / 64 + 3) / 4);
+    const double small_cost = static_cast<double>(full) * (4.5 + quarter * 1.3 * width) + (rest > 0 ? 4.5 + quarter * (rest <= 256 ? 0.6 : 1.3) * width : 0.0);
+    if (small_cost < best_cost) {
+      best = 5;
+      best_cost = small_cost;
+    }
+  }
   if (cost_out != nullptr) *cost_out = best_cost;
   return best;
 }
@@ -65,19 +80,19 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
 // in operand order with the pass that puts them there), a factor for each weight width, the output's way to memory
 // (rms errors of 10, 8 and 13 %).
 double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form) {
-  struct Times { double step[5], out_mb, launches, bits2, bits3, bits6, bits8; };
-  static const Times forms[3] = {{{0.81, 0.85, 1.39, 1.09, 1.12}, 0.20, 0.5, 1.09, 1.11, 1.69, 1.58},
-                                 {{1.12, 1.10, 1.72, 1.40, 1.40}, 0.18, 2.2, 1.06, 1.08, 1.56, 1.50},
-                                 {{0.94, 1.05, 2.03, 1.32, 1.35}, 0.19, 5.5, 0.95, 0.96, 1.88, 1.74}};
-  static const struct { int tm, tn, capacity; double fixed; } tiles[5] = {
-      {128, 128, 512, 4.5}, {128, 256, 256, 5.5}, {256, 256, 256, 7.0}, {256, 192, 256, 6.0}, {128, 96, 256, 7.5}};
+  struct Times { double step[6], out_mb, launches, bits2, bits3, bits6, bits8; };
+  static const Times forms[3] = {{{0.81, 0.85, 1.39, 1.09, 1.12, 1.10}, 0.20, 0.5, 1.09, 1.11, 1.69, 1.58},
+                                 {{1.12, 1.10, 1.72, 1.40, 1.40, 1.30}, 0.18, 2.2, 1.06, 1.08, 1.56, 1.50},
+                                 {{0.94, 1.05, 2.03, 1.32, 1.35, 1.15}, 0.19, 5.5, 0.95, 0.96, 1.88, 1.74}};
+  static const struct { int tm, tn, capacity; double fixed; } tiles[6] = {
+      {128, 128, 512, 4.5}, {128, 256, 256, 5.5}, {256, 256, 256, 7.0}, {256, 192, 256, 6.0}, {128, 96, 256, 7.5}, {64, 64, 512, 4.5}};
   const Times &f = forms[form];
   const int tile = choose_tile_with_cost(M, N, K, bits, nullptr, form == PRICE_BYTES);
   const auto &sh = tiles[tile];
   const double width = bits == 2 ? f.bits2 : bits == 3 ? f.bits3 : bits == 6 ? f.bits6 : bits == 8 ? f.bits8 : 1.0;
-  const double steps = static_cast<double>(K / 64) / (tile == 4 ? 4.0 : 1.0), step = f.step[tile] * width;
+  const double steps = static_cast<double>(K / 64) / (tile >= 4 ? 4.0 : 1.0), step = f.step[tile] * width;
   const int64_t count = ((M + sh.tm - 1) / sh.tm) * ((N + sh.tn - 1) / sh.tn), rest = count % sh.capacity;
-  const double rest_step = tile == 0 && rest <= 256 ? 0.55 * step : step;  // (alone on its CU)
+  const double rest_step = sh.capacity == 512 && rest <= 256 ? (tile == 0 ? 0.55 : 0.5) * step : step;  // (alone on its CU)
   return static_cast<double>(count / sh.capacity) * (sh.fixed + steps * step) + (rest > 0 ? sh.fixed + steps * rest_step : 0.0) +
          2.0 * static_cast<double>(M) * static_cast<double>(N) / 1.0e6 * f.out_mb + f.launches;
 }
@@ -96,7 +111,8 @@ int apply_value_map(void *out, int64_t count, const uint16_t *table, hipStream_t
 // none), chosen with the cost model above plus the second launch (3 us and the partial tiles, written and
 // read back, at 3 TB/s):
 // every part keeps at least sixteen K-steps, the partial tiles stay within 64 MB, and the split has to
-// promise 15 % over the best single launch.  OQ_GEMM_WG_SPLIT overrides (1 = never).
+// promise 15 % over the best single launch (5 % over 64x64 tiles, whose price is the better known: 128 x 4096 x 14336).
+// OQ_GEMM_WG_SPLIT overrides (1 = never).
 // `cost_out`: the time of the split launch, if it is one.
 int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_out = nullptr) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = K / 64;
@@ -108,10 +124,10 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
   }
   if (debug_env(ENV_GEMM_TILE) != nullptr) return 1;  // a forced tile is a forced single launch
   double single = 0.0;
-  choose_tile_with_cost(M, N, K, bits, &single);
+  const int tile = choose_tile_with_cost(M, N, K, bits, &single);
   const double width = bits == 4 ? 1.0 : 1.28;
   int best = 1;
-  double best_cost = 0.85 * single;
+  double best_cost = (tile == 5 ? 0.95 : 0.85) * single;
   for (int s = 2; s <= 8; ++s) {
     if (!allowed(s)) continue;
     const int64_t groups = tiles * s;
@@ -136,7 +152,7 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
 // (3-bit) 333 -> 300 us, 4608 x 3072 x 3072 even (85 us), 2048 x 3072 x 12288 (3-bit) 155 -> 175 us.  It has to promise
 // 5 % over the best launch without it; with two codes a byte 20 % where the decoded operands outgrow the 256 MB last-level cache, which
 // the codes, a quarter of their size, do not (6144 x 4096 x 16384, 3-bit: 711 -> 998 us).  Where that launch takes the
-// 128 x 96 tile it keeps the problem: four wavefronts that share K and add four partial sums leave a smaller error than
+// 128 x 96 or the 64 x 64 tile it keeps the problem: four wavefronts that share K and add four partial sums leave a smaller error than
 // one running sum (2048 x 4096 x 14336 in fp32: 7.3e-8 of the result against 2.3e-7), and a workspace does not change
 // the bits of a result.
 static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr) {
@@ -146,7 +162,7 @@ static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byt
   if (cost_out != nullptr) *cost_out = dense;
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
   if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
-  if (choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes) == 4) return -1;
+  if (choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes) >= 4) return -1;
   const double share = byte_codes || 2.0 * k * (m + n) <= 268435456.0 ? 0.95 : 0.8;
   return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES) ? tile : -1;
 }

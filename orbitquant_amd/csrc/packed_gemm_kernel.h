@@ -91,13 +91,14 @@ static_assert(kEpiLdsBytes <= kTableBytes, "the epilogue reuses the table block"
 //   KSPLIT = 4: all four work on the SAME [32 FM x 32 FN] output tile, each over a quarter of K
 //               (for short-and-wide problems whose output has too few tiles to fill the chip);
 //               the partial tiles are then summed through LDS in a fixed order, each wavefront
-//               ending up with one 32-row slice of the tile, which it scales and stores.  FM = 4.
+//               ending up with a quarter of the tile (FM = 4: one 32-row slice; FM = 2: half of one),
+//               which it scales and stores.
 // NBUF = K-steps of packed operands held in registers (NBUF-1 of them in flight from memory).
 template <int AM, int BITS, int FM, int FN, int KSPLIT = 1, int NBUF = (FM * FN >= 12 ? 2 : 3)>
 __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, const float *act_cents, const uint8_t *a_codes,
                                                           const uint8_t *w_packed, const uint16_t *map_table, int K32, int M32,
                                                           int N32, int levels_splits, GemmArgs rest) {
-  static_assert(KSPLIT == 1 || (KSPLIT == 4 && FM == 4), "K split: four wavefronts, four row slices");
+  static_assert(KSPLIT == 1 || (KSPLIT == 4 && (FM == 4 || (FM == 2 && FN == 2))), "K split: four wavefronts, a quarter of the tile each");
   // What the first loads need comes as leading scalar arguments: the first fourteen dwords of a kernel's
   // arguments are handed over in scalar registers when a wavefront starts (the build asks for that with
   // -mllvm -amdgpu-kernarg-preload-count=16), so centroids and packed operands are requested without
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   // packed operands of NBUF consecutive K-steps
   uint4 pa[NBUF][FM][kAVec];
   uint32_t pw[NBUF][FN][BITS];
-  int steps = static_cast<int>(g.K / 64) / KSPLIT;  // K-steps of this wavefront
+  int steps = static_cast<int>(g.K / 64);  // K-steps of this wavefront
   if constexpr (KSPLIT == 1 && (AM == A_NIBBLE || AM == A_U8)) {
     if (g.k_splits > 1) {  // this workgroup's share of the K-steps
       const int z = blockIdx.y;
@@ -236,11 +237,13 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
       for (int j = 0; j < FN; ++j) wp[j] += static_cast<int64_t>(first) * (8 * BITS);
     }
   }
-  if constexpr (KSPLIT > 1) {
+  if constexpr (KSPLIT > 1) {  // (at least one step each: the launcher asks for K >= 256)
+    const int all = steps, w = __builtin_amdgcn_readfirstlane(wave), first = all * w / KSPLIT;
+    steps = all * (w + 1) / KSPLIT - first;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) ap[i] += static_cast<int64_t>(wave) * steps * kAStep;  // (A_STAGED: every ap[i] is the same base)
+    for (int i = 0; i < FM; ++i) ap[i] += static_cast<int64_t>(first) * kAStep;  // (A_STAGED: every ap[i] is the same base)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) wp[j] += static_cast<int64_t>(wave) * steps * (8 * BITS);
+    for (int j = 0; j < FN; ++j) wp[j] += static_cast<int64_t>(first) * (8 * BITS);
   }
   // operand `e` (A row-tile e < FM, else weight column-tile e-FM) of K-step ks into buffer B
   auto fetch_one = [&](auto buf, int e, int ks) {
@@ -518,72 +521,105 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
                           reinterpret_cast<unsigned char *>(lds), out_map, 64 * FM,
                           window_ahead ? reinterpret_cast<const uint16_t *>(map_window) : nullptr);
   } else {
-    // Reduce-scatter over the wavefronts in four rounds, one per row slice: in round s every wavefront parks
-    // slice s of its partial tile in LDS (slot = its own number) and wavefront s adds the other three to its
-    // own, in the order s-1, s-2, s-3 (mod 4).  The accumulator slices are registers, so which one is sent or
-    // summed has to be a compile-time index: this way it is the round's number, the same instructions for all
-    // four wavefronts (a scheme in which each wavefront sends a different slice per round needs four copies
-    // of every round, each fetched by one wavefront alone, and measured 0.5 us slower a launch).  Every barrier
-    // (and the epilogue, which has one of its own) is reached by all four in the same place.
-    // Slot of wavefront v: [FN tiles][4 runs][64 lanes] of float4.
+    // FM = 2: each wavefront parks all four of its 32 x 32 tiles, one slot of 4 KB each in the 64 KB of the tables, and
+    // adds up the four copies of one, its own first and the others in the order of the rounds below.
     float4 *slots = reinterpret_cast<float4 *>(lds);
-    f32x16 slice[1][FN];
     EpiFactors<1> mine;
     mine.rn = epi.rn;
     mine.bv = epi.bv;
     mine.sc[0] = 1.0f;
+    if constexpr (FM == 2) {
+      static_assert(kTableBytes >= 16 * 4096, "sixteen parked tiles");
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+      for (int t = 0; t < 4; ++t) {
+        const f32x16 part = acc[t >> 1][t & 1];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) slice[0][j][e] = 0.0f;
-    auto round = [&](auto st) __attribute__((always_inline)) {
-      constexpr int S = decltype(st)::value;
-      if (wave != S) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const f32x16 t = acc[S][j];  // whole-tile copies keep the accumulators in registers
-#pragma unroll
-          for (int a4 = 0; a4 < 4; ++a4)
-            slots[((wave * FN + j) * 4 + a4) * 64 + lane] = make_float4(t[4 * a4 + 0], t[4 * a4 + 1], t[4 * a4 + 2], t[4 * a4 + 3]);
-        }
+        for (int a4 = 0; a4 < 4; ++a4)
+          slots[((wave * 4 + t) * 4 + a4) * 64 + lane] = make_float4(part[4 * a4 + 0], part[4 * a4 + 1], part[4 * a4 + 2], part[4 * a4 + 3]);
       }
       __syncthreads();
-      if (wave == S) {
-        mine.sc[0] = epi.sc[S];
-        // the twelve reads of a tile are issued before its first sum (one LDS round trip a tile, not one a read)
+      f32x16 sum[1][1];
+      float4 part[4][4];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          float4 part[3][4];
+      for (int d = 0; d < 4; ++d)
 #pragma unroll
-          for (int d = 1; d < 4; ++d)
+        for (int a4 = 0; a4 < 4; ++a4) part[d][a4] = slots[(((((wave + 4 - d) & 3) * 4 + wave) * 4 + a4) * 64) + lane];
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        sum[0][0][4 * a4 + 0] = ((part[0][a4].x + part[1][a4].x) + part[2][a4].x) + part[3][a4].x;
+        sum[0][0][4 * a4 + 1] = ((part[0][a4].y + part[1][a4].y) + part[2][a4].y) + part[3][a4].y;
+        sum[0][0][4 * a4 + 2] = ((part[0][a4].z + part[1][a4].z) + part[2][a4].z) + part[3][a4].z;
+        sum[0][0][4 * a4 + 3] = ((part[0][a4].w + part[1][a4].w) + part[2][a4].w) + part[3][a4].w;
+      }
+      mine.sc[0] = wave < 2 ? epi.sc[0] : epi.sc[1];
+      __syncthreads();  // the slots are read: the epilogue takes the block
+      gemm_epilogue<1, 1>(sum, static_cast<int64_t>(pid_m) * TM, static_cast<int64_t>(pid_n) * TN, 32 * (wave >> 1), 32 * (wave & 1), TN, tid, g.M,
+                          g.N, g.row_scale, g.row_norms, g.bias, g.bias_dtype, mine, g.out, g.out_dtype,
+                          reinterpret_cast<unsigned char *>(lds), g.out_map, TM,
+                          window_ahead ? reinterpret_cast<const uint16_t *>(map_window) : nullptr);
+    } else {
+      // Reduce-scatter over the wavefronts in four rounds, one per row slice: in round s every wavefront parks
+      // slice s of its partial tile in LDS (slot = its own number) and wavefront s adds the other three to its
+      // own, in the order s-1, s-2, s-3 (mod 4).  The accumulator slices are registers, so which one is sent or
+      // summed has to be a compile-time index: this way it is the round's number, the same instructions for all
+      // four wavefronts (a scheme in which each wavefront sends a different slice per round needs four copies
+      // of every round, each fetched by one wavefront alone, and measured 0.5 us slower a launch).  Every barrier
+      // (and the epilogue, which has one of its own) is reached by all four in the same place.
+      // Slot of wavefront v: [FN tiles][4 runs][64 lanes] of float4.
+      f32x16 slice[1][FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) slice[0][j][e] = 0.0f;
+      auto round = [&](auto st) __attribute__((always_inline)) {
+        constexpr int S = decltype(st)::value;
+        if (wave != S) {
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const f32x16 t = acc[S][j];  // whole-tile copies keep the accumulators in registers
 #pragma unroll
             for (int a4 = 0; a4 < 4; ++a4)
-              part[d - 1][a4] = slots[((((S + 4 - d) & 3) * FN + j) * 4 + a4) * 64 + lane];
-          __builtin_amdgcn_sched_barrier(0);
-          f32x16 sum = acc[S][j];
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-#pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-              sum[4 * a4 + 0] += part[d][a4].x;
-              sum[4 * a4 + 1] += part[d][a4].y;
-              sum[4 * a4 + 2] += part[d][a4].z;
-              sum[4 * a4 + 3] += part[d][a4].w;
-            }
-          slice[0][j] = sum;
-          __builtin_amdgcn_sched_barrier(0);
+              slots[((wave * FN + j) * 4 + a4) * 64 + lane] = make_float4(t[4 * a4 + 0], t[4 * a4 + 1], t[4 * a4 + 2], t[4 * a4 + 3]);
+          }
         }
-      }
-      if (S < 3) __syncthreads();  // the slots are written again by the next round
-    };
-    round(std::integral_constant<int, 0>{});
-    round(std::integral_constant<int, 1>{});
-    round(std::integral_constant<int, 2>{});
-    round(std::integral_constant<int, 3>{});
-    gemm_epilogue<1, FN>(slice, static_cast<int64_t>(pid_m) * TM, static_cast<int64_t>(pid_n) * TN, 32 * wave, 0, TN, tid, g.M,
-                         g.N, g.row_scale, g.row_norms, g.bias, g.bias_dtype, mine, g.out, g.out_dtype,
-                         reinterpret_cast<unsigned char *>(lds), g.out_map, TM,
-                         window_ahead ? reinterpret_cast<const uint16_t *>(map_window) : nullptr);
+        __syncthreads();
+        if (wave == S) {
+          mine.sc[0] = epi.sc[S];
+          // the twelve reads of a tile are issued before its first sum (one LDS round trip a tile, not one a read)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            float4 part[3][4];
+#pragma unroll
+            for (int d = 1; d < 4; ++d)
+#pragma unroll
+              for (int a4 = 0; a4 < 4; ++a4)
+                part[d - 1][a4] = slots[((((S + 4 - d) & 3) * FN + j) * 4 + a4) * 64 + lane];
+            __builtin_amdgcn_sched_barrier(0);
+            f32x16 sum = acc[S][j];
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+              for (int a4 = 0; a4 < 4; ++a4) {
+                sum[4 * a4 + 0] += part[d][a4].x;
+                sum[4 * a4 + 1] += part[d][a4].y;
+                sum[4 * a4 + 2] += part[d][a4].z;
+                sum[4 * a4 + 3] += part[d][a4].w;
+              }
+            slice[0][j] = sum;
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if (S < 3) __syncthreads();  // the slots are written again by the next round
+      };
+      round(std::integral_constant<int, 0>{});
+      round(std::integral_constant<int, 1>{});
+      round(std::integral_constant<int, 2>{});
+      round(std::integral_constant<int, 3>{});
+      gemm_epilogue<1, FN>(slice, static_cast<int64_t>(pid_m) * TM, static_cast<int64_t>(pid_n) * TN, 32 * wave, 0, TN, tid, g.M,
+                           g.N, g.row_scale, g.row_norms, g.bias, g.bias_dtype, mine, g.out, g.out_dtype,
+                           reinterpret_cast<unsigned char *>(lds), g.out_map, TM,
+                           window_ahead ? reinterpret_cast<const uint16_t *>(map_window) : nullptr);
+    }
   }
 #ifdef OQ_GEMM_STAMPS
   OQ_STAMP(5);  // epilogue issued
@@ -630,6 +666,7 @@ int launch_cfg(GemmArgs g, hipStream_t stream) {
 
 template <int AM, int BITS>
 int launch_bits(const GemmArgs &g, int tile, hipStream_t stream) {
+  if (tile == 5) return launch_cfg<AM, BITS, 2, 2, 4>(g, stream);
   if (tile == 4) return launch_cfg<AM, BITS, 4, 3, 4>(g, stream);
   if (tile == 3) return launch_cfg<AM, BITS, 4, 3>(g, stream);
   if constexpr (AM == A_NIBBLE) {

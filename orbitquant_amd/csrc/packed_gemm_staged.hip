@@ -21,6 +21,7 @@ int gemm_staged_dispatch(const void *x, const float *token_scale, const uint8_t 
   const int tile = gemm_choose_tile(M, N, K, bits);
   auto go = [&](auto bits_c) {
     constexpr int BITS = decltype(bits_c)::value;
+    if (tile == 5) return launch_cfg<A_STAGED, BITS, 2, 2, 4>(g, stream);
     if (tile == 4) return launch_cfg<A_STAGED, BITS, 4, 3, 4>(g, stream);
     if (tile == 3 || tile == 2) return launch_cfg<A_STAGED, BITS, 4, 3>(g, stream);
     if (tile == 1) return launch_cfg<A_STAGED, BITS, 2, 4>(g, stream);

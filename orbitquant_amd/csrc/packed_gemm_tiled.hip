@@ -36,6 +36,7 @@ __global__ __launch_bounds__(256) void tile_activations_kernel(const uint16_t *x
 
 template <int AM, int BITS>
 int launch_tiled(const GemmArgs &g, int tile, hipStream_t stream) {
+  if (tile == 5) return launch_cfg<AM, BITS, 2, 2, 4>(g, stream);
   if (tile == 4) return launch_cfg<AM, BITS, 4, 3, 4>(g, stream);
   if (tile == 3) return launch_cfg<AM, BITS, 4, 3>(g, stream);
   if (tile == 1 || tile == 2) return launch_cfg<AM, BITS, 2, 4>(g, stream);
@@ -59,7 +60,7 @@ int launch_tiled_bits(const GemmArgs &g, int bits, int tile, hipStream_t stream)
 int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits);  // packed_gemm.hip
 
 // Tile of the decode-first GEMM, -1 where looking the weights up in every tile is as fast, or where that launch takes
-// the 128 x 96 tile, for the reasons given at gemm_choose_dense: its sums are more exact, and the same with and without
+// the 128 x 96 or the 64 x 64 tile, for the reasons given at gemm_choose_dense: its sums are more exact, and the same with and without
 // a workspace.  Both sides pay for the activations' pass.  Asked for 10 %, the prices send 412 of 750
 // measured shapes to it, 12 of them to more than 3 % more time (rows of some hundred values); without the price of
 // values (gemm_price), 512 x 7488 with three bits took 73 us instead of 53 at 2 to 64 tokens.
@@ -68,7 +69,7 @@ static int tiled_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool f1
   const double passes = static_cast<double>(K) * (static_cast<double>(N) * (2.0 + bits / 8.0) + static_cast<double>(M) * 4.0);
   const int tile = dense_choose_tile(M, N, K, M, f16 ? MF_F16 : MF_BF16, passes, &dense);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
-  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_tile(M, N, K, bits) == 4) return -1;
+  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_tile(M, N, K, bits) >= 4) return -1;
   return dense < 0.9 * gemm_price(M, N, K, bits, PRICE_VALUES) ? tile : -1;
 }
 

@@ -355,6 +355,23 @@ def test_packed_linear_k_split_kernel(dev, m, n, k, wbits, library_switch):
     assert torch.equal(got, again)  # fixed summation order: bitwise reproducible
 
 
+@pytest.mark.parametrize(("m", "n", "k", "wbits", "abits"), [
+    (65, 72, 256, 4, 4), (64, 64, 320, 4, 4), (130, 136, 1152, 3, 4), (17, 8, 832, 2, 3), (300, 200, 1472, 4, 6), (129, 264, 2304, 6, 8)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_packed_linear_small_tiles_share_k(dev, m, n, k, wbits, abits, out_dtype, library_switch):
+    """64 x 64 tiles, K shared by the four wavefronts in parts that differ by a step where it has to be."""
+    library_switch("OQ_GEMM_TILE", "5")
+    rng = np.random.default_rng(m + n + k)
+    layer = make_layer(rng, n, k, wbits, abits)
+    _, x32 = make_x(rng, m, k, torch.bfloat16)
+    x32[2] = 0
+    codes, s = oracle_c.rotate_quantize(x32, layer["perm"], layer["signs"], layer["ba"], layer["block"], 1e-10, layer["inv"])
+    fmt = "nibble" if abits <= 4 else "u8"
+    got = run_packed_linear(dev, layer, codes, s, fmt, out_dtype)
+    check_outputs(got, oracle_linear(layer, codes, s, out_dtype), s, layer["r"].float().numpy(), k, f"small tiles, {fmt}")
+    assert torch.equal(got, run_packed_linear(dev, layer, codes, s, fmt, out_dtype))  # fixed summation order
+
+
 @pytest.mark.parametrize(("m", "n", "k", "wbits", "abits", "splits"), [
     (128, 256, 2048, 4, 4, 2), (65, 520, 4096, 4, 4, 4), (300, 136, 8192, 3, 3, 8), (129, 96, 4608, 2, 4, 3),
     (200, 264, 3072, 6, 4, 2), (130, 128, 2048, 8, 4, 2), (256, 384, 4096, 4, 6, 4), (100, 72, 2048, 3, 8, 2)])
