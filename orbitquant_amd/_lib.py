@@ -26,6 +26,7 @@ EXPORTS = (
 )
 
 _lib = None
+_torch_ops = None   # the compiled module of the custom ops (csrc/torch_ops.cpp), or the ImportError that kept it away
 
 
 class OrbitQuantHipError(RuntimeError):
@@ -103,7 +104,45 @@ def load() -> ctypes.CDLL:
     lib.oq_unpack_lowbit.restype = c_int
     lib.oq_unpack_lowbit.argtypes = [vp, c_int, c_i64, vp, vp]
     _lib = lib
+    if hasattr(_torch_ops, "bind"):
+        _bind(lib)
     return lib
+
+
+def _bind(lib: ctypes.CDLL) -> None:
+    names = ("oq_quantized_linear", "oq_quantized_linear_group", "oq_packed_linear_workspace_bytes", "oq_rotate_plan_bytes",
+             "oq_matmul_packed_adaln_int4")
+    _torch_ops.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names})
+
+
+def torch_ops():
+    """The compiled module that implements the custom ops on the GPU; raises where it is not built."""
+    global _torch_ops
+    if _torch_ops is None:
+        try:
+            from . import _torch_ops as module
+        except ImportError as exc:
+            _torch_ops = exc
+        else:
+            _torch_ops = module
+            if _lib is not None:
+                _bind(_lib)
+    if isinstance(_torch_ops, ImportError):
+        raise OrbitQuantHipError(f"the custom ops' compiled module is missing or of another torch ({_torch_ops}): "
+                                 "build it with `python -m orbitquant_amd.build`")
+    return _torch_ops
+
+
+def register_gpu_ops(library, names: tuple[str, ...]) -> None:
+    """Loads the module, which registers the ops' GPU implementations; where it cannot be loaded, `names` raise when
+    they are called on a GPU (importing the package needs no build)."""
+    try:
+        torch_ops()
+    except OrbitQuantHipError:
+        def missing(*args, **kwargs):
+            torch_ops()
+        for name in names:
+            library.impl(name, missing, "CUDA")
 
 
 def check(rc: int, what: str) -> None:

@@ -46,8 +46,10 @@ def quantize_adaln_weight(weight: torch.Tensor, *, group_size: int) -> tuple[tor
 
 
 _LIB = torch.library.Library("orbitquant_amd", "FRAGMENT")
-_LIB.define("adaln_int4_linear(Tensor x, Tensor packed_weight, Tensor scales, Tensor? bias, int out_features, "
-            "int in_features, int group_size) -> Tensor")
+_SCHEMA = ("(Tensor x, Tensor packed_weight, Tensor scales, Tensor? bias, int out_features, "
+           "int in_features, int group_size) -> Tensor")
+_LIB.define("adaln_int4_linear" + _SCHEMA)
+_LIB.define("adaln_int4_linear_general" + _SCHEMA)   # what csrc/torch_ops.cpp hands on: unusual operands, and errors
 
 
 def _adaln_forward(x, packed_weight, scales, bias, out_features, in_features, group_size):
@@ -59,7 +61,7 @@ def _adaln_fake(x, packed_weight, scales, bias, out_features, in_features, group
     return x.new_empty((*x.shape[:-1], out_features), dtype=torch.bfloat16)
 
 
-_LIB.impl("adaln_int4_linear", _adaln_forward, "CUDA")
+_LIB.impl("adaln_int4_linear_general", _adaln_forward, "CUDA")
 torch.library.register_fake("orbitquant_amd::adaln_int4_linear", _adaln_fake, lib=_LIB)
 _adaln_int4_linear = torch.ops.orbitquant_amd.adaln_int4_linear.default
 
@@ -130,7 +132,7 @@ class RTNInt4Linear(nn.Module):
             raise ValueError(f"expected last dimension {self.in_features}, got {x.shape[-1]}")
         if x.device.type != "cuda":
             raise RuntimeError("RTNInt4Linear runs on AMD GPUs only (torch device 'cuda'); there is no CPU fallback")
-        self.last_effective_runtime_mode = "hip_packed_adaln_int4"
+        self.__dict__["last_effective_runtime_mode"] = "hip_packed_adaln_int4"
         return _adaln_int4_linear(x, self.packed_weight, self.scales, self.bias, self.out_features, self.in_features, self.group_size)
 
     def extra_repr(self) -> str:

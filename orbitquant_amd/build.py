@@ -1,4 +1,5 @@
-"""Compile the gfx950 HIP kernels into `orbitquant_amd/liborbitquant_hip.so`.
+"""Compile the gfx950 HIP kernels into `orbitquant_amd/liborbitquant_hip.so`, and the custom ops' host code
+(csrc/torch_ops.cpp, against the installed torch) into `orbitquant_amd/_torch_ops.so`.
 
     python -m orbitquant_amd.build
 
@@ -83,8 +84,28 @@ def _compile(item, obj_dir: Path = None) -> Path:
     return obj
 
 
+def build_torch_ops() -> Path:
+    """Host code only: the ops' checks and allocations; the kernels are in the library it calls."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    out = PKG / "_torch_ops.so"
+    includes = [f"-I{p}" for p in cpp_extension.include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"]]]
+    torch_lib = Path(torch.__file__).parent / "lib"
+    cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + includes +
+           [str(CSRC / "torch_ops.cpp"), "-o", str(out), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+    t0 = time.time()
+    subprocess.run(cmd, check=True)
+    print(f"  compiled torch_ops.cpp in {time.time() - t0:.1f}s", flush=True)
+    return out
+
+
 def build(verbose: bool = True) -> Path:
     OBJ_DIR.mkdir(exist_ok=True)
+    build_torch_ops()
     with ThreadPoolExecutor(max_workers=4) as pool:
         objects = list(pool.map(_compile, SOURCES.items()))
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB)] + [str(o) for o in objects]

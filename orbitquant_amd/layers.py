@@ -27,20 +27,22 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from . import ops
+from . import _lib, ops
 from .codebooks import get_codebook
 from .config import OrbitQuantConfig
 from .rotations import get_rpbh_rotation
 from .weights import quantize_weight
 
 _LIB = torch.library.Library("orbitquant_amd", "DEF")
-_LIB.define(
-    "quantized_linear(Tensor x, Tensor permutation, Tensor signs, Tensor act_centroids, "
+_SCHEMA = (
+    "(Tensor x, Tensor permutation, Tensor signs, Tensor act_centroids, "
     "Tensor act_boundaries, Tensor packed_weight_indices, Tensor row_norms, Tensor weight_centroids, "
     "Tensor? bias, int block_size, float eps, float inv_sqrt_block, int activation_bits, "
     "int weight_bits, int out_features, Tensor? input_map=None, Tensor? output_map=None, "
     "Tensor? rotate_plan=None) -> Tensor"
 )
+_LIB.define("quantized_linear" + _SCHEMA)
+_LIB.define("quantized_linear_general" + _SCHEMA)   # what csrc/torch_ops.cpp hands on: unusual operands, and errors
 
 
 def quantized_linear_forward(
@@ -81,7 +83,8 @@ def _quantized_linear_fake(
     return x.new_empty((*x.shape[:-1], out_features))
 
 
-_LIB.impl("quantized_linear", quantized_linear_forward, "CUDA")
+_LIB.impl("quantized_linear_general", quantized_linear_forward, "CUDA")
+_lib.register_gpu_ops(_LIB, ("quantized_linear", "adaln_int4_linear"))
 torch.library.register_fake("orbitquant_amd::quantized_linear", _quantized_linear_fake, lib=_LIB)
 _quantized_linear = torch.ops.orbitquant_amd.quantized_linear.default   # (the overload itself: no lookup per call)
 
@@ -308,7 +311,7 @@ class OrbitLinear(nn.Module):
         out_table = self._buffers["_output_activation_table"]
         if out_table is not None and out_table.dtype != x.dtype:
             raise ValueError(f"the fused output activation was built for {out_table.dtype}, got {x.dtype}")
-        self.last_effective_runtime_mode = "hip_packed"
+        self.__dict__["last_effective_runtime_mode"] = "hip_packed"   # (past Module.__setattr__, a microsecond)
         if self.share_input_quantization and not torch.compiler.is_compiling():
             return self._forward_shared(x, table, out_table)
         packed, weight_bits, weight_centroids = self._matmul_weight(x.numel() // self.in_features)

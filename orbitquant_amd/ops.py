@@ -543,10 +543,15 @@ def quantized_linear_group(
     import ctypes
 
     _require_gpu(x, "x")
+    weights = list(weights)
+    # (the usual call, without Python per matrix; None: an operand to convert or copy, or an error to name)
+    outs = _lib.torch_ops().quantized_linear_group(x, permutation, signs, boundaries, act_centroids, weights, int(block_size), float(eps),
+                                                   float(inv_sqrt_block), int(activation_bits), input_map, plan)
+    if outs is not None:
+        return outs
     dim = x.shape[-1]
     rows = x if x.dim() == 2 and x.is_contiguous() else x.contiguous().reshape(-1, dim)
     m = rows.shape[0]
-    weights = list(weights)
     if not 1 <= len(weights) <= 64:
         raise ValueError("a group holds 1 to 64 matrices")
     permutation = _operand(permutation, "permutation", x, dtype=torch.int32, numel=dim)

@@ -1,0 +1,93 @@
+"""The custom ops' compiled implementation against the Python one it hands unusual calls to: the same results, the same
+refusals."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def layer():
+    if not torch.cuda.is_available():
+        pytest.skip("needs an AMD GPU")
+    from orbitquant_amd import OrbitLinear, recipe
+
+    torch.manual_seed(0)
+    return OrbitLinear.from_linear(torch.nn.Linear(384, 136), config=recipe("w4a4")).cuda()
+
+
+def arguments(layer, x, **changed):
+    a = dict(x=x, permutation=layer._rotation_permutation, signs=layer._rotation_signs, act_centroids=layer._activation_codebook_centroids,
+             act_boundaries=layer._activation_codebook_boundaries, packed_weight_indices=layer.packed_weight_indices, row_norms=layer.row_norms,
+             weight_centroids=layer._weight_codebook_centroids, bias=layer.bias.to(x.dtype), block_size=layer.rotation.block_size,
+             eps=layer.activation_eps, inv_sqrt_block=layer.rotation.normalization, activation_bits=4, weight_bits=4, out_features=136,
+             input_map=None, output_map=None, rotate_plan=layer._rotation_plan)
+    return {**a, **changed}
+
+
+def both(a):
+    op = torch.ops.orbitquant_amd
+    return op.quantized_linear(**a), op.quantized_linear_general(**a)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 384), (384,), (3, 7, 384), (0, 384), (130, 384)])
+def test_same_results(layer, shape, dtype):
+    x = torch.randn(*shape, device="cuda").to(dtype)
+    for changed in ({}, {"bias": None}, {"rotate_plan": None}, {"rotate_plan": layer._rotation_plan.clone()}, {"bias": layer.bias.double().float()},
+                    {"row_norms": torch.stack([layer.row_norms, layer.row_norms], 1)[:, 0]}):
+        got, want = both(arguments(layer, x, **changed))
+        assert got.dtype == dtype and got.shape == want.shape == (*shape[:-1], 136) and torch.equal(got, want)
+
+
+def test_views_and_tables(layer):
+    from orbitquant_amd import ops
+
+    x = torch.randn(64, 768, device="cuda").bfloat16()
+    table = ops.activation_table(torch.nn.functional.gelu, torch.bfloat16, "cuda")
+    for view in (x[:, ::2], x[:, 384:], x[::2, :384], x.t()[:384].t()):
+        got, want = both(arguments(layer, view, input_map=table, output_map=table))
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("wrong", [
+    {"signs": torch.ones(383, dtype=torch.int8)}, {"permutation": torch.arange(384)}, {"row_norms": torch.ones(136)}, {"weight_bits": 3},
+    {"packed_weight_indices": torch.zeros(10, dtype=torch.uint8)}, {"bias": torch.zeros(5)}, {"input_map": torch.zeros(65536, dtype=torch.float16)},
+    {"rotate_plan": torch.zeros(16, dtype=torch.uint8)}])
+def test_same_refusals(layer, wrong):
+    a = arguments(layer, torch.randn(8, 384, device="cuda").bfloat16(), **{k: v.cuda() if isinstance(v, torch.Tensor) else v for k, v in wrong.items()})
+    op = torch.ops.orbitquant_amd
+    for call in (op.quantized_linear, op.quantized_linear_general):
+        with pytest.raises(ValueError):
+            call(**a)
+
+
+def test_a_plan_of_another_shape_is_refused(layer):
+    from orbitquant_amd import ops
+
+    other = ops.rotate_plan(layer._rotation_permutation, layer._rotation_signs, layer._activation_codebook_boundaries, block_size=64, inv_sqrt_block=0.125)
+    with pytest.raises(ValueError, match="built for"):
+        torch.ops.orbitquant_amd.quantized_linear(**arguments(layer, torch.randn(8, 384, device="cuda").bfloat16(), rotate_plan=other))
+
+
+@pytest.mark.parametrize("m", [1, 40, 200])
+def test_group_equals_its_members(layer, m):
+    from orbitquant_amd import OrbitLinear, OrbitLinearGroup, recipe
+
+    torch.manual_seed(1)
+    linears = [layer] + [OrbitLinear.from_linear(torch.nn.Linear(384, n, bias=False), config=recipe("w4a4")).cuda() for n in (64, 8)]
+    x = torch.randn(2, m, 384, device="cuda").bfloat16()
+    for view in (x, x.transpose(0, 1)):
+        for got, l in zip(OrbitLinearGroup(*linears)(view), linears):
+            assert torch.equal(got, l(view))
+
+
+def test_under_fake_tensors(layer):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        y = layer(mode.from_tensor(torch.empty(3, 384, dtype=torch.bfloat16, device="meta")).to("cuda"))
+        assert y.shape == (3, 136) and y.dtype == torch.bfloat16
