@@ -116,7 +116,7 @@ bool token_linear_supported(int x_dtype, int64_t M, int64_t N, int64_t K, int le
                             const int32_t *perm, const int8_t *signs);
 int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map, int64_t K, const int32_t *perm,
                           const int8_t *signs, const float *boundaries, const float *act_cents, int levels,
-                          int64_t block, float eps, float inv_sqrt_block, const uint8_t *packed_w, int bits,
+                          int64_t block, float eps, float inv_sqrt_block, const void *plan, const uint8_t *packed_w, int bits,
                           const uint16_t *row_norms, const float *w_cents, const void *bias, int bias_dtype,
                           int64_t N, void *out, int out_dtype, const uint16_t *out_map, hipStream_t stream, bool *launched);
 int generic_matmul_float(const void *x, int x_dtype, const float *token_scale, const uint8_t *packed_w,
@@ -418,7 +418,7 @@ int oq_quantized_linear(const void *x, int x_dtype, const uint16_t *input_map, i
   if (aligned16(packed_w) && token_linear_supported(x_dtype, M, N, K, levels, w_bits, x, perm, signs)) {
     bool launched = false;
     const int rc = token_linear_dispatch(x, x_dtype, input_map, K, perm, signs, boundaries, act_centroids, levels, block,
-                                         eps, inv_sqrt_block, packed_w, w_bits, row_norms, w_centroids, bias,
+                                         eps, inv_sqrt_block, rotate_plan, packed_w, w_bits, row_norms, w_centroids, bias,
                                          bias_dtype, N, out, out_dtype, output_map, s, &launched);
     if (rc != OQ_OK || launched) return rc;
   }

@@ -19,6 +19,9 @@
 //     denominator outside [2^-80, 2^20], anything not finite) take the IEEE division instead;
 //     the test is one packed instruction pair per two bf16 values while the row is read.
 //
+// With few rows a wavefront alone on a block of 1024 to 4096 values is a long chain of dependent steps, so there WB
+// wavefronts share a block: each keeps 1 / WB of it in registers, and the butterflies between them go through LDS once.
+//
 // The sum of squares keeps the documented order: [passes][256 lanes][8], tree over the lanes.
 // Compiled without FMA contraction.
 #pragma once
@@ -66,8 +69,18 @@ struct FastArgs {
   const uint16_t *map;
 };
 
+inline void fast_args_fill(FastArgs &a, const void *x, int64_t M, int64_t K, const void *plan, int levels, int64_t block, float eps) {
+  a.x = x; a.M = M; a.K = K; a.plan = static_cast<const unsigned char *>(plan);
+  a.levels = levels; a.block = static_cast<int>(block); a.eps = eps;
+  a.levels_pow2 = 2;
+  while (a.levels_pow2 < levels) a.levels_pow2 <<= 1;
+  a.passes = static_cast<int>((K + kPass - 1) / kPass);
+  const int64_t unit = block > kLaneSpan ? block : kLaneSpan;
+  a.units = static_cast<int>((K + unit - 1) / unit);
+}
+
 // LDS: cells (2048) | thresholds (1024) | centroids (1024) | reduction slots (64) | staging
-constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then one flag per wavefront
+constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then four flags
 
 // The row is staged once, in its own type; behind it, for a launch with an input map, the map's 16 KB window
 // (value_map.h).  Long rows are bound by how many wavefronts a CU holds, and that by LDS and registers: with a second,
@@ -191,30 +204,152 @@ __device__ __forceinline__ void count_below(const uint2 (&ent)[kChunk], const fl
 // little-endian stream; the norm is stored as bf16.
 enum EmitMode { EMIT_NIBBLE = 0, EMIT_U8 = 1, EMIT_ANY = 2, EMIT_WEIGHT = 3 };
 
-// One row.  `smem`: fast_lds_bytes(K, DT) bytes (and kWideBytes more if MAPPED), 16-byte aligned.  All 64 * waves threads of the
-// workgroup make the call.
-template <int DT, int LOG_H, int EMIT, bool MAPPED = false>
+// Phase B of a row whose blocks of H values are shared by WB wavefronts each (EMIT_NIBBLE / EMIT_U8).  A wavefront
+// rotates its GW steps of 512 slots as far as its registers reach and writes them to LDS; behind one barrier a thread
+// takes CT consecutive columns of the WB parts, does the butterflies between the parts and makes their codes.
+template <int DT, int H, int EMIT, int WB, int GW, typename Request, typename Rotate>
+__device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned char *smem, const int64_t row, const int tid, const int waves,
+                                                     const uint32_t modes, const uint2 *cells, const float *thr, float cell_scale,
+                                                     float cell_offset, uint8_t *codes_row, int4 (&ea)[GW], int4 (&eb)[GW], Request request,
+                                                     Rotate rotate_step) {
+  constexpr int SPAN = GW * kLaneSpan;   // slots a wavefront keeps, and the distance between the parts
+  constexpr int CT = kChunk * GW / WB;   // columns a thread takes
+  constexpr int N = CT * WB;             // values it turns into codes: 8 or 16
+  static_assert(SPAN * WB == H && CT >= 1 && N % kChunk == 0);
+  const int lane = tid & 63, wave = tid >> 6, team = wave / WB, teams = waves / WB, part = wave % WB;
+  float *buffer = reinterpret_cast<float *>(smem + fast_lds_bytes(a.K, DT));  // [K]
+  const bool plain = (modes & 1u) != 0u, searched = (modes & 2u) != 0u, signs_left = (modes & 4u) != 0u;
+#pragma nounroll
+  for (int u = team; u < a.units && team < teams; u += teams) {
+    if (u != team) request(u);
+    const int first = u * H + part * SPAN;
+    float y[GW][kChunk];
+#pragma unroll
+    for (int j = 0; j < GW; ++j) rotate_step(ea[j], eb[j], first + j * kLaneSpan, plain, signs_left, y[j]);
+    if constexpr (GW > 1) {
+#pragma unroll
+      for (int dist = 1; dist < GW; dist <<= 1)
+#pragma unroll
+        for (int j = 0; j < GW; ++j)
+          if ((j & dist) == 0)
+#pragma unroll
+            for (int e = 0; e < kChunk; ++e) {
+              const float l = y[j][e], r = y[j + dist][e];
+              y[j][e] = l + r;
+              y[j + dist][e] = l - r;
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < GW; ++j) {
+      float4 *dst = reinterpret_cast<float4 *>(buffer + first + j * kLaneSpan + lane * kChunk);
+      dst[0] = make_float4(y[j][0], y[j][1], y[j][2], y[j][3]);
+      dst[1] = make_float4(y[j][4], y[j][5], y[j][6], y[j][7]);
+    }
+  }
+  __syncthreads();
+#pragma nounroll
+  for (int u = team; u < a.units && team < teams; u += teams) {
+    const int column = u * H + (part * 64 + lane) * CT;
+    float z[WB][CT];
+#pragma unroll
+    for (int v = 0; v < WB; ++v) {
+      const float *src = buffer + column + v * SPAN;
+      if constexpr (CT % 4 == 0) {
+#pragma unroll
+        for (int c = 0; c < CT; c += 4) {
+          const float4 q = *reinterpret_cast<const float4 *>(src + c);
+          z[v][c] = q.x; z[v][c + 1] = q.y; z[v][c + 2] = q.z; z[v][c + 3] = q.w;
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) z[v][c] = src[c];
+      }
+    }
+#pragma unroll
+    for (int dist = 1; dist < WB; dist <<= 1)
+#pragma unroll
+      for (int v = 0; v < WB; ++v)
+        if ((v & dist) == 0)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            const float l = z[v][c], r = z[v + dist][c];
+            z[v][c] = l + r;
+            z[v + dist][c] = l - r;
+          }
+    int code[N];
+#pragma unroll
+    for (int at = 0; at < N; at += kChunk) {
+      float value[kChunk];
+      int eight[kChunk];
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) value[e] = z[(at + e) / CT][(at + e) % CT];
+      if (!searched) {
+        uint2 ent[kChunk];
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) ent[e] = cells[plan::cell_of(value[e], cell_scale, cell_offset)];
+        count_below(ent, value, eight);
+      } else {
+        rq::bucketize_many<kChunk>(thr, a.levels_pow2, value, eight);
+      }
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) code[at + e] = eight[e];
+    }
+#pragma unroll
+    for (int v = 0; v < WB; ++v) {
+      constexpr int kBits = EMIT == EMIT_NIBBLE ? 4 : 8;
+      uint64_t run = 0;  // this thread's CT codes of part v
+#pragma unroll
+      for (int c = CT - 1; c >= 0; --c) run = (run << kBits) | static_cast<uint32_t>(code[v * CT + c]);
+      const int slot = column + v * SPAN;
+      if constexpr (EMIT == EMIT_U8) {
+        uint8_t *dst = codes_row + slot;
+        if constexpr (CT == 8) *reinterpret_cast<uint2 *>(dst) = make_uint2(static_cast<uint32_t>(run), static_cast<uint32_t>(run >> 32));
+        else if constexpr (CT == 4) *reinterpret_cast<uint32_t *>(dst) = static_cast<uint32_t>(run);
+        else if constexpr (CT == 2) *reinterpret_cast<uint16_t *>(dst) = static_cast<uint16_t>(run);
+        else *dst = static_cast<uint8_t>(run);
+      } else {
+        uint8_t *dst = codes_row + slot / 2;
+        uint32_t w = static_cast<uint32_t>(run);
+        if constexpr (CT == 8) *reinterpret_cast<uint32_t *>(dst) = w;
+        else if constexpr (CT == 4) *reinterpret_cast<uint16_t *>(dst) = static_cast<uint16_t>(w);
+        else if constexpr (CT == 2) *dst = static_cast<uint8_t>(w);
+        else {  // one code: the lanes of a quad hand theirs to its first lane
+          w |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0xB1, 0xF, 0xF, true)) << 4;
+          w |= static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w), 0x4E, 0xF, 0xF, true)) << 8;
+          if ((lane & 3) == 0) *reinterpret_cast<uint16_t *>(dst) = static_cast<uint16_t>(w);
+        }
+      }
+    }
+  }
+}
+
+// One row.  `smem`: fast_lds_bytes(K, DT) bytes (and kWideBytes more if MAPPED, 4 K more if WB > 1), 16-byte aligned.
+// All 64 * waves threads of the workgroup make the call.  `after_loads` is called once by every thread, when it waits for
+// no load of its own any more but the gather entries.
+template <int DT, int LOG_H, int EMIT, bool MAPPED = false, int WB = 1, bool ANYWHERE = (WB > 1), typename AfterLoads>
 __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsigned char *smem, const int64_t row,
-                                                         const int tid, const int waves) {
+                                                         const int tid, const int waves, AfterLoads after_loads) {
   static_assert(!MAPPED || DT == OQ_BF16, "the input map's LDS window is one of bf16 bit patterns");
   constexpr int H = 1 << LOG_H;
   constexpr int G = H > kLaneSpan ? H / kLaneSpan : 1;  // steps of 512 values a unit is made of
+  static_assert(WB == 1 || (!MAPPED && G % WB == 0 && (EMIT == EMIT_NIBBLE || EMIT == EMIT_U8)), "shared blocks: codes of unmapped rows");
   const int lane = tid & 63, wave = tid >> 6;
   const int64_t K = a.K;
   const plan::PlanHeader *hdr = reinterpret_cast<const plan::PlanHeader *>(a.plan);
   uint2 *cells = reinterpret_cast<uint2 *>(smem + kCellsAt);
   float *thr = reinterpret_cast<float *>(smem + kThrAt);
   float *cent = reinterpret_cast<float *>(smem + kCentAt);
-  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..11] per-wavefront flags
+  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..7] per-wavefront flags
   unsigned char *stage = smem + kStageAt;
   const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset);
   const uint16_t *signs_by_position = reinterpret_cast<const uint16_t *>(gather + K), *signs_by_slot = signs_by_position + K;
 
   // A plan built for another shape must not be walked.  No codes are written then, and the row's norm
   // is stored as NaN, so that the mismatch cannot pass for a result: every output computed from it is NaN.
-  // (The gather entries are absolute LDS addresses, valid because this kernel's LDS block starts at 0.)
+  // (The gather entries are LDS addresses for a block of LDS that starts at 0; ANYWHERE adds where it starts.)
   if (hdr->magic != plan::kMagic || hdr->K != static_cast<uint32_t>(K) || hdr->block != static_cast<uint32_t>(H) ||
-      hdr->levels != static_cast<uint32_t>(a.levels) || lds_byte_address(smem) != 0u) {
+      hdr->levels != static_cast<uint32_t>(a.levels) || (!ANYWHERE && lds_byte_address(smem) != 0u)) {
+    after_loads();
     if (tid == 0) {
       if (a.norms != nullptr) a.norms[row] = __builtin_nanf("");
       if constexpr (EMIT == EMIT_WEIGHT) a.norms_bf16[row] = 0x7fc0;
@@ -234,6 +369,30 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
                                           : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
   const float cent_v = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(table_idx, a.levels - 1)] : 0.0f;
 
+  const uint32_t lds_at = ANYWHERE ? lds_byte_address(smem) : 0u;
+
+  // The gather entries of the first step(s) of this wavefront, where few rows are waited for: with the row, not behind it
+  constexpr int GW = G / WB;  // steps a wavefront keeps
+  const int team = wave / WB, teams = waves / WB, part = wave % WB;  // WB > 1: wavefronts of one block
+  const unsigned char *gather_bytes = reinterpret_cast<const unsigned char *>(gather);  // uniform
+  int4 early_a[GW], early_b[GW];
+  auto request_shared = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < GW; ++j) {
+      const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + lane * kChunk, Ki - kChunk));
+      early_a[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
+      early_b[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
+    }
+  };
+  if constexpr (WB > 1) request_shared(team);
+  int4 ea_next, eb_next;
+  auto request_entries = [&](int first) {
+    const uint32_t c = static_cast<uint32_t>(min(first + lane * kChunk, Ki - kChunk));
+    ea_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
+    eb_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
+  };
+  if constexpr (WB == 1 && ANYWHERE) request_entries(wave * (G * kLaneSpan));
+
   // an input map's window goes to LDS first (every wavefront looks values up in it as it reads the row)
   const uint16_t *hot = nullptr;
   if constexpr (MAPPED) {
@@ -246,7 +405,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // ---- phase A: stage the row with its signs, sum of squares ----------------------------------
   // Virtual lane t of the documented [passes][256 lanes][8] order is lane t % 64 of group t / 64;
   // wavefront w owns the groups w, w + waves, ... with all their passes, and keeps four passes of
-  // a group requested ahead of the one it is summing.  (Adding a lane's first pass to +0 is exact.)
+  // a group (fp32: two) requested ahead of the one it is summing; eight, the whole of most rows, cost few rows 0.35 us.  (Adding a lane's first pass to +0 is exact.)
   constexpr int kElem = DT == OQ_F32 ? 4 : 2;
   const unsigned char *xrow = static_cast<const unsigned char *>(a.x) + row * K * kElem;  // uniform
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -353,7 +512,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   bool tiny = tiny32;
   if constexpr (DT == OQ_BF16) tiny = min(tiny_acc & 0xffffu, tiny_acc >> 16) < 0x2effu;
   const bool wave_tiny = __builtin_amdgcn_ballot_w64(tiny) != 0;
-  if (lane == 0) red[4 + wave] = wave_tiny ? 1.0f : 0.0f;
+  if (lane == 0 && wave < 4) red[4 + wave] = wave_tiny ? 1.0f : 0.0f;  // (four wavefronts at most read the row)
   if (tid < 256) {
     cells[tid] = cell_v;
     thr[tid] = thr_v;
@@ -366,6 +525,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
                                    : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[idx];
     cent[idx] = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(idx, a.levels - 1)] : 0.0f;
   }
+  after_loads();
   __syncthreads();
   const float total = (red[0] + red[1]) + (red[2] + red[3]);
   const float s_norm = sqrtf(total);
@@ -375,7 +535,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   rc.rl = __builtin_fmaf(-rc.d, rc.rh, 1.0f) * rc.rh;
   bool row_plain = !(rc.d >= 0x1p-80f && rc.d <= 0x1p20f);
 #pragma nounroll
-  for (int w = 0; w < waves; ++w) row_plain = row_plain || red[4 + w] != 0.0f;
+  for (int w = 0; w < min(waves, 4); ++w) row_plain = row_plain || red[4 + w] != 0.0f;
   if (tid == 0 && a.norms != nullptr) a.norms[row] = s_norm;
   const float weight_denominator = s_norm < a.eps ? a.eps : s_norm;  // clamp_min(eps): a NaN norm stays NaN
   Reciprocal weight_rc{};
@@ -395,19 +555,70 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (hdr->cells != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
   const uint32_t neg1 = (lane & 1) ? 0x80000000u : 0u, neg2 = (lane & 2) ? 0x80000000u : 0u;
-  // The gather entries of a step are requested one step ahead (past the last step: the row's
-  // last chunk again, never used).
-  int4 ea_next, eb_next;
-  const unsigned char *gather_bytes = reinterpret_cast<const unsigned char *>(gather);  // uniform
-  auto request_entries = [&](int first) {
-    const uint32_t c = static_cast<uint32_t>(min(first + lane_first, Ki - kChunk));
-    ea_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
-    eb_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
-  };
-  request_entries(wave * (G * kLaneSpan));
   float xv[kChunk];  // the gathered inputs of a step
 #pragma unroll
   for (int e = 0; e < kChunk; ++e) xv[e] = 0.0f;
+  // Slots first + 8 lane .. + 7, gathered through their entries, divided by the norm, butterflies up to distance 256
+  auto rotate_step = [&](int4 ea, int4 eb, int first, bool plain, bool signs_left, float (&out)[kChunk]) __attribute__((always_inline)) {
+    uint32_t ent[kChunk] = {static_cast<uint32_t>(ea.x), static_cast<uint32_t>(ea.y), static_cast<uint32_t>(ea.z),
+                            static_cast<uint32_t>(ea.w), static_cast<uint32_t>(eb.x), static_cast<uint32_t>(eb.y),
+                            static_cast<uint32_t>(eb.z), static_cast<uint32_t>(eb.w)};
+    if constexpr (DT == OQ_BF16) {
+      if constexpr (ANYWHERE) {
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) ent[e] += lds_at;
+      }
+      // A bf16 value is the upper half of its fp32: the 16-bit LDS load that writes only the upper
+      // half of its destination needs no conversion, as long as the lower halves are zero (xv was
+      // zeroed before the loop and is only ever written by these loads).
+      asm volatile("ds_read_u16_d16_hi %0, %8\n\tds_read_u16_d16_hi %1, %9\n\tds_read_u16_d16_hi %2, %10\n\t"
+                   "ds_read_u16_d16_hi %3, %11\n\tds_read_u16_d16_hi %4, %12\n\tds_read_u16_d16_hi %5, %13\n\t"
+                   "ds_read_u16_d16_hi %6, %14\n\tds_read_u16_d16_hi %7, %15\n\ts_waitcnt lgkmcnt(0)"
+                   : "+v"(xv[0]), "+v"(xv[1]), "+v"(xv[2]), "+v"(xv[3]), "+v"(xv[4]), "+v"(xv[5]), "+v"(xv[6]), "+v"(xv[7])
+                   : "v"(ent[0]), "v"(ent[1]), "v"(ent[2]), "v"(ent[3]), "v"(ent[4]), "v"(ent[5]), "v"(ent[6]), "v"(ent[7])
+                   : "memory");
+    } else {
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) {  // the entries are LDS addresses (the workgroup's LDS starts at 0)
+        if constexpr (DT == OQ_F32) {
+          xv[e] = __uint_as_float(lds_read_u32(2u * ent[e] - plan::kStageAddress + lds_at));
+        } else {
+          xv[e] = f16_bits_to_f32(lds_read_u16(ent[e] + lds_at));
+        }
+      }
+    }
+    if (signs_left) {
+      const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(first + lane_first, Ki - kChunk));
+      const uint32_t w[4] = {sg.x, sg.y, sg.z, sg.w};
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) xv[e] = __uint_as_float(__float_as_uint(xv[e]) ^ (((e & 1) != 0 ? w[e / 2] : w[e / 2] << 16) & 0x80000000u));
+    }
+    if constexpr (EMIT == EMIT_WEIGHT) {
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) out[e] = xv[e];
+    } else if (!plain) {
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) out[e] = divide_fast(xv[e], rc);
+    } else {
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) out[e] = xv[e] / rc.d;
+    }
+    rq::fwht_regs<kChunk>(out, H);
+    if constexpr (H > 8) stage_xor1(out, neg1);
+    if constexpr (H > 16) stage_xor2(out, neg2);
+    if constexpr (H > 32) stage_xor4(out);
+    if constexpr (H > 64) stage_xor8(out);
+    if constexpr (H > 128) rq::swap_stage<16>(out);
+    if constexpr (H > 256) rq::swap_stage<32>(out);
+  };
+  if constexpr (WB > 1) {
+    rotate_shared_blocks<DT, H, EMIT, WB, GW>(a, smem, row, tid, waves, row_modes, cells, thr, cell_scale, cell_offset, codes_row,
+                                          early_a, early_b, request_shared, rotate_step);
+    return;
+  }
+  // The gather entries of a step are requested one step ahead (past the last step: the row's
+  // last chunk again, never used).
+  if constexpr (!ANYWHERE) request_entries(wave * (G * kLaneSpan));
 #pragma nounroll
   for (int u = wave; u < a.units; u += waves) {
     float y[G][kChunk];
@@ -421,52 +632,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       // chunk instead: their blocks are their own, and nothing of theirs is stored.
       const int4 ea = ea_next, eb = eb_next;
       request_entries(j + 1 < G ? unit_base + (j + 1) * kLaneSpan : unit_base + waves * (G * kLaneSpan));
-      const uint32_t ent[kChunk] = {static_cast<uint32_t>(ea.x), static_cast<uint32_t>(ea.y), static_cast<uint32_t>(ea.z),
-                                    static_cast<uint32_t>(ea.w), static_cast<uint32_t>(eb.x), static_cast<uint32_t>(eb.y),
-                                    static_cast<uint32_t>(eb.z), static_cast<uint32_t>(eb.w)};
-      if constexpr (DT == OQ_BF16) {
-        // A bf16 value is the upper half of its fp32: the 16-bit LDS load that writes only the upper
-        // half of its destination needs no conversion, as long as the lower halves are zero (xv was
-        // zeroed before the loop and is only ever written by these loads).
-        asm volatile("ds_read_u16_d16_hi %0, %8\n\tds_read_u16_d16_hi %1, %9\n\tds_read_u16_d16_hi %2, %10\n\t"
-                     "ds_read_u16_d16_hi %3, %11\n\tds_read_u16_d16_hi %4, %12\n\tds_read_u16_d16_hi %5, %13\n\t"
-                     "ds_read_u16_d16_hi %6, %14\n\tds_read_u16_d16_hi %7, %15\n\ts_waitcnt lgkmcnt(0)"
-                     : "+v"(xv[0]), "+v"(xv[1]), "+v"(xv[2]), "+v"(xv[3]), "+v"(xv[4]), "+v"(xv[5]), "+v"(xv[6]), "+v"(xv[7])
-                     : "v"(ent[0]), "v"(ent[1]), "v"(ent[2]), "v"(ent[3]), "v"(ent[4]), "v"(ent[5]), "v"(ent[6]), "v"(ent[7])
-                     : "memory");
-      } else {
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) {  // the entries are LDS addresses (the workgroup's LDS starts at 0)
-          if constexpr (DT == OQ_F32) {
-            xv[e] = __uint_as_float(lds_read_u32(2u * ent[e] - plan::kStageAddress));
-          } else {
-            xv[e] = f16_bits_to_f32(lds_read_u16(ent[e]));
-          }
-        }
-      }
-      if (signs_left) {
-        const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(unit_base + j * kLaneSpan + lane_first, Ki - kChunk));
-        const uint32_t w[4] = {sg.x, sg.y, sg.z, sg.w};
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) xv[e] = __uint_as_float(__float_as_uint(xv[e]) ^ (((e & 1) != 0 ? w[e / 2] : w[e / 2] << 16) & 0x80000000u));
-      }
-      if constexpr (EMIT == EMIT_WEIGHT) {
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) y[j][e] = xv[e];
-      } else if (!plain) {
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) y[j][e] = divide_fast(xv[e], rc);
-      } else {
-#pragma unroll
-        for (int e = 0; e < kChunk; ++e) y[j][e] = xv[e] / rc.d;
-      }
-      rq::fwht_regs<kChunk>(y[j], H);
-      if constexpr (H > 8) stage_xor1(y[j], neg1);
-      if constexpr (H > 16) stage_xor2(y[j], neg2);
-      if constexpr (H > 32) stage_xor4(y[j]);
-      if constexpr (H > 64) stage_xor8(y[j]);
-      if constexpr (H > 128) rq::swap_stage<16>(y[j]);
-      if constexpr (H > 256) rq::swap_stage<32>(y[j]);
+      rotate_step(ea, eb, unit_base + j * kLaneSpan, plain, signs_left, y[j]);
     }
     // distances 512 and up: between the steps of the unit, in registers, one slot of every step at a time
     if constexpr (G > 1) {

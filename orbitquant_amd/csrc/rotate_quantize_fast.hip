@@ -1,5 +1,7 @@
 // Rotate plan construction and the launcher of the plan-based rotate+quantize kernel
 // (rotate_quantize_fast.h).
+#include <stdlib.h>
+
 #include "rotate_quantize_fast.h"
 
 namespace oq {
@@ -130,7 +132,13 @@ constexpr int waves_per_simd(int log_h, bool mapped) { return log_h <= 9 ? (mapp
 template <int DT, int LOG_H, int EMIT, bool MAPPED>
 __global__ __launch_bounds__(512, waves_per_simd(LOG_H, MAPPED)) void rotate_quantize_fast_kernel(FastArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  rotate_quantize_row_fast<DT, LOG_H, EMIT, MAPPED>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6);
+  rotate_quantize_row_fast<DT, LOG_H, EMIT, MAPPED>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6, [] {});
+}
+
+template <int DT, int LOG_H, int EMIT, int WB>
+__global__ __launch_bounds__(1024) void rotate_quantize_shared_kernel(FastArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  rotate_quantize_row_fast<DT, LOG_H, EMIT, false, WB>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6, [] {});
 }
 
 template <int DT, int LOG_H, int EMIT, bool MAPPED = false>
@@ -142,8 +150,41 @@ int launch_emit(const FastArgs &a, int waves, size_t smem, hipStream_t stream) {
   return check_launch("rotate_quantize (plan)");
 }
 
+template <int DT, int LOG_H, int WB>
+int launch_shared(const FastArgs &a, hipStream_t stream) {
+  const size_t smem = fast_lds_bytes(a.K, DT) + 4u * static_cast<size_t>(a.K);
+  auto kern = a.code_format == OQ_CODES_NIBBLE ? rotate_quantize_shared_kernel<DT, LOG_H, EMIT_NIBBLE, WB> : rotate_quantize_shared_kernel<DT, LOG_H, EMIT_U8, WB>;
+  if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
+    return fail(OQ_ERR_LAUNCH, "rotate_quantize: cannot reserve %zu bytes of LDS", smem);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.M)), dim3(static_cast<unsigned>(64 * WB * a.units)), smem, stream, a);
+  return check_launch("rotate_quantize (plan, shared blocks)");
+}
+
+// Few rows: blocks of 1024 and more shared by as many wavefronts as sixteen a row allow; -1: not one of those launches.
+// Up to 4096 wavefronts the chip takes them all at once, or nearly; rows of one or two blocks, which would otherwise
+// have one or two wavefronts each, gain up to 1024 rows.  Measured against the better of the other two kernels: K = 4096
+// = one block, 1 / 333 / 1024 rows 5.8 / 9.4 / 12.0 -> 4.8 / 6.2 / 10.2 us; 12288 in three blocks, 1 / 256 rows 8.7 / 12.1
+// -> 7.4 / 8.4 us; 3072 in three, 1 / 512 rows 5.2 / 6.3 -> 4.4 / 6.0 us, but 1024 rows 7.2 -> 8.7 us; 14336 in seven,
+// 256 rows 10.8 -> 9.4 us, 333 rows 12.5 -> 16.3 us.
+template <int DT, int LOG_H>
+int launch_few(const FastArgs &a, hipStream_t stream) {
+  if constexpr (LOG_H >= 10) {
+    if (a.map != nullptr || a.packed != nullptr || a.codes == nullptr || a.values != nullptr) return -1;
+    int wb = 1;
+    while (wb < (1 << (LOG_H - 9)) && a.units * wb * 2 <= 16) wb *= 2;
+    if (a.M * a.units * wb > 4096 && (a.units > 2 || a.M > 1024)) return -1;
+    if constexpr (LOG_H >= 12)
+      if (wb == 8) return launch_shared<DT, LOG_H, 8>(a, stream);
+    if constexpr (LOG_H >= 11)
+      if (wb == 4) return launch_shared<DT, LOG_H, 4>(a, stream);
+    if (wb == 2) return launch_shared<DT, LOG_H, 2>(a, stream);
+  }
+  return -1;
+}
+
 template <int DT, int LOG_H>
 int launch_one(const FastArgs &a, int waves, size_t smem, hipStream_t stream) {
+  if (const int rc = launch_few<DT, LOG_H>(a, stream); rc >= 0) return rc;
   if (a.map != nullptr) {  // an input map: bf16 rows into codes only (the forms the layers use); -1 sends the rest to the plain kernel
     if constexpr (DT == OQ_BF16) {
       if (a.packed == nullptr && a.codes != nullptr && a.values == nullptr) {
@@ -216,8 +257,7 @@ int quantize_weight_fast(const void *w, int w_dtype, int64_t N, int64_t K, const
   if (!aligned16(w) || !aligned16(plan)) return fail(OQ_ERR_INVALID, "quantize_weight: w and the plan must be 16-byte aligned");
   if (N == 0) return OQ_OK;
   FastArgs a{};
-  a.x = w; a.M = N; a.K = K; a.plan = static_cast<const unsigned char *>(plan);
-  a.levels = levels; a.block = static_cast<int>(block); a.eps = eps;
+  fast_args_fill(a, w, N, K, plan, levels, block, eps);
   a.raw_bounds = boundaries; a.inv_sqrt_block = inv_sqrt_block; a.pack_bits = bits;
   a.packed = packed_out; a.packed_aligned = (reinterpret_cast<uintptr_t>(packed_out) & 7u) == 0;
   a.norms_bf16 = row_norms_out;
@@ -234,11 +274,8 @@ int rotate_quantize_fast(const void *x, int x_dtype, int64_t M, int64_t K, const
       (codes_out != nullptr && !aligned16(codes_out)) || (values_out != nullptr && !aligned16(values_out)))
     return -1;
   FastArgs a{};
-  a.x = x; a.M = M; a.K = K; a.plan = static_cast<const unsigned char *>(plan);
+  fast_args_fill(a, x, M, K, plan, levels, block, eps);
   a.cents = values_mode != OQ_VALUES_NONE ? centroids : nullptr;
-  a.levels = levels;
-  a.block = static_cast<int>(block);
-  a.eps = eps;
   a.codes = static_cast<uint8_t *>(codes_out); a.code_format = code_format;
   a.values = values_mode == OQ_VALUES_NONE ? nullptr : values_out; a.values_mode = values_mode;
   a.norms = norms_out;
@@ -251,11 +288,6 @@ static int launch_fast(FastArgs &a, int x_dtype, hipStream_t stream) {
   const int64_t K = a.K, block = a.block;
   int log_h = 0;
   while ((int64_t{1} << log_h) < block) ++log_h;
-  a.levels_pow2 = 2;
-  while (a.levels_pow2 < a.levels) a.levels_pow2 <<= 1;
-  a.passes = static_cast<int>((K + kPass - 1) / kPass);
-  const int64_t unit = block > kLaneSpan ? block : kLaneSpan;
-  a.units = static_cast<int>((K + unit - 1) / unit);
   // Wavefronts per row (each owns whole units): four, which is also what staging the row uses,
   // eight for rows of sixteen units and more (measured on 32760 rows: 5120 values in 5 units of 1024, 165 us on four
   // against 201 us on five; 13824 values in 27 units of 512, 458 us on eight, 454 on four, and few rows are sooner done on eight).

@@ -1,6 +1,7 @@
 // Dispatch of the one-token quantized linear (token_linear_impl.h): decides whether the single
 // launch applies, and builds the arguments of its two halves.
 #include "packed_gemv_body.h"
+#include "rotate_quantize_fast.h"
 #include "rotate_quantize_row.h"
 
 namespace oq {
@@ -8,6 +9,10 @@ namespace oq {
 int token_linear_launch_w2(const rq::RqArgs &q, const gemv::GemvArgs &g, int x_dtype, size_t rq_bytes, hipStream_t stream);
 int token_linear_launch_w3(const rq::RqArgs &q, const gemv::GemvArgs &g, int x_dtype, size_t rq_bytes, hipStream_t stream);
 int token_linear_launch_w4(const rq::RqArgs &q, const gemv::GemvArgs &g, int x_dtype, size_t rq_bytes, hipStream_t stream);
+
+int token_linear_plan_launch_w2(const rqf::FastArgs &q, const gemv::GemvArgs &g, int x_dtype, hipStream_t stream);
+int token_linear_plan_launch_w3(const rqf::FastArgs &q, const gemv::GemvArgs &g, int x_dtype, hipStream_t stream);
+int token_linear_plan_launch_w4(const rqf::FastArgs &q, const gemv::GemvArgs &g, int x_dtype, hipStream_t stream);
 
 namespace {
 constexpr size_t kLdsPerWorkgroup = 160 * 1024;  // gfx950
@@ -29,7 +34,7 @@ bool token_linear_supported(int x_dtype, int64_t M, int64_t N, int64_t K, int le
 
 int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map, int64_t K, const int32_t *perm,
                           const int8_t *signs, const float *boundaries, const float *act_cents, int levels,
-                          int64_t block, float eps, float inv_sqrt_block, const uint8_t *packed_w, int bits,
+                          int64_t block, float eps, float inv_sqrt_block, const void *plan, const uint8_t *packed_w, int bits,
                           const uint16_t *row_norms, const float *w_cents, const void *bias, int bias_dtype,
                           int64_t N, void *out, int out_dtype, const uint16_t *out_map, hipStream_t stream, bool *launched) {
   *launched = false;
@@ -50,6 +55,16 @@ int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map,
   g.act_cents = act_cents; g.a_levels = levels; g.w = packed_w; g.row_norms = row_norms; g.w_cents = w_cents;
   g.bias = bias; g.bias_dtype = bias_dtype; g.M = 1; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype; g.out_map = out_map;
   *launched = true;
+  // with a plan: blocks of 128 to 4096 (rows of K % 128 == 0 have no smaller ones unless the caller asks for them)
+  if (plan != nullptr && (reinterpret_cast<uintptr_t>(plan) & 15u) == 0 && input_map == nullptr && block >= 128 && block <= 4096) {
+    rqf::FastArgs f{};
+    rqf::fast_args_fill(f, x, 1, K, plan, levels, block, eps);
+    switch (bits) {
+      case 2: return token_linear_plan_launch_w2(f, g, x_dtype, stream);
+      case 3: return token_linear_plan_launch_w3(f, g, x_dtype, stream);
+      default: return token_linear_plan_launch_w4(f, g, x_dtype, stream);
+    }
+  }
   switch (bits) {
     case 2: return token_linear_launch_w2(q, g, x_dtype, rq_bytes, stream);
     case 3: return token_linear_launch_w3(q, g, x_dtype, rq_bytes, stream);

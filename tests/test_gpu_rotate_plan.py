@@ -153,6 +153,34 @@ def test_rows_that_take_the_ieee_division(dev, dtype):
     assert np.array_equal(got[ok].view(np.int32), want_norms[ok].view(np.int32))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,h", [(1024, 1024), (9216, 1024), (8192, 1024), (2048, 2048), (14336, 2048), (4096, 4096), (8192, 4096), (12288, 4096), (16384, 4096)])
+@pytest.mark.parametrize("m,bits", [(1, 4), (12, 3), (12, 6)])
+def test_blocks_shared_by_wavefronts(dev, k, h, m, bits, dtype):
+    """Few rows: two to eight wavefronts a block, eight or sixteen values each; slow rows, and a codebook without cells."""
+    from oracle import oracle_c
+
+    perm, signs, hh, inv, cents, bounds, t = constants(dev, k, h, bits)
+    x = make_rows(16, k, torch.float32, seed=k + bits)[:m]
+    if m > 1:
+        x[1, 7] = 1e-30 if dtype != torch.float16 else 6e-8
+        x[2] *= 1e12 if dtype != torch.float16 else 30.0
+        x[4, 100] = float("inf")
+        x[6, 5] = float("nan")
+    x = x.to(dtype)
+    fmt = "nibble" if bits <= 4 else "u8"
+    for table in (bounds, np.sort(np.concatenate([bounds[:-1], bounds[:1] * (1 + 1e-7)])).astype(np.float32)):
+        t["bounds"] = torch.from_numpy(table).to(dev)
+        (codes, _, norms), (codes_plain, _, _) = both_kernels(x.to(dev), t, h, inv, code_format=fmt)
+        with np.errstate(all="ignore"):
+            want, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, signs, table, h, 1e-10, inv)
+        if fmt == "nibble":
+            want = (want[:, 0::2] | (want[:, 1::2] << 4)).astype(np.uint8)
+        assert np.array_equal(codes.cpu().numpy(), want) and torch.equal(codes, codes_plain)
+        got, ok = norms.cpu().numpy(), ~np.isnan(want_norms)
+        assert np.array_equal(np.isnan(got), ~ok) and np.array_equal(got[ok].view(np.int32), want_norms[ok].view(np.int32))
+
+
 @pytest.mark.parametrize("levels", [2, 3, 5, 16, 64, 100, 256])
 def test_any_codebook_size_and_awkward_boundaries(dev, levels):
     """Boundary sets for which no cell table exists (more than 64 levels, clustered boundaries)

@@ -83,6 +83,20 @@ def test_one_token_single_launch_equals_two_launches(dev, k, n, wbits, abits, dt
     assert torch.equal(one_call(c), want)
 
 
+@pytest.mark.parametrize(("k", "n", "wbits", "abits", "dtype", "block", "with_bias"),
+                         [c for c in ONE_TOKEN if c[5] != 64 and c[0] < 8192] + [(5120, 4096, 4, 4, torch.bfloat16, "paper", False),
+                                                                                (2304, 5000, 2, 4, torch.float16, "paper", True)])
+def test_one_token_with_a_plan_equals_two_launches_without(dev, k, n, wbits, abits, dtype, block, with_bias):
+    from orbitquant_amd import ops
+
+    c = make_case(dev, 1, k, n, wbits, abits, dtype, block, with_bias, seed=k + n)
+    plan = ops.rotate_plan(c["perm"], c["signs"], c["bounds"], block_size=c["kw"]["block_size"], inv_sqrt_block=c["kw"]["inv_sqrt_block"])
+    want = two_calls(c)
+    assert torch.equal(one_call(dict(c, kw=dict(c["kw"], plan=plan))), want)
+    c["x"][0, 3] = 1e-30 if dtype == torch.bfloat16 else 6e-8      # the IEEE division
+    assert torch.equal(one_call(dict(c, kw=dict(c["kw"], plan=plan))), two_calls(c))
+
+
 def test_one_token_with_input_map(dev):
     from orbitquant_amd import ops
 
