@@ -10,6 +10,7 @@
 
 #include "dense_gemm.h"
 #include "gemm_epilogue.h"
+#include "rotate_plan.h"
 
 namespace oq {
 
@@ -220,7 +221,7 @@ int oq_rotate_quantize(const void *x, int x_dtype, int64_t M, int64_t K, const i
                                   nullptr, rotate_plan, as_stream(stream));
 }
 
-uint64_t oq_rotate_plan_bytes(int64_t K) { return K > 0 ? 3136u + 8u * static_cast<uint64_t>(K) : 0u; }
+uint64_t oq_rotate_plan_bytes(int64_t K) { return K > 0 ? plan::plan_bytes(K) : 0u; }
 
 int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
                          int64_t block, float inv_sqrt_block, void *plan_out, void *stream) {

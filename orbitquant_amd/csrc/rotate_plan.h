@@ -20,6 +20,7 @@
 //   3136  gather      uint32[K]
 //   3136 + 4K  signs by input position  uint16[K]   (0x8000: negative)
 //   3136 + 6K  signs by slot            uint16[K]
+//   3136 + 8K  weight cells             uint2[256]   the same table over the boundaries as they are
 #pragma once
 
 #include "oq_common.h"
@@ -44,12 +45,17 @@ struct PlanHeader {
   float cell_offset;
   float inv_sqrt_block;  // the factor folded into the thresholds
   uint32_t bijective;    // the permutation takes every position once
-  uint32_t reserved[7];
+  uint32_t weight_cells; // kCells, or 0: as `cells`, of the unfolded boundaries
+  float weight_cell_scale, weight_cell_offset;
+  uint32_t reserved[4];
 };
 static_assert(sizeof(PlanHeader) == 64, "the header is 64 bytes");
 
+// (K a multiple of 8 wherever the weight cells are read: an eight-byte boundary)
+__host__ __device__ inline size_t weight_cells_offset(int64_t K) { return static_cast<size_t>(kGatherOffset) + 8u * static_cast<size_t>(K); }
+
 __host__ __device__ inline size_t plan_bytes(int64_t K) {
-  return static_cast<size_t>(kGatherOffset) + 8u * static_cast<size_t>(K);
+  return static_cast<size_t>(kGatherOffset) + 8u * static_cast<size_t>(K) + static_cast<size_t>(kCells) * 8u;
 }
 
 // The cell of a value: one fused multiply-add and one saturating conversion to 0..255.  Any

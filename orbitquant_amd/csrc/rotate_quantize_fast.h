@@ -356,7 +356,9 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     }
     return;
   }
-  const float cell_scale = hdr->cell_scale, cell_offset = hdr->cell_offset;
+  const float cell_scale = EMIT == EMIT_WEIGHT ? hdr->weight_cell_scale : hdr->cell_scale;
+  const float cell_offset = EMIT == EMIT_WEIGHT ? hdr->weight_cell_offset : hdr->cell_offset;
+  const uint2 *plan_cells = reinterpret_cast<const uint2 *>(a.plan + (EMIT == EMIT_WEIGHT ? plan::weight_cells_offset(K) : plan::kCellsOffset));
   const bool bijective = hdr->bijective != 0u;  // (uniform: the signs go on while the row is staged)
 
   // tables: entry tid is requested now and stored to LDS after the row has been requested (loads
@@ -364,7 +366,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   const int nthreads = waves * 64;
   const int Ki = static_cast<int>(K);
   const int table_idx = min(tid, 255);
-  const uint2 cell_v = reinterpret_cast<const uint2 *>(a.plan + plan::kCellsOffset)[table_idx];
+  const uint2 cell_v = plan_cells[table_idx];
   const float thr_v = EMIT == EMIT_WEIGHT ? (table_idx < a.levels - 1 ? a.raw_bounds[table_idx] : __builtin_inff())
                                           : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
   const float cent_v = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(table_idx, a.levels - 1)] : 0.0f;
@@ -520,7 +522,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   }
 #pragma nounroll
   for (int idx = tid + nthreads; idx < 256; idx += nthreads) {  // workgroups of fewer than 256 threads only
-    cells[idx] = reinterpret_cast<const uint2 *>(a.plan + plan::kCellsOffset)[idx];
+    cells[idx] = plan_cells[idx];
     thr[idx] = EMIT == EMIT_WEIGHT ? (idx < a.levels - 1 ? a.raw_bounds[idx] : __builtin_inff())
                                    : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[idx];
     cent[idx] = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(idx, a.levels - 1)] : 0.0f;
@@ -552,7 +554,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // The two rare modes (IEEE division for this row, binary search instead of the cell table) pass
   // through an empty asm statement inside the loop on purpose: as loop invariants the compiler
   // clones the whole loop per combination.
-  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (hdr->cells != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
+  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | ((EMIT == EMIT_WEIGHT ? hdr->weight_cells : hdr->cells) != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
   const uint32_t neg1 = (lane & 1) ? 0x80000000u : 0u, neg2 = (lane & 2) ? 0x80000000u : 0u;
   float xv[kChunk];  // the gathered inputs of a step
@@ -669,8 +671,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
         for (int e = 1; e < kChunk; ++e) least = __builtin_fminf(least, __builtin_fabsf(unit[e]));
         // divide_fast is the IEEE quotient for numerators of 2^-80 and more and the rows it takes at all (NaN and
         // infinities make a row's norm one, so those rows take the other branch); the compiler's division, eleven
-        // instructions a value instead of four, remains for the rest.  With the wide stores below, 14336 x 4096 into
-        // four bits: 145 -> 139 us; bound by instruction issue, the search through the boundaries first.
+        // instructions a value instead of four, remains for the rest.  14336 x 4096 into four bits,
+        // the plan included: 89 us; 108 with a search of four dependent LDS reads per value in place of the cells.
         if (weight_plain || __builtin_amdgcn_ballot_w64(least < 0x1p-80f) != 0) {
 #pragma unroll
           for (int e = 0; e < kChunk; ++e) unit[e] = unit[e] / weight_denominator;
@@ -678,7 +680,14 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
 #pragma unroll
           for (int e = 0; e < kChunk; ++e) unit[e] = divide_fast(unit[e], weight_rc);
         }
-        rq::bucketize_many<kChunk>(thr, a.levels_pow2, unit, code);
+        if (!searched) {
+          uint2 ent[kChunk];
+#pragma unroll
+          for (int e = 0; e < kChunk; ++e) ent[e] = cells[plan::cell_of(unit[e], cell_scale, cell_offset)];
+          count_below(ent, unit, code);
+        } else {
+          rq::bucketize_many<kChunk>(thr, a.levels_pow2, unit, code);
+        }
       } else if (!searched) {
         uint2 ent[kChunk];
 #pragma unroll

@@ -65,7 +65,6 @@ __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *p
     return;
   }
   const int nb = levels - 1;
-  if (tid == 0) bad = 0;
   // thresholds: bisection between -inf and +inf in the ordered code (RN(t * c) is non-decreasing in t)
   float t = __builtin_inff();
   if (tid < nb) {
@@ -86,40 +85,52 @@ __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *p
       t = ordered_to_float(lo);
     }
   }
-  thr[tid] = t;
   reinterpret_cast<float *>(out + plan::kThresholdsOffset)[tid] = t;
-  __syncthreads();
-
-  // cells over [first threshold, last threshold]
-  const float lo = thr[0], hi = thr[nb > 0 ? nb - 1 : 0];
-  float scale = static_cast<float>(plan::kCells) / (hi - lo);
-  float offset = -lo * scale;
-  bool usable = levels >= 3 && levels <= 64 && hi > lo && scale < 3.0e38f && __builtin_fabsf(offset) < 3.0e38f;
-  if (usable) {
-    // thresholds ascend, so their cells do: the first with cell >= tid, the first with cell > tid
-    int first = 0, last = 0;
-    for (int j = 0; j < nb; ++j) {
-      const int cj = static_cast<int>(plan::cell_of(thr[j], scale, offset));
-      if (cj < tid) first = j + 1;
-      if (cj <= tid) last = j + 1;
-      if (j > 0 && !(thr[j - 1] <= thr[j])) bad = 1;  // not ascending (or NaN): no table
+  // A bucketize table over `count` ascending values in thr: cells between the first and the last.  The same for all threads.
+  struct Map { float scale, offset; bool usable; };
+  auto make_cells = [&](float value, uint2 *cells) -> Map {
+    __syncthreads();
+    thr[tid] = value;
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    const float lo = thr[0], hi = thr[nb > 0 ? nb - 1 : 0];
+    Map m;
+    m.scale = static_cast<float>(plan::kCells) / (hi - lo);
+    m.offset = -lo * m.scale;
+    m.usable = levels >= 3 && levels <= 64 && hi > lo && m.scale < 3.0e38f && __builtin_fabsf(m.offset) < 3.0e38f;
+    uint2 cell = make_uint2(__float_as_uint(__builtin_inff()), 0u);
+    if (m.usable) {
+      // the values ascend, so their cells do: the first with cell >= tid, the first with cell > tid
+      int first = 0, last = 0;
+      for (int j = 0; j < nb; ++j) {
+        const int cj = static_cast<int>(plan::cell_of(thr[j], m.scale, m.offset));
+        if (cj < tid) first = j + 1;
+        if (cj <= tid) last = j + 1;
+        if (j > 0 && !(thr[j - 1] <= thr[j])) bad = 1;  // not ascending (or NaN): no table
+      }
+      if (last - first > 1) bad = 1;
+      cell = make_uint2(__float_as_uint(last > first ? thr[first] : __builtin_inff()), static_cast<uint32_t>(first));
     }
-    if (last - first > 1) bad = 1;
-    reinterpret_cast<uint2 *>(out + plan::kCellsOffset)[tid] =
-        make_uint2(__float_as_uint(last > first ? thr[first] : __builtin_inff()), static_cast<uint32_t>(first));
-  } else {
-    reinterpret_cast<uint2 *>(out + plan::kCellsOffset)[tid] = make_uint2(__float_as_uint(__builtin_inff()), 0u);
-  }
-  __syncthreads();
+    cells[tid] = cell;
+    __syncthreads();
+    m.usable = m.usable && bad == 0;
+    return m;
+  };
+  const Map folded = make_cells(t, reinterpret_cast<uint2 *>(out + plan::kCellsOffset));
+  const Map raw = (K & 7) == 0 ? make_cells(tid < nb ? boundaries[tid] : __builtin_inff(), reinterpret_cast<uint2 *>(out + plan::weight_cells_offset(K)))
+                               : Map{0.0f, 0.0f, false};
   if (tid == 0) {
     plan::PlanHeader *h = reinterpret_cast<plan::PlanHeader *>(out);  // (`bijective` is the last workgroup's to write)
     h->magic = plan::kMagic;
     h->K = static_cast<uint32_t>(K);
     h->block = static_cast<uint32_t>(block);
     h->levels = static_cast<uint32_t>(levels);
-    h->cells = (usable && bad == 0) ? plan::kCells : 0;
-    h->cell_scale = scale;
-    h->cell_offset = offset;
+    h->cells = folded.usable ? plan::kCells : 0;
+    h->cell_scale = folded.scale;
+    h->cell_offset = folded.offset;
+    h->weight_cells = raw.usable ? plan::kCells : 0;
+    h->weight_cell_scale = raw.scale;
+    h->weight_cell_offset = raw.offset;
     h->inv_sqrt_block = c;
     for (uint32_t &r : h->reserved) r = 0u;
   }

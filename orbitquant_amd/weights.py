@@ -58,7 +58,7 @@ def quantize_weight(
 
         device = weight.device
         # (one launch for the matrix: at 256 rows a launch, one workgroup a CU, 14336 x 4096 took 56 launches of 16 us
-        # and some 200 us of Python; one launch 139 us)
+        # and some 200 us of Python; one launch 84 us)
         return ops.quantize_weight(
             weight, rotation.permutation.to(torch.int32).to(device), rotation.signs.to(torch.int8).to(device),
             codebook.boundaries.to(device), bits=bits, block_size=rotation.block_size, eps=eps,

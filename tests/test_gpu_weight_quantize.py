@@ -189,3 +189,20 @@ def test_rows_with_infinities_and_nan(dev, dtype):
         assert np.array_equal(got[row], want[row])
         alone, _ = gpu_quantize(dev, w[row : row + 1], perm, signs, bounds, block, inv, bits)
         assert torch.equal(alone, packed.view(7, -1)[row])
+
+
+@pytest.mark.parametrize("kind", ["crowded", "repeated", "wide", "two"])
+def test_boundaries_with_and_without_cells(dev, kind):
+    """Boundaries too close for one cell each, equal ones, far apart ones, a single one; weights that sit on them."""
+    k, n = 512, 40
+    perm, signs, block, inv = o.rpbh_constants(k, 0, "paper")
+    _, bounds = reference_tables(k, 4)
+    bounds = {"crowded": np.sort(np.concatenate([bounds[:8], bounds[7] * (1 + np.arange(7) * 1e-6)])), "repeated": np.repeat(bounds[::2], 2)[:15],
+              "wide": bounds * np.float32(40), "two": bounds[7:8]}[kind].astype(np.float32)
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(3))
+    w[3] = 0                                        # every value is zero
+    w[5] = 0
+    w[5, 9] = 1.0                                   # every value is +-1/sqrt(block)
+    packed, norms = gpu_quantize(dev, w, perm, signs, bounds, block, inv, 4)
+    want_packed, want_norms, _ = o.quantize_weight(w.numpy(), perm, signs, bounds, block, 1e-10, 4, norm_order="sumsq_v1")
+    assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
