@@ -45,10 +45,12 @@ def quantize_weight(
     bits: int,
     eps: float,
     row_tile: int = 4096,
+    constants: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """-> (packed uint8 [ceil(N*K*bits/8)], row_norms bfloat16 [N]), on the GPU for a GPU weight the
     kernel takes, else on the CPU.  `row_tile` bounds the rows whose fp32 copies the host path holds at a
-    time; the result does not depend on it, and a GPU weight is one launch without such copies."""
+    time; the result does not depend on it, and a GPU weight is one launch without such copies.
+    `constants`: permutation (int32), signs (int8) and boundaries where they are on the weight's device already."""
     if weight.ndim != 2:
         raise ValueError("weight must be a matrix")
     n, k = weight.shape
@@ -59,9 +61,11 @@ def quantize_weight(
         device = weight.device
         # (one launch for the matrix: at 256 rows a launch, one workgroup a CU, 14336 x 4096 took 56 launches of 16 us
         # and some 200 us of Python; one launch 84 us)
+        if constants is None:
+            constants = (rotation.permutation.to(torch.int32).to(device), rotation.signs.to(torch.int8).to(device),
+                         codebook.boundaries.to(device))
         return ops.quantize_weight(
-            weight, rotation.permutation.to(torch.int32).to(device), rotation.signs.to(torch.int8).to(device),
-            codebook.boundaries.to(device), bits=bits, block_size=rotation.block_size, eps=eps,
+            weight, *constants, bits=bits, block_size=rotation.block_size, eps=eps,
             inv_sqrt_block=rotation.normalization)
     # Tiles must end on a byte boundary of the flat stream: rows * k * bits % 8 == 0.
     align = 8
