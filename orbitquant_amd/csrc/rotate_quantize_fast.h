@@ -7,9 +7,8 @@
 //   * a row is cut into units of max(block, 512) values; a wavefront owns whole units and keeps a
 //     unit in registers (block / 512 steps of 8 values per lane), so butterfly distances of 512
 //     and more are register operations too and nothing is regrouped through LDS;
-//   * lane exchanges are two instructions per value: DPP adds and subtracts restricted to the
-//     lower / upper lanes of a pair by their bank masks (distances 4 and 8 lanes), an exclusive-or
-//     plus a DPP add inside quads, lane-group swaps of register pairs for 16 and 32 lanes;
+//   * lane exchanges are one instruction per value inside sixteen lanes (a DPP multiply-add), one and a
+//     half for 16 and 32 lanes (lane-group swaps of register pairs, left swapped until the codes are packed);
 //   * permutation, sign, the 1/sqrt(block) factor and the bucketize table come from the plan;
 //     the signs are applied to the row as it is staged, four exclusive-ors for eight 16-bit values;
 //   * x / (s + eps) is four instructions: q = fma(x, rh, x * rl) with rh + rl = 1 / (s + eps) to
@@ -91,78 +90,81 @@ __host__ __device__ inline size_t fast_lds_bytes(int64_t K, int dtype) {
 }
 
 // ---- lane-exchange butterflies, eight values per call -------------------------------------------
-// y'[lane] = (lane & J) ? y[lane ^ J] - y[lane] : y[lane] + y[lane ^ J]
-// The leading s_nop covers the two wait states a DPP read needs after a vector write of the same
-// register (the values of the previous stage); inside a block eight other instructions separate
-// a value's write from its next DPP read.
-#define OQ_DPP_PAIR(ADD, SUB)                                                                      \
-  asm("s_nop 1\n\t" ADD(0) SUB(0) ADD(1) SUB(1) ADD(2) SUB(2) ADD(3) SUB(3) ADD(4) SUB(4) ADD(5) SUB(5) ADD(6) SUB(6) ADD(7) SUB(7) \
-      : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]), "=&v"(d[4]), "=&v"(d[5]), "=&v"(d[6]), "=&v"(d[7])                 \
-      : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]))
+// One instruction a value: y += s * y[partner], s = -1 in the upper lane of a pair and 1 in the lower one (the product is
+// exact, so it is the rounded sum or difference).  That leaves l + r in the lane that held r if it is the lower one, and
+// l - r in the lane that held l if it is the upper one: the inputs are gathered with the lane bits of these stages
+// inverted, and the outputs stand where they belong.  Partners within eight lanes are lane ^ 1, lane ^ 2 and lane ^ 7
+// (what a DPP operand reaches), so the bits that number a lane's slots are those of logical_lane().
+// (Two instructions a value, an exclusive-or or a second masked add with each DPP add, and swapping registers back after
+// the last two stages, took 28 vector instructions a value of a block of 4096 instead of 23.)
+__device__ __forceinline__ int logical_lane(int lane) { return lane ^ ((lane & 4) ? 3 : 0); }
 
-__device__ __forceinline__ void stage_xor4(float (&y)[kChunk]) {
-  float d[kChunk];
-#define OQ_A(i) "v_add_f32_dpp %" #i ", %" OQ_IN(i) ", %" OQ_IN(i) " row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-#define OQ_S(i) "v_sub_f32_dpp %" #i ", %" OQ_IN(i) ", %" OQ_IN(i) " row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
-#define OQ_IN(i) OQ_IN_##i
-#define OQ_IN_0 "8"
-#define OQ_IN_1 "9"
-#define OQ_IN_2 "10"
-#define OQ_IN_3 "11"
-#define OQ_IN_4 "12"
-#define OQ_IN_5 "13"
-#define OQ_IN_6 "14"
-#define OQ_IN_7 "15"
-  OQ_DPP_PAIR(OQ_A, OQ_S);
-#undef OQ_A
-#undef OQ_S
-#pragma unroll
-  for (int e = 0; e < kChunk; ++e) y[e] = d[e];
-}
+// The bits of the logical lane that the DPP stages of a block of H values go over.
+constexpr int inverted_lanes(int H) { return H > 64 ? 15 : H > 32 ? 7 : H > 16 ? 3 : H > 8 ? 1 : 0; }
 
-__device__ __forceinline__ void stage_xor8(float (&y)[kChunk]) {
-  float d[kChunk];
-#define OQ_A(i) "v_add_f32_dpp %" #i ", %" OQ_IN(i) ", %" OQ_IN(i) " row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-#define OQ_S(i) "v_sub_f32_dpp %" #i ", %" OQ_IN(i) ", %" OQ_IN(i) " row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-  OQ_DPP_PAIR(OQ_A, OQ_S);
-#undef OQ_A
-#undef OQ_S
-#pragma unroll
-  for (int e = 0; e < kChunk; ++e) y[e] = d[e];
-}
-
-// Inside a quad no mask tells the lower lane of a pair from the upper one: the upper lane's own
-// value is negated by an exclusive-or with `neg` (the sign bit in the upper lanes), then one DPP add.
-#define OQ_QUAD_STAGE(NAME, PERM)                                                                                     \
-  __device__ __forceinline__ void NAME(float (&y)[kChunk], uint32_t neg) {                                            \
-    float d[kChunk];                                                                                                  \
-    asm("v_xor_b32 %0, %16, %8\n\tv_xor_b32 %1, %16, %9\n\tv_xor_b32 %2, %16, %10\n\tv_xor_b32 %3, %16, %11\n\t"      \
-        "v_xor_b32 %4, %16, %12\n\tv_xor_b32 %5, %16, %13\n\tv_xor_b32 %6, %16, %14\n\tv_xor_b32 %7, %16, %15\n\t"    \
-        "v_add_f32_dpp %0, %8, %0 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                            \
-        "v_add_f32_dpp %1, %9, %1 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                            \
-        "v_add_f32_dpp %2, %10, %2 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        "v_add_f32_dpp %3, %11, %3 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        "v_add_f32_dpp %4, %12, %4 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        "v_add_f32_dpp %5, %13, %5 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        "v_add_f32_dpp %6, %14, %6 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        "v_add_f32_dpp %7, %15, %7 " PERM " row_mask:0xf bank_mask:0xf\n\t"                                           \
-        : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]), "=&v"(d[4]), "=&v"(d[5]), "=&v"(d[6]), "=&v"(d[7])      \
-        : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(y[4]), "v"(y[5]), "v"(y[6]), "v"(y[7]), "v"(neg));          \
-    _Pragma("unroll") for (int e = 0; e < kChunk; ++e) y[e] = d[e];                                                   \
+// The leading s_nop covers the two wait states a DPP read needs after a vector write of the same register; between two
+// stages of a block seven other instructions separate a value's write from its next DPP read.
+#define OQ_DPP1(i, S, PERM) "v_fmac_f32_dpp %" #i ", %" #i ", %" #S " " PERM " row_mask:0xf bank_mask:0xf\n\t"
+#define OQ_DPP8(S, PERM)                                                                                        \
+  OQ_DPP1(0, S, PERM) OQ_DPP1(1, S, PERM) OQ_DPP1(2, S, PERM) OQ_DPP1(3, S, PERM) OQ_DPP1(4, S, PERM) OQ_DPP1(5, S, PERM) \
+  OQ_DPP1(6, S, PERM) OQ_DPP1(7, S, PERM)
+#define OQ_EIGHT(y) "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7])
+template <int H>
+__device__ __forceinline__ void lane_stages(float (&y)[kChunk], float s1, float s2, float s4, float s8) {
+  if constexpr (H > 64) {
+    asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[1,0,3,2]") OQ_DPP8(9, "quad_perm:[2,3,0,1]") OQ_DPP8(10, "row_half_mirror") OQ_DPP8(11, "row_ror:8")
+        : OQ_EIGHT(y) : "v"(s1), "v"(s2), "v"(s4), "v"(s8));
+  } else {
+    if constexpr (H > 8) asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[1,0,3,2]") : OQ_EIGHT(y) : "v"(s1));
+    if constexpr (H > 16) asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[2,3,0,1]") : OQ_EIGHT(y) : "v"(s2));
+    if constexpr (H > 32) asm("s_nop 1\n\t" OQ_DPP8(8, "row_half_mirror") : OQ_EIGHT(y) : "v"(s4));
   }
-OQ_QUAD_STAGE(stage_xor1, "quad_perm:[1,0,3,2]")
-OQ_QUAD_STAGE(stage_xor2, "quad_perm:[2,3,0,1]")
-#undef OQ_QUAD_STAGE
-#undef OQ_DPP_PAIR
-#undef OQ_IN
-#undef OQ_IN_0
-#undef OQ_IN_1
-#undef OQ_IN_2
-#undef OQ_IN_3
-#undef OQ_IN_4
-#undef OQ_IN_5
-#undef OQ_IN_6
-#undef OQ_IN_7
+}
+#undef OQ_EIGHT
+#undef OQ_DPP8
+#undef OQ_DPP1
+
+// Butterflies between lanes 16 and 32 apart: registers e and e + 1 (e + 2) swap halves, lane for lane, and sum and
+// difference are register operations.  They stay swapped: of what register bit 0 (1) and lane bit 4 (5) number, each
+// now numbers the other's (codes are swapped back, four packed registers for eight values, by restore_lanes).
+template <int J>
+__device__ __forceinline__ void swapped_stage(float (&y)[kChunk]) {
+  constexpr int D = J == 16 ? 1 : 2;
+#pragma unroll
+  for (int e = 0; e < kChunk; ++e) {
+    if ((e & D) != 0) continue;
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 r;
+    if constexpr (J == 16) r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[e]), __float_as_uint(y[e + D]), false, false);
+    else r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(y[e + D]), false, false);
+    const float lo = __uint_as_float(r.x), hi = __uint_as_float(r.y);
+    y[e] = lo + hi;
+    y[e + D] = lo - hi;
+  }
+}
+
+// word[k]: code k in the lower half and code k + 4 in the upper one, of lanes whose registers swapped_stage left
+// swapped (H > 128: 16 lanes apart, H > 256: 32 as well).  Afterwards they are the codes k and k + 4 of the lane's own slots.
+template <int H>
+__device__ __forceinline__ void restore_lanes(uint32_t (&word)[4]) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  if constexpr (H > 128) {
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) {
+      const u32x2 r = __builtin_amdgcn_permlane16_swap(word[k], word[k + 1], false, false);
+      word[k] = r.x;
+      word[k + 1] = r.y;
+    }
+  }
+  if constexpr (H > 256) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const u32x2 r = __builtin_amdgcn_permlane32_swap(word[k], word[k + 2], false, false);
+      word[k] = r.x;
+      word[k + 2] = r.y;
+    }
+  }
+}
 
 __device__ __forceinline__ uint16_t lds_read_u16(uint32_t byte_addr) {
   return *reinterpret_cast<__attribute__((address_space(3))) const uint16_t *>(static_cast<uintptr_t>(byte_addr));
@@ -217,6 +219,7 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
   constexpr int N = CT * WB;             // values it turns into codes: 8 or 16
   static_assert(SPAN * WB == H && CT >= 1 && N % kChunk == 0);
   const int lane = tid & 63, wave = tid >> 6, team = wave / WB, teams = waves / WB, part = wave % WB;
+  const int slot_lane = logical_lane(lane);
   float *buffer = reinterpret_cast<float *>(smem + fast_lds_bytes(a.K, DT));  // [K]
   const bool plain = (modes & 1u) != 0u, searched = (modes & 2u) != 0u, signs_left = (modes & 4u) != 0u;
 #pragma nounroll
@@ -241,7 +244,7 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
     }
 #pragma unroll
     for (int j = 0; j < GW; ++j) {
-      float4 *dst = reinterpret_cast<float4 *>(buffer + first + j * kLaneSpan + lane * kChunk);
+      float4 *dst = reinterpret_cast<float4 *>(buffer + first + j * kLaneSpan + slot_lane * kChunk);
       dst[0] = make_float4(y[j][0], y[j][1], y[j][2], y[j][3]);
       dst[1] = make_float4(y[j][4], y[j][5], y[j][6], y[j][7]);
     }
@@ -334,6 +337,9 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   constexpr int G = H > kLaneSpan ? H / kLaneSpan : 1;  // steps of 512 values a unit is made of
   static_assert(WB == 1 || (!MAPPED && G % WB == 0 && (EMIT == EMIT_NIBBLE || EMIT == EMIT_U8)), "shared blocks: codes of unmapped rows");
   const int lane = tid & 63, wave = tid >> 6;
+  const int slot_lane = logical_lane(lane), slot_first = slot_lane * kChunk;       // the slots a lane ends up with
+  const int gather_first = (slot_lane ^ inverted_lanes(H)) * kChunk;               // and those whose inputs it starts from
+  constexpr bool kSwapped = WB == 1 && EMIT != EMIT_ANY && H > 128;                // codes are swapped back, not values
   const int64_t K = a.K;
   const plan::PlanHeader *hdr = reinterpret_cast<const plan::PlanHeader *>(a.plan);
   uint2 *cells = reinterpret_cast<uint2 *>(smem + kCellsAt);
@@ -381,7 +387,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   auto request_shared = [&](int u) {
 #pragma unroll
     for (int j = 0; j < GW; ++j) {
-      const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + lane * kChunk, Ki - kChunk));
+      const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + gather_first, Ki - kChunk));
       early_a[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
       early_b[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
     }
@@ -389,7 +395,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   if constexpr (WB > 1) request_shared(team);
   int4 ea_next, eb_next;
   auto request_entries = [&](int first) {
-    const uint32_t c = static_cast<uint32_t>(min(first + lane * kChunk, Ki - kChunk));
+    const uint32_t c = static_cast<uint32_t>(min(first + gather_first, Ki - kChunk));
     ea_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
     eb_next = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
   };
@@ -556,7 +562,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // clones the whole loop per combination.
   const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | ((EMIT == EMIT_WEIGHT ? hdr->weight_cells : hdr->cells) != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
-  const uint32_t neg1 = (lane & 1) ? 0x80000000u : 0u, neg2 = (lane & 2) ? 0x80000000u : 0u;
+  const float s1 = (slot_lane & 1) ? -1.0f : 1.0f, s2 = (slot_lane & 2) ? -1.0f : 1.0f;
+  const float s4 = (slot_lane & 4) ? -1.0f : 1.0f, s8 = (slot_lane & 8) ? -1.0f : 1.0f;
   float xv[kChunk];  // the gathered inputs of a step
 #pragma unroll
   for (int e = 0; e < kChunk; ++e) xv[e] = 0.0f;
@@ -590,7 +597,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       }
     }
     if (signs_left) {
-      const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(first + lane_first, Ki - kChunk));
+      const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(first + gather_first, Ki - kChunk));
       const uint32_t w[4] = {sg.x, sg.y, sg.z, sg.w};
 #pragma unroll
       for (int e = 0; e < kChunk; ++e) xv[e] = __uint_as_float(__float_as_uint(xv[e]) ^ (((e & 1) != 0 ? w[e / 2] : w[e / 2] << 16) & 0x80000000u));
@@ -606,12 +613,14 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       for (int e = 0; e < kChunk; ++e) out[e] = xv[e] / rc.d;
     }
     rq::fwht_regs<kChunk>(out, H);
-    if constexpr (H > 8) stage_xor1(out, neg1);
-    if constexpr (H > 16) stage_xor2(out, neg2);
-    if constexpr (H > 32) stage_xor4(out);
-    if constexpr (H > 64) stage_xor8(out);
-    if constexpr (H > 128) rq::swap_stage<16>(out);
-    if constexpr (H > 256) rq::swap_stage<32>(out);
+    lane_stages<H>(out, s1, s2, s4, s8);
+    if constexpr (kSwapped) {
+      swapped_stage<16>(out);
+      if constexpr (H > 256) swapped_stage<32>(out);
+    } else {
+      if constexpr (H > 128) rq::swap_stage<16>(out);
+      if constexpr (H > 256) rq::swap_stage<32>(out);
+    }
   };
   if constexpr (WB > 1) {
     rotate_shared_blocks<DT, H, EMIT, WB, GW>(a, smem, row, tid, waves, row_modes, cells, thr, cell_scale, cell_offset, codes_row,
@@ -660,7 +669,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     // bucketize against the folded thresholds and emit
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      const int c0 = unit_base + j * kLaneSpan + lane_first;  // >= K: an idle lane of the row's last unit
+      const int c0 = unit_base + j * kLaneSpan + slot_first;  // >= K: an idle lane of the row's last unit
       int code[kChunk];
       if constexpr (EMIT == EMIT_WEIGHT) {
         float unit[kChunk];
@@ -696,16 +705,20 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       } else {
         rq::bucketize_many<kChunk>(thr, a.levels_pow2, y[j], code);
       }
+      uint32_t word[4];  // codes e and e + 4 of the lane's slots
+      if constexpr (EMIT != EMIT_ANY) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) word[e] = (static_cast<uint32_t>(code[e + 4]) << 16) | static_cast<uint32_t>(code[e]);
+        if constexpr (kSwapped) restore_lanes<H>(word);
+      }
       if (c0 < Ki) {
         if constexpr (EMIT == EMIT_NIBBLE) {
-          uint32_t w = static_cast<uint32_t>(code[7]);
-#pragma unroll
-          for (int e = kChunk - 2; e >= 0; --e) w = (w << 4) | static_cast<uint32_t>(code[e]);  // one shift-or each
-          *reinterpret_cast<uint32_t *>(codes_row + static_cast<uint32_t>(c0) / 2u) = w;
+          *reinterpret_cast<uint32_t *>(codes_row + static_cast<uint32_t>(c0) / 2u) = (((((word[3] << 4) | word[2]) << 4) | word[1]) << 4) | word[0];
         } else if constexpr (EMIT == EMIT_U8) {
+          const uint32_t even = (word[1] << 8) | word[0], odd = (word[3] << 8) | word[2];
           uint2 w;
-          w.x = ((((static_cast<uint32_t>(code[3]) << 8) | code[2]) << 8 | code[1]) << 8) | code[0];
-          w.y = ((((static_cast<uint32_t>(code[7]) << 8) | code[6]) << 8 | code[5]) << 8) | code[4];
+          w.x = __builtin_amdgcn_perm(odd, even, 0x05040100u);
+          w.y = __builtin_amdgcn_perm(odd, even, 0x07060302u);
           *reinterpret_cast<uint2 *>(codes_row + static_cast<uint32_t>(c0)) = w;
         } else if constexpr (EMIT == EMIT_WEIGHT) {
           // eight indices = pack_bits whole bytes at a byte boundary of the stream (K is a multiple of 8)
@@ -713,9 +726,9 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
           uint32_t half[2];              // four indices each
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            half[h] = static_cast<uint32_t>(code[4 * h + 3]);
+            half[h] = h == 0 ? word[3] & 0xffffu : word[3] >> 16;
 #pragma unroll
-            for (int e = 2; e >= 0; --e) half[h] = (half[h] << bits) | static_cast<uint32_t>(code[4 * h + e]);
+            for (int e = 2; e >= 0; --e) half[h] = (half[h] << bits) | (h == 0 ? word[e] & 0xffffu : word[e] >> 16);
           }
           uint8_t *dst = a.packed + (row * K + c0) / 8 * bits;
           if (bits == 4 && a.packed_aligned) {

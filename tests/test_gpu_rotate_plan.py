@@ -91,6 +91,31 @@ def test_every_block_size(dev, log_h):
         assert torch.equal(packed, packed_plain)
 
 
+@pytest.mark.parametrize("log_h", range(3, 13))
+def test_every_block_size_in_byte_codes_and_weight_indices(dev, log_h):
+    """What a lane holds after the last stages (16 and 32 lanes apart) is not its own slots: codes are put back as they
+    are packed, by emitter and width.  The other weight widths have their own packing, 1000 rows their own kernel."""
+    from oracle import oracle_c, oracle_np
+    from orbitquant_amd import ops
+
+    h = 1 << log_h
+    k = max(h, 8) * 3
+    perm, signs, hh, inv, cents, bounds, t = constants(dev, k, h, 6)
+    for m in (19, 1100):
+        x = make_rows(m, k, torch.float16, seed=log_h)
+        (codes, _, _), _ = both_kernels(x.to(dev), t, h, inv, code_format="u8")
+        want, _ = oracle_c.rotate_quantize(x.float().numpy(), perm, signs, bounds, h, 1e-10, inv)
+        assert np.array_equal(codes.cpu().numpy(), want), (h, m)
+    for bits in (3, 4, 6, 8):
+        edges = np.linspace(-3, 3, 2 ** bits - 1).astype(np.float32) / np.float32(np.sqrt(k))
+        w = torch.randn(9, k, generator=torch.Generator().manual_seed(bits))
+        packed, norms = ops.quantize_weight(w.to(dev), t["perm"], t["signs"], torch.from_numpy(edges).to(dev), bits=bits, block_size=h,
+                                            eps=1e-10, inv_sqrt_block=float(inv))
+        want_packed, want_norms, _ = oracle_np.quantize_weight(w.numpy(), perm, signs, edges, h, 1e-10, bits, norm_order="sumsq_v1")
+        assert np.array_equal(packed.cpu().numpy(), want_packed), (h, bits)
+        assert torch.equal(norms.cpu(), want_norms)
+
+
 @pytest.mark.parametrize("k,h", [(520, 8), (1048, 8), (2056, 8), (24 * 64, 64), (17 * 128, 128), (9 * 256, 256)])
 def test_ragged_rows(dev, k, h):
     """Rows that are not a multiple of 512: the last unit has idle lanes."""
