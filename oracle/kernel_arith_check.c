@@ -8,6 +8,9 @@
  *                             (orbitquant_amd/csrc/rotate_quantize_fast.h, divide_fast), for the
  *                             operand ranges the kernel admits: 2^-80 <= |x| or x == 0, 2^-80 <= d <= 2^20,
  *                             |x| <= d * 2^9 (a value never exceeds the norm of its row)
+ *   oqk_short_quotient_mismatches  for x of 8 or 11 significant bits, q = fma(x, rh, x * rl) with rl = RN(fma(-d, rh, 1) / d)
+ *                             against x / d, over ALL significands of x and d (short_quotient_fails there lists the d
+ *                             for which some x is rounded wrongly)
  *   oqk_fold_threshold        the largest float t with RN(t * c) <= b, by bisection over the
  *                             ordered floats (rotate_quantize_fast.hip, rotate_plan_build_kernel)
  *
@@ -34,7 +37,7 @@ static float divide_fast(float x, float d, float rh, float rl) {
 /* mode 0: x has a bf16 significand (8 bits), 1: fp16 significand (11 bits), 2: any fp32 significand;
  * + 16: the control, a sequence that is NOT exact (the first quotient without its correction),
  * which this check must catch.  Every fourth denominator has a special significand (all ones, one, all ones but the last ...). */
-int64_t oqk_division_mismatches(int64_t pairs, uint64_t seed, int mode, float *first_x, float *first_d) {
+static int64_t sampled_mismatches(int64_t pairs, uint64_t seed, int mode, float *first_x, float *first_d, const uint32_t *skip, int64_t skips) {
   int64_t bad = 0;
 #pragma omp parallel for reduction(+ : bad) schedule(static)
   for (int64_t chunk = 0; chunk < 1024; ++chunk) {
@@ -58,8 +61,11 @@ int64_t oqk_division_mismatches(int64_t pairs, uint64_t seed, int mode, float *f
       if (xe < -80) xe = -80;
       const float x = from_bits(((uint32_t)(r2 >> 63) << 31) | ((uint32_t)(xe + 127) << 23) | xm);
       const float rh = 1.0f / d;
-      const float rl = fmaf(-d, rh, 1.0f) * rh;
-      const float want = x / d, got = (mode & 16) ? fmaf(x, rh, x * rl) : divide_fast(x, d, rh, rl);
+      const float rl = (mode & 32) ? fmaf(-d, rh, 1.0f) / d : fmaf(-d, rh, 1.0f) * rh;
+      int skipped = 0;
+      for (int64_t j = 0; j < skips; ++j) skipped |= skip[j] == dm;
+      if (skipped) continue;
+      const float want = x / d, got = (mode & 48) ? fmaf(x, rh, x * rl) : divide_fast(x, d, rh, rl);
       if (to_bits(want) != to_bits(got)) {
         if (bad == 0 && first_x != 0) { *first_x = x; *first_d = d; }
         ++bad;
@@ -67,6 +73,35 @@ int64_t oqk_division_mismatches(int64_t pairs, uint64_t seed, int mode, float *f
     }
   }
   return bad;
+}
+
+int64_t oqk_division_mismatches(int64_t pairs, uint64_t seed, int mode, float *first_x, float *first_d) {
+  return sampled_mismatches(pairs, seed, mode, first_x, first_d, 0, 0);
+}
+
+/* The short quotient on the same samples (modes 0 and 1), denominators with a significand in `skip` left out. */
+int64_t oqk_short_quotient_sample(int64_t pairs, uint64_t seed, int mode, float *first_x, float *first_d, const uint32_t *skip, int64_t skips) {
+  return sampled_mismatches(pairs, seed, mode | 32, first_x, first_d, skip, skips);
+}
+
+/* The denominators' significands for which some x of `xbits` significant bits gives a quotient that is not x / d, in
+ * ascending order into found[0 .. most); returns how many there are. */
+int64_t oqk_short_quotient_mismatches(int xbits, uint32_t *found, int64_t most) {
+  static unsigned char wrong[1 << 23];
+#pragma omp parallel for schedule(static)
+  for (int64_t m = 0; m < (1 << 23); ++m) {
+    const float d = from_bits(0x3f800000u | (uint32_t)m), rh = 1.0f / d, rl = fmaf(-d, rh, 1.0f) / d;
+    int bad = 0;
+    for (int i = 1 << (xbits - 1); i < (1 << xbits); ++i) {
+      const float x = (float)i;
+      bad |= fmaf(x, rh, x * rl) != x / d;
+    }
+    wrong[m] = (unsigned char)bad;
+  }
+  int64_t count = 0;
+  for (int64_t m = 0; m < (1 << 23); ++m)
+    if (wrong[m] && count++ < most) found[count - 1] = (uint32_t)m;
+  return count;
 }
 
 static uint32_t float_to_ordered(float f) { const uint32_t u = to_bits(f); return (u & 0x80000000u) ? ~u : (u | 0x80000000u); }

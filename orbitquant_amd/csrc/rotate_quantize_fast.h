@@ -14,7 +14,7 @@
 //   * x / (s + eps) is four instructions: q = fma(x, rh, x * rl) with rh + rl = 1 / (s + eps) to
 //     twice the working precision is a faithful quotient, and one residual correction
 //     fma(fma(-q, d, x), rh, q) with rh the correctly rounded reciprocal rounds it correctly
-//     (Markstein).  Rows whose magnitudes could make a residual inexact (a value below 2^-80, a
+//     (Markstein); 16-bit inputs do without it (short_quotient_fails).  Rows whose magnitudes could make a residual inexact (a value below 2^-80, a
 //     denominator outside [2^-80, 2^20], anything not finite) take the IEEE division instead;
 //     the test is one packed instruction pair per two bf16 values while the row is read.
 //
@@ -173,11 +173,27 @@ __device__ __forceinline__ uint16_t lds_read_u16(uint32_t byte_addr) {
 // ---- the division -------------------------------------------------------------------------------
 struct Reciprocal {
   float d, rh, rl;
-  bool plain;  // this row takes the IEEE division
 };
 __device__ __forceinline__ float divide_fast(float x, const Reciprocal &r) {
   const float q = __builtin_fmaf(x, r.rh, x * r.rl);
   return __builtin_fmaf(__builtin_fmaf(-q, r.d, x), r.rh, q);
+}
+
+// 16-bit inputs need no correction when rl is the rounded quotient of 1 - d rh and d.  x has 8 (fp16: 11) significant bits
+// and d 24, so x / d lies at least 2^-49 of itself from a midpoint of two floats, and q = fma(x, rh, x * rl) lies about as
+// close to x / d: which pairs it rounds wrongly was counted over all of them, 2^7 (2^10) by 2^23 significands.  They are
+// one x each of the d below, whose rows take the IEEE division (two instructions fewer a value: 4608 x 12288 66 -> 63 us).
+template <int DT>
+__device__ __forceinline__ bool short_quotient_fails(float d) {
+  const uint32_t m = __float_as_uint(d) & 0x7fffffu;
+  if constexpr (DT == OQ_F32) return false;
+  bool fails = m == 0x50ab43u || m == 0x792863u;
+  if constexpr (DT == OQ_F16) {
+    constexpr uint32_t more[10] = {0x5562afu, 0x56edffu, 0x59c6cbu, 0x5eca3fu, 0x6828ebu, 0x722cf3u, 0x742bcbu, 0x74458fu, 0x7453bbu, 0x7f3c33u};
+#pragma unroll
+    for (int i = 0; i < 10; ++i) fails = fails || m == more[i];
+  }
+  return fails;
 }
 
 // code = entry.count + (entry.threshold < value) for eight values: the compares first, into eight
@@ -540,8 +556,10 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   Reciprocal rc;
   rc.d = s_norm + a.eps;
   rc.rh = 1.0f / rc.d;
-  rc.rl = __builtin_fmaf(-rc.d, rc.rh, 1.0f) * rc.rh;
-  bool row_plain = !(rc.d >= 0x1p-80f && rc.d <= 0x1p20f);
+  constexpr bool kShortQuotient = DT != OQ_F32;
+  const float remainder = __builtin_fmaf(-rc.d, rc.rh, 1.0f);
+  rc.rl = kShortQuotient ? remainder / rc.d : remainder * rc.rh;
+  bool row_plain = !(rc.d >= 0x1p-80f && rc.d <= 0x1p20f) || short_quotient_fails<DT>(rc.d);
 #pragma nounroll
   for (int w = 0; w < min(waves, 4); ++w) row_plain = row_plain || red[4 + w] != 0.0f;
   if (tid == 0 && a.norms != nullptr) a.norms[row] = s_norm;
@@ -607,7 +625,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       for (int e = 0; e < kChunk; ++e) out[e] = xv[e];
     } else if (!plain) {
 #pragma unroll
-      for (int e = 0; e < kChunk; ++e) out[e] = divide_fast(xv[e], rc);
+      for (int e = 0; e < kChunk; ++e) out[e] = kShortQuotient ? __builtin_fmaf(xv[e], rc.rh, xv[e] * rc.rl) : divide_fast(xv[e], rc);
     } else {
 #pragma unroll
       for (int e = 0; e < kChunk; ++e) out[e] = xv[e] / rc.d;

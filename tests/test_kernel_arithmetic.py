@@ -25,6 +25,11 @@ def checks():
     f32p = ctypes.POINTER(ctypes.c_float)
     lib.oqk_division_mismatches.restype = ctypes.c_int64
     lib.oqk_division_mismatches.argtypes = [ctypes.c_int64, ctypes.c_uint64, ctypes.c_int, f32p, f32p]
+    u32p = ctypes.POINTER(ctypes.c_uint32)
+    lib.oqk_short_quotient_sample.restype = ctypes.c_int64
+    lib.oqk_short_quotient_sample.argtypes = [ctypes.c_int64, ctypes.c_uint64, ctypes.c_int, f32p, f32p, u32p, ctypes.c_int64]
+    lib.oqk_short_quotient_mismatches.restype = ctypes.c_int64
+    lib.oqk_short_quotient_mismatches.argtypes = [ctypes.c_int, u32p, ctypes.c_int64]
     lib.oqk_fold_threshold.restype = ctypes.c_float
     lib.oqk_fold_threshold.argtypes = [ctypes.c_float, ctypes.c_float]
     lib.oqk_fold_mismatches.restype = ctypes.c_int64
@@ -42,6 +47,25 @@ def test_four_instruction_division_is_the_ieee_quotient(checks, mode):
 def test_the_division_check_catches_an_inexact_sequence(checks):
     x, d = ctypes.c_float(), ctypes.c_float()
     assert checks.oqk_division_mismatches(200_000_000, 5, 16, ctypes.byref(x), ctypes.byref(d)) > 0
+
+
+SHORT_QUOTIENT_FAILS = {8: [0x50ab43, 0x792863],
+                        11: [0x50ab43, 0x5562af, 0x56edff, 0x59c6cb, 0x5eca3f, 0x6828eb, 0x722cf3, 0x742bcb, 0x74458f, 0x7453bb, 0x792863, 0x7f3c33]}
+
+
+@pytest.mark.parametrize("xbits", [8, 11])
+def test_quotients_of_16_bit_inputs_without_the_correction(checks, xbits):
+    """All significands: the denominators with a wrong quotient are those whose rows the kernel sends to the IEEE division.
+    And a sample over the admitted exponents, where products may be subnormal."""
+    found = (ctypes.c_uint32 * 64)()
+    count = checks.oqk_short_quotient_mismatches(xbits, found, 64)
+    assert list(found[:min(count, 64)]) == SHORT_QUOTIENT_FAILS[xbits]
+    source = (ROOT / "orbitquant_amd/csrc/rotate_quantize_fast.h").read_text()
+    assert all(f"0x{m:06x}u" in source for m in SHORT_QUOTIENT_FAILS[xbits])
+    x, d = ctypes.c_float(), ctypes.c_float()
+    skip = (ctypes.c_uint32 * count)(*SHORT_QUOTIENT_FAILS[xbits])
+    bad = checks.oqk_short_quotient_sample(300_000_000, 77, int(xbits == 11), ctypes.byref(x), ctypes.byref(d), skip, count)
+    assert bad == 0, f"{bad} quotients differ, first x={x.value!r} d={d.value!r}"
 
 
 @pytest.mark.parametrize("block", [8, 64, 128, 512, 2048, 4096])
