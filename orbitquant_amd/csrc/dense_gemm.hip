@@ -34,6 +34,7 @@ struct DenseArgs {
   int bias_dtype;
   int M, N, steps;           // steps of 128 operand bytes
   int tiles_m, tiles_n;
+  int whole;                 // tiles done as such; a workgroup after them does a part of one of the others (launch_dense)
   void *out;
   int out_dtype;
   OutMap out_map;
@@ -61,26 +62,15 @@ __device__ __forceinline__ T mfma_piece(uint4 w, uint4 a, T c) {
 // its bytes only behind a barrier that comes after this wait.
 constexpr int kCopiesArrived = 0x0f70;
 
+template <int FM, int FN> constexpr int kStageBytes = 2 * (FM + FN) * 4096;
+
+// One tile of 64 FM x 64 FN outputs, number (pid_m, pid_n) of its size.  `stage0` has room for the epilogue's kEpiLdsBytes.
 template <int MF, int FM, int FN>
-__global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
-  constexpr int kBlocks = 2 * (FM + FN), kStage = kBlocks * 4096;
+__device__ __forceinline__ void dense_tile(const DenseArgs &g, const int pid_m, const int pid_n, unsigned char *stage0, unsigned char *stage1) {
+  constexpr int kBlocks = 2 * (FM + FN);
   constexpr int kPerWave = (kBlocks + 3) / 4;
   constexpr int TM = 64 * FM, TN = 64 * FN;
-  // two LDS objects, not one array: the compiler then knows that a copy into one stage does not touch the operands
-  // being read from the other, and waits for neither
-  __shared__ __attribute__((aligned(1024))) unsigned char stage0[kStage > kEpiLdsBytes ? kStage : kEpiLdsBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char stage1[kStage];
-
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // consecutive tiles to the same XCD (workgroup ids go round-robin over the eight), any tile count
-  const int total = g.tiles_m * g.tiles_n;
-  const int xcd = blockIdx.x & 7, base = total >> 3, extra = total & 7;
-  const int bid = xcd * base + min(xcd, extra) + (static_cast<int>(blockIdx.x) >> 3);
-  constexpr int GROUP_M = 4;  // groups of four tile rows walked column by column
-  const int width = GROUP_M * g.tiles_n, group = bid / width, first_m = group * GROUP_M;
-  const int gsz = min(g.tiles_m - first_m, GROUP_M), in_group = bid - group * width;
-  const int pid_m = first_m + in_group % gsz, pid_n = in_group / gsz;
-
   const int wm = (wave >> 1) * FM, wn = (wave & 1) * FN;  // in tiles of 32
   const int a_tiles = (g.M + 31) / 32, w_tiles = (g.N + 31) / 32;
   const uint8_t *src[kPerWave];
@@ -210,15 +200,71 @@ __global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
                         g.row_scale, g.row_norms, g.bias, g.bias_dtype, epi, g.out, g.out_dtype, stage0, g.out_map, TM, nullptr);
 }
 
+// Tile `id` in the order in which neighbours share operands: groups of four tile rows walked column by column.
+__device__ __forceinline__ void tile_at(const DenseArgs &g, int id, int *pid_m, int *pid_n) {
+  constexpr int GROUP_M = 4;
+  const int width = GROUP_M * g.tiles_n, group = id / width, first_m = group * GROUP_M;
+  const int gsz = min(g.tiles_m - first_m, GROUP_M), in_group = id - group * width;
+  *pid_m = first_m + in_group % gsz;
+  *pid_n = in_group / gsz;
+}
+
+// SM, SN: the tiles after the first g.whole are cut into SM x SN parts of a workgroup each (1, 1: no tile is).
+template <int MF, int FM, int FN, int SM, int SN>
+__global__ __launch_bounds__(256, 1) void dense_gemm_kernel(DenseArgs g) {
+  constexpr int kStage = kStageBytes<FM, FN>;
+  // two LDS objects, not one array: the compiler then knows that a copy into one stage does not touch the operands
+  // being read from the other, and waits for neither
+  __shared__ __attribute__((aligned(1024))) unsigned char stage0[kStage > kEpiLdsBytes ? kStage : kEpiLdsBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char stage1[kStage];
+  // consecutive tiles to the same XCD (workgroup ids go round-robin over the eight), any tile count
+  auto spread = [](int block, int total) { return (block & 7) * (total >> 3) + min(block & 7, total & 7) + (block >> 3); };
+  const int block = static_cast<int>(blockIdx.x);
+  int pid_m, pid_n;
+  if (SM * SN == 1 || block < g.whole) {
+    tile_at(g, spread(block, g.whole), &pid_m, &pid_n);
+    dense_tile<MF, FM, FN>(g, pid_m, pid_n, stage0, stage1);
+  } else if constexpr (SM * SN > 1) {
+    const int part = spread(block - g.whole, (g.tiles_m * g.tiles_n - g.whole) * SM * SN);
+    tile_at(g, g.whole + part / (SM * SN), &pid_m, &pid_n);
+    pid_m = pid_m * SM + part % SM;
+    pid_n = pid_n * SN + part / SM % SN;
+    if (pid_m * (64 * FM / SM) >= g.M || pid_n * (64 * FN / SN) >= g.N) return;  // (a part wholly past the matrix; the whole workgroup leaves)
+    dense_tile<MF, FM / SM, FN / SN>(g, pid_m, pid_n, stage0, stage1);
+  }
+}
+
+template <int MF, int FM, int FN, int SM, int SN>
+int launch_parts(const DenseArgs &g, hipStream_t stream) {
+  const int64_t blocks = g.whole + (static_cast<int64_t>(g.tiles_m) * g.tiles_n - g.whole) * SM * SN;
+  auto kern = dense_gemm_kernel<MF, FM, FN, SM, SN>;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g);
+  return check_launch("dense_gemm");
+}
+
 template <int MF, int FM, int FN>
 int launch_dense(DenseArgs g, hipStream_t stream) {
   g.tiles_m = (g.M + 64 * FM - 1) / (64 * FM);
   g.tiles_n = (g.N + 64 * FN - 1) / (64 * FN);
   const int64_t total = static_cast<int64_t>(g.tiles_m) * g.tiles_n;
   if (total > 0x7fffffffLL) return fail(OQ_ERR_UNSUPPORTED, "dense_gemm: too many tiles");
-  auto kern = dense_gemm_kernel<MF, FM, FN>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(total)), dim3(256), 0, stream, g);
-  return check_launch("dense_gemm");
+  g.whole = static_cast<int>(total);
+  // The last round of 256 workgroups, one to a CU, takes as long for one tile as for 256.  Where it is at most half (a
+  // quarter) full its tiles are cut into two (four) parts, a workgroup each, which still are one round.  A part multiplies
+  // fewer values per operand byte (a K-step of 128 x 128 takes half as long as one of 256 x 256, not a quarter), so fuller
+  // rounds stay whole: 136 tiles of 256 x 256 in parts 252 -> 276 us.  Three-bit linears, passes included: 4608 x 12288 x 3072
+  // (96 tiles in the last round) 334 -> 321 us, 4352 x 12288 x 3072 (48) 326 -> 306 us, 6144 x 14336 x 4096 (64) 659 -> 630 us;
+  // 256 x 192: 3072 x 6144 x 4096 (128) 178 -> 170 us; 256 x 128: 4096 x 4608 x 4096 (64) 199 -> 191 us; int8, 4608 x 36864 x
+  // 4096 (32) 714 -> 695 us with its quantizer and passes.
+  if constexpr (FM == 4) {
+    const int rest = static_cast<int>(total % 256);
+    if (total > 256 && rest > 0 && rest <= 128) {
+      g.whole -= rest;
+      if constexpr (FN == 4) return rest <= 64 ? launch_parts<MF, FM, FN, 2, 2>(g, stream) : launch_parts<MF, FM, FN, 1, 2>(g, stream);
+      else return launch_parts<MF, FM, FN, 2, 1>(g, stream);
+    }
+  }
+  return launch_parts<MF, FM, FN, 1, 1>(g, stream);
 }
 
 template <int MF>
@@ -243,7 +289,8 @@ double launch_warmth(double operations) {
 // one to a CU (each part of the rows in rounds of its own), each with a fixed prologue and epilogue and a time per
 // K-step of 128 operand bytes that grows with the length of the launch (a step of the 256 x 256 tile: 0.96 us in bf16
 // at 2e10 operations, 1.14 us from 1e12 on) and by up to a quarter where the operands outgrow the 256 MB last-level
-// cache; on top come the passes, the output's way to memory and the launches.  Fitted to 5000 timings of single calls,
+// cache; on top come the passes, the output's way to memory and the launches.  (That a last round up to half full is cut
+// into parts is left out: launches that it would bring here keep the kernel they have.)  Fitted to 5000 timings of single calls,
 // 256 to 16384 in each dimension, all tiles (rms error 9 %); the tile it picks is 1 % behind the best one on average.
 int dense_choose_tile(int64_t M, int64_t N, int64_t K, int64_t rows_at_a_time, int mf, double pass_bytes, double *cost_out) {
   if (K % 64 != 0 || N % 8 != 0 || M > 0x7fff0000LL || N > 0x7fff0000LL || K > 0x0fffffffLL) return -1;

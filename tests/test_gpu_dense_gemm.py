@@ -66,6 +66,27 @@ def test_same_bits_as_the_packed_gemm(dev, library_switch, tile, m, k, n, wbits,
     assert torch.equal(multiply(o, m, k, n, wbits, abits, dtype, table), want)
 
 
+@pytest.mark.parametrize("tile,n", [(0, 4088), (0, 4728), (1, 3064), (2, 2040), (2, 2616)])
+def test_last_round_of_workgroups_in_parts(dev, library_switch, tile, n):
+    """More than 256 tiles and a last round that is at most half full: its tiles are cut into two parts or four, of which
+    some lie wholly past the matrix (seventeen rows of tiles, four rows in the last; columns likewise)."""
+    from orbitquant_amd import ops
+
+    m, k = 4100, 192
+    o = operands(dev, m, k, n, 3, 4, seed=n)
+    library_switch("OQ_GEMM_TILE", 0)
+    library_switch("OQ_DENSE_GEMM", "never")
+    want = multiply(o, m, k, n, 3, 4, torch.float32)
+    library_switch("OQ_DENSE_GEMM", tile)
+    assert torch.equal(multiply(o, m, k, n, 3, 4, torch.float32), want)
+    o = operands(dev, m, k, n, 4, 4, seed=n + 1)
+    table = torch.tensor(A_TABLE, dtype=torch.int8, device=dev)
+    got = ops.packed_linear_int8(o["codes"], o["norms"], table, o["packed"], o["rn"], table, scale=0.01, out_features=n, in_features=k,
+                                 output_dtype=torch.float32)
+    sums = (looked_up(o["codes"], m, k, table) @ looked_up(o["packed"], n, k, table).T).float()
+    assert torch.equal(got, sums * (o["norms"] * 0.01)[:, None] * o["rn"].float())
+
+
 def test_chosen_for_large_problems_only_and_only_with_a_workspace(dev):
     from orbitquant_amd import _lib, ops
 
