@@ -113,11 +113,13 @@ template <bool BYTES, int BITS, int R, int WAVES, bool LATE, bool ASTAGE = false
 __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *lds, int64_t group, Produce produce) {
   static_assert(!ASTAGE || (!BYTES && !LATE), "staged activation values: nibble codes that exist at launch");
   static_assert(MB == 1 || (!ASTAGE && !LATE), "several row blocks: plain launches with table lookups");
-  static_assert(R * MB <= WAVES, "every epilogue item (64 per row block and row step) needs a thread");
+  // the epilogue's items, 64 per row block and row step, are a thread each: kRounds rounds of kRoundBlocks row blocks
+  constexpr int kRounds = R * MB > WAVES ? R * MB / WAVES : 1, kRoundBlocks = MB / kRounds;
+  static_assert(kRoundBlocks * kRounds == MB && R * kRoundBlocks <= WAVES, "a round is whole row blocks");
   constexpr int kAVec = BYTES ? 2 : 1;      // 16-byte loads of activation codes per lane and K-step
   constexpr int kAStep = 64 * kAVec;        // bytes of one activation row per K-step of 128
-  static_assert(WAVES * MB * R * 64 * 16 <= kGemvTableBytes, "partial sums reuse the table block");
-  float *partial = reinterpret_cast<float *>(lds);  // [WAVES][MB][R][64][4], after the main loop
+  static_assert(WAVES * kRoundBlocks * R * 64 * 16 <= kGemvTableBytes, "partial sums reuse the table block");
+  float *partial = reinterpret_cast<float *>(lds);  // [WAVES][kRoundBlocks][R][64][4], after the main loop
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, grp = lane >> 4;
@@ -235,8 +237,8 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
     }
   };
 
-  // Epilogue operands of the item this thread will finish (item = tid when tid < 64*R*MB: row
-  // block tid / (64*R), row step (tid / 64) % R, accumulator lane tid % 64).  They
+  // Epilogue operands of the items this thread will finish (item = tid when tid < 64*R*kRoundBlocks: row
+  // block tid / (64*R) of the round, row step (tid / 64) % R, accumulator lane tid % 64).  They
   // are requested BEFORE the stream, by every thread, without a branch (clamped indices, a
   // readable stand-in address for an absent operand) and stay untouched, as raw bits, until the
   // epilogue.  A wavefront's loads return in order: a use of one of these values before the main
@@ -253,9 +255,11 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
   const uint32_t ep_bias_lo = *reinterpret_cast<const uint16_t *>(bias_at);
   const uint32_t ep_bias_hi = *reinterpret_cast<const uint16_t *>(bias_at + (bias_size - 2));
   const float *scale_at = has_scale ? g.row_scale : g.w_cents;
-  float ep_sc_raw[4];
+  float ep_sc_raw[kRounds][4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) ep_sc_raw[e] = scale_at[has_scale ? min(16 * ep_mb + 4 * (ep_l >> 4) + e, g.M - 1) : 0];
+  for (int p = 0; p < kRounds; ++p)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ep_sc_raw[p][e] = scale_at[has_scale ? min(16 * (p * kRoundBlocks + ep_mb) + 4 * (ep_l >> 4) + e, g.M - 1) : 0];
 
   // ---- then the packed stream ------------------------------------------------------
   // Batches in flight: two for the plain stream (decode of one overlaps the loads of the next);
@@ -327,43 +331,47 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
   for (int i = 0; i < NB; ++i) consume(s + i * kDepth, b[i], std::true_type{});
 
   // ---- cross-wave sum in LDS (the tables are dead), fixed order ------------------------
-  __syncthreads();
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+  for (int p = 0; p < kRounds; ++p) {
+    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < R; ++j)
-      *reinterpret_cast<float4 *>(partial + (((wave * MB + mb) * R + j) * 64 + lane) * 4) =
-          make_float4(acc[mb][j][0], acc[mb][j][1], acc[mb][j][2], acc[mb][j][3]);
-  __syncthreads();
-  // accumulator e of lane l in row block mb: token row 16*mb + 4*(l/16) + e, weight row l%16
-  if (tid < 64 * R * MB && ep_n < g.N) {
-    const int ep_item = ep_mb * R + ep_j;
-    float4 sum = *reinterpret_cast<const float4 *>(partial + (ep_item * 64 + ep_l) * 4);
-    for (int w = 1; w < WAVES; ++w) {
-      const float4 p = *reinterpret_cast<const float4 *>(partial + ((w * MB * R + ep_item) * 64 + ep_l) * 4);
-      sum.x += p.x; sum.y += p.y; sum.z += p.z; sum.w += p.w;
-    }
-    const float v[4] = {sum.x, sum.y, sum.z, sum.w};
-    const float ep_rn = bf16_bits_to_f32(static_cast<uint16_t>(ep_rn_bits));
-    const float ep_bv = has_bias ? dyn_bits_to_f32(bias_size == 4 ? (ep_bias_lo | (ep_bias_hi << 16)) : ep_bias_lo, g.bias_dtype) : 0.0f;
+    for (int mb = 0; mb < kRoundBlocks; ++mb)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = 16 * ep_mb + 4 * (ep_l >> 4) + e;
-      if (m >= g.M) continue;
-      float sc = has_scale ? ep_sc_raw[e] : 1.0f;
-      if constexpr (LATE) {  // produced by this launch: read where it is used
-        if (g.row_scale != nullptr) sc = g.row_scale[m];
+      for (int j = 0; j < R; ++j) {
+        const f32x4 &sums = acc[p * kRoundBlocks + mb][j];
+        *reinterpret_cast<float4 *>(partial + (((wave * kRoundBlocks + mb) * R + j) * 64 + lane) * 4) = make_float4(sums[0], sums[1], sums[2], sums[3]);
       }
-      const float y = v[e] * sc * ep_rn + ep_bv;
-      const int64_t o = static_cast<int64_t>(m) * g.N + ep_n;
-      if (g.out_dtype == OQ_F32) {
-        static_cast<float *>(g.out)[o] = y;
-      } else {
-        // (a launch of its own for the map took 3 - 4 us; here it is one two-byte load per value: a decoder layer's
-        // linears of one token as a graph 65.0 -> 62.6 us, of sixteen tokens launched eagerly 139 -> 132 us)
-        uint16_t bits = g.out_dtype == OQ_BF16 ? f32_to_bf16_bits(y) : f32_to_f16_bits(y);
-        if (g.out_map != nullptr) bits = g.out_map[bits];
-        static_cast<uint16_t *>(g.out)[o] = bits;
+    __syncthreads();
+    // accumulator e of lane l in row block mb: token row 16*mb + 4*(l/16) + e, weight row l%16
+    if (tid < 64 * R * kRoundBlocks && ep_n < g.N) {
+      const int ep_item = ep_mb * R + ep_j;
+      float4 sum = *reinterpret_cast<const float4 *>(partial + (ep_item * 64 + ep_l) * 4);
+      for (int w = 1; w < WAVES; ++w) {
+        const float4 q = *reinterpret_cast<const float4 *>(partial + ((w * kRoundBlocks * R + ep_item) * 64 + ep_l) * 4);
+        sum.x += q.x; sum.y += q.y; sum.z += q.z; sum.w += q.w;
+      }
+      const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+      const float ep_rn = bf16_bits_to_f32(static_cast<uint16_t>(ep_rn_bits));
+      const float ep_bv = has_bias ? dyn_bits_to_f32(bias_size == 4 ? (ep_bias_lo | (ep_bias_hi << 16)) : ep_bias_lo, g.bias_dtype) : 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = 16 * (p * kRoundBlocks + ep_mb) + 4 * (ep_l >> 4) + e;
+        if (m >= g.M) continue;
+        float sc = has_scale ? ep_sc_raw[p][e] : 1.0f;
+        if constexpr (LATE) {  // produced by this launch: read where it is used
+          if (g.row_scale != nullptr) sc = g.row_scale[m];
+        }
+        const float y = v[e] * sc * ep_rn + ep_bv;
+        const int64_t o = static_cast<int64_t>(m) * g.N + ep_n;
+        if (g.out_dtype == OQ_F32) {
+          static_cast<float *>(g.out)[o] = y;
+        } else {
+          // (a launch of its own for the map took 3 - 4 us; here it is one two-byte load per value: a decoder layer's
+          // linears of one token as a graph 65.0 -> 62.6 us, of sixteen tokens launched eagerly 139 -> 132 us)
+          uint16_t bits = g.out_dtype == OQ_BF16 ? f32_to_bf16_bits(y) : f32_to_f16_bits(y);
+          if (g.out_map != nullptr) bits = g.out_map[bits];
+          static_cast<uint16_t *>(g.out)[o] = bits;
+        }
       }
     }
   }

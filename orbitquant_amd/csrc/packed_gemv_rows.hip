@@ -2,8 +2,8 @@
 // of sixteen token rows per workgroup (MB), so that the weights are still streamed and decoded
 // once.  The tile kernel is the wrong tool there: its 128-row tiles are mostly padding, and a
 // short-and-long matrix (4096 rows of 14336 values) gives it 32 workgroups for 256 CUs.
-// Launch shapes (rows per workgroup, K-split) follow the rule of the sixteen-token launches, so a
-// token row's sums do not depend on how many rows are computed with it.
+// The K-split follows the rule of the sixteen-token launches, so a token row's sums do not depend on
+// how many rows are computed with it.
 #include "packed_gemv_body.h"
 
 namespace oq {
@@ -30,8 +30,15 @@ template <bool BYTES, int BITS, int MB>
 int launch_shape(const GemvArgs &g, hipStream_t stream) {
   const int waves = gemv_waves(g.N, g.K);
   if (waves == 16) return launch<BYTES, BITS, 1, 16, MB>(g, stream);
-  if (g.N <= 16 * 512) return launch<BYTES, BITS, 1, 8, MB>(g, stream);
-  return launch<BYTES, BITS, 2, 8, MB>(g, stream);
+  // As many rows a workgroup as leave one workgroup a CU: MB operands of activations are looked up for every R of
+  // weights (values of a byte-code operand twice as dearly), and two workgroups on a CU look the activations up twice.  With 16
+  // rows up to N = 8192 and 32 from there: 33 tokens 4096 x 14336 26.3 -> 22.5 us, 2048 x 8192 16.0 -> 14.3 us, 6-bit
+  // activations 3072 x 12288 32.6 -> 24.4 us; 17 tokens 8192 x 8192 23.6 -> 22.0 us, 4096 x 14336 19.0 -> 19.2 us.  Beyond
+  // 64 rows a CU a second round starts either way, and smaller steps fill it better: 17 tokens 4096 x 18432 23.4 us on
+  // 32 rows, 28.4 on 64.  The sums do not depend on it.
+  if (g.N <= 16 * 256) return launch<BYTES, BITS, 1, 8, MB>(g, stream);
+  if (g.N <= 32 * 256 || g.N > 64 * 256) return launch<BYTES, BITS, 2, 8, MB>(g, stream);
+  return launch<BYTES, BITS, 4, 8, MB>(g, stream);
 }
 
 template <bool BYTES, int BITS>

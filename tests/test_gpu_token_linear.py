@@ -225,3 +225,23 @@ def test_shared_input_quantization_under_inference_mode(dev, monkeypatch):
         got = [layer(x) for layer in (q, k)]
     assert len(calls) == 2
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("n", [1040, 4104, 8200, 14328, 16400])
+@pytest.mark.parametrize(("m", "wbits", "abits"), [(17, 4, 4), (33, 3, 4), (64, 2, 3), (47, 4, 6)])
+def test_a_row_among_many_is_what_it_is_among_sixteen(dev, m, n, wbits, abits):
+    """17 to 64 tokens: 16, 32 or 64 weight rows a workgroup, one or two rounds of sums (33 tokens on 64 rows), the last
+    workgroup ragged.  The split of K is that of sixteen tokens, and so are the bits."""
+    from orbitquant_amd import ops
+
+    k = 1152
+    c = make_case(dev, m, k, n, wbits, abits, torch.bfloat16, "paper", True, seed=m + n)
+    fmt = "nibble" if abits <= 4 else "u8"
+    codes, _, norms = ops.rotate_quantize(c["x"], c["perm"], c["signs"], c["bounds"], code_format=fmt, **c["kw"])
+
+    def multiply(rows):
+        return ops.packed_linear(codes[rows].contiguous(), norms[rows].contiguous(), c["cents"], c["packed"], c["rn"], c["wcents"], code_format=fmt,
+                                 activation_bits=abits, weight_bits=wbits, out_features=n, in_features=k, bias=c["bias"], output_dtype=torch.float32)
+
+    want = torch.cat([multiply(slice(at, min(at + 16, m))) for at in range(0, m, 16)])
+    assert torch.equal(multiply(slice(0, m)), want)
