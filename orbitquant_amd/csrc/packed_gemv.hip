@@ -55,8 +55,10 @@ int launch_waves(const GemvArgs &g, int waves, hipStream_t stream) {
 
 template <bool BYTES, int BITS>
 int launch_bits(const GemvArgs &g, hipStream_t stream) {
-  // rows per workgroup (16*R) and K-split (wavefronts per workgroup); OQ_GEMV_CFG="R,WAVES" overrides
-  int r = g.N <= 16 * 512 ? 1 : 2, waves = gemv_waves(g.N, g.K);
+  // rows per workgroup (16*R) and K-split (wavefronts per workgroup); OQ_GEMV_CFG="R,WAVES" overrides.  Beyond 4096 rows
+  // a CU has more than one workgroup of sixteen rows, and each decodes the activations: on 32 rows 4 tokens 4096 x 8192
+  // 13.8 -> 12.5 us with the quantizer, 8 tokens 2048 x 8192 12.5 -> 11.0 us, 16 tokens 1152 x 4608 10.8 -> 10.4 us; 64 rows lose (15 % there).
+  int r = g.N <= 16 * 256 ? 1 : 2, waves = gemv_waves(g.N, g.K);
   if (const char *cfg = debug_env(ENV_GEMV_CFG)) {
     int cr = 0, cw = 0;
     if (sscanf(cfg, "%d,%d", &cr, &cw) == 2 && (cr == 1 || cr == 2 || cr == 4) && (cw == 4 || cw == 8 || cw == 16)) {
