@@ -108,7 +108,7 @@ def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[s
     copy that nothing waits for: the tensors are views of it, 256 bytes apart or more.  (A copy each is a synchronization
     each, which waits for everything the stream was given before:
     a weight of 14336 x 4096 converted and read back 287 -> 149 us.)"""
-    if device.type != "cuda":
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():   # (a graph would read the buffer again at each replay)
         return {name: t.to(device) for name, t in tensors.items()}
     starts, total = {}, 0
     for name, t in tensors.items():

@@ -91,3 +91,21 @@ def test_under_fake_tensors(layer):
     with FakeTensorMode(allow_non_fake_inputs=True) as mode:
         y = layer(mode.from_tensor(torch.empty(3, 384, dtype=torch.bfloat16, device="meta")).to("cuda"))
         assert y.shape == (3, 136) and y.dtype == torch.bfloat16
+
+
+def test_constants_made_under_capture_are_not_one_buffer(monkeypatch):
+    """A captured copy would read the pinned buffer again at each replay, when it holds something else: there the copies
+    are the blocking ones, which a capture refuses."""
+    from orbitquant_amd import layers
+
+    tensors = {"a": torch.arange(5, dtype=torch.int32), "b": torch.ones(3)}
+    device = torch.device("cuda:0")
+
+    def shared():
+        there = layers._on_device(tensors, device)
+        assert all(torch.equal(there[name].cpu(), t) for name, t in tensors.items())
+        return there["a"].untyped_storage().data_ptr() == there["b"].untyped_storage().data_ptr()
+
+    assert shared()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert not shared()
