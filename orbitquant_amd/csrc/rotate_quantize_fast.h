@@ -103,7 +103,9 @@ __device__ __forceinline__ int logical_lane(int lane) { return lane ^ ((lane & 4
 constexpr int inverted_lanes(int H) { return H > 64 ? 15 : H > 32 ? 7 : H > 16 ? 3 : H > 8 ? 1 : 0; }
 
 // The leading s_nop covers the two wait states a DPP read needs after a vector write of the same register; between two
-// stages of a block seven other instructions separate a value's write from its next DPP read.
+// stages of a block seven other instructions separate a value's write from its next DPP read.  The closing one covers the
+// same two before a lane-group swap: the compiler keeps them behind its own instructions, but does not see what a block
+// writes (without it a swap came one scalar instruction behind the write of its operand wherever the scheduler put it there).
 #define OQ_DPP1(i, S, PERM) "v_fmac_f32_dpp %" #i ", %" #i ", %" #S " " PERM " row_mask:0xf bank_mask:0xf\n\t"
 #define OQ_DPP8(S, PERM)                                                                                        \
   OQ_DPP1(0, S, PERM) OQ_DPP1(1, S, PERM) OQ_DPP1(2, S, PERM) OQ_DPP1(3, S, PERM) OQ_DPP1(4, S, PERM) OQ_DPP1(5, S, PERM) \
@@ -112,7 +114,7 @@ constexpr int inverted_lanes(int H) { return H > 64 ? 15 : H > 32 ? 7 : H > 16 ?
 template <int H>
 __device__ __forceinline__ void lane_stages(float (&y)[kChunk], float s1, float s2, float s4, float s8) {
   if constexpr (H > 64) {
-    asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[1,0,3,2]") OQ_DPP8(9, "quad_perm:[2,3,0,1]") OQ_DPP8(10, "row_half_mirror") OQ_DPP8(11, "row_ror:8")
+    asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[1,0,3,2]") OQ_DPP8(9, "quad_perm:[2,3,0,1]") OQ_DPP8(10, "row_half_mirror") OQ_DPP8(11, "row_ror:8") "s_nop 1"
         : OQ_EIGHT(y) : "v"(s1), "v"(s2), "v"(s4), "v"(s8));
   } else {
     if constexpr (H > 8) asm("s_nop 1\n\t" OQ_DPP8(8, "quad_perm:[1,0,3,2]") : OQ_EIGHT(y) : "v"(s1));
@@ -313,6 +315,8 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
 #pragma unroll
       for (int e = 0; e < kChunk; ++e) code[at + e] = eight[e];
     }
+    // (one code a part and lane goes to its neighbours by DPP below, straight from count_below's additions: the wait states, as in lane_stages)
+    if constexpr (CT == 1 && EMIT == EMIT_NIBBLE) asm("s_nop 1" : "+v"(code[0]), "+v"(code[1]), "+v"(code[2]), "+v"(code[3]), "+v"(code[4]), "+v"(code[5]), "+v"(code[6]), "+v"(code[7]));
 #pragma unroll
     for (int v = 0; v < WB; ++v) {
       constexpr int kBits = EMIT == EMIT_NIBBLE ? 4 : 8;
