@@ -113,7 +113,7 @@ def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[s
     for name, t in tensors.items():
         starts[name] = total
         total += (t.numel() * t.element_size() + 255) & -256
-    host = torch.empty(total, dtype=torch.uint8, pin_memory=True)
+    host = torch.empty(total, dtype=torch.uint8, device="cpu", pin_memory=True)   # (whatever the default device is)
     for name, t in tensors.items():
         host[starts[name] : starts[name] + t.numel() * t.element_size()].view(t.dtype).copy_(t.reshape(-1))
     there = host.to(device, non_blocking=True)

@@ -109,3 +109,18 @@ def test_constants_made_under_capture_are_not_one_buffer(monkeypatch):
     assert shared()
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     assert not shared()
+
+
+def test_layers_are_made_and_moved_under_a_default_device():
+    """`torch.device("cuda")` as a context: what torch makes without a device is on the GPU, pinned memory is not."""
+    from orbitquant_amd import OrbitLinear, recipe
+
+    config = recipe("w4a4")
+    host = OrbitLinear.from_linear(torch.nn.Linear(384, 136), config=config)
+    weight = torch.randn(136, 384, device="cuda").bfloat16()
+    want = OrbitLinear.from_weight(weight, bias=None, config=config)   # (and the caches are filled)
+    x = torch.randn(3, 384, device="cuda").bfloat16()
+    with torch.device("cuda"):
+        got = OrbitLinear.from_weight(weight, bias=None, config=config)
+        assert torch.equal(got(x), want(x)) and torch.equal(got.to(torch.bfloat16).cuda()(x), want(x))
+        assert host.cuda()(x).shape == (3, 136)
