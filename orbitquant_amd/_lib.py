@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(os.environ.get("ORBITQUANT_HIP_LIB") or Path(__file__).resolve().parent / "liborbitquant_hip.so")
@@ -27,6 +28,7 @@ EXPORTS = (
 
 _lib = None
 _torch_ops = None   # the compiled module of the custom ops (csrc/torch_ops.cpp), or the ImportError that kept it away
+_warned = False
 
 
 class OrbitQuantHipError(RuntimeError):
@@ -116,7 +118,8 @@ def _bind(lib: ctypes.CDLL) -> None:
 
 
 def torch_ops():
-    """The compiled module that implements the custom ops on the GPU; raises where it is not built."""
+    """The compiled module that implements the custom ops on the GPU; None where it is not built, or built for another
+    torch: the same calls then go through Python, to the same kernels."""
     global _torch_ops
     if _torch_ops is None:
         try:
@@ -127,22 +130,25 @@ def torch_ops():
             _torch_ops = module
             if _lib is not None:
                 _bind(_lib)
-    if isinstance(_torch_ops, ImportError):
-        raise OrbitQuantHipError(f"the custom ops' compiled module is missing or of another torch ({_torch_ops}): "
-                                 "build it with `python -m orbitquant_amd.build`")
-    return _torch_ops
+    return None if isinstance(_torch_ops, ImportError) else _torch_ops
 
 
-def register_gpu_ops(library, names: tuple[str, ...]) -> None:
-    """Loads the module, which registers the ops' GPU implementations; where it cannot be loaded, `names` raise when
-    they are called on a GPU (importing the package needs no build)."""
-    try:
-        torch_ops()
-    except OrbitQuantHipError:
-        def missing(*args, **kwargs):
-            torch_ops()
-        for name in names:
-            library.impl(name, missing, "CUDA")
+def warn_without_torch_ops() -> None:
+    global _warned
+    if not _warned:
+        _warned = True
+        warnings.warn(f"the custom ops' compiled module is missing or of another torch ({_torch_ops}): calls take some "
+                      "microseconds more; build it with `python -m orbitquant_amd.build`", RuntimeWarning, stacklevel=3)
+
+
+def register_gpu_op(library, name: str, in_python) -> None:
+    """The GPU implementation of a custom op: the compiled module's, which its loading registers, or where that cannot
+    be loaded `in_python`."""
+    if torch_ops() is None:
+        def call(*args, **kwargs):
+            warn_without_torch_ops()
+            return in_python(*args, **kwargs)
+        library.impl(name, call, "CUDA")
 
 
 def check(rc: int, what: str) -> None:

@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from . import ops
+from . import _lib, ops
 from .config import OrbitQuantConfig
 from .packing import pack_lowbit, packed_length
 
@@ -62,6 +62,7 @@ def _adaln_fake(x, packed_weight, scales, bias, out_features, in_features, group
 
 
 _LIB.impl("adaln_int4_linear_general", _adaln_forward, "CUDA")
+_lib.register_gpu_op(_LIB, "adaln_int4_linear", _adaln_forward)
 torch.library.register_fake("orbitquant_amd::adaln_int4_linear", _adaln_fake, lib=_LIB)
 _adaln_int4_linear = torch.ops.orbitquant_amd.adaln_int4_linear.default
 

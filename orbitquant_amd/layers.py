@@ -84,7 +84,7 @@ def _quantized_linear_fake(
 
 
 _LIB.impl("quantized_linear_general", quantized_linear_forward, "CUDA")
-_lib.register_gpu_ops(_LIB, ("quantized_linear", "adaln_int4_linear"))
+_lib.register_gpu_op(_LIB, "quantized_linear", quantized_linear_forward)
 torch.library.register_fake("orbitquant_amd::quantized_linear", _quantized_linear_fake, lib=_LIB)
 _quantized_linear = torch.ops.orbitquant_amd.quantized_linear.default   # (the overload itself: no lookup per call)
 

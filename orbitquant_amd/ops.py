@@ -545,10 +545,14 @@ def quantized_linear_group(
     _require_gpu(x, "x")
     weights = list(weights)
     # (the usual call, without Python per matrix; None: an operand to convert or copy, or an error to name)
-    outs = _lib.torch_ops().quantized_linear_group(x, permutation, signs, boundaries, act_centroids, weights, int(block_size), float(eps),
-                                                   float(inv_sqrt_block), int(activation_bits), input_map, plan)
-    if outs is not None:
-        return outs
+    module = _lib.torch_ops()
+    if module is None:
+        _lib.warn_without_torch_ops()
+    else:
+        outs = module.quantized_linear_group(x, permutation, signs, boundaries, act_centroids, weights, int(block_size), float(eps),
+                                             float(inv_sqrt_block), int(activation_bits), input_map, plan)
+        if outs is not None:
+            return outs
     dim = x.shape[-1]
     rows = x if x.dim() == 2 and x.is_contiguous() else x.contiguous().reshape(-1, dim)
     m = rows.shape[0]

@@ -3,6 +3,10 @@ refusals."""
 
 from __future__ import annotations
 
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -124,3 +128,26 @@ def test_layers_are_made_and_moved_under_a_default_device():
         got = OrbitLinear.from_weight(weight, bias=None, config=config)
         assert torch.equal(got(x), want(x)) and torch.equal(got.to(torch.bfloat16).cuda()(x), want(x))
         assert host.cuda()(x).shape == (3, 136)
+
+
+def test_without_the_compiled_module():
+    """Forwards of every kind are those of the general implementations, where they raised (another process: the ops are
+    registered when the package is imported)."""
+    program = """
+import sys
+sys.modules["orbitquant_amd._torch_ops"] = None      # importing it raises ImportError
+import torch
+from orbitquant_amd import OrbitLinear, OrbitLinearGroup, RTNInt4Linear, recipe
+torch.manual_seed(0)
+linears = [OrbitLinear.from_linear(torch.nn.Linear(384, n), config=recipe("w4a4")).cuda() for n in (136, 64)]
+adaln = RTNInt4Linear.from_linear(torch.nn.Linear(384, 136), config=recipe("w4a4")).cuda()
+for m in (1, 40):
+    x = torch.randn(m, 384, device="cuda").bfloat16()
+    alone = [l(x) for l in linears]
+    assert all(torch.equal(a, b) for a, b in zip(OrbitLinearGroup(*linears)(x), alone)) and alone[0].shape == (m, 136)
+    general = torch.ops.orbitquant_amd.adaln_int4_linear_general
+    assert torch.equal(adaln(x), general(x, adaln.packed_weight, adaln.scales, adaln.bias, 136, 384, adaln.group_size))
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=Path(__file__).resolve().parent.parent, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stderr
+    assert "RuntimeWarning" in done.stderr

@@ -8,6 +8,8 @@ import ctypes
 import hashlib
 import json
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -251,3 +253,33 @@ def test_the_wrappers_do_without_private_names_of_torch(monkeypatch):
     assert module._current_device is torch.cuda.current_device
     monkeypatch.setattr(torch.cuda, "current_stream", lambda index: type("Stream", (), {"cuda_stream": 100 + index})())
     assert module._stream(type("Tensor", (), {"device": torch.device("cuda", 3)})()) == 103
+
+
+def test_the_ops_run_in_python_where_their_compiled_module_cannot_be_loaded():
+    """Another torch, or no build of it: the package imports, and the ops' GPU implementations are the Python ones, which
+    say so once.  (Another process: the ops are registered when the package is imported.)"""
+    program = """
+import sys, warnings
+sys.modules["orbitquant_amd._torch_ops"] = None      # importing it raises ImportError
+warnings.simplefilter("error")
+import torch
+from orbitquant_amd import _lib, adaln, layers, ops
+assert _lib.torch_ops() is None
+names = ("quantized_linear", "quantized_linear_general", "adaln_int4_linear", "adaln_int4_linear_general")
+assert all(torch._C._dispatch_has_kernel_for_dispatch_key("orbitquant_amd::" + name, "CUDA") for name in names)
+
+class Library:
+    def impl(self, name, function, key):
+        self.registered = name, function, key
+
+library = Library()
+_lib.register_gpu_op(library, "an_op", lambda *args, **kwargs: (args, kwargs))
+name, function, key = library.registered
+assert (name, key) == ("an_op", "CUDA")
+warnings.simplefilter("always")
+with warnings.catch_warnings(record=True) as said:
+    assert function(1, x=2) == function(1, x=2) == ((1,), {"x": 2})
+assert len(said) == 1 and "orbitquant_amd.build" in str(said[0].message)
+"""
+    done = subprocess.run([sys.executable, "-c", program], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr
