@@ -181,6 +181,16 @@ Tensor adaln_int4_linear(const Tensor &x, const Tensor &packed, const Tensor &sc
   return rc == OQ_OK ? out : general();
 }
 
+// A tuple of the six things that make up a matrix, of the types that the casts below take.
+bool entry_usable(PyObject *w) {
+  if (!PyTuple_Check(w) || PyTuple_GET_SIZE(w) != 6) return false;
+  for (const int i : {0, 1, 2})
+    if (!THPVariable_Check(PyTuple_GET_ITEM(w, i))) return false;
+  for (const int i : {3, 4})
+    if (!PyLong_Check(PyTuple_GET_ITEM(w, i))) return false;
+  return PyTuple_GET_ITEM(w, 5) == Py_None || THPVariable_Check(PyTuple_GET_ITEM(w, 5));
+}
+
 // `ops.quantized_linear_group` for the usual call; None: the Python side.  `weights`: its list of (packed, row norms,
 // centroids, bits, rows, bias).
 pybind11::object quantized_linear_group(const Tensor &x, const Tensor &permutation, const Tensor &signs, const Tensor &act_boundaries,
@@ -200,6 +210,7 @@ pybind11::object quantized_linear_group(const Tensor &x, const Tensor &permutati
   uint64_t need = 0;
   std::vector<Tensor> keep;
   for (size_t i = 0; i < count; ++i) {
+    if (!entry_usable(weights[i].ptr())) return pybind11::none();
     const pybind11::tuple w = weights[i];
     const Tensor p = w[0].cast<Tensor>(), n = w[1].cast<Tensor>(), c = w[2].cast<Tensor>();
     const OptTensor b = w[5].is_none() ? OptTensor() : OptTensor(w[5].cast<Tensor>());

@@ -151,3 +151,29 @@ for m in (1, 40):
     done = subprocess.run([sys.executable, "-c", program], cwd=Path(__file__).resolve().parent.parent, capture_output=True, text=True, timeout=100)
     assert done.returncode == 0, done.stderr
     assert "RuntimeWarning" in done.stderr
+
+
+def test_group_entries_of_other_forms(layer):
+    """What is no tuple of six tensors and plain numbers is the Python implementation's to take or to refuse."""
+    import numpy as np
+
+    from orbitquant_amd import ops
+
+    x = torch.randn(5, 384, device="cuda").bfloat16()
+    entry = (layer.packed_weight_indices, layer.row_norms, layer._weight_codebook_centroids, 4, 136, None)
+
+    def call(*weights):
+        return ops.quantized_linear_group(
+            x, layer._rotation_permutation, layer._rotation_signs, layer._activation_codebook_boundaries, layer._activation_codebook_centroids,
+            weights, block_size=layer.rotation.block_size, eps=layer.activation_eps, inv_sqrt_block=layer.rotation.normalization,
+            activation_bits=4, plan=layer._rotation_plan)
+
+    want, = call(entry)
+    for other in (list(entry), (*entry[:3], np.int64(4), np.int32(136), None)):
+        got, same = call(other, entry)
+        assert torch.equal(got, want) and torch.equal(same, want)
+    for wrong in ((*entry, None), entry[:5]):
+        with pytest.raises(ValueError, match="unpack"):
+            call(entry, wrong)
+    with pytest.raises(AttributeError):
+        call((None, *entry[1:]))
