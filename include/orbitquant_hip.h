@@ -80,8 +80,9 @@ const char *oq_version(void);
  * centroids    fp32 [levels]; only read when values_mode != OQ_VALUES_NONE (else may be NULL)
  * block        power of two dividing K;  K <= 16384
  * rotate_plan  NULL, or the plan oq_rotate_plan_build made from these perm, signs, boundaries,
- *              levels, K, block and inv_sqrt_block: launches of more than 16 rows then take the
- *              plan-based kernel (a third of the instructions, the same results bit for bit)
+ *              levels, K, block and inv_sqrt_block: launches of more than 16 rows, and fewer where a row
+ *              has several blocks or blocks of 1024 to 4096, then take the plan-based kernel (a third of
+ *              the instructions, the same results bit for bit)
  * codes_out    NULL or [M, K] u8 / [M, K/2] u8 per code_format
  * values_out   NULL or per values_mode
  * norms_out    fp32 [M]: the raw norm s (no eps); may be NULL
@@ -124,7 +125,10 @@ int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *
  *
  * w            [N, K] of w_dtype, row-major, 16-byte aligned;  K a multiple of 8, K <= 16384
  * rotate_plan  the plan oq_rotate_plan_build made from the layer's perm and signs with THESE
- *              boundaries, levels, K, block and inv_sqrt_block (only its gather entries are used)
+ *              boundaries, levels, K, block and inv_sqrt_block.  Its bucketize table is used where it is
+ *              one over `boundaries`; a plan of the same perm, signs, levels, K and block over others (the
+ *              layer's activation plan, say) gives the same indices from a search (14336 x 4096 into four bits:
+ *              108 us instead of 89, a plan's launch included)
  * boundaries   fp32 [levels-1] of the weight codebook;  2 <= levels <= 2^bits, 1 <= bits <= 8
  * block        power of two dividing K, 8 <= block <= 4096
  */

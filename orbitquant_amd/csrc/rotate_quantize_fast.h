@@ -79,7 +79,7 @@ inline void fast_args_fill(FastArgs &a, const void *x, int64_t M, int64_t K, con
 }
 
 // LDS: cells (2048) | thresholds (1024) | centroids (1024) | reduction slots (64) | staging
-constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then four flags
+constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then five flags
 
 // The row is staged once, in its own type; behind it, for a launch with an input map, the map's 16 KB window
 // (value_map.h).  Long rows are bound by how many wavefronts a CU holds, and that by LDS and registers: with a second,
@@ -220,7 +220,8 @@ __device__ __forceinline__ void count_below(const uint2 (&ent)[kChunk], const fl
 // the output arguments at run time (values modes, no codes, ...).  EMIT_WEIGHT is the weight side
 // of the layer (src/orbitquant/layers.py:121-125,201-215 of the reference): the row is rotated
 // as it is, multiplied by 1/sqrt(block), THEN divided by max(norm, eps) with the IEEE division,
-// searched in the unfolded boundaries, and its indices are packed `pack_bits` wide into the flat
+// searched in the unfolded boundaries (the plan's table over them, where the call's are the ones it was built from),
+// and its indices are packed `pack_bits` wide into the flat
 // little-endian stream; the norm is stored as bf16.
 enum EmitMode { EMIT_NIBBLE = 0, EMIT_U8 = 1, EMIT_ANY = 2, EMIT_WEIGHT = 3 };
 
@@ -365,7 +366,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   uint2 *cells = reinterpret_cast<uint2 *>(smem + kCellsAt);
   float *thr = reinterpret_cast<float *>(smem + kThrAt);
   float *cent = reinterpret_cast<float *>(smem + kCentAt);
-  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..7] per-wavefront flags
+  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..7] per-wavefront flags, [8] the table is another's
   unsigned char *stage = smem + kStageAt;
   const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset);
   const uint16_t *signs_by_position = reinterpret_cast<const uint16_t *>(gather + K), *signs_by_slot = signs_by_position + K;
@@ -541,6 +542,17 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   if constexpr (DT == OQ_BF16) tiny = min(tiny_acc & 0xffffu, tiny_acc >> 16) < 0x2effu;
   const bool wave_tiny = __builtin_amdgcn_ballot_w64(tiny) != 0;
   if (lane == 0 && wave < 4) red[4 + wave] = wave_tiny ? 1.0f : 0.0f;  // (four wavefronts at most read the row)
+  if constexpr (EMIT == EMIT_WEIGHT) {
+    // The plan's table decides the indices only if it is one over the boundaries of this call: boundary j is the j-th
+    // of the table, in the cell it falls into (a table has 63 boundaries at most, a lane of the first wavefront each;
+    // 14336 x 4096: 77.4 -> 78.3 us).
+    if (wave == 0) {
+      const uint2 there = plan_cells[plan::cell_of(thr_v, cell_scale, cell_offset)];
+      const bool other = lane < a.levels - 1 && (there.x != __float_as_uint(thr_v) || there.y != static_cast<uint32_t>(lane));
+      const bool others = __builtin_amdgcn_ballot_w64(other) != 0;
+      if (lane == 0) red[8] = others ? 1.0f : 0.0f;
+    }
+  }
   if (tid < 256) {
     cells[tid] = cell_v;
     thr[tid] = thr_v;
@@ -582,7 +594,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // The two rare modes (IEEE division for this row, binary search instead of the cell table) pass
   // through an empty asm statement inside the loop on purpose: as loop invariants the compiler
   // clones the whole loop per combination.
-  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | ((EMIT == EMIT_WEIGHT ? hdr->weight_cells : hdr->cells) != 0 ? 0u : 2u) | (bijective ? 0u : 4u));
+  const bool has_cells = EMIT == EMIT_WEIGHT ? hdr->weight_cells != 0 && red[8] == 0.0f : hdr->cells != 0;
+  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (has_cells ? 0u : 2u) | (bijective ? 0u : 4u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
   const float s1 = (slot_lane & 1) ? -1.0f : 1.0f, s2 = (slot_lane & 2) ? -1.0f : 1.0f;
   const float s4 = (slot_lane & 4) ? -1.0f : 1.0f, s8 = (slot_lane & 8) ? -1.0f : 1.0f;

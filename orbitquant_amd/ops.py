@@ -213,7 +213,8 @@ def rotate_quantize(
     """-> (codes or None, values or None, norms[...]).
 
     plan: None, or `rotate_plan(...)` of the same permutation, signs, boundaries, block and
-    factor: more than 16 rows then take the plan-based kernel (same results, much faster).
+    factor: more than 16 rows, and fewer where a row has several blocks or blocks of 1024 to 4096,
+    then take the plan-based kernel (same results, much faster).
 
     input_map: None, or the table of an elementwise function f (`activation_table`): the
     result is that of rotate_quantize(f(x)), bit for bit, without f(x) ever being stored.

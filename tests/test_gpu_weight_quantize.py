@@ -206,3 +206,34 @@ def test_boundaries_with_and_without_cells(dev, kind):
     packed, norms = gpu_quantize(dev, w, perm, signs, bounds, block, inv, 4)
     want_packed, want_norms, _ = o.quantize_weight(w.numpy(), perm, signs, bounds, block, 1e-10, 4, norm_order="sumsq_v1")
     assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
+
+
+@pytest.mark.parametrize("k", [24, 1152, 4096])
+@pytest.mark.parametrize("change", ["activation codebook", "one boundary", "signed zero", "none"])
+def test_a_plan_over_other_boundaries_decides_nothing(dev, k, change):
+    """The indices are those of the call's own boundaries, whatever boundaries the plan was built from."""
+    from orbitquant_amd import _lib, ops
+
+    lib = _lib.load()
+    n, bits = 21, 4
+    perm, signs, block, inv = o.rpbh_constants(k, 5, "paper")
+    bounds = (np.linspace(-2.5, 2.5, 15) / np.sqrt(k)).astype(np.float32)
+    bounds[7] = 0.0
+    other = bounds.copy()
+    if change == "activation codebook":
+        other = (bounds * np.float32(1.4) + np.float32(0.1 / np.sqrt(k))).astype(np.float32)
+    elif change == "one boundary":
+        other[11] = np.nextafter(other[11], np.float32(1))
+    elif change == "signed zero":
+        other[7] = -0.0
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(k)).bfloat16()
+    w[2] = 0
+    t = lambda a: torch.from_numpy(a).to(dev)
+    plan = ops.rotate_plan(t(perm.astype(np.int32)), t(signs), t(other), block_size=block, inv_sqrt_block=float(inv))
+    weight, mine = w.to(dev), t(bounds)
+    packed = torch.zeros(n * k * bits // 8, dtype=torch.uint8, device=dev)
+    norms = torch.zeros(n, dtype=torch.bfloat16, device=dev)
+    assert lib.oq_quantize_weight(weight.data_ptr(), _lib.OQ_BF16, n, k, plan.data_ptr(), mine.data_ptr(), 16, block, 1e-10, float(inv), bits,
+                                  packed.data_ptr(), norms.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    want_packed, want_norms, _ = o.quantize_weight(w.float().numpy(), perm, signs, bounds, block, 1e-10, bits, norm_order="sumsq_v1")
+    assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
