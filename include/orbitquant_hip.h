@@ -101,8 +101,9 @@ int oq_rotate_quantize(const void *x, int x_dtype, int64_t M, int64_t K,
  * inv_sqrt_block, the bucketize table), built once per layer by one small launch and kept by
  * the caller in device memory next to the layer's other constants: oq_rotate_plan_bytes(K)
  * bytes, 16-byte aligned.  No counterpart in the reference, whose kernels re-derive all of it per
- * row (packed_matmul.cu:581-657).  A plan is only valid for the arguments it was built from; a
- * call that passes a plan built for another K, block or levels writes nothing.
+ * row (packed_matmul.cu:581-657).  A plan is only valid for the arguments it was built from,
+ * and for the library that built it; a call that passes a plan built for another K, block or levels, or
+ * by a library of another layout, writes no codes, and NaN for the norms.
  */
 uint64_t oq_rotate_plan_bytes(int64_t K);
 int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels,

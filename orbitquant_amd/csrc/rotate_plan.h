@@ -28,7 +28,7 @@
 namespace oq {
 namespace plan {
 
-constexpr uint32_t kMagic = 0x4f51504cu;  // "OQPL"
+constexpr uint32_t kMagic = 0x4f51504du;  // one more for every change of the layout or of what an entry means: a kept plan of another build is refused, not misread
 constexpr int kCells = 256;
 constexpr int kThresholdsOffset = 64;
 constexpr int kCellsOffset = kThresholdsOffset + 256 * 4;

@@ -303,3 +303,26 @@ def test_layer_uses_the_plan_and_matches_the_two_call_path(dev):
                              weight_bits=4, out_features=256, in_features=1152, bias=layer.bias.to(torch.bfloat16),
                              output_dtype=torch.bfloat16)
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("m", [1, 32])
+def test_a_kept_plan_of_an_earlier_layout_is_loud(dev, m):
+    """The layout with signs merged into two sets of gather entries had the first byte 0x4c.  A plan of it holds other
+    things at the places that are read now."""
+    from orbitquant_amd import _lib, ops
+
+    perm, signs, h, inv, cents, bounds, t = constants(dev, 2048, 256, 4)
+    plan = ops.rotate_plan(t["perm"], t["signs"], t["bounds"], block_size=256, inv_sqrt_block=float(inv))
+    earlier = plan.clone()
+    assert bytes(plan[:4].tolist()) != b"LPQO"
+    earlier[:4] = torch.tensor(list(b"LPQO"), dtype=torch.uint8, device=dev)
+    x = make_rows(32, 2048, torch.bfloat16, seed=3)[:m].to(dev)
+    for kept, loud in ((plan, False), (earlier, True)):
+        codes, _, norms = ops.rotate_quantize(x, t["perm"], t["signs"], t["bounds"], block_size=256, eps=1e-10, inv_sqrt_block=float(inv),
+                                              code_format="u8", plan=kept)
+        assert bool(torch.isnan(norms).all()) == loud
+    weight = torch.randn(8, 2048, device=dev)
+    packed, weight_norms = torch.zeros(8 * 2048 // 2, dtype=torch.uint8, device=dev), torch.zeros(8, dtype=torch.bfloat16, device=dev)
+    assert _lib.load().oq_quantize_weight(weight.data_ptr(), _lib.OQ_F32, 8, 2048, earlier.data_ptr(), t["bounds"].data_ptr(), 16, 256, 1e-10, float(inv), 4,
+                                          packed.data_ptr(), weight_norms.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    assert bool(torch.isnan(weight_norms).all()) and not packed.any()
