@@ -120,6 +120,14 @@ def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[s
     return {name: there[starts[name] : starts[name] + t.numel() * t.element_size()].view(t.dtype).view(t.shape) for name, t in tensors.items()}
 
 
+def _constants_on(device: torch.device, tensors: dict[str, torch.Tensor]) -> dict[str, torch.Tensor]:
+    """`_on_device`, with a storage for every type: torch saves no storage that is viewed as more than one."""
+    there = _on_device(tensors, device)
+    if device.type != "cuda":
+        return there
+    return {name: t if t.dtype == torch.float32 else t.clone() for name, t in there.items()}
+
+
 def _wait_for(device: torch.device) -> None:
     """Waits for what the current stream was given.  A module that was built or moved may be called on any stream at once,
     as torch's own may, so its constants, its indices and its rotate plan have to be there when the call that makes them
@@ -167,7 +175,7 @@ class OrbitLinear(nn.Module):
             self.bias = nn.Parameter(bias.detach().clone(), requires_grad=False)
         device = packed_weight_indices.device
         if constants is None:   # (`from_weight` has them on the device already)
-            constants = _on_device(self._constants(), device)
+            constants = _constants_on(device, self._constants())
         for name, tensor in constants.items():
             self.register_buffer(name, tensor, persistent=False)
         self.register_buffer("_rotation_plan", None, persistent=False)
@@ -287,7 +295,7 @@ class OrbitLinear(nn.Module):
         constants = quantizer_constants = None
         if device.type == "cuda":
             activation_codebook = get_codebook(in_features, config.activation_bits, config.codebook_version)
-            constants = _on_device({**_host_constants(rotation, activation_codebook, codebook), "weight_boundaries": codebook.boundaries}, device)
+            constants = _constants_on(device, {**_host_constants(rotation, activation_codebook, codebook), "weight_boundaries": codebook.boundaries})
             quantizer_constants = (constants["_rotation_permutation"], constants["_rotation_signs"], constants.pop("weight_boundaries"))
         packed, row_norms = quantize_weight(
             weight, rotation=rotation, codebook=codebook, bits=config.weight_bits,
@@ -323,7 +331,7 @@ class OrbitLinear(nn.Module):
         result = super()._apply(fn, recurse=recurse)
         # integer / fp32 constants must survive .to(dtype=...) casts unchanged
         device = self.packed_weight_indices.device
-        for name, tensor in _on_device(self._constants(), device).items():
+        for name, tensor in _constants_on(device, self._constants()).items():
             setattr(self, name, tensor)
         self._build_rotation_plan()
         self._nibble_weight_copy = None   # rebuilt on the new device / from uncast centroids when next needed

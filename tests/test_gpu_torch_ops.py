@@ -177,3 +177,29 @@ def test_group_entries_of_other_forms(layer):
             call(entry, wrong)
     with pytest.raises(AttributeError):
         call((None, *entry[1:]))
+
+
+@pytest.mark.parametrize("how", ["from_weight", "moved", "cast"])
+def test_layers_are_saved_whole(how):
+    """torch.save takes a module, or its buffers, only where no storage is viewed as more than one type."""
+    import copy
+    import io
+
+    from orbitquant_amd import OrbitLinear, recipe
+
+    torch.manual_seed(0)
+    weight = torch.randn(136, 384)
+    layer = OrbitLinear.from_weight(weight.cuda() if how == "from_weight" else weight, bias=None, config=recipe("w4a6")).cuda()
+    if how == "cast":
+        layer = layer.to(torch.bfloat16)
+    x = torch.randn(5, 384, device="cuda").bfloat16()
+    for saved in (layer, dict(layer.named_buffers()), layer.state_dict()):
+        file = io.BytesIO()
+        torch.save(saved, file)
+        file.seek(0)
+        restored = torch.load(file, weights_only=False)
+        if saved is layer:
+            assert torch.equal(restored(x), layer(x))
+        else:
+            assert all(torch.equal(t, saved[name]) and t.dtype == saved[name].dtype for name, t in restored.items())
+    assert torch.equal(copy.deepcopy(layer)(x), layer(x))
