@@ -283,6 +283,14 @@ class OrbitLinear(nn.Module):
             self._rotation_permutation, self._rotation_signs, self._activation_codebook_boundaries,
             block_size=self.rotation.block_size, inv_sqrt_block=self.rotation.normalization)
 
+    def __setstate__(self, state) -> None:
+        super().__setstate__(state)
+        # a module pickled whole has its plan with it, which is of the build that made it
+        plan = self._buffers.get("_rotation_plan")
+        if plan is not None and plan.device.type == "cuda" and plan.numel() != int(_lib.load().oq_rotate_plan_bytes(self.in_features)):
+            self._build_rotation_plan()
+            _wait_for(plan.device)
+
     def _constants(self) -> dict[str, torch.Tensor]:
         return _host_constants(self.rotation, self.activation_codebook, self.weight_codebook)
 

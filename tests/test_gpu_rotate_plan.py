@@ -326,3 +326,22 @@ def test_a_kept_plan_of_an_earlier_layout_is_loud(dev, m):
     assert _lib.load().oq_quantize_weight(weight.data_ptr(), _lib.OQ_F32, 8, 2048, earlier.data_ptr(), t["bounds"].data_ptr(), 16, 256, 1e-10, float(inv), 4,
                                           packed.data_ptr(), weight_norms.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
     assert bool(torch.isnan(weight_norms).all()) and not packed.any()
+
+
+def test_a_layer_pickled_with_an_earlier_plan(dev):
+    """A module saved whole by a build whose plans were 2048 bytes shorter computes what it did."""
+    import io
+
+    from orbitquant_amd import OrbitLinear, recipe
+
+    torch.manual_seed(0)
+    layer = OrbitLinear.from_linear(torch.nn.Linear(1152, 256), config=recipe("w4a4")).to(dev)
+    x = make_rows(40, 1152, torch.bfloat16, seed=4).to(dev)
+    want = layer(x)
+    for cut in (0, 2048):
+        layer._rotation_plan = layer._rotation_plan[: layer._rotation_plan.numel() - cut].clone()
+        file = io.BytesIO()
+        torch.save(layer, file)
+        file.seek(0)
+        restored = torch.load(file, weights_only=False)
+        assert torch.equal(restored(x), want) and torch.equal(restored(x[:1]), want[:1])
