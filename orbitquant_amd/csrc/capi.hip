@@ -131,7 +131,7 @@ int generic_linear_codes(const void *codes, int code_format, const float *token_
                          hipStream_t stream);
 int unpack_dispatch(const uint8_t *packed, int bits, int64_t count, uint8_t *out, hipStream_t stream);
 bool gemm_supported(int64_t K, int bits);
-double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits);
+double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits, bool without_small = false);
 int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float *act_cents, int a_levels,
                   const uint8_t *w, int bits, const uint16_t *row_norms, const float *w_cents,
                   const void *bias, int bias_dtype, int64_t M, int64_t N, int64_t K, void *out,
@@ -327,7 +327,8 @@ static int int8_choose_tile(int64_t M, int64_t N, int64_t K) {
   double cost = 0.0;
   const int tile = dense_choose_tile(M, N, K, dense_rows_at_a_time(M, K, MF_I8), MF_I8, 1.5 * static_cast<double>(K) * static_cast<double>(M + N), &cost);
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
-  return cost < 0.9 * gemm_call_price(M, N, K, 4) ? tile : -1;
+  // (its sums are whole numbers: the 64x64 tiles, which sum in fp32, take no problem from it that the larger ones leave)
+  return cost < 0.9 * fmax(gemm_call_price(M, N, K, 4), gemm_call_price(M, N, K, 4, true)) ? tile : -1;
 }
 
 uint64_t oq_packed_linear_int8_workspace_bytes(int64_t M, int64_t N, int64_t K) {

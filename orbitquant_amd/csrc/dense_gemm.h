@@ -12,7 +12,7 @@ uint64_t operand_order_bytes(int64_t rows, int64_t K, int value_bytes);
 int decode_operands(const uint8_t *packed, int bits, const float *cents, int levels, int64_t rows, int64_t K, bool f16, void *out,
                     hipStream_t stream);
 int decode_operands_int8(const uint8_t *packed, const int8_t *table, int64_t rows, int64_t K, void *out, hipStream_t stream);
-double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form);  // packed_gemm.hip
+double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form, bool without_small = false);  // packed_gemm.hip
 int dense_choose_tile(int64_t M, int64_t N, int64_t K, int64_t rows_at_a_time, int mf, double pass_bytes, double *cost_out);
 int dense_gemm(int mf, const void *a, const void *w, const float *row_scale, float scale, const uint16_t *row_norms, const void *bias, int bias_dtype,
                int64_t M, int64_t N, int64_t K, void *out, int out_dtype, const uint16_t *out_map, int tile, hipStream_t stream);

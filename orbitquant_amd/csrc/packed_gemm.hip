@@ -16,7 +16,8 @@ int gemm_launch_bytes(const GemmArgs &g, int bits, int tile, hipStream_t stream)
 // widths other than 4 pay for their longer index extraction, least on the largest tile.
 // byte_codes: one activation code per byte (eight single lookups per operand instead of four pair lookups);
 // a K-step then costs 1.07-1.23 times as much, least on the tiles with many columns per activation row.
-static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, double *cost_out, bool byte_codes = false) {
+// without_small: as if there were no 64x64 tiles.
+static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, double *cost_out, bool byte_codes = false, bool without_small = false) {
   const bool can_split = K % 256 == 0;  // a quarter of the K-steps per wavefront
   const char *force = debug_env(ENV_GEMM_TILE);
   if (force != nullptr && force[0] >= '0' && force[0] <= '3') return force[0] - '0';
@@ -55,7 +56,7 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
       best_cost = cost;
     }
   }
-  if (K >= 256 && bits <= 4) {  // (a quarter of the K-steps, more or less one, for each wavefront)
+  if (K >= 256 && bits <= 4 && !without_small) {  // (a quarter of the K-steps, more or less one, for each wavefront)
     // 64x64 tiles, shared along K the same way: few tokens or few rows, which leave the chip empty on larger tiles.  Twice
     // the lookups per product, so only where the tiles fit about one round: 256 x 1152 x 1152 12.4 -> 7.0 us, 128 x 4096 x
     // 4096 19.3 -> 13.1 us, 77 x 8192 x 8192 25.9 -> 23.5 us, but 333 x 14336 x 4096 54 us on 128x96 and 65 on these.  Of
@@ -79,7 +80,7 @@ static int choose_tile_with_cost(int64_t M, int64_t N, int64_t K, int bits, doub
 // dimension: a time per K-step and tile for each form of the activations (two codes a byte, one code a byte, values
 // in operand order with the pass that puts them there), a factor for each weight width, the output's way to memory
 // (rms errors of 10, 8 and 13 %).
-double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form) {
+double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form, bool without_small) {
   struct Times { double step[6], out_mb, launches, bits2, bits3, bits6, bits8; };
   static const Times forms[3] = {{{0.81, 0.85, 1.39, 1.09, 1.12, 1.10}, 0.20, 0.5, 1.09, 1.11, 1.69, 1.58},
                                  {{1.12, 1.10, 1.72, 1.40, 1.40, 1.30}, 0.18, 2.2, 1.06, 1.08, 1.56, 1.50},
@@ -87,7 +88,7 @@ double gemm_price(int64_t M, int64_t N, int64_t K, int bits, int form) {
   static const struct { int tm, tn, capacity; double fixed; } tiles[6] = {
       {128, 128, 512, 4.5}, {128, 256, 256, 5.5}, {256, 256, 256, 7.0}, {256, 192, 256, 6.0}, {128, 96, 256, 7.5}, {64, 64, 512, 4.5}};
   const Times &f = forms[form];
-  const int tile = choose_tile_with_cost(M, N, K, bits, nullptr, form == PRICE_BYTES);
+  const int tile = choose_tile_with_cost(M, N, K, bits, nullptr, form == PRICE_BYTES, without_small);
   const auto &sh = tiles[tile];
   const double width = bits == 2 ? f.bits2 : bits == 3 ? f.bits3 : bits == 6 ? f.bits6 : bits == 8 ? f.bits8 : 1.0;
   const double steps = static_cast<double>(K / 64) / (tile >= 4 ? 4.0 : 1.0), step = f.step[tile] * width;
@@ -112,9 +113,16 @@ int apply_value_map(void *out, int64_t count, const uint16_t *table, hipStream_t
 // read back, at 3 TB/s):
 // every part keeps at least sixteen K-steps, the partial tiles stay within 64 MB, and the split has to
 // promise 15 % over the best single launch (5 % over 64x64 tiles, whose price is the better known: 128 x 4096 x 14336).
+// The more partial sums, the smaller their error (K = 8192 in fp32: 1.6e-7 of the result with eight, 2.1e-7 with four),
+// so the 64x64 tiles, whose four wavefronts make four, take no problem from a split into more parts, though they are
+// faster there (512 x 1152 x 8192 18.3 us against 23.0 in six parts, 100 x 4096 x 8192, 2-bit, 21.8 against 24.4 in eight);
+// nor does a split into fewer take one from the 128x96 tiles because 64x64 ones look better still (512 x 8192 x 8192 in
+// two parts 87 us, 82 in one launch).
 // OQ_GEMM_WG_SPLIT overrides (1 = never).
 // `cost_out`: the time of the split launch, if it is one.
-int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_out = nullptr) {
+static int sums_of_tile(int tile) { return tile >= 4 ? 4 : 1; }
+
+int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr, bool without_small = false) {
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), steps = K / 64;
   auto allowed = [&](int s) { return s >= 2 && s <= 8 && steps / s >= 16 && M * N * 4 * s <= (64ll << 20); };
   if (const char *force = debug_env(ENV_GEMM_WG_SPLIT)) {
@@ -123,25 +131,30 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
     return s < 1 ? 1 : s;
   }
   if (debug_env(ENV_GEMM_TILE) != nullptr) return 1;  // a forced tile is a forced single launch
-  double single = 0.0;
-  const int tile = choose_tile_with_cost(M, N, K, bits, &single);
   const double width = bits == 4 ? 1.0 : 1.28;
-  int best = 1;
-  double best_cost = (tile == 5 ? 0.95 : 0.85) * single;
-  for (int s = 2; s <= 8; ++s) {
-    if (!allowed(s)) continue;
-    const int64_t groups = tiles * s;
-    const double per_step = (groups <= 256 ? 0.5 : 0.8) * width;
-    const double rounds = static_cast<double>((groups + 511) / 512);
-    const double cost = rounds * (4.5 + static_cast<double>(steps / s) * per_step) + 3.0 +
-                        static_cast<double>(M) * static_cast<double>(N) * (8.0 * s + 2.0) / 3.0e6;  // partial tiles written, then read
-    if (cost < best_cost) {
-      best = s;
-      best_cost = cost;
+  auto choose = [&](double limit, int least) {  // (of the shares in `least` parts or more)
+    int best = 1;
+    for (int s = least; s <= 8; ++s) {
+      if (!allowed(s)) continue;
+      const int64_t groups = tiles * s;
+      const double per_step = (groups <= 256 ? 0.5 : 0.8) * width;
+      const double rounds = static_cast<double>((groups + 511) / 512);
+      const double cost = rounds * (4.5 + static_cast<double>(steps / s) * per_step) + 3.0 +
+                          static_cast<double>(M) * static_cast<double>(N) * (8.0 * s + 2.0) / 3.0e6;  // partial tiles written, then read
+      if (cost < limit) {
+        best = s;
+        limit = cost;
+      }
     }
-  }
-  if (cost_out != nullptr && best > 1) *cost_out = best_cost;
-  return best;
+    if (cost_out != nullptr && best > 1) *cost_out = limit;
+    return best;
+  };
+  double single = 0.0, single_large = 0.0;
+  const int tile = choose_tile_with_cost(M, N, K, bits, &single);
+  choose_tile_with_cost(M, N, K, bits, &single_large, false, true);
+  const int large = choose(0.85 * single_large, 2);  // what it would be without 64x64 tiles
+  if (without_small || tile != 5 || large > sums_of_tile(choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes))) return large;
+  return choose(0.95 * single, large > 1 ? large : sums_of_tile(choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes, true)));
 }
 
 // Tile of the decode-first GEMM (dense_gemm.hip) for a launch that has the workspace for it, -1 for the others.  The
@@ -155,25 +168,26 @@ int gemm_choose_splits(int64_t M, int64_t N, int64_t K, int bits, double *cost_o
 // 128 x 96 or the 64 x 64 tile it keeps the problem: four wavefronts that share K and add four partial sums leave a smaller error than
 // one running sum (2048 x 4096 x 14336 in fp32: 7.3e-8 of the result against 2.3e-7), and a workspace does not change
 // the bits of a result.
-static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr) {
+static int gemm_choose_dense(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, double *cost_out = nullptr, bool without_small = false) {
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   double dense = 0.0;
   const int tile = dense_choose_tile(M, N, K, dense_rows_at_a_time(M, K, MF_BF16), MF_BF16, k * (m * (byte_codes ? 3.0 : 2.5) + n * (2.0 + bits / 8.0)), &dense);
   if (cost_out != nullptr) *cost_out = dense;
   if (tile < 0 || debug_env(ENV_DENSE_GEMM) != nullptr) return tile;
-  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits) > 1) return -1;
-  if (choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes) >= 4) return -1;
+  if (debug_env(ENV_GEMM_TILE) != nullptr || gemm_choose_splits(M, N, K, bits, byte_codes, nullptr, without_small) > 1) return -1;
+  if (choose_tile_with_cost(M, N, K, bits, nullptr, byte_codes, without_small) >= 4) return -1;
   const double share = byte_codes || 2.0 * k * (m + n) <= 268435456.0 ? 0.95 : 0.8;
-  return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES) ? tile : -1;
+  return dense < share * gemm_price(M, N, K, bits, byte_codes ? PRICE_BYTES : PRICE_NIBBLES, without_small) ? tile : -1;
 }
 
 // What a call on two codes a byte takes with the workspace it asks for: decoded first, shared between workgroups
 // along K (where the two prices differ, the lower one), or the single launch.
-double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits) {
+// `without_small`: as if there were no 64x64 tiles.
+double gemm_call_price(int64_t M, int64_t N, int64_t K, int bits, bool without_small) {
   double dense = 0.0, split = 0.0;
-  if (gemm_choose_dense(M, N, K, bits, false, &dense) >= 0) return dense;
-  const double single = gemm_price(M, N, K, bits, PRICE_NIBBLES);
-  return gemm_choose_splits(M, N, K, bits, &split) > 1 && split < single ? split : single;
+  if (gemm_choose_dense(M, N, K, bits, false, &dense, without_small) >= 0) return dense;
+  const double single = gemm_price(M, N, K, bits, PRICE_NIBBLES, without_small);
+  return gemm_choose_splits(M, N, K, bits, false, &split, without_small) > 1 && split < single ? split : single;
 }
 
 bool gemm_supported(int64_t K, int bits) {
@@ -184,7 +198,7 @@ bool gemm_supported(int64_t K, int bits) {
 // problems), or partial tiles (0: it is a launch that needs neither).  `decoded` false: without the decoded operands.
 uint64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, bool decoded) {
   if (gemm_choose_dense(M, N, K, bits, byte_codes) >= 0) return decoded ? dense_workspace_bytes(M, N, K, MF_BF16) : 0u;
-  const int splits = gemm_choose_splits(M, N, K, bits);
+  const int splits = gemm_choose_splits(M, N, K, bits, byte_codes);
   return splits > 1 ? static_cast<uint64_t>(M) * static_cast<uint64_t>(N) * 4u * static_cast<uint64_t>(splits) : 0u;
 }
 
@@ -220,7 +234,7 @@ int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float
   int tile = choose_tile_with_cost(M, N, K, bits, nullptr, a_mode == A_U8);
   g.k_splits = 1;
   if (const char *where = debug_env(ENV_GEMM_STAMPS)) g.stamps = reinterpret_cast<uint64_t *>(strtoull(where, nullptr, 0));  // builds with -DOQ_GEMM_STAMPS: a device buffer for the kernel's phase stamps
-  const int splits = gemm_choose_splits(M, N, K, bits);
+  const int splits = gemm_choose_splits(M, N, K, bits, a_mode == A_U8);
   if (splits > 1 && workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 &&
       workspace_bytes >= static_cast<uint64_t>(M) * static_cast<uint64_t>(N) * 4u * static_cast<uint64_t>(splits)) {
     g.k_splits = splits;

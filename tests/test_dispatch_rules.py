@@ -96,3 +96,23 @@ def test_the_decoded_activations_are_bounded(lib, m, n, k):
     assert operand_order(n, k) < size <= part + operand_order(n, k) and size < operand_order(m, k) + operand_order(n, k)
     size = lib.oq_packed_linear_int8_workspace_bytes(4 * m, n, k)
     assert operand_order(n, k, 1) < size <= part + operand_order(n, k, 1)
+
+
+PARTS = [   # (tokens, rows, values, weight bits, parts of K that a launch adds up in fp32; 0: four wavefronts' parts in one launch)
+    (65, 8192, 12288, 2, 8), (65, 8192, 16384, 4, 8), (1259, 280, 8448, 4, 8), (100, 4608, 8192, 3, 7), (256, 2048, 8192, 2, 7),
+    (128, 3072, 8192, 4, 7), (512, 1152, 8192, 4, 6), (87, 4864, 9728, 3, 6), (200, 3072, 16384, 2, 5), (200, 3072, 8192, 4, 5),
+    (200, 4608, 4608, 2, 0), (67, 8856, 3328, 3, 0), (1912, 2160, 6656, 2, 0), (256, 14336, 8192, 4, 0), (512, 8192, 8192, 4, 0),
+    (2048, 2048, 8192, 4, 0)]
+
+
+@pytest.mark.parametrize("abits", [4, 6])
+@pytest.mark.parametrize("m,n,k,wbits,parts", PARTS)
+def test_64x64_tiles_do_not_lessen_the_partial_sums(lib, m, n, k, wbits, parts, abits):
+    """The fewer partial sums, the larger their error (about 1.6e-7 of the result with eight, 2.1e-7 with four)."""
+    fmt = _lib.OQ_CODES_U8 if abits > 4 else _lib.OQ_CODES_NIBBLE
+    assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, fmt, abits) == 4 * m * n * parts
+
+
+@pytest.mark.parametrize("m,n,k", [(829, 3568, 12608), (1217, 1552, 6464), (5807, 680, 15936), (772, 4888, 2048), (299, 14224, 8000), (4668, 880, 5312)])
+def test_64x64_tiles_take_no_whole_numbers_into_fp32(lib, m, n, k):
+    assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) == operand_order(m, k, 1) + operand_order(n, k, 1)
