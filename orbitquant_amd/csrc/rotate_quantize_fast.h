@@ -236,7 +236,8 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
   constexpr int SPAN = GW * kLaneSpan;   // slots a wavefront keeps, and the distance between the parts
   constexpr int CT = kChunk * GW / WB;   // columns a thread takes
   constexpr int N = CT * WB;             // values it turns into codes: 8 or 16
-  static_assert(SPAN * WB == H && CT >= 1 && N % kChunk == 0);
+  static_assert(SPAN * WB == H && N % kChunk == 0);
+  static_assert(CT == 1 || CT == 2 || CT == 4 || CT == 8, "the columns that the stores below have a case for");
   const int lane = tid & 63, wave = tid >> 6, team = wave / WB, teams = waves / WB, part = wave % WB;
   const int slot_lane = logical_lane(lane);
   float *buffer = reinterpret_cast<float *>(smem + fast_lds_bytes(a.K, DT));  // [K]

@@ -188,7 +188,8 @@ int launch_few(const FastArgs &a, hipStream_t stream) {
       if (wb == 8) return launch_shared<DT, LOG_H, 8>(a, stream);
     if constexpr (LOG_H >= 11)
       if (wb == 4) return launch_shared<DT, LOG_H, 4>(a, stream);
-    if (wb == 2) return launch_shared<DT, LOG_H, 2>(a, stream);
+    if constexpr (LOG_H <= 11)  // (a row of 16384 values has four blocks of 4096 at most, which four wavefronts share at least)
+      if (wb == 2) return launch_shared<DT, LOG_H, 2>(a, stream);
   }
   return -1;
 }
