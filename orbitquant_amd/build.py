@@ -92,11 +92,14 @@ def build_torch_ops() -> Path:
     from torch.utils import cpp_extension
 
     out = PKG / "_torch_ops.so"
+    sources = [CSRC / "torch_ops.cpp", PKG.parent / "include/orbitquant_hip.h", Path(torch.__file__).parent / "version.py"]
+    if INCREMENTAL and out.exists() and out.stat().st_mtime > max(p.stat().st_mtime for p in sources):
+        return out
     includes = [f"-I{p}" for p in cpp_extension.include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"]]]
     torch_lib = Path(torch.__file__).parent / "lib"
     cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + includes +
-           [str(CSRC / "torch_ops.cpp"), "-o", str(out), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+           [str(sources[0]), "-o", str(out), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
     t0 = time.time()
     subprocess.run(cmd, check=True)
     print(f"  compiled torch_ops.cpp in {time.time() - t0:.1f}s", flush=True)
@@ -105,9 +108,10 @@ def build_torch_ops() -> Path:
 
 def build(verbose: bool = True) -> Path:
     OBJ_DIR.mkdir(exist_ok=True)
-    build_torch_ops()
     with ThreadPoolExecutor(max_workers=4) as pool:
+        torch_ops = pool.submit(build_torch_ops)
         objects = list(pool.map(_compile, SOURCES.items()))
+        torch_ops.result()
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB)] + [str(o) for o in objects]
     subprocess.run(cmd, check=True)
     if verbose:

@@ -283,3 +283,23 @@ assert len(said) == 1 and "orbitquant_amd.build" in str(said[0].message)
 """
     done = subprocess.run([sys.executable, "-c", program], cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, done.stderr
+
+
+def test_an_incremental_build_compiles_the_ops_only_after_a_change(monkeypatch, tmp_path):
+    import os
+
+    from orbitquant_amd import build
+
+    ran = []
+    monkeypatch.setattr(build.subprocess, "run", lambda command, **kw: ran.append(command))
+    monkeypatch.setattr(build, "PKG", tmp_path / "package")
+    (tmp_path / "package").mkdir()
+    (tmp_path / "include").mkdir()
+    header, out = tmp_path / "include" / "orbitquant_hip.h", tmp_path / "package" / "_torch_ops.so"
+    header.touch()
+    out.touch()
+    for incremental, changed, times in ((True, False, 0), (True, True, 1), (False, False, 2)):
+        monkeypatch.setattr(build, "INCREMENTAL", incremental)
+        later = out.stat().st_mtime + (5 if changed else -5)
+        os.utime(header, (later, later))
+        assert build.build_torch_ops() == out and len(ran) == times
