@@ -63,3 +63,28 @@ def test_a_layer_is_complete_when_the_call_returns(source, how, monkeypatch):
             there = layer(x)
         torch.cuda.current_stream().wait_stream(other)
         assert torch.equal(here, there)
+
+
+def test_a_capture_refuses_to_make_or_move_a_layer(source):
+    """Its constants come from host memory, which a captured copy would read again at each replay.  The capture itself
+    goes on, and replays what else was given to it."""
+    from orbitquant_amd import OrbitLinear, recipe
+
+    layer = made("converted", source)
+    config = recipe("w4a4")
+    weight, moved = source.weight.detach().cuda(), made("converted", source)
+    x = torch.randn(4, K, device="cuda").bfloat16()
+    want = layer(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captur"):
+            OrbitLinear.from_weight(weight, bias=None, config=config)
+        with pytest.raises(RuntimeError, match="captur"):
+            moved.to(torch.bfloat16)
+        y = layer(x)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(made("converted", source)(x), want)
