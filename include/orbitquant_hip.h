@@ -97,8 +97,8 @@ int oq_rotate_quantize(const void *x, int x_dtype, int64_t M, int64_t K,
 
 /*
  * The rotate plan: everything the rotate+quantize kernel can know about a layer before it sees
- * a token (permutation and signs merged into gather offsets, the boundaries folded with
- * inv_sqrt_block, the bucketize table), built once per layer by one small launch and kept by
+ * a token (the permutation as gather offsets, the signs by position, the boundaries folded with
+ * inv_sqrt_block, the bucketize tables), built once per layer by one small launch and kept by
  * the caller in device memory next to the layer's other constants: oq_rotate_plan_bytes(K)
  * bytes, 16-byte aligned.  No counterpart in the reference, whose kernels re-derive all of it per
  * row (packed_matmul.cu:581-657).  A plan is only valid for the arguments it was built from,
@@ -129,7 +129,7 @@ int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *
  *              boundaries, levels, K, block and inv_sqrt_block.  Its bucketize table is used where it is
  *              one over `boundaries`; a plan of the same perm, signs, levels, K and block over others (the
  *              layer's activation plan, say) gives the same indices from a search (14336 x 4096 into four bits:
- *              108 us instead of 89, a plan's launch included)
+ *              99 us instead of 78)
  * boundaries   fp32 [levels-1] of the weight codebook;  2 <= levels <= 2^bits, 1 <= bits <= 8
  * block        power of two dividing K, 8 <= block <= 4096
  */

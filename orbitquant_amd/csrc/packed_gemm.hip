@@ -113,7 +113,8 @@ int apply_value_map(void *out, int64_t count, const uint16_t *table, hipStream_t
 // read back, at 3 TB/s):
 // every part keeps at least sixteen K-steps, the partial tiles stay within 64 MB, and the split has to
 // promise 15 % over the best single launch (5 % over 64x64 tiles, whose price is the better known: 128 x 4096 x 14336).
-// The more partial sums, the smaller their error (K = 8192 in fp32: 1.6e-7 of the result with eight, 2.1e-7 with four),
+// The more partial sums, the smaller their error (in fp32, 512 x 1152 x 8192: 2.5e-7 of the result with six, 3.7e-7 with
+// four; 65 x 8192 x 12288, 2-bit: 1.7e-7 with eight, 5.6e-7 with four),
 // so the 64x64 tiles, whose four wavefronts make four, take no problem from a split into more parts, though they are
 // faster there (512 x 1152 x 8192 18.3 us against 23.0 in six parts, 100 x 4096 x 8192, 2-bit, 21.8 against 24.4 in eight);
 // nor does a split into fewer take one from the 128x96 tiles because 64x64 ones look better still (512 x 8192 x 8192 in

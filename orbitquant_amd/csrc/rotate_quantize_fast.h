@@ -717,7 +717,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
         // divide_fast is the IEEE quotient for numerators of 2^-80 and more and the rows it takes at all (NaN and
         // infinities make a row's norm one, so those rows take the other branch); the compiler's division, eleven
         // instructions a value instead of four, remains for the rest.  14336 x 4096 into four bits,
-        // the plan included: 89 us; 108 with a search of four dependent LDS reads per value in place of the cells.
+        // the plan included: 84 us; 105 with a search of four dependent LDS reads per value in place of the cells.
         if (weight_plain || __builtin_amdgcn_ballot_w64(least < 0x1p-80f) != 0) {
 #pragma unroll
           for (int e = 0; e < kChunk; ++e) unit[e] = unit[e] / weight_denominator;

@@ -12,7 +12,7 @@ using namespace rqf;
 // ---- plan construction: once per layer, twice per converted weight ----------
 // Workgroup 0 makes the header and the tables, the last one checks that the permutation is one, the others write 256
 // gather entries and signs each (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
-// for rows of some thousand values).
+// for rows of some thousand values; 6.2 us with the second table and the check).
 // Floats in an order-preserving integer code, so that "the largest float t with RN(t * c) <= b" can
 // be found by bisection over all of them.
 __device__ __forceinline__ uint32_t float_to_ordered(float f) {

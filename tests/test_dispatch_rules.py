@@ -108,7 +108,7 @@ PARTS = [   # (tokens, rows, values, weight bits, parts of K that a launch adds 
 @pytest.mark.parametrize("abits", [4, 6])
 @pytest.mark.parametrize("m,n,k,wbits,parts", PARTS)
 def test_64x64_tiles_do_not_lessen_the_partial_sums(lib, m, n, k, wbits, parts, abits):
-    """The fewer partial sums, the larger their error (about 1.6e-7 of the result with eight, 2.1e-7 with four)."""
+    """The fewer partial sums, the larger their error (512 x 1152 x 8192 in fp32: 2.5e-7 of the result with six, 3.7e-7 with four)."""
     fmt = _lib.OQ_CODES_U8 if abits > 4 else _lib.OQ_CODES_NIBBLE
     assert lib.oq_packed_linear_workspace_bytes(m, n, k, wbits, fmt, abits) == 4 * m * n * parts
 
