@@ -170,72 +170,87 @@ __device__ __forceinline__ float lane_table(const float *__restrict__ cents, int
   return t;
 }
 
-// Build the block with WAVES wavefronts: wavefront w writes rows [w*256/WAVES, (w+1)*256/WAVES),
-// four rows per 16-byte-per-lane store.  The caller puts a barrier between this and the first lookup.
-// A_SINGLE: the activation half holds single-code entries (one code per byte, up to 256 levels)
-// instead of the pair table of two 4-bit codes.
-// W_ONLY: the activation half of every row is left alone (it then holds something else: the
-// small-M kernel parks decoded activation values there).
-template <int BITS, int WAVES, bool A_SINGLE = false, bool W_ONLY = false>
-__device__ __forceinline__ void build_row_tables(uint32_t *lds, const float *__restrict__ w_cents,
-                                                 const float *__restrict__ act_cents, int a_levels) {
+// The weight half of the block alone, for single-code entries (6- and 8-bit weights): wavefront w writes the groups of
+// eight rows w, w + WAVES, ... that an index can reach, eight rows per 16-byte-per-lane store.  The activation half of
+// every row is left alone (the small-M kernel parks decoded activation values there).
+template <int BITS, int WAVES>
+__device__ __forceinline__ void build_single_w_rows(uint32_t *lds, const float *__restrict__ w_cents) {
+  static_assert(BITS > 4, "pair tables: write_w_rows");
   constexpr int kLevels = 1 << BITS;
-  constexpr bool kPair = BITS <= 4;
-  constexpr int kRowsPerWave = 256 / WAVES;
+  constexpr int kGroups = kLevels / 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float a_tab = 0.0f;
-  if constexpr (!W_ONLY) a_tab = A_SINGLE ? lane_table<64>(act_cents, a_levels) : lane_table<16>(act_cents, a_levels);
   float w_tab = 0.0f;
   if constexpr (kLevels <= 64) w_tab = lane_table<kLevels>(w_cents, kLevels);
-  if constexpr (W_ONLY) {
-    // only the rows an index can reach (16, 64 or 256), eight rows per 16-byte-per-lane store
-    // (a weight half is eight lanes wide), the groups of eight rows dealt round the wavefronts
-    constexpr int kRows = kPair ? (kLevels * kLevels < 256 ? kLevels * kLevels : 256) : kLevels;
-    constexpr int kGroups = (kRows + 7) / 8;
 #pragma unroll
-    for (int i = 0; i < (kGroups + WAVES - 1) / WAVES; ++i) {
-      const int grp8 = wave + WAVES * i;
-      if (grp8 >= kGroups) break;  // the same for the whole wavefront
-      const int e = 8 * grp8 + (lane >> 3);
-      uint32_t ew;
-      if constexpr (kLevels <= 64) {
-        if constexpr (kPair) ew = pack16(__shfl(w_tab, e & (kLevels - 1)), __shfl(w_tab, (e >> BITS) & (kLevels - 1)), false);
-        else ew = pack16(__shfl(w_tab, e & (kLevels - 1)), __shfl(w_tab, e & (kLevels - 1)), false);
-      } else {
-        const float v = w_cents[e];
-        ew = pack16(v, v, false);
-      }
-      *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned char *>(lds) + e * 256 + (lane & 7) * 16) = make_uint4(ew, ew, ew, ew);
-    }
-    return;
+  for (int i = 0; i < (kGroups + WAVES - 1) / WAVES; ++i) {
+    const int grp8 = wave + WAVES * i;
+    if (grp8 >= kGroups) break;  // the same for the whole wavefront
+    const int e = 8 * grp8 + (lane >> 3);
+    float v;
+    if constexpr (kLevels <= 64) v = __shfl(w_tab, e & (kLevels - 1));
+    else v = w_cents[e];
+    const uint32_t ew = pack16(v, v, false);
+    *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned char *>(lds) + e * 256 + (lane & 7) * 16) = make_uint4(ew, ew, ew, ew);
   }
+}
+
+// Both halves, built by WAVES wavefronts from centroids that every lane fetches for itself with the kernel's first loads
+// (request_row_seeds): an entry is then one conversion, and the block costs the one memory round trip that the launch
+// begins with anyway.  Lane l writes 16-byte chunk l % 16 of rows  wave * 256 / WAVES + 4 i + l / 16:  a weight copy (chunks
+// 0..7) or an activation copy; the caller puts a barrier between this and the first lookup.  Entries of pairs repeat with
+// i: the lower code every fourth i (rows go up in sixteens), the upper one, of four bits, only changes then.
+// A_SINGLE: the activation half holds single-code entries (one code per byte, up to 256 levels) instead of the pair table of
+// two 4-bit codes.  Weight rows that no index reaches hold arbitrary entries.
+// (Centroids through scalar loads, each behind a comparison with the level count, handed round by wavefront shuffles: the
+// tables of a launch on sixteen tokens stood 4.4 us after its start, and stand 2.1 us after it; 16 tokens through 14336 x
+// 4096 with the quantizer 24.4 -> 23.1 us, q, k and v of 4096 x 4096 21.4 -> 19.5 us.)
+template <int BITS, int WAVES, bool A_SINGLE>
+struct RowSeeds {
+  static constexpr int kRows = 256 / WAVES, kIters = kRows / 4;
+  static constexpr bool kPairs = BITS <= 4 && !A_SINGLE, kSingles = BITS > 4 && A_SINGLE;
+  static constexpr int kLo = kPairs && kIters > 4 ? 4 : kIters;
+  static constexpr int kHi = kSingles ? 1 : kPairs && BITS == 4 && kIters >= 4 ? kIters / 4 : kIters;
+  static_assert(kRows % 16 == 0, "sixteen wavefronts at most");
+  float lo[kLo], hi[kHi];
+  static __device__ __forceinline__ int lo_slot(int i) { return i % kLo; }
+  static __device__ __forceinline__ int hi_slot(int i) { return kSingles ? 0 : i * kHi / kIters; }
+  // the codes of row e's entry: of the activation table for lanes of its copies, of the weight table for the others
+  static __device__ __forceinline__ int row(int i) { return static_cast<int>(threadIdx.x >> 6) * kRows + 4 * i + static_cast<int>((threadIdx.x & 63) >> 4); }
+  static __device__ __forceinline__ int lo_code(int e, bool is_a) { return is_a ? (A_SINGLE ? e : e & 15) : e & ((1 << BITS) - 1); }
+  static __device__ __forceinline__ int hi_code(int e, bool is_a) {
+    return is_a ? (A_SINGLE ? e : e >> 4) : BITS <= 4 ? (e >> BITS) & ((1 << BITS) - 1) : e & ((1 << BITS) - 1);
+  }
+};
+
+template <int BITS, int WAVES, bool A_SINGLE>
+__device__ __forceinline__ void request_row_seeds(RowSeeds<BITS, WAVES, A_SINGLE> &seeds, const float *__restrict__ w_cents,
+                                                  const float *__restrict__ act_cents, int a_levels) {
+  typedef RowSeeds<BITS, WAVES, A_SINGLE> S;
+  const bool is_a = (threadIdx.x & 8) != 0;
+  const float *table = is_a ? act_cents : w_cents;
+  const int last = is_a ? a_levels - 1 : (1 << BITS) - 1;
 #pragma unroll
-  for (int i = 0; i < kRowsPerWave / 4; ++i) {
-    const int e = wave * kRowsPerWave + 4 * i + (lane >> 4);  // the row this lane writes to
-    uint32_t ea;
-    if constexpr (A_SINGLE) {
-      float v = __shfl(a_tab, e & 63);
-      if (a_levels > 64) v = e < a_levels ? act_cents[e] : 0.0f;  // wide tables: one vector load per row
-      else if (e >= a_levels) v = 0.0f;
-      ea = pack16(v, v, false);
-    } else {
-      ea = pack16(__shfl(a_tab, e & 15), __shfl(a_tab, e >> 4), false);
-    }
-    uint32_t ew;
-    if constexpr (kLevels <= 64) {
-      if constexpr (kPair) {
-        ew = (e < kLevels * kLevels)
-                 ? pack16(__shfl(w_tab, e & (kLevels - 1)), __shfl(w_tab, (e >> BITS) & (kLevels - 1)), false)
-                 : 0u;
-      } else {
-        const float v = __shfl(w_tab, e & (kLevels - 1));
-        ew = (e < kLevels) ? pack16(v, v, false) : 0u;
-      }
-    } else {
-      const float v = w_cents[e];  // 256 single-code entries: one vector load per row
-      ew = pack16(v, v, false);
-    }
-    const uint32_t d = (lane & 8) ? ea : ew;
+  for (int i = 0; i < S::kLo; ++i) seeds.lo[i] = table[min(S::lo_code(S::row(i), is_a), last)];
+#pragma unroll
+  for (int i = 0; i < S::kHi; ++i)
+    seeds.hi[i] = S::kSingles ? 0.0f : table[min(S::hi_code(S::row(i * (S::kIters / S::kHi)), is_a), last)];
+}
+
+template <int BITS, int WAVES, bool A_SINGLE>
+__device__ __forceinline__ void write_row_seeds(uint32_t *lds, const RowSeeds<BITS, WAVES, A_SINGLE> &seeds, int a_levels) {
+  typedef RowSeeds<BITS, WAVES, A_SINGLE> S;
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63;
+  const bool is_a = (lane & 8) != 0;
+  const int levels = is_a ? a_levels : 1 << BITS;  // codes past the table read zero
+#pragma unroll
+  for (int i = 0; i < S::kIters; ++i) {
+    const int e = S::row(i);
+    const float lo = S::lo_code(e, is_a) < levels ? seeds.lo[S::lo_slot(i)] : 0.0f;
+    const float hi = S::kSingles ? lo : S::hi_code(e, is_a) < levels ? seeds.hi[S::hi_slot(i)] : 0.0f;
+    const f32x2_t pair = {lo, hi};
+    const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2_t));
     *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned char *>(lds) + e * 256 + (lane & 15) * 16) = make_uint4(d, d, d, d);
   }
 }
@@ -243,7 +258,7 @@ __device__ __forceinline__ void build_row_tables(uint32_t *lds, const float *__r
 // The same block for a 256-thread workgroup whose thread t already holds the two dwords of row t
 // (loaded with its first vector loads, before any bulk load): wavefront w writes rows 64w..64w+63;
 // 16-byte chunk c of a row is a weight copy (c < 8) or an activation copy; lane l writes chunk l%16
-// of row 64w + 4i + l/16.  Fewer shuffles than build_row_tables, at the price of a vector-load latency.
+// of row 64w + 4i + l/16.  
 __device__ __forceinline__ void write_row_tables(uint32_t *lds, uint32_t my_w, uint32_t my_a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll

@@ -17,10 +17,9 @@
 // entry e 32 times in bytes 0..127 of row e, activation entry e in bytes
 // 128..255; lane l reads copy l%32, a byte-indexed lookup is one v_perm_b32 plus
 // one ds_read_b32).  The packed stream is requested first thing (right behind the few epilogue
-// operands, which are not touched before the epilogue); the tables are
-// built meanwhile from centroids fetched with SCALAR loads, which do not queue
-// behind the vector loads of the stream, and spread over the lanes so that every lane can pick the two values of its table entry with
-// wavefront shuffles.  After the main loop the same LDS holds the partial sums.
+// operands, which are not touched before the epilogue, and the centroids of the
+// table entries that a lane writes, which arrive ahead of the stream); the tables are
+// built while it is on its way.  After the main loop the same LDS holds the partial sums.
 //
 // The kernel body is a device function here, shared by the plain small-M kernel
 // (packed_gemv.hip) and by the one-token linear that quantizes its input in the same launch.
@@ -173,6 +172,10 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
     fetch_w(s0, bt);
   };
 
+  // the centroids that this lane's table rows need: requested first, branch-free, written where the tables are built
+  RowSeeds<BITS, WAVES, BYTES> seeds;
+  if constexpr (!ASTAGE) request_row_seeds(seeds, g.w_cents, g.act_cents, g.a_levels);
+
   // ASTAGE: the codes this thread decodes (groups of eight values, 4 bytes; requested before
   // everything else so that they are not queued behind the stream), and the address of the lane's
   // operand of K-step 0, MFMA 0: value (row, 32*grp) of the staged activations.
@@ -278,12 +281,10 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
   }
 
   // ---- tables (built while the stream is in flight) ---------------------------------------
-  if constexpr (kRowsDirect) {
-    __builtin_amdgcn_sched_barrier(0);  // nothing that waits for a value above the requests
-    write_w_rows<BITS, WAVES>(lds, w_row_lo, w_row_hi);
-  } else {
-    build_row_tables<BITS, WAVES, BYTES, ASTAGE>(lds, g.w_cents, g.act_cents, g.a_levels);
-  }
+  __builtin_amdgcn_sched_barrier(0);  // nothing that waits for a value above the requests
+  if constexpr (kRowsDirect) write_w_rows<BITS, WAVES>(lds, w_row_lo, w_row_hi);
+  else if constexpr (ASTAGE) build_single_w_rows<BITS, WAVES>(lds, g.w_cents);
+  else write_row_seeds(lds, seeds, g.a_levels);
   if constexpr (ASTAGE) {
     const float a_tab = (lane & 15) < g.a_levels ? a_tab_early : 0.0f;  // centroid l % 16 in lane l (codes past the table read zero)
 #pragma unroll

@@ -796,3 +796,30 @@ def test_matmul_packed_weight_large_m_bf16_under_graph_capture(dev, bits, m):
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
         assert torch.equal(call(), eager)   # eager work between the replays
+
+
+@pytest.mark.parametrize("wbits", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize(("abits", "m"), [(2, 16), (3, 9), (4, 16), (3, 40), (6, 16), (7, 33)])
+@pytest.mark.parametrize(("n", "k"), [(40, 2048), (4100, 1152)])
+def test_streaming_tables_of_every_width(dev, wbits, abits, m, n, k):
+    """The table block of the streaming kernels, by eight and by sixteen wavefronts: every entry that a code can reach, and zero for
+    codes past the activation table.  Reference in fp64 over the bf16 operand values; K products of relative error 2^-24 each
+    and at most K / 32 + 16 additions of partial sums stay below 1e-5 of the row's absolute sum."""
+    from orbitquant_amd import ops
+
+    g = torch.Generator().manual_seed(n + 8 * wbits + abits)
+    nibble = abits <= 4
+    codes = torch.randint(0, 16 if nibble else 1 << abits, (m, k), generator=g)
+    index = torch.randint(0, 1 << wbits, (n, k), generator=g)
+    a_table, w_table = torch.randn(1 << abits, generator=g), torch.randn(1 << wbits, generator=g)
+    packed_codes = (codes[:, 0::2] | codes[:, 1::2] << 4).to(torch.uint8) if nibble else codes.to(torch.uint8)
+    bits = ((index.flatten()[:, None] >> torch.arange(wbits)) & 1).flatten().view(-1, 8)
+    packed = (bits << torch.arange(8)).sum(1).to(torch.uint8)
+    norms, row_norms = torch.rand(m, generator=g), torch.rand(n, generator=g).bfloat16()
+    out = ops.packed_linear(packed_codes.to(dev), norms.to(dev), a_table.to(dev), packed.to(dev), row_norms.to(dev), w_table.to(dev),
+                            code_format="nibble" if nibble else "u8", activation_bits=abits, weight_bits=wbits, out_features=n, in_features=k,
+                            output_dtype=torch.float32)
+    a = torch.cat([a_table.bfloat16().double(), torch.zeros(16, dtype=torch.float64)])[codes]
+    w = w_table.bfloat16().double()[index]
+    scale = norms.double()[:, None] * row_norms.double()[None]
+    assert bool(((out.cpu().double() - a @ w.T * scale).abs() <= 1e-5 * (a.abs() @ w.abs().T) * scale).all())
