@@ -39,7 +39,7 @@ PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 SOURCES = {
     "capi.hip": [],
     "rotate_quantize.hip": ["-ffp-contract=off"],
-    "rotate_quantize_fast.hip": ["-ffp-contract=off"],
+    "rotate_quantize_fast.hip": ["-ffp-contract=off"] + PRELOAD,
     "packed_generic.hip": [],
     "adaln_int4.hip": [],
     "pack_utils.hip": [],

@@ -150,7 +150,7 @@ int rotate_quantize_dispatch(const void *x, int x_dtype, int64_t M, int64_t K, c
                                          inv_sqrt_block, codes_out, code_format, values_out, values_mode, norms_out,
                                          input_map, &checked, &vec_checked))
       return rc;
-    const int rc = rotate_quantize_fast(x, x_dtype, M, K, plan, levels, block, eps, centroids, codes_out, code_format,
+    const int rc = rotate_quantize_fast(x, x_dtype, M, K, plan, perm, signs, levels, block, eps, centroids, codes_out, code_format,
                                         values_out, values_mode, norms_out, input_map, stream);
     if (rc >= 0) return rc;
   }

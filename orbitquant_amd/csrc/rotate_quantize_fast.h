@@ -20,6 +20,11 @@
 //
 // With few rows a wavefront alone on a block of 1024 to 4096 values is a long chain of dependent steps, so there WB
 // wavefronts share a block: each keeps 1 / WB of it in registers, and the butterflies between them go through LDS once.
+// Such a launch is one chain of memory round trips (a microsecond each, of lines that no cache near by holds) and of steps
+// that wait for each other, so everything it reads is requested when it starts: the plan's header is checked behind the
+// row, not in front of it, and as nothing of the plan that lies behind the header may be touched before that, the gather
+// entries and signs are made from the permutation and the signs themselves.  One row of 4096 / 14336 values, launch to
+// launch: 4.50 / 7.70 -> 4.21 / 7.05 us; 16 rows 4.78 / 8.45 -> 4.49 / 7.57 us.
 //
 // The sum of squares keeps the documented order: [passes][256 lanes][8], tree over the lanes.
 // Compiled without FMA contraction.
@@ -45,6 +50,8 @@ struct FastArgs {
   const void *x;
   int64_t M, K;
   const unsigned char *plan;
+  const int32_t *perm;  // WB > 1 only: what the plan was built from
+  const int8_t *signs;
   const float *cents;  // only for the values modes
   int levels, levels_pow2;
   int block;
@@ -68,18 +75,25 @@ struct FastArgs {
   const uint16_t *map;
 };
 
-inline void fast_args_fill(FastArgs &a, const void *x, int64_t M, int64_t K, const void *plan, int levels, int64_t block, float eps) {
-  a.x = x; a.M = M; a.K = K; a.plan = static_cast<const unsigned char *>(plan);
+// Units of max(block, 512) values per row.
+__host__ __device__ inline int row_units(int64_t K, int64_t block) {
+  const int64_t unit = block > kLaneSpan ? block : kLaneSpan;
+  return static_cast<int>((K + unit - 1) / unit);
+}
+
+inline void fast_args_fill(FastArgs &a, const void *x, int64_t M, int64_t K, const void *plan, const int32_t *perm, const int8_t *signs,
+                           int levels, int64_t block, float eps) {
+  a.x = x; a.M = M; a.K = K; a.plan = static_cast<const unsigned char *>(plan); a.perm = perm; a.signs = signs;
   a.levels = levels; a.block = static_cast<int>(block); a.eps = eps;
   a.levels_pow2 = 2;
   while (a.levels_pow2 < levels) a.levels_pow2 <<= 1;
   a.passes = static_cast<int>((K + kPass - 1) / kPass);
-  const int64_t unit = block > kLaneSpan ? block : kLaneSpan;
-  a.units = static_cast<int>((K + unit - 1) / unit);
+  a.units = row_units(K, block);
 }
 
 // LDS: cells (2048) | thresholds (1024) | centroids (1024) | reduction slots (64) | staging
-constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;  // kRedAt: four group sums, then five flags
+// kRedAt: four group sums, then five flags (WB > 1: four group sums, then a byte for every wavefront)
+constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;
 
 // The row is staged once, in its own type; behind it, for a launch with an input map, the map's 16 KB window
 // (value_map.h).  Long rows are bound by how many wavefronts a CU holds, and that by LDS and registers: with a second,
@@ -87,6 +101,19 @@ constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStage
 // with one copy and 122 registers 72 and 457 us.
 __host__ __device__ inline size_t fast_lds_bytes(int64_t K, int dtype) {
   return static_cast<size_t>(kStageAt) + (dtype == OQ_F32 ? 4u : 2u) * static_cast<size_t>(K);
+}
+
+// With shared blocks (WB > 1) a buffer of the row in fp32 follows, for the butterflies between wavefronts, and in it - for
+// rows of up to kFewPasses passes behind it - the squares' partial sums: [passes][64 lanes][4 groups].
+constexpr int kFewPasses = 4;
+__host__ __device__ inline size_t shared_sums_at(int64_t K, int dtype) {
+  const bool few = K <= static_cast<int64_t>(kFewPasses) * kPass;
+  return fast_lds_bytes(K, dtype) + (few ? 4u * static_cast<size_t>(K) : 0u);
+}
+__host__ __device__ inline size_t shared_lds_bytes(int64_t K, int dtype) {
+  const size_t passes = static_cast<size_t>((K + kPass - 1) / kPass), sums = shared_sums_at(K, dtype) + 1024u * passes;
+  const size_t buffer = fast_lds_bytes(K, dtype) + 4u * static_cast<size_t>(K);
+  return sums > buffer ? sums : buffer;
 }
 
 // ---- lane-exchange butterflies, eight values per call -------------------------------------------
@@ -231,8 +258,8 @@ enum EmitMode { EMIT_NIBBLE = 0, EMIT_U8 = 1, EMIT_ANY = 2, EMIT_WEIGHT = 3 };
 template <int DT, int H, int EMIT, int WB, int GW, typename Request, typename Rotate>
 __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned char *smem, const int64_t row, const int tid, const int waves,
                                                      const uint32_t modes, const uint2 *cells, const float *thr, float cell_scale,
-                                                     float cell_offset, uint8_t *codes_row, int4 (&ea)[GW], int4 (&eb)[GW], Request request,
-                                                     Rotate rotate_step) {
+                                                     float cell_offset, uint8_t *codes_row, int4 (&ea)[GW], int4 (&eb)[GW], uint2 (&sg)[GW],
+                                                     Request request, Rotate rotate_step) {
   constexpr int SPAN = GW * kLaneSpan;   // slots a wavefront keeps, and the distance between the parts
   constexpr int CT = kChunk * GW / WB;   // columns a thread takes
   constexpr int N = CT * WB;             // values it turns into codes: 8 or 16
@@ -241,14 +268,14 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
   const int lane = tid & 63, wave = tid >> 6, team = wave / WB, teams = waves / WB, part = wave % WB;
   const int slot_lane = logical_lane(lane);
   float *buffer = reinterpret_cast<float *>(smem + fast_lds_bytes(a.K, DT));  // [K]
-  const bool plain = (modes & 1u) != 0u, searched = (modes & 2u) != 0u, signs_left = (modes & 4u) != 0u;
+  const bool plain = (modes & 1u) != 0u, searched = (modes & 2u) != 0u;
 #pragma nounroll
   for (int u = team; u < a.units && team < teams; u += teams) {
     if (u != team) request(u);
     const int first = u * H + part * SPAN;
     float y[GW][kChunk];
 #pragma unroll
-    for (int j = 0; j < GW; ++j) rotate_step(ea[j], eb[j], first + j * kLaneSpan, plain, signs_left, y[j]);
+    for (int j = 0; j < GW; ++j) rotate_step(ea[j], eb[j], sg[j], first + j * kLaneSpan, plain, true, y[j]);
     if constexpr (GW > 1) {
 #pragma unroll
       for (int dist = 1; dist < GW; dist <<= 1)
@@ -348,9 +375,9 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
   }
 }
 
-// One row.  `smem`: fast_lds_bytes(K, DT) bytes (and kWideBytes more if MAPPED, 4 K more if WB > 1), 16-byte aligned.
-// All 64 * waves threads of the workgroup make the call.  `after_loads` is called once by every thread, when it waits for
-// no load of its own any more but the gather entries.
+// One row.  `smem`: fast_lds_bytes(K, DT) bytes (kWideBytes more if MAPPED), shared_lds_bytes(K, DT) if WB > 1, 16-byte
+// aligned.  All 64 * waves threads of the workgroup make the call.  `after_loads` is called once by every thread, when it
+// has requested all it needs from memory (WB > 1), or waits for no load of its own any more but the gather entries.
 template <int DT, int LOG_H, int EMIT, bool MAPPED = false, int WB = 1, bool ANYWHERE = (WB > 1), typename AfterLoads>
 __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsigned char *smem, const int64_t row,
                                                          const int tid, const int waves, AfterLoads after_loads) {
@@ -372,17 +399,73 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset);
   const uint16_t *signs_by_position = reinterpret_cast<const uint16_t *>(gather + K), *signs_by_slot = signs_by_position + K;
 
+  const int nthreads = waves * 64;
+  const int Ki = static_cast<int>(K);
+  const int table_idx = min(tid, 255);
+  uint2 cell_v;
+  float thr_v;
+  constexpr int kElem = DT == OQ_F32 ? 4 : 2;
+  const unsigned char *xrow = static_cast<const unsigned char *>(a.x) + row * K * kElem;  // uniform
+  const int lane_first = lane * kChunk;
+  constexpr int kBatch = DT == OQ_F32 || WB > 1 ? 2 : 4;
+  struct Ring { uint4 lo[kBatch], hi[kBatch], signs[kBatch]; };  // requested chunks of 512 values (fp32: both halves; 16-bit: lo only) and their signs
+  auto request_row = [&](Ring &ring, int b, int i0) {  // chunks past the row: i0 >= Ki
+    ring.lo[b] = make_uint4(0u, 0u, 0u, 0u);
+    ring.hi[b] = ring.lo[b];
+    ring.signs[b] = ring.lo[b];
+    if (i0 < Ki) {
+      if constexpr (WB == 1) ring.signs[b] = *reinterpret_cast<const uint4 *>(signs_by_position + static_cast<uint32_t>(i0));
+      const uint4 *src = reinterpret_cast<const uint4 *>(xrow + static_cast<uint32_t>(i0) * kElem);
+      ring.lo[b] = src[0];
+      if constexpr (DT == OQ_F32) ring.hi[b] = src[1];
+    }
+  };
+
+  // WB > 1: everything but the plan's header and what depends on it is requested first - the tables, which lie at the
+  // plan's beginning, the wavefront's first chunks of the row, the positions and signs of its first step(s)
+  const uint32_t lds_at = ANYWHERE ? lds_byte_address(smem) : 0u;
+  constexpr int GW = G / WB;  // steps a wavefront keeps
+  const int team = wave / WB, part = wave % WB;  // wavefronts of one block
+  int4 early_a[GW], early_b[GW];
+  uint2 early_signs[GW];
+  auto request_shared = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < GW; ++j) {
+      const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + gather_first, Ki - kChunk));
+      early_a[j] = reinterpret_cast<const int4 *>(a.perm)[c / 4u];
+      early_b[j] = reinterpret_cast<const int4 *>(a.perm)[c / 4u + 1u];
+      early_signs[j] = *reinterpret_cast<const uint2 *>(a.signs + c);
+    }
+  };
+  Ring early;
+  if constexpr (WB > 1) {
+    cell_v = reinterpret_cast<const uint2 *>(a.plan + plan::kCellsOffset)[table_idx];
+    thr_v = reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) request_row(early, b, (wave + b * waves) * kLaneSpan + lane_first);
+    request_shared(team);
+    asm volatile("" ::: "memory");  // (requested here, and not moved to where they are first used)
+  }
+
   // A plan built for another shape must not be walked.  No codes are written then, and the row's norm
   // is stored as NaN, so that the mismatch cannot pass for a result: every output computed from it is NaN.
   // (The gather entries are LDS addresses for a block of LDS that starts at 0; ANYWHERE adds where it starts.)
-  if (hdr->magic != plan::kMagic || hdr->K != static_cast<uint32_t>(K) || hdr->block != static_cast<uint32_t>(H) ||
-      hdr->levels != static_cast<uint32_t>(a.levels) || (!ANYWHERE && lds_byte_address(smem) != 0u)) {
-    after_loads();
+  auto refuse = [&]() __attribute__((always_inline)) {
     if (tid == 0) {
       if (a.norms != nullptr) a.norms[row] = __builtin_nanf("");
       if constexpr (EMIT == EMIT_WEIGHT) a.norms_bf16[row] = 0x7fc0;
     }
-    return;
+  };
+// (an expression, not a lambda: behind its truth value the compiler kept five registers too many for eight wavefronts a SIMD)
+#define OQ_PLAN_IS_ANOTHERS                                                                                                        \
+  (hdr->magic != plan::kMagic || hdr->K != static_cast<uint32_t>(K) || hdr->block != static_cast<uint32_t>(H) ||                   \
+   hdr->levels != static_cast<uint32_t>(a.levels) || (!ANYWHERE && lds_byte_address(smem) != 0u))
+  if constexpr (WB == 1) {
+    if (OQ_PLAN_IS_ANOTHERS) {
+      after_loads();
+      refuse();
+      return;
+    }
   }
   const float cell_scale = EMIT == EMIT_WEIGHT ? hdr->weight_cell_scale : hdr->cell_scale;
   const float cell_offset = EMIT == EMIT_WEIGHT ? hdr->weight_cell_offset : hdr->cell_offset;
@@ -391,30 +474,15 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
 
   // tables: entry tid is requested now and stored to LDS after the row has been requested (loads
   // return in order); workgroups of fewer than 256 threads fetch the rest when they store.
-  const int nthreads = waves * 64;
-  const int Ki = static_cast<int>(K);
-  const int table_idx = min(tid, 255);
-  const uint2 cell_v = plan_cells[table_idx];
-  const float thr_v = EMIT == EMIT_WEIGHT ? (table_idx < a.levels - 1 ? a.raw_bounds[table_idx] : __builtin_inff())
-                                          : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
+  if constexpr (WB == 1) {
+    cell_v = plan_cells[table_idx];
+    thr_v = EMIT == EMIT_WEIGHT ? (table_idx < a.levels - 1 ? a.raw_bounds[table_idx] : __builtin_inff())
+                                : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
+  }
   const float cent_v = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(table_idx, a.levels - 1)] : 0.0f;
 
-  const uint32_t lds_at = ANYWHERE ? lds_byte_address(smem) : 0u;
-
-  // The gather entries of the first step(s) of this wavefront, where few rows are waited for: with the row, not behind it
-  constexpr int GW = G / WB;  // steps a wavefront keeps
-  const int team = wave / WB, teams = waves / WB, part = wave % WB;  // WB > 1: wavefronts of one block
+  // The gather entries of a wavefront's next step, requested one step ahead
   const unsigned char *gather_bytes = reinterpret_cast<const unsigned char *>(gather);  // uniform
-  int4 early_a[GW], early_b[GW];
-  auto request_shared = [&](int u) {
-#pragma unroll
-    for (int j = 0; j < GW; ++j) {
-      const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + gather_first, Ki - kChunk));
-      early_a[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u);
-      early_b[j] = *reinterpret_cast<const int4 *>(gather_bytes + c * 4u + 16u);
-    }
-  };
-  if constexpr (WB > 1) request_shared(team);
   int4 ea_next, eb_next;
   auto request_entries = [&](int first) {
     const uint32_t c = static_cast<uint32_t>(min(first + gather_first, Ki - kChunk));
@@ -433,116 +501,132 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   }
 
   // ---- phase A: stage the row with its signs, sum of squares ----------------------------------
-  // Virtual lane t of the documented [passes][256 lanes][8] order is lane t % 64 of group t / 64;
-  // wavefront w owns the groups w, w + waves, ... with all their passes, and keeps four passes of
-  // a group (fp32: two) requested ahead of the one it is summing; eight, the whole of most rows, cost few rows 0.35 us.  (Adding a lane's first pass to +0 is exact.)
-  constexpr int kElem = DT == OQ_F32 ? 4 : 2;
-  const unsigned char *xrow = static_cast<const unsigned char *>(a.x) + row * K * kElem;  // uniform
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
   uint32_t tiny_acc = 0xffffffffu;   // bf16: running minimum of (2 T - 1) - 2 |x| per half, T = bits of 2^-80
   bool tiny32 = false;               // fp32: a nonzero value below 2^-80 was seen
   const uint32_t kMadMul = 0xfffefffeu, kMadAdd = 0x2eff2effu;
-  const int lane_first = lane * kChunk;
-  constexpr int kBatch = DT == OQ_F32 ? 2 : 4;
-#pragma nounroll
-  for (int grp = wave; grp < 4; grp += waves) {  // uniform over the wavefront
-    float q = 0.0f;
-    uint4 raw_lo[kBatch], raw_hi[kBatch], raw_signs[kBatch];  // a ring of requested chunks (fp32: both halves; 16-bit: raw_lo only) and their signs
-    auto request = [&](int b, int p) {
-      const int i0 = p * kPass + grp * kLaneSpan + lane_first;  // chunks past the row: i0 >= Ki
-      raw_lo[b] = make_uint4(0u, 0u, 0u, 0u);
-      raw_hi[b] = raw_lo[b];
-      raw_signs[b] = raw_lo[b];
+  // Slot b of the ring, values i0 .. i0 + 7 (none: i0 >= Ki), to LDS; their squares' sum
+  auto take_chunk = [&](const Ring &ring, int b, int i0) __attribute__((always_inline)) -> float {
+    float f[kChunk];
+    if constexpr (DT == OQ_F32) {
       if (i0 < Ki) {
-        raw_signs[b] = *reinterpret_cast<const uint4 *>(signs_by_position + static_cast<uint32_t>(i0));
-        const uint4 *src = reinterpret_cast<const uint4 *>(xrow + static_cast<uint32_t>(i0) * kElem);
-        raw_lo[b] = src[0];
-        if constexpr (DT == OQ_F32) raw_hi[b] = src[1];
-      }
-    };
-#pragma unroll
-    for (int b = 0; b < kBatch; ++b) request(b, b);
-#pragma nounroll
-    for (int pb = 0; pb < a.passes; pb += kBatch) {
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int chunk0 = (pb + b) * kPass + grp * kLaneSpan;
-        const int i0 = chunk0 + lane_first;
-        if (chunk0 < Ki) {  // uniform over the wavefront; chunks wholly past the row would add +0
-          float f[kChunk];
-          if constexpr (DT == OQ_F32) {
-            if (i0 < Ki) {
-              uint4 lo = raw_lo[b], hi = raw_hi[b];
-              if (bijective) {
-                const uint4 sg = raw_signs[b];
-                lo.x ^= sg.x << 16; lo.y ^= sg.x & 0x80000000u; lo.z ^= sg.y << 16; lo.w ^= sg.y & 0x80000000u;
-                hi.x ^= sg.z << 16; hi.y ^= sg.z & 0x80000000u; hi.z ^= sg.w << 16; hi.w ^= sg.w & 0x80000000u;
-              }
-              uint4 *dst = reinterpret_cast<uint4 *>(stage + 4 * i0);
-              dst[0] = lo;
-              dst[1] = hi;
-            }
-            const uint32_t w[kChunk] = {raw_lo[b].x, raw_lo[b].y, raw_lo[b].z, raw_lo[b].w,
-                                        raw_hi[b].x, raw_hi[b].y, raw_hi[b].z, raw_hi[b].w};
-#pragma unroll
-            for (int e = 0; e < kChunk; ++e) {
-              f[e] = __uint_as_float(w[e]);
-              tiny32 = tiny32 || (f[e] != 0.0f && __builtin_fabsf(f[e]) < 0x1p-80f);
-            }
-          } else {
-            uint4 in = raw_lo[b];
-            if constexpr (MAPPED) {
-              // (lanes past the row's end look up an ordinary value instead of their zero padding, which lies
-              // outside the window and would send the whole wavefront to the table in memory; they add +0 as before)
-              const bool live = i0 < Ki;
-              uint4 one[1] = {live ? in : make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u)};
-              map_words8_many<OQ_BF16, 1, kWideLog2>(one, a.map, hot, kWideLoBf16);
-              in = live ? one[0] : make_uint4(0u, 0u, 0u, 0u);
-            }
-            const uint32_t w[4] = {in.x, in.y, in.z, in.w};
-            if (i0 < Ki) {
-              const uint4 sg = raw_signs[b];
-              *reinterpret_cast<uint4 *>(stage + 2 * i0) = bijective ? make_uint4(w[0] ^ sg.x, w[1] ^ sg.y, w[2] ^ sg.z, w[3] ^ sg.w) : in;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              if constexpr (DT == OQ_BF16) {
-                f[2 * j] = __uint_as_float(w[j] << 16);
-                f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-                uint32_t g;
-                asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(g) : "v"(w[j]), "v"(kMadMul), "v"(kMadAdd));
-                tiny_acc = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, tiny_acc),
-                                                                                  __builtin_bit_cast(u16x2, g)));
-              } else {
-                f[2 * j] = f16_bits_to_f32(static_cast<uint16_t>(w[j] & 0xffffu));
-                f[2 * j + 1] = f16_bits_to_f32(static_cast<uint16_t>(w[j] >> 16));
-              }
-            }
-          }
-#ifdef OQ_RQ_TIMING_NO_SUMSQ  // timing experiment only: what the pass would cost if the sums came from elsewhere
-          q = q + f[0];
-#else
-          float sq[kChunk];
-#pragma unroll
-          for (int e = 0; e < kChunk; ++e) sq[e] = f[e] * f[e];
-          q = q + (((sq[0] + sq[1]) + (sq[2] + sq[3])) + ((sq[4] + sq[5]) + (sq[6] + sq[7])));
-#endif
+        uint4 lo = ring.lo[b], hi = ring.hi[b];
+        if (WB == 1 && bijective) {
+          const uint4 sg = ring.signs[b];
+          lo.x ^= sg.x << 16; lo.y ^= sg.x & 0x80000000u; lo.z ^= sg.y << 16; lo.w ^= sg.y & 0x80000000u;
+          hi.x ^= sg.z << 16; hi.y ^= sg.z & 0x80000000u; hi.z ^= sg.w << 16; hi.w ^= sg.w & 0x80000000u;
         }
-        if (pb + kBatch < a.passes) request(b, pb + b + kBatch);  // refill the slot: four passes stay in flight
+        uint4 *dst = reinterpret_cast<uint4 *>(stage + 4 * i0);
+        dst[0] = lo;
+        dst[1] = hi;
+      }
+      const uint32_t w[kChunk] = {ring.lo[b].x, ring.lo[b].y, ring.lo[b].z, ring.lo[b].w,
+                                  ring.hi[b].x, ring.hi[b].y, ring.hi[b].z, ring.hi[b].w};
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) {
+        f[e] = __uint_as_float(w[e]);
+        tiny32 = tiny32 || (f[e] != 0.0f && __builtin_fabsf(f[e]) < 0x1p-80f);
+      }
+    } else {
+      uint4 in = ring.lo[b];
+      if constexpr (MAPPED) {
+        // (lanes past the row's end look up an ordinary value instead of their zero padding, which lies
+        // outside the window and would send the whole wavefront to the table in memory; they add +0 as before)
+        const bool live = i0 < Ki;
+        uint4 one[1] = {live ? in : make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u)};
+        map_words8_many<OQ_BF16, 1, kWideLog2>(one, a.map, hot, kWideLoBf16);
+        in = live ? one[0] : make_uint4(0u, 0u, 0u, 0u);
+      }
+      const uint32_t w[4] = {in.x, in.y, in.z, in.w};
+      if (i0 < Ki) {
+        const uint4 sg = ring.signs[b];
+        *reinterpret_cast<uint4 *>(stage + 2 * i0) = WB == 1 && bijective ? make_uint4(w[0] ^ sg.x, w[1] ^ sg.y, w[2] ^ sg.z, w[3] ^ sg.w) : in;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (DT == OQ_BF16) {
+          f[2 * j] = __uint_as_float(w[j] << 16);
+          f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+          uint32_t g;
+          asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(g) : "v"(w[j]), "v"(kMadMul), "v"(kMadAdd));
+          tiny_acc = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, tiny_acc),
+                                                                            __builtin_bit_cast(u16x2, g)));
+        } else {
+          f[2 * j] = f16_bits_to_f32(static_cast<uint16_t>(w[j] & 0xffffu));
+          f[2 * j + 1] = f16_bits_to_f32(static_cast<uint16_t>(w[j] >> 16));
+        }
       }
     }
+#ifdef OQ_RQ_TIMING_NO_SUMSQ  // timing experiment only: what the pass would cost if the sums came from elsewhere
+    return f[0];
+#else
+    float sq[kChunk];
+#pragma unroll
+    for (int e = 0; e < kChunk; ++e) sq[e] = f[e] * f[e];
+    return ((sq[0] + sq[1]) + (sq[2] + sq[3])) + ((sq[4] + sq[5]) + (sq[6] + sq[7]));
+#endif
+  };
+  // a group's sum over its 64 lanes
+  auto over_lanes = [](float q) __attribute__((always_inline)) -> float {
     q = q + rq::lane_xor<1>(q);
     q = q + rq::lane_xor<2>(q);
     q = q + rq::lane_xor<4>(q);
     q = q + rq::lane_xor<8>(q);
     q = q + rq::lane_xor<16>(q);
     q = q + rq::lane_xor<32>(q);
-    if (lane == 0) red[grp] = q;
+    return q;
+  };
+  float *sums = reinterpret_cast<float *>(smem + shared_sums_at(K, DT));  // WB > 1: [passes][64 lanes][4 groups]
+  if constexpr (WB > 1) {
+    // All wavefronts read the row, a chunk each (rows of more chunks than wavefronts: two or more); a lane's sums over the
+    // passes are put together from LDS, in their order.  (Read by four wavefronts, a group each, a row of 14336 values took
+    // 4.6 us to stage, and takes 1.9.)
+    after_loads();
+    const int chunks = Ki / kLaneSpan;  // (rows are whole blocks of 1024 and more)
+#pragma nounroll
+    for (int c0 = wave; c0 < chunks; c0 += kBatch * waves) {
+      if (c0 != wave) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) request_row(early, b, (c0 + b * waves) * kLaneSpan + lane_first);
+      }
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const int c = c0 + b * waves;
+        if (c < chunks) sums[((c >> 2) * 64 + lane) * 4 + (c & 3)] = take_chunk(early, b, c * kLaneSpan + lane_first);
+      }
+    }
+  } else {
+    // Virtual lane t of the documented [passes][256 lanes][8] order is lane t % 64 of group t / 64; wavefront w owns the
+    // groups w, w + waves, ... with all their passes, and keeps four passes of a group (fp32: two) requested ahead of the
+    // one it is summing; eight, the whole of most rows, cost few rows 0.35 us.
+#pragma nounroll
+    for (int grp = wave; grp < 4; grp += waves) {  // uniform over the wavefront
+      float q = 0.0f;
+      Ring ring;
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) request_row(ring, b, b * kPass + grp * kLaneSpan + lane_first);
+#pragma nounroll
+      for (int pb = 0; pb < a.passes; pb += kBatch) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+          const int chunk0 = (pb + b) * kPass + grp * kLaneSpan;
+          if (chunk0 < Ki) q = q + take_chunk(ring, b, chunk0 + lane_first);  // uniform over the wavefront; chunks wholly past the row would add +0
+          if (pb + kBatch < a.passes) request_row(ring, b, (pb + b + kBatch) * kPass + grp * kLaneSpan + lane_first);  // refill the slot: four passes stay in flight
+        }
+      }
+      q = over_lanes(q);  // (adding a lane's first pass to +0 was exact)
+      if (lane == 0) red[grp] = q;
+    }
   }
   bool tiny = tiny32;
   if constexpr (DT == OQ_BF16) tiny = min(tiny_acc & 0xffffu, tiny_acc >> 16) < 0x2effu;
   const bool wave_tiny = __builtin_amdgcn_ballot_w64(tiny) != 0;
-  if (lane == 0 && wave < 4) red[4 + wave] = wave_tiny ? 1.0f : 0.0f;  // (four wavefronts at most read the row)
+  uint8_t *wave_flags = reinterpret_cast<uint8_t *>(red + 4);  // WB > 1
+  if constexpr (WB > 1) {
+    if (lane == 0) wave_flags[wave] = wave_tiny ? 1 : 0;
+  } else {
+    if (lane == 0 && wave < 4) red[4 + wave] = wave_tiny ? 1.0f : 0.0f;  // (four wavefronts at most read the row)
+  }
   if constexpr (EMIT == EMIT_WEIGHT) {
     // The plan's table decides the indices only if it is one over the boundaries of this call: boundary j is the j-th
     // of the table, in the cell it falls into (a table has 63 boundaries at most, a lane of the first wavefront each;
@@ -566,9 +650,53 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
                                    : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[idx];
     cent[idx] = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(idx, a.levels - 1)] : 0.0f;
   }
-  after_loads();
+  if constexpr (WB == 1) {
+    after_loads();
+  } else {
+    if (OQ_PLAN_IS_ANOTHERS) {
+      refuse();
+      return;
+    }
+  }
+#undef OQ_PLAN_IS_ANOTHERS
   __syncthreads();
-  const float total = (red[0] + red[1]) + (red[2] + red[3]);
+  float total;
+  bool any_tiny;
+  if constexpr (WB > 1) {
+    any_tiny = __builtin_amdgcn_ballot_w64(wave_flags[min(lane, waves - 1)] != 0) != 0;
+    float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (a.passes <= kFewPasses) {  // every wavefront makes the four group sums for itself
+#pragma unroll
+      for (int p = 0; p < kFewPasses; ++p) {
+        if (p >= a.passes) break;
+        const float4 t = reinterpret_cast<const float4 *>(sums)[p * 64 + lane];
+        // (of a row that ends within a pass the groups that it has)
+        q[0] = q[0] + t.x;
+        q[1] = p * kPass + kLaneSpan < Ki ? q[1] + t.y : q[1];
+        q[2] = p * kPass + 2 * kLaneSpan < Ki ? q[2] + t.z : q[2];
+        q[3] = p * kPass + 3 * kLaneSpan < Ki ? q[3] + t.w : q[3];
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) q[g] = over_lanes(q[g]);
+    } else {  // four wavefronts make one each: long rows have more sums than they are worth reading sixteen times
+      if (wave < 4) {
+        float mine = 0.0f;
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+          if (p * kPass + wave * kLaneSpan < Ki) mine = mine + sums[(p * 64 + lane) * 4 + wave];
+        mine = over_lanes(mine);
+        if (lane == 0) red[wave] = mine;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int g = 0; g < 4; ++g) q[g] = red[g];
+    }
+    total = (q[0] + q[1]) + (q[2] + q[3]);
+  } else {
+    const float4 groups = *reinterpret_cast<const float4 *>(red), flags = *reinterpret_cast<const float4 *>(red + 4);
+    total = (groups.x + groups.y) + (groups.z + groups.w);
+    any_tiny = flags.x != 0.0f || (waves > 1 && flags.y != 0.0f) || (waves > 2 && flags.z != 0.0f) || (waves > 3 && flags.w != 0.0f);
+  }
   const float s_norm = sqrtf(total);
   Reciprocal rc;
   rc.d = s_norm + a.eps;
@@ -576,9 +704,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   constexpr bool kShortQuotient = DT != OQ_F32;
   const float remainder = __builtin_fmaf(-rc.d, rc.rh, 1.0f);
   rc.rl = kShortQuotient ? remainder / rc.d : remainder * rc.rh;
-  bool row_plain = !(rc.d >= 0x1p-80f && rc.d <= 0x1p20f) || short_quotient_fails<DT>(rc.d);
-#pragma nounroll
-  for (int w = 0; w < min(waves, 4); ++w) row_plain = row_plain || red[4 + w] != 0.0f;
+  const bool row_plain = !(rc.d >= 0x1p-80f && rc.d <= 0x1p20f) || short_quotient_fails<DT>(rc.d) || any_tiny;
   if (tid == 0 && a.norms != nullptr) a.norms[row] = s_norm;
   const float weight_denominator = s_norm < a.eps ? a.eps : s_norm;  // clamp_min(eps): a NaN norm stays NaN
   Reciprocal weight_rc{};
@@ -604,10 +730,15 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
 #pragma unroll
   for (int e = 0; e < kChunk; ++e) xv[e] = 0.0f;
   // Slots first + 8 lane .. + 7, gathered through their entries, divided by the norm, butterflies up to distance 256
-  auto rotate_step = [&](int4 ea, int4 eb, int first, bool plain, bool signs_left, float (&out)[kChunk]) __attribute__((always_inline)) {
+  // (WB > 1: their positions in the row and their signs, instead of the plan's entries)
+  auto rotate_step = [&](int4 ea, int4 eb, uint2 slot_signs, int first, bool plain, bool signs_left, float (&out)[kChunk]) __attribute__((always_inline)) {
     uint32_t ent[kChunk] = {static_cast<uint32_t>(ea.x), static_cast<uint32_t>(ea.y), static_cast<uint32_t>(ea.z),
                             static_cast<uint32_t>(ea.w), static_cast<uint32_t>(eb.x), static_cast<uint32_t>(eb.y),
                             static_cast<uint32_t>(eb.z), static_cast<uint32_t>(eb.w)};
+    if constexpr (WB > 1) {
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) ent[e] = 2u * ent[e] + plan::kStageAddress;
+    }
     if constexpr (DT == OQ_BF16) {
       if constexpr (ANYWHERE) {
 #pragma unroll
@@ -632,7 +763,11 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
         }
       }
     }
-    if (signs_left) {
+    if constexpr (WB > 1) {
+      const uint32_t w[2] = {slot_signs.x, slot_signs.y};
+#pragma unroll
+      for (int e = 0; e < kChunk; ++e) xv[e] = __uint_as_float(__float_as_uint(xv[e]) ^ ((w[e / 4] << (24 - 8 * (e & 3))) & 0x80000000u));
+    } else if (signs_left) {
       const uint4 sg = *reinterpret_cast<const uint4 *>(signs_by_slot + min(first + gather_first, Ki - kChunk));
       const uint32_t w[4] = {sg.x, sg.y, sg.z, sg.w};
 #pragma unroll
@@ -660,7 +795,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   };
   if constexpr (WB > 1) {
     rotate_shared_blocks<DT, H, EMIT, WB, GW>(a, smem, row, tid, waves, row_modes, cells, thr, cell_scale, cell_offset, codes_row,
-                                          early_a, early_b, request_shared, rotate_step);
+                                          early_a, early_b, early_signs, request_shared, rotate_step);
     return;
   }
   // The gather entries of a step are requested one step ahead (past the last step: the row's
@@ -679,7 +814,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
       // chunk instead: their blocks are their own, and nothing of theirs is stored.
       const int4 ea = ea_next, eb = eb_next;
       request_entries(j + 1 < G ? unit_base + (j + 1) * kLaneSpan : unit_base + waves * (G * kLaneSpan));
-      rotate_step(ea, eb, unit_base + j * kLaneSpan, plain, signs_left, y[j]);
+      rotate_step(ea, eb, make_uint2(0u, 0u), unit_base + j * kLaneSpan, plain, signs_left, y[j]);
     }
     // distances 512 and up: between the steps of the unit, in registers, one slot of every step at a time
     if constexpr (G > 1) {

@@ -146,9 +146,18 @@ __global__ __launch_bounds__(512, waves_per_simd(LOG_H, MAPPED)) void rotate_qua
   rotate_quantize_row_fast<DT, LOG_H, EMIT, MAPPED>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6, [] {});
 }
 
+// The arguments come one by one: the first sixteen dwords are in registers when a wavefront starts
+// (-amdgpu-kernarg-preload-count), where a struct has to be fetched before the first request can be made.
 template <int DT, int LOG_H, int EMIT, int WB>
-__global__ __launch_bounds__(1024) void rotate_quantize_shared_kernel(FastArgs a) {
+__global__ __launch_bounds__(1024) void rotate_quantize_shared_kernel(const void *x, const int32_t *perm, const int8_t *signs,
+                                                                      const unsigned char *plan, uint8_t *codes, float *norms, int K,
+                                                                      int levels, int levels_pow2, float eps) {
   extern __shared__ __align__(16) unsigned char smem[];
+  FastArgs a{};
+  a.x = x; a.perm = perm; a.signs = signs; a.plan = plan; a.codes = codes; a.norms = norms; a.K = K; a.levels = levels;
+  a.levels_pow2 = levels_pow2; a.eps = eps; a.block = 1 << LOG_H;
+  a.passes = (K + rqf::kPass - 1) / rqf::kPass;
+  a.units = row_units(K, 1 << LOG_H);
   rotate_quantize_row_fast<DT, LOG_H, EMIT, false, WB>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6, [] {});
 }
 
@@ -163,11 +172,12 @@ int launch_emit(const FastArgs &a, int waves, size_t smem, hipStream_t stream) {
 
 template <int DT, int LOG_H, int WB>
 int launch_shared(const FastArgs &a, hipStream_t stream) {
-  const size_t smem = fast_lds_bytes(a.K, DT) + 4u * static_cast<size_t>(a.K);
+  const size_t smem = shared_lds_bytes(a.K, DT);
   auto kern = a.code_format == OQ_CODES_NIBBLE ? rotate_quantize_shared_kernel<DT, LOG_H, EMIT_NIBBLE, WB> : rotate_quantize_shared_kernel<DT, LOG_H, EMIT_U8, WB>;
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "rotate_quantize: cannot reserve %zu bytes of LDS", smem);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.M)), dim3(static_cast<unsigned>(64 * WB * a.units)), smem, stream, a);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.M)), dim3(static_cast<unsigned>(64 * WB * a.units)), smem, stream, a.x, a.perm, a.signs,
+                     a.plan, a.codes, a.norms, static_cast<int>(a.K), a.levels, a.levels_pow2, a.eps);
   return check_launch("rotate_quantize (plan, shared blocks)");
 }
 
@@ -181,6 +191,7 @@ template <int DT, int LOG_H>
 int launch_few(const FastArgs &a, hipStream_t stream) {
   if constexpr (LOG_H >= 10) {
     if (a.map != nullptr || a.packed != nullptr || a.codes == nullptr || a.values != nullptr) return -1;
+    if (((reinterpret_cast<uintptr_t>(a.perm) | reinterpret_cast<uintptr_t>(a.signs)) & 15u) != 0) return -1;
     int wb = 1;
     while (wb < (1 << (LOG_H - 9)) && a.units * wb * 2 <= 16) wb *= 2;
     if (a.M * a.units * wb > 4096 && (a.units > 2 || a.M > 1024)) return -1;
@@ -269,15 +280,15 @@ int quantize_weight_fast(const void *w, int w_dtype, int64_t N, int64_t K, const
   if (!aligned16(w) || !aligned16(plan)) return fail(OQ_ERR_INVALID, "quantize_weight: w and the plan must be 16-byte aligned");
   if (N == 0) return OQ_OK;
   FastArgs a{};
-  fast_args_fill(a, w, N, K, plan, levels, block, eps);
+  fast_args_fill(a, w, N, K, plan, nullptr, nullptr, levels, block, eps);
   a.raw_bounds = boundaries; a.inv_sqrt_block = inv_sqrt_block; a.pack_bits = bits;
   a.packed = packed_out; a.packed_aligned = (reinterpret_cast<uintptr_t>(packed_out) & 7u) == 0;
   a.norms_bf16 = row_norms_out;
   return launch_fast(a, w_dtype, stream);
 }
 
-int rotate_quantize_fast(const void *x, int x_dtype, int64_t M, int64_t K, const void *plan, int levels, int64_t block,
-                         float eps, const float *centroids, void *codes_out, int code_format, void *values_out,
+int rotate_quantize_fast(const void *x, int x_dtype, int64_t M, int64_t K, const void *plan, const int32_t *perm, const int8_t *signs,
+                         int levels, int64_t block, float eps, const float *centroids, void *codes_out, int code_format, void *values_out,
                          int values_mode, float *norms_out, const uint16_t *input_map, hipStream_t stream) {
   auto aligned16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   int log_h = 0;
@@ -286,7 +297,7 @@ int rotate_quantize_fast(const void *x, int x_dtype, int64_t M, int64_t K, const
       (codes_out != nullptr && !aligned16(codes_out)) || (values_out != nullptr && !aligned16(values_out)))
     return -1;
   FastArgs a{};
-  fast_args_fill(a, x, M, K, plan, levels, block, eps);
+  fast_args_fill(a, x, M, K, plan, perm, signs, levels, block, eps);
   a.cents = values_mode != OQ_VALUES_NONE ? centroids : nullptr;
   a.codes = static_cast<uint8_t *>(codes_out); a.code_format = code_format;
   a.values = values_mode == OQ_VALUES_NONE ? nullptr : values_out; a.values_mode = values_mode;

@@ -58,7 +58,7 @@ int token_linear_dispatch(const void *x, int x_dtype, const uint16_t *input_map,
   // with a plan: blocks of 128 to 4096 (rows of K % 128 == 0 have no smaller ones unless the caller asks for them)
   if (plan != nullptr && (reinterpret_cast<uintptr_t>(plan) & 15u) == 0 && input_map == nullptr && block >= 128 && block <= 4096) {
     rqf::FastArgs f{};
-    rqf::fast_args_fill(f, x, 1, K, plan, levels, block, eps);
+    rqf::fast_args_fill(f, x, 1, K, plan, perm, signs, levels, block, eps);
     switch (bits) {
       case 2: return token_linear_plan_launch_w2(f, g, x_dtype, stream);
       case 3: return token_linear_plan_launch_w3(f, g, x_dtype, stream);

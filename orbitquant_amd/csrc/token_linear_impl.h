@@ -59,7 +59,7 @@ __global__ __launch_bounds__(64 * WAVES) void token_linear_plan_kernel(rqf::Fast
 
 template <int DT, int LOG_H, int BITS, int R, int WAVES>
 int launch_plan_waves(const rqf::FastArgs &q, const gemv::GemvArgs &g, hipStream_t stream) {
-  const size_t scratch = rqf::fast_lds_bytes(q.K, DT) + (LOG_H >= 10 ? 4u * static_cast<size_t>(q.K) : 0u);
+  const size_t scratch = LOG_H >= 10 ? rqf::shared_lds_bytes(q.K, DT) : rqf::fast_lds_bytes(q.K, DT);
   const size_t smem = scratch + static_cast<size_t>((q.K / 2 + 15) & ~static_cast<int64_t>(15)) + 16;
   auto kern = token_linear_plan_kernel<DT, LOG_H, BITS, R, WAVES>;
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))

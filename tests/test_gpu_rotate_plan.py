@@ -345,3 +345,34 @@ def test_a_layer_pickled_with_an_earlier_plan(dev):
         file.seek(0)
         restored = torch.load(file, weights_only=False)
         assert torch.equal(restored(x), want) and torch.equal(restored(x[:1]), want[:1])
+
+
+@pytest.mark.parametrize("m", [1, 12])
+def test_shared_blocks_refuse_a_plan_for_another_shape(dev, m):
+    """Few rows check the plan behind their first requests: still no codes, and NaN norms."""
+    from orbitquant_amd import _lib, ops
+
+    _, _, _, inv, _, _, t = constants(dev, 4096, 4096, 4)
+    _, _, _, other_inv, _, _, other = constants(dev, 2048, 2048, 4)
+    wrong = ops.rotate_plan(other["perm"], other["signs"], other["bounds"], block_size=2048, inv_sqrt_block=float(other_inv))
+    x = make_rows(16, 4096, torch.bfloat16, seed=5)[:m].contiguous().to(dev)
+    codes, norms = torch.full((m, 2048), 0xAB, dtype=torch.uint8, device=dev), torch.full((m,), -1.0, device=dev)
+    rc = _lib.load().oq_rotate_quantize(x.data_ptr(), 2, m, 4096, t["perm"].data_ptr(), t["signs"].data_ptr(), t["bounds"].data_ptr(), None, 16,
+                                        4096, 1e-10, float(inv), wrong.data_ptr(), codes.data_ptr(), 1, None, 0, norms.data_ptr(), None)
+    torch.cuda.synchronize()
+    assert rc == 0 and bool((codes == 0xAB).all()) and bool(torch.isnan(norms).all())
+
+
+@pytest.mark.parametrize("which", ["perm", "signs"])
+def test_few_rows_with_an_unaligned_permutation(dev, which):
+    """The shared form reads the permutation and the signs in pieces of sixteen and eight bytes; others take another kernel."""
+    from oracle import oracle_c
+
+    perm, signs, h, inv, _, bounds, t = constants(dev, 4096, 4096, 4)
+    x = make_rows(8, 4096, torch.bfloat16, seed=6)
+    t[which] = torch.cat([t[which][:1], t[which]])[1:]
+    assert t[which].data_ptr() % 8 != 0
+    (codes, _, norms), (plain, _, _) = both_kernels(x.to(dev), t, h, inv, code_format="u8")
+    want, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, signs, bounds, h, 1e-10, inv)
+    assert torch.equal(codes, plain) and np.array_equal(codes.cpu().numpy(), want)
+    assert np.array_equal(norms.cpu().numpy().view(np.int32), want_norms.view(np.int32))
