@@ -109,6 +109,12 @@ uint64_t oq_rotate_plan_bytes(int64_t K);
 int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels,
                          int64_t K, int64_t block, float inv_sqrt_block, void *plan_out, void *stream);
 
+/* The same launch, which also copies perm and signs to perm_copy int32 [K] and signs_copy int8 [K]: for a caller whose
+ * constants came to the device in one buffer and that wants them in memory of their own. */
+int oq_rotate_plan_build_copy(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
+                              int64_t block, float inv_sqrt_block, void *plan_out, int32_t *perm_copy, int8_t *signs_copy,
+                              void *stream);
+
 /*
  * The weight side of a layer on the GPU: what the packed matmuls read, made from a float weight
  * matrix.  Replaces the reference's device-side weight quantization

@@ -93,8 +93,6 @@ int rotate_quantize_dispatch(const void *x, int x_dtype, int64_t M, int64_t K, c
                              int levels, int64_t block, float eps, float inv_sqrt_block,
                              void *codes_out, int code_format, void *values_out, int values_mode,
                              float *norms_out, const uint16_t *input_map, const void *plan, hipStream_t stream);
-int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
-                      int64_t block, float inv_sqrt_block, void *plan_out, hipStream_t stream);
 int quantize_weight_fast(const void *w, int w_dtype, int64_t N, int64_t K, const void *plan, const float *boundaries,
                          int levels, int64_t block, float eps, float inv_sqrt_block, int bits, uint8_t *packed_out,
                          uint16_t *row_norms_out, hipStream_t stream);
@@ -225,7 +223,13 @@ uint64_t oq_rotate_plan_bytes(int64_t K) { return K > 0 ? plan::plan_bytes(K) : 
 
 int oq_rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
                          int64_t block, float inv_sqrt_block, void *plan_out, void *stream) {
-  return rotate_plan_build(perm, signs, boundaries, levels, K, block, inv_sqrt_block, plan_out, as_stream(stream));
+  return rotate_plan_build(perm, signs, boundaries, levels, K, block, inv_sqrt_block, plan_out, nullptr, nullptr, as_stream(stream));
+}
+
+int oq_rotate_plan_build_copy(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K, int64_t block,
+                              float inv_sqrt_block, void *plan_out, int32_t *perm_copy, int8_t *signs_copy, void *stream) {
+  if (perm_copy == nullptr || signs_copy == nullptr) return fail(OQ_ERR_INVALID, "rotate_plan_build_copy: null copy");
+  return rotate_plan_build(perm, signs, boundaries, levels, K, block, inv_sqrt_block, plan_out, perm_copy, signs_copy, as_stream(stream));
 }
 
 int oq_rotate_quantize_mapped(const void *x, int x_dtype, const uint16_t *input_map, int64_t M, int64_t K,

@@ -68,7 +68,7 @@ __device__ __forceinline__ uint32_t cell_of(float v, float scale, float offset) 
 
 // Host side (rotate_quantize_fast.hip).
 int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
-                      int64_t block, float inv_sqrt_block, void *plan_out, hipStream_t stream);
+                      int64_t block, float inv_sqrt_block, void *plan_out, int32_t *perm_copy, int8_t *signs_copy, hipStream_t stream);
 // -1: this plan / shape has no fast kernel (the caller takes the plain one); else a status.
 int rotate_quantize_fast(const void *x, int x_dtype, int64_t M, int64_t K, const void *plan, const int32_t *perm, const int8_t *signs,
                          int levels, int64_t block, float eps, const float *centroids, void *codes_out, int code_format, void *values_out,

@@ -11,7 +11,7 @@ using namespace rqf;
 
 // ---- plan construction: once per layer, twice per converted weight ----------
 // Workgroup 0 makes the header and the tables, the last one checks that the permutation is one, the others write 256
-// gather entries and signs each (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
+// gather entries and signs each, and copies of the two where the caller wants its own (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
 // for rows of some thousand values; 6.2 us with the second table and the check).
 // Floats in an order-preserving integer code, so that "the largest float t with RN(t * c) <= b" can
 // be found by bisection over all of them.
@@ -25,7 +25,7 @@ __device__ __forceinline__ float ordered_to_float(uint32_t o) {
 
 __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *perm, const int8_t *signs,
                                                                  const float *boundaries, int levels, int K, int block,
-                                                                 float c, unsigned char *out) {
+                                                                 float c, unsigned char *out, int32_t *perm_copy, int8_t *signs_copy) {
   __shared__ float thr[256];
   __shared__ int bad;
   const int tid = threadIdx.x;
@@ -57,7 +57,12 @@ __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *p
     const int i = (static_cast<int>(blockIdx.x) - 1) * 256 + tid;
     if (i < K) {
       const uint32_t p = static_cast<uint32_t>(perm[i]);
-      const uint16_t sign = signs[i] < 0 ? 0x8000u : 0u;
+      const int8_t signed_one = signs[i];
+      const uint16_t sign = signed_one < 0 ? 0x8000u : 0u;
+      if (perm_copy != nullptr) {
+        perm_copy[i] = static_cast<int32_t>(p);
+        signs_copy[i] = signed_one;
+      }
       gather[i] = plan::kStageAddress + 2u * p;
       by_slot[i] = sign;
       if (p < static_cast<uint32_t>(K)) by_position[p] = sign;
@@ -245,9 +250,10 @@ int launch_dtype(const FastArgs &a, int log_h, int waves, size_t smem, hipStream
 }  // namespace
 
 int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *boundaries, int levels, int64_t K,
-                      int64_t block, float inv_sqrt_block, void *plan_out, hipStream_t stream) {
+                      int64_t block, float inv_sqrt_block, void *plan_out, int32_t *perm_copy, int8_t *signs_copy, hipStream_t stream) {
   if (perm == nullptr || signs == nullptr || boundaries == nullptr || plan_out == nullptr)
     return fail(OQ_ERR_INVALID, "rotate_plan_build: null pointer");
+  if ((perm_copy == nullptr) != (signs_copy == nullptr)) return fail(OQ_ERR_INVALID, "rotate_plan_build: one copy without the other");
   if (levels < 2 || levels > 256) return fail(OQ_ERR_INVALID, "rotate_plan_build: levels=%d not in [2, 256]", levels);
   if (K <= 0 || K > 16384) return fail(OQ_ERR_UNSUPPORTED, "rotate_plan_build: K=%lld not in [1, 16384]", (long long)K);
   if (block <= 0 || (block & (block - 1)) != 0 || K % block != 0)
@@ -256,7 +262,7 @@ int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *bou
     return fail(OQ_ERR_INVALID, "rotate_plan_build: inv_sqrt_block must be positive and finite");
   if ((reinterpret_cast<uintptr_t>(plan_out) & 15u) != 0) return fail(OQ_ERR_INVALID, "rotate_plan_build: the plan must be 16-byte aligned");
   hipLaunchKernelGGL(rotate_plan_build_kernel, dim3(static_cast<unsigned>(2 + (K + 255) / 256)), dim3(256), 0, stream, perm, signs, boundaries, levels,
-                     static_cast<int>(K), static_cast<int>(block), inv_sqrt_block, static_cast<unsigned char *>(plan_out));
+                     static_cast<int>(K), static_cast<int>(block), inv_sqrt_block, static_cast<unsigned char *>(plan_out), perm_copy, signs_copy);
   return check_launch("rotate_plan_build");
 }
 

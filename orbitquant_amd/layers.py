@@ -24,6 +24,8 @@ There is no dequantized-weight or CPU fallback on this path.
 
 from __future__ import annotations
 
+from functools import lru_cache
+
 import numpy as np
 import torch
 from torch import nn
@@ -32,7 +34,7 @@ from . import _lib, ops
 from .codebooks import get_codebook
 from .config import OrbitQuantConfig
 from .rotations import get_rpbh_rotation
-from .weights import quantize_weight
+from .weights import quantize_weight, quantized_on_gpu
 
 _LIB = torch.library.Library("orbitquant_amd", "DEF")
 _SCHEMA = (
@@ -104,23 +106,40 @@ def _host_constants(rotation, activation_codebook, weight_codebook) -> dict[str,
     }
 
 
+class _Packed(dict):
+    """Tensors on the host, and `host`, a pinned buffer that holds them one behind the other, 256 bytes apart or more."""
+
+    def __init__(self, tensors: dict[str, torch.Tensor]) -> None:
+        super().__init__(tensors)
+        self.sizes = [(t.numel() * t.element_size() + 255) & -256 for t in tensors.values()]
+        self.host = torch.empty(sum(self.sizes), dtype=torch.uint8, device="cpu", pin_memory=True)   # (whatever the default device is)
+        raw, at = self.host.numpy(), 0   # (numpy's slices and copies, not torch's: the quantizer's launch comes 17 us sooner)
+        for t, size in zip(tensors.values(), self.sizes):
+            values = t.contiguous().numpy().reshape(-1).view(np.uint8)
+            raw[at : at + values.size] = values
+            at += size
+
+
+@lru_cache(maxsize=16)
+def _conversion_constants(dim: int, seed: int, block_size, weight_bits: int, activation_bits: int, version: int) -> _Packed:
+    """What a conversion takes to the GPU.  It depends on these numbers alone, like the rotation and the codebooks it is made
+    of; a model's layers have a few of them (some 70 KB each).  Packing them anew took 38 of the 82 us that lay before the
+    quantizer's launch."""
+    rotation, codebook = get_rpbh_rotation(dim, seed, block_size), get_codebook(dim, weight_bits, version)
+    return _Packed({**_host_constants(rotation, get_codebook(dim, activation_bits, version), codebook), "weight_boundaries": codebook.boundaries})
+
+
 def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[str, torch.Tensor]:
     """`tensors` (on the host) on `device`.  For a GPU they are packed into one pinned buffer and taken there in one
     copy on the current stream: the tensors are views of it, 256 bytes apart or more.  The copy is not waited for; who
     hands the tensors on calls `_wait_for` first.  (A copy each is a synchronization each.)"""
     if device.type != "cuda" or torch.cuda.is_current_stream_capturing():   # (a graph would read the buffer again at each replay)
         return {name: t.to(device) for name, t in tensors.items()}
-    sizes = [(t.numel() * t.element_size() + 255) & -256 for t in tensors.values()]
-    host = torch.empty(sum(sizes), dtype=torch.uint8, device="cpu", pin_memory=True)   # (whatever the default device is)
-    raw, at = host.numpy(), 0   # (numpy's slices and copies, not torch's: the quantizer's launch comes 17 us sooner)
-    for t, size in zip(tensors.values(), sizes):
-        values = t.contiguous().numpy().reshape(-1).view(np.uint8)
-        raw[at : at + values.size] = values
-        at += size
-    there = host.to(device, non_blocking=True)
+    packed = tensors if isinstance(tensors, _Packed) else _Packed(tensors)
+    there = packed.host.to(device, non_blocking=True)
     typed = {dtype: there.view(dtype) for dtype in {t.dtype for t in tensors.values()}}
     views, at = {}, 0
-    for (name, t), size in zip(tensors.items(), sizes):
+    for (name, t), size in zip(packed.items(), packed.sizes):
         first = at // t.element_size()
         view = typed[t.dtype][first : first + t.numel()]
         views[name] = view if t.dim() == 1 else view.view(t.shape)
@@ -156,6 +175,7 @@ class OrbitLinear(nn.Module):
         row_norms: torch.Tensor,
         module_name: str = "",
         constants: dict[str, torch.Tensor] | None = None,
+        rotation_plan: torch.Tensor | None = None,
     ) -> None:
         super().__init__()
         self.in_features = in_features
@@ -179,12 +199,13 @@ class OrbitLinear(nn.Module):
         else:
             self.bias = nn.Parameter(bias.detach().clone(), requires_grad=False)
         device = packed_weight_indices.device
-        if constants is None:   # (`from_weight` has them on the device already)
-            constants = _on_device(self._constants(), device)
-        for name, tensor in _separate(constants).items():
+        if constants is None:   # (`from_weight` has them on the device already, in storages of their own)
+            constants = _separate(_on_device(self._constants(), device))
+        for name, tensor in constants.items():
             self.register_buffer(name, tensor, persistent=False)
-        self.register_buffer("_rotation_plan", None, persistent=False)
-        self._build_rotation_plan()
+        self.register_buffer("_rotation_plan", rotation_plan, persistent=False)
+        if rotation_plan is None:
+            self._build_rotation_plan()
         self.last_effective_runtime_mode: str | None = None
         self._input_activation = None  # (fn, dtype) once fuse_input_activation() was called
         self.register_buffer("_input_activation_table", None, persistent=False)
@@ -305,19 +326,31 @@ class OrbitLinear(nn.Module):
         rotation = get_rpbh_rotation(in_features, config.rotation_seed, config.block_size)
         codebook = get_codebook(in_features, config.weight_bits, config.codebook_version)
         device = weight.device
-        constants = quantizer_constants = None
+        constants = quantizer_constants = plan = None
         if device.type == "cuda":
-            activation_codebook = get_codebook(in_features, config.activation_bits, config.codebook_version)
-            constants = _on_device({**_host_constants(rotation, activation_codebook, codebook), "weight_boundaries": codebook.boundaries}, device)
-            quantizer_constants = (constants["_rotation_permutation"], constants["_rotation_signs"], constants.pop("weight_boundaries"))
+            constants = _on_device(_conversion_constants(in_features, config.rotation_seed, config.block_size, config.weight_bits,
+                                                         config.activation_bits, config.codebook_version), device)
+            boundaries = constants.pop("weight_boundaries")
+            if quantized_on_gpu(weight, rotation):
+                # the quantizer's plan; its launch also gives the layer a permutation and signs in storages of their own
+                # (two copies behind the quantizer, 9 us, when they were cloned), and where the weights have as many bits as the
+                # activations it is the layer's plan too
+                own = {name: torch.empty_like(constants[name]) for name in ("_rotation_permutation", "_rotation_signs")}
+                plan = ops.rotate_plan(constants["_rotation_permutation"], constants["_rotation_signs"], boundaries,
+                                       block_size=rotation.block_size, inv_sqrt_block=rotation.normalization, copies=tuple(own.values()))
+                quantizer_constants = (constants["_rotation_permutation"], constants["_rotation_signs"], boundaries)
+                constants.update(own)
+            else:
+                constants = _separate(constants)
         packed, row_norms = quantize_weight(
             weight, rotation=rotation, codebook=codebook, bits=config.weight_bits,
-            eps=config.activation_eps, row_tile=config.weight_row_tile_size, constants=quantizer_constants)
+            eps=config.activation_eps, row_tile=config.weight_row_tile_size, constants=quantizer_constants, plan=plan)
         return cls(
             in_features=in_features, out_features=out_features, config=config,
             bias=None if bias is None else bias.detach(),
             packed_weight_indices=packed.to(device), row_norms=row_norms.to(device),
-            module_name=module_name, constants=constants)
+            module_name=module_name, constants=constants,
+            rotation_plan=plan if config.weight_bits == config.activation_bits else None)
 
     @classmethod
     def empty_from_linear(cls, layer: nn.Linear, *, config: OrbitQuantConfig, module_name: str = "") -> "OrbitLinear":

@@ -124,10 +124,11 @@ class _OnDevice:
 
 
 def rotate_plan(permutation: torch.Tensor, signs: torch.Tensor, boundaries: torch.Tensor, *, block_size: int,
-                inv_sqrt_block: float) -> torch.Tensor:
+                inv_sqrt_block: float, copies: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:
     """The rotate plan of a layer (`oq_rotate_plan_build`): a uint8 blob on the constants' device
     that `rotate_quantize(plan=...)` and `quantized_linear(plan=...)` take to run the plan-based
-    kernel.  Built by one small launch; valid for exactly these constants."""
+    kernel.  Built by one small launch; valid for exactly these constants.  `copies`: two tensors of the
+    permutation's and the signs' form that the launch fills with them."""
     _require_gpu(permutation, "permutation")
     dim = permutation.numel()
     permutation = _operand(permutation, "permutation", permutation, dtype=torch.int32)
@@ -136,19 +137,23 @@ def rotate_plan(permutation: torch.Tensor, signs: torch.Tensor, boundaries: torc
     lib = _lib.load()
     plan = torch.empty(int(lib.oq_rotate_plan_bytes(dim)), dtype=torch.uint8, device=permutation.device)
     with _OnDevice(permutation):
-        rc = lib.oq_rotate_plan_build(permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(),
-                                      boundaries.numel() + 1, dim, int(block_size), float(inv_sqrt_block),
-                                      plan.data_ptr(), _stream(permutation))
+        args = (permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(), boundaries.numel() + 1, dim, int(block_size),
+                float(inv_sqrt_block), plan.data_ptr())
+        if copies is None:
+            rc = lib.oq_rotate_plan_build(*args, _stream(permutation))
+        else:
+            rc = lib.oq_rotate_plan_build_copy(*args, *(t.data_ptr() for t in copies), _stream(permutation))
     _lib.check(rc, "oq_rotate_plan_build")
     plan._oq_plan_of = (int(dim), int(block_size), int(boundaries.numel() + 1))
     return plan
 
 
 def quantize_weight(weight: torch.Tensor, permutation: torch.Tensor, signs: torch.Tensor, boundaries: torch.Tensor, *,
-                    bits: int, block_size: int, eps: float, inv_sqrt_block: float,
-                    row_tile: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+                    bits: int, block_size: int, eps: float, inv_sqrt_block: float, row_tile: int | None = None,
+                    plan: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """The weight side of a layer on the GPU (`oq_quantize_weight`): -> (packed uint8
-    [ceil(N*K*bits/8)], row_norms bfloat16 [N]) on the weight's device.  `row_tile` bounds the
+    [ceil(N*K*bits/8)], row_norms bfloat16 [N]) on the weight's device.  `plan`: `rotate_plan` of these
+    constants, where there is one already.  `row_tile` bounds the
     rows converted per launch (the launches write disjoint byte ranges of the same stream, so the
     result does not depend on it; tiles end on byte boundaries because K is a multiple of 8)."""
     _require_gpu(weight, "weight")
@@ -161,7 +166,10 @@ def quantize_weight(weight: torch.Tensor, permutation: torch.Tensor, signs: torc
     permutation = _operand(permutation, "permutation", w, dtype=torch.int32, numel=k)
     signs = _operand(signs, "signs", w, dtype=torch.int8, numel=k)
     boundaries = _operand(boundaries, "boundaries", w, dtype=torch.float32)
-    plan = rotate_plan(permutation, signs, boundaries, block_size=block_size, inv_sqrt_block=inv_sqrt_block)
+    if plan is None:
+        plan = rotate_plan(permutation, signs, boundaries, block_size=block_size, inv_sqrt_block=inv_sqrt_block)
+    else:
+        plan = _plan_operand(plan, w, k, block_size, boundaries.numel() + 1)
     packed = torch.empty((n * k * bits + 7) // 8, dtype=torch.uint8, device=w.device)
     norms = torch.empty(n, dtype=torch.bfloat16, device=w.device)
     lib = _lib.load()

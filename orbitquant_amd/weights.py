@@ -37,6 +37,13 @@ def quantize_weight_indices(
     return codebook.quantize_indices(unit)
 
 
+def quantized_on_gpu(weight: torch.Tensor, rotation: RPBHRotation) -> bool:
+    """Whether the GPU's quantizer takes this weight."""
+    k = weight.shape[1]
+    return (weight.device.type == "cuda" and k % 8 == 0 and k <= 16384 and 8 <= rotation.block_size <= 4096
+            and weight.dtype in (torch.float32, torch.float16, torch.bfloat16))
+
+
 def quantize_weight(
     weight: torch.Tensor,
     *,
@@ -46,16 +53,17 @@ def quantize_weight(
     eps: float,
     row_tile: int = 4096,
     constants: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
+    plan: torch.Tensor | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """-> (packed uint8 [ceil(N*K*bits/8)], row_norms bfloat16 [N]), on the GPU for a GPU weight the
     kernel takes, else on the CPU.  `row_tile` bounds the rows whose fp32 copies the host path holds at a
     time; the result does not depend on it, and a GPU weight is one launch without such copies.
-    `constants`: permutation (int32), signs (int8) and boundaries where they are on the weight's device already."""
+    `constants`: permutation (int32), signs (int8) and boundaries where they are on the weight's device already, and
+    `plan` the rotate plan of these."""
     if weight.ndim != 2:
         raise ValueError("weight must be a matrix")
     n, k = weight.shape
-    if (weight.device.type == "cuda" and k % 8 == 0 and k <= 16384 and 8 <= rotation.block_size <= 4096
-            and weight.dtype in (torch.float32, torch.float16, torch.bfloat16)):
+    if quantized_on_gpu(weight, rotation):
         from . import ops
 
         device = weight.device
@@ -66,7 +74,7 @@ def quantize_weight(
                          codebook.boundaries.to(device))
         return ops.quantize_weight(
             weight, *constants, bits=bits, block_size=rotation.block_size, eps=eps,
-            inv_sqrt_block=rotation.normalization)
+            inv_sqrt_block=rotation.normalization, plan=plan)
     # Tiles must end on a byte boundary of the flat stream: rows * k * bits % 8 == 0.
     align = 8
     while (align // 2) * k * bits % 8 == 0 and align > 1:

@@ -237,3 +237,21 @@ def test_a_plan_over_other_boundaries_decides_nothing(dev, k, change):
                                   packed.data_ptr(), norms.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
     want_packed, want_norms, _ = o.quantize_weight(w.float().numpy(), perm, signs, bounds, block, 1e-10, bits, norm_order="sumsq_v1")
     assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
+
+
+@pytest.mark.parametrize("bits", [(4, 4), (3, 4)])
+def test_a_converted_layer_has_what_a_built_one_has(dev, bits):
+    """One plan where weights and activations share a codebook, constants in storages of their own."""
+    import io
+
+    from orbitquant_amd import OrbitLinear, OrbitQuantConfig
+
+    config = OrbitQuantConfig(weight_bits=bits[0], activation_bits=bits[1])
+    w = torch.randn(136, 384, generator=torch.Generator().manual_seed(4)).bfloat16().to(dev)
+    for layer in (OrbitLinear.from_weight(w, bias=None, config=config), OrbitLinear.from_weight(w, bias=None, config=config)):
+        built = OrbitLinear(in_features=384, out_features=136, config=config, bias=None, packed_weight_indices=layer.packed_weight_indices,
+                            row_norms=layer.row_norms)
+        for (name, a), (other, b) in zip(layer.named_buffers(), built.named_buffers()):
+            assert name == other and a.dtype == b.dtype and torch.equal(a, b), name
+        torch.save(layer, io.BytesIO())
+        layer._rotation_signs.neg_()      # (a layer's constants are its own: the next one is not made of them)
