@@ -92,8 +92,9 @@ inline void fast_args_fill(FastArgs &a, const void *x, int64_t M, int64_t K, con
 }
 
 // LDS: cells (2048) | thresholds (1024) | centroids (1024) | reduction slots (64) | staging
-// kRedAt: four group sums, then five flags (WB > 1: four group sums, then a byte for every wavefront)
+// kRedAt: four group sums, then six flags (WB > 1: four group sums, then a byte for every wavefront)
 constexpr int kCellsAt = 0, kThrAt = 2048, kCentAt = 3072, kRedAt = 4096, kStageAt = plan::kStageAddress;
+constexpr int kFoldValues = 1100;  // values a wavefront, from which on a weight row has thresholds of its own
 
 // The row is staged once, in its own type; behind it, for a launch with an input map, the map's 16 KB window
 // (value_map.h).  Long rows are bound by how many wavefronts a CU holds, and that by LDS and registers: with a second,
@@ -241,6 +242,30 @@ __device__ __forceinline__ void count_below(const uint2 (&ent)[kChunk], const fl
       : "v"(ent[0].x), "v"(ent[1].x), "v"(ent[2].x), "v"(ent[3].x), "v"(ent[4].x), "v"(ent[5].x), "v"(ent[6].x), "v"(ent[7].x),
         "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
         "v"(ent[0].y), "v"(ent[1].y), "v"(ent[2].y), "v"(ent[3].y), "v"(ent[4].y), "v"(ent[5].y), "v"(ent[6].y), "v"(ent[7].y));
+}
+
+// ---- a weight row's thresholds --------------------------------------------------------------------
+// Floats in an order-preserving integer code, and `steps` floats further up.
+__device__ __forceinline__ uint32_t float_to_ordered(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float ordered_to_float(uint32_t o) {
+  return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+}
+__device__ __forceinline__ float float_above(float f, int steps) { return ordered_to_float(float_to_ordered(f) + static_cast<uint32_t>(steps)); }
+
+// The largest float t with op(t) <= b, where op rounds an exact product or quotient (`scale` is the inverse factor) once:
+// the largest below the middle between b and the next float, taken back through the factor in fp64.  Whether it is one
+// is looked at: `found` stays true only if op says so on both sides (an infinity or NaN anywhere says no).
+template <typename Op>
+__device__ __forceinline__ float largest_below(float b, double scale, bool &found, Op op) {
+  b = b + 0.0f;  // (-0 is 0)
+  const double middle = 0.5 * (static_cast<double>(b) + static_cast<double>(float_above(b, 1)));
+  const float near = static_cast<float>(middle * scale) + 0.0f;
+  const float below = float_above(near, -1);
+  found = found && op(below) <= b && !(op(float_above(near, 1)) <= b);
+  return op(near) <= b ? near : below;
 }
 
 // What a launch writes: EMIT_NIBBLE / EMIT_U8 are the two hot forms (codes only), EMIT_ANY reads
@@ -394,7 +419,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   uint2 *cells = reinterpret_cast<uint2 *>(smem + kCellsAt);
   float *thr = reinterpret_cast<float *>(smem + kThrAt);
   float *cent = reinterpret_cast<float *>(smem + kCentAt);
-  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..7] per-wavefront flags, [8] the table is another's
+  float *red = reinterpret_cast<float *>(smem + kRedAt);       // [0..3] group sums, [4..7] per-wavefront flags, [8] the table is another's, [9] a weight row has thresholds
   unsigned char *stage = smem + kStageAt;
   const uint32_t *gather = reinterpret_cast<const uint32_t *>(a.plan + plan::kGatherOffset);
   const uint16_t *signs_by_position = reinterpret_cast<const uint16_t *>(gather + K), *signs_by_slot = signs_by_position + K;
@@ -641,14 +666,14 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   if (tid < 256) {
     cells[tid] = cell_v;
     thr[tid] = thr_v;
-    cent[tid] = cent_v;
+    if constexpr (EMIT == EMIT_ANY) cent[tid] = cent_v;
   }
 #pragma nounroll
   for (int idx = tid + nthreads; idx < 256; idx += nthreads) {  // workgroups of fewer than 256 threads only
     cells[idx] = plan_cells[idx];
     thr[idx] = EMIT == EMIT_WEIGHT ? (idx < a.levels - 1 ? a.raw_bounds[idx] : __builtin_inff())
                                    : reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[idx];
-    cent[idx] = (EMIT == EMIT_ANY && a.cents != nullptr) ? a.cents[min(idx, a.levels - 1)] : 0.0f;
+    if constexpr (EMIT == EMIT_ANY) cent[idx] = a.cents != nullptr ? a.cents[min(idx, a.levels - 1)] : 0.0f;
   }
   if constexpr (WB == 1) {
     after_loads();
@@ -721,8 +746,39 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   // The two rare modes (IEEE division for this row, binary search instead of the cell table) pass
   // through an empty asm statement inside the loop on purpose: as loop invariants the compiler
   // clones the whole loop per combination.
+  // A weight's index counts the boundaries below RN(RN(y c) / n), which ascends with y: boundary j is below it just where
+  // t_j is below y, t_j the largest float whose quotient is not above the boundary.  So the row's norm goes into the
+  // thresholds, a lane of the first wavefront each (the largest product first, then the largest y of that product), and a
+  // value is compared as it leaves the butterflies: no product and no division for each, six of its 36 vector instructions.  The
+  // cells of the table are scaled by c / n and keep their places if every t_j falls into the cell of its boundary; a row of
+  // which one does not, or whose quotients are not those of divide_fast either, is divided value by value.  The thresholds
+  // are some 170 instructions of one wavefront: rows with fewer than kFoldValues values a wavefront are divided too (12288 x
+  // 3072, three wavefronts a row, 59.2 -> 60.1 us).  With the plan's launch: 14336 x 4096 into four bits 91.3 -> 87.8 us, of
+  // fp32 140 -> 128 us, 4096 x 14336 79.6 -> 75.8 us, 5120 x 13824 88.1 -> 80.6 us.
+  bool folded = false;
+  float folded_scale = 0.0f;
+  if constexpr (EMIT == EMIT_WEIGHT) {
+    folded_scale = cell_scale * (a.inv_sqrt_block / weight_denominator);
+    if (hdr->weight_cells != 0 && red[8] == 0.0f && !weight_plain && Ki >= kFoldValues * waves) {  // uniform over the workgroup
+      if (wave == 0) {
+        const bool mine = lane < a.levels - 1;
+        bool found = true;  // (thr_v: boundary `lane`)
+        const float product = largest_below(thr_v, static_cast<double>(weight_denominator), found,
+                                            [&](float u) __attribute__((always_inline)) { return u / weight_denominator; });
+        const float threshold = largest_below(product, 1.0 / static_cast<double>(a.inv_sqrt_block), found,
+                                              [&](float y) __attribute__((always_inline)) { return y * a.inv_sqrt_block; });
+        const uint32_t cell = plan::cell_of(thr_v, cell_scale, cell_offset);
+        found = found && plan::cell_of(threshold, folded_scale, cell_offset) == cell;
+        const bool all = __builtin_amdgcn_ballot_w64(mine && !found) == 0;
+        if (all && mine) cells[cell].x = __float_as_uint(threshold);
+        if (lane == 0) red[9] = all ? 1.0f : 0.0f;
+      }
+      __syncthreads();
+      folded = red[9] != 0.0f;
+    }
+  }
   const bool has_cells = EMIT == EMIT_WEIGHT ? hdr->weight_cells != 0 && red[8] == 0.0f : hdr->cells != 0;
-  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (has_cells ? 0u : 2u) | (bijective ? 0u : 4u));
+  const uint32_t row_modes = __builtin_amdgcn_readfirstlane((row_plain ? 1u : 0u) | (has_cells ? 0u : 2u) | (bijective ? 0u : 4u) | (folded ? 8u : 0u));
   uint8_t *codes_row = a.codes + row * (EMIT == EMIT_NIBBLE ? K / 2 : K);  // uniform; used by EMIT_NIBBLE / EMIT_U8 only
   const float s1 = (slot_lane & 1) ? -1.0f : 1.0f, s2 = (slot_lane & 2) ? -1.0f : 1.0f;
   const float s4 = (slot_lane & 4) ? -1.0f : 1.0f, s8 = (slot_lane & 8) ? -1.0f : 1.0f;
@@ -842,7 +898,12 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     for (int j = 0; j < G; ++j) {
       const int c0 = unit_base + j * kLaneSpan + slot_first;  // >= K: an idle lane of the row's last unit
       int code[kChunk];
-      if constexpr (EMIT == EMIT_WEIGHT) {
+      if (EMIT == EMIT_WEIGHT && (modes_now & 8u) != 0u) {
+        uint2 ent[kChunk];
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) ent[e] = cells[plan::cell_of(y[j][e], folded_scale, cell_offset)];
+        count_below(ent, y[j], code);
+      } else if constexpr (EMIT == EMIT_WEIGHT) {
         float unit[kChunk];
 #pragma unroll
         for (int e = 0; e < kChunk; ++e) unit[e] = y[j][e] * a.inv_sqrt_block;
@@ -851,8 +912,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
         for (int e = 1; e < kChunk; ++e) least = __builtin_fminf(least, __builtin_fabsf(unit[e]));
         // divide_fast is the IEEE quotient for numerators of 2^-80 and more and the rows it takes at all (NaN and
         // infinities make a row's norm one, so those rows take the other branch); the compiler's division, eleven
-        // instructions a value instead of four, remains for the rest.  14336 x 4096 into four bits,
-        // the plan included: 84 us; 105 with a search of four dependent LDS reads per value in place of the cells.
+        // instructions a value instead of four, remains for the rest.  (14336 x 4096 into four bits,
+        // the plan included, all rows this way: 84 us; 105 with a search of four dependent LDS reads per value in place of the cells.)
         if (weight_plain || __builtin_amdgcn_ballot_w64(least < 0x1p-80f) != 0) {
 #pragma unroll
           for (int e = 0; e < kChunk; ++e) unit[e] = unit[e] / weight_denominator;

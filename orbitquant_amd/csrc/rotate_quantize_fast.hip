@@ -13,16 +13,7 @@ using namespace rqf;
 // Workgroup 0 makes the header and the tables, the last one checks that the permutation is one, the others write 256
 // gather entries and signs each, and copies of the two where the caller wants its own (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
 // for rows of some thousand values; 6.2 us with the second table and the check).
-// Floats in an order-preserving integer code, so that "the largest float t with RN(t * c) <= b" can
-// be found by bisection over all of them.
-__device__ __forceinline__ uint32_t float_to_ordered(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float ordered_to_float(uint32_t o) {
-  return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
-}
-
+// (A folded threshold, "the largest float t with RN(t * c) <= b", is found by bisection over all floats.)
 __global__ __launch_bounds__(256) void rotate_plan_build_kernel(const int32_t *perm, const int8_t *signs,
                                                                  const float *boundaries, int levels, int K, int block,
                                                                  float c, unsigned char *out, int32_t *perm_copy, int8_t *signs_copy) {

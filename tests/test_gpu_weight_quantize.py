@@ -239,6 +239,38 @@ def test_a_plan_over_other_boundaries_decides_nothing(dev, k, change):
     assert np.array_equal(packed.cpu().numpy(), want_packed) and torch.equal(norms.cpu(), want_norms)
 
 
+@pytest.mark.parametrize("bits", [2, 4, 6])
+@pytest.mark.parametrize(("k", "dtype"), [(4096, torch.bfloat16), (2048, torch.float32), (12288, torch.float16), (13824, torch.bfloat16), (14336, torch.float32), (5120, torch.bfloat16)])
+def test_rows_with_thresholds_of_their_own_equal_divided_ones(dev, k, dtype, bits):
+    """Long rows compare with boundaries that carry the row's norm; a plan over other boundaries has every value divided
+    and searched.  The same indices, for norms and values of every size, a boundary at zero, and values next to boundaries."""
+    from orbitquant_amd import ops
+
+    n = 96
+    perm, signs, block, inv = o.rpbh_constants(k, 2, "paper")
+    levels = 1 << bits
+    bounds = (np.linspace(-2.4, 2.4, levels - 1) / np.sqrt(k)).astype(np.float32)
+    bounds[levels // 2 - 1] = 0.0
+    g = torch.Generator().manual_seed(k + bits)
+    w = torch.randn(n, k, generator=g)
+    w[:40] *= 10.0 ** torch.linspace(-6 if dtype == torch.float16 else -30, 3 if dtype == torch.float16 else 8, 40)[:, None]
+    w[40] = 0
+    w[41, 1:] = 0                                    # every value is +-1 / sqrt(block) of the row's norm
+    w[42] = torch.round(w[42])                       # few distinct sums, many of them zero
+    w[43, ::2] = 0
+    w = w.to(dtype).to(dev)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    args = (w, t(perm.astype(np.int32)), t(signs), t(bounds))
+    kw = dict(bits=bits, block_size=block, eps=1e-10, inv_sqrt_block=float(inv))
+    other = ops.rotate_plan(*args[1:3], t((bounds * np.float32(1.3)).astype(np.float32)), block_size=block, inv_sqrt_block=float(inv))
+    packed, norms = ops.quantize_weight(*args, **kw)
+    divided, divided_norms = ops.quantize_weight(*args, **kw, plan=other)
+    assert torch.equal(packed, divided) and torch.equal(norms, divided_norms)
+    rows = [0, 20, 39, 41, 42, 95]
+    want, _, _ = o.quantize_weight(w[rows].float().cpu().numpy(), perm, signs, bounds, block, 1e-10, bits, norm_order="sumsq_v1")
+    assert np.array_equal(packed.view(n, -1)[rows].cpu().numpy().reshape(-1), want)
+
+
 @pytest.mark.parametrize("bits", [(4, 4), (3, 4)])
 def test_a_converted_layer_has_what_a_built_one_has(dev, bits):
     """One plan where weights and activations share a codebook, constants in storages of their own."""
