@@ -275,9 +275,16 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
 #pragma unroll
     for (int i = 0; i < NB; ++i) fetch_w(s_begin + i * kDepth, b[i]);
   };
+  // Batches requested in front of the tables, the others behind the barrier.  A wavefront that requests more than its CU has
+  // room for waits where it requests, and every other one then waits for its tables: launches of q, k and v on 64 rows a
+  // workgroup reached the barrier 5.4 to 7 us after their start, when most of their weights had arrived.  Behind one
+  // batch of 32 wavefront rows and more, and with several token blocks, the second one is late enough: q, k and v of
+  // 4096 x 4096, 1 / 16 tokens with the quantizer 15.2 -> 14.4 / 18.3 -> 17.3 us, 33 tokens 4096 x 14336 22.0 -> 21.3 us, 64 tokens
+  // 2048 x 8192 12.5 -> 12.1 us; smaller launches lose by it (1 token 4096 x 14336 14.1 -> 14.5 us).
+  constexpr int kAhead = R * WAVES >= 32 || MB > 1 ? 1 : NB;
   if constexpr (!LATE) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) fetch(s_begin + i * kDepth, b[i]);
+    for (int i = 0; i < kAhead; ++i) fetch(s_begin + i * kDepth, b[i]);
   }
 
   // ---- tables (built while the stream is in flight) ---------------------------------------
@@ -311,6 +318,9 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
     for (int i = 0; i < NB; ++i) fetch_a(s_begin + i * kDepth, b[i]);
   } else {
     __syncthreads();
+#pragma unroll
+    for (int i = kAhead; i < NB; ++i) fetch(s_begin + i * kDepth, b[i]);
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // Every fetch is issued unconditionally (past the end of the wavefront's share it re-reads
