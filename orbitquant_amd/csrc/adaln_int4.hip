@@ -228,13 +228,13 @@ int adaln_int4_dispatch(const uint16_t *x, const uint8_t *packed, const uint16_t
   const bool stream_form = fast && group % 32 == 0 && K >= 32 && (reinterpret_cast<uintptr_t>(packed) & 15u) == 0 &&
                            (static_cast<int64_t>(a.group) * a.groups / 2) % 16 == 0;
   if (stream_form) {
-    hipLaunchKernelGGL(adaln_int4_stream_kernel, dim3(static_cast<unsigned>((N + 15) / 16)), dim3(256), 0, stream, a);
+    launch_kernel(adaln_int4_stream_kernel, dim3(static_cast<unsigned>((N + 15) / 16)), dim3(256), 0, stream, a);
   } else if (fast) {
     const int64_t blocks = (N + 63) / 64;
-    hipLaunchKernelGGL(adaln_int4_mfma_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+    launch_kernel(adaln_int4_mfma_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
   } else {
     const int64_t row_groups = (M + 3) / 4;
-    hipLaunchKernelGGL(adaln_int4_generic_kernel, dim3(static_cast<unsigned>(N), static_cast<unsigned>(row_groups < 65535 ? row_groups : 65535)),
+    launch_kernel(adaln_int4_generic_kernel, dim3(static_cast<unsigned>(N), static_cast<unsigned>(row_groups < 65535 ? row_groups : 65535)),
                        dim3(256), 0, stream, a);
   }
   return check_launch("adaln_int4");
@@ -250,7 +250,7 @@ int adaln_quantize_dispatch(const void *w, int w_dtype, int64_t N, int64_t K, in
   a.w = w; a.w_dtype = w_dtype; a.N = N; a.K = K; a.group = static_cast<int>(group); a.groups = static_cast<int>((K + group - 1) / group);
   a.packed = packed; a.scales = scales;
   const int64_t blocks = (N * a.groups + 3) / 4;
-  hipLaunchKernelGGL(adaln_quantize_kernel, dim3(static_cast<unsigned>(blocks < 65536 ? blocks : 65536)), dim3(256), 0, stream, a);
+  launch_kernel(adaln_quantize_kernel, dim3(static_cast<unsigned>(blocks < 65536 ? blocks : 65536)), dim3(256), 0, stream, a);
   return check_launch("adaln_quantize");
 }
 

@@ -238,7 +238,7 @@ template <int MF, int FM, int FN, int SM, int SN>
 int launch_parts(const DenseArgs &g, hipStream_t stream) {
   const int64_t blocks = g.whole + (static_cast<int64_t>(g.tiles_m) * g.tiles_n - g.whole) * SM * SN;
   auto kern = dense_gemm_kernel<MF, FM, FN, SM, SN>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g);
+  launch_kernel(kern, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g);
   return check_launch("dense_gemm");
 }
 

@@ -108,7 +108,7 @@ int decode_operands(const uint8_t *packed, int bits, const float *cents, int lev
   auto go = [&](auto bits_c) {
     constexpr int BITS = decltype(bits_c)::value;
     auto kern = f16 ? decode_operands_kernel<BITS, true> : decode_operands_kernel<BITS, false>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, packed, cents, levels, static_cast<int>(rows), static_cast<int>(K),
+    launch_kernel(kern, grid, dim3(256), 0, stream, packed, cents, levels, static_cast<int>(rows), static_cast<int>(K),
                        static_cast<int>(row_tiles), static_cast<uint4 *>(out));
     return check_launch("decode_operands");
   };
@@ -124,7 +124,7 @@ int decode_operands(const uint8_t *packed, int bits, const float *cents, int lev
 
 int decode_operands_int8(const uint8_t *packed, const int8_t *table, int64_t rows, int64_t K, void *out, hipStream_t stream) {
   const int64_t row_tiles = (rows + 31) / 32;
-  hipLaunchKernelGGL(decode_operands_int8_kernel, dim3(pass_blocks(row_tiles, ((K + 127) / 128 + 3) / 4)), dim3(256), 0, stream, packed, table,
+  launch_kernel(decode_operands_int8_kernel, dim3(pass_blocks(row_tiles, ((K + 127) / 128 + 3) / 4)), dim3(256), 0, stream, packed, table,
                      static_cast<int>(rows), static_cast<int>(K), static_cast<int>(row_tiles), static_cast<uint4 *>(out));
   return check_launch("decode_operands_int8");
 }

@@ -120,7 +120,7 @@ void launch_dequantize_rows(const uint8_t *packed, const uint16_t *row_norms, co
   const uint32_t stride = blocks * 256, last_dword = static_cast<uint32_t>(N * K / 8 * BITS / 4 - 1);
   auto kern = out_dtype == OQ_F32 ? dequantize_rows_kernel<BITS, OQ_F32>
               : out_dtype == OQ_F16 ? dequantize_rows_kernel<BITS, OQ_F16> : dequantize_rows_kernel<BITS, OQ_BF16>;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, reinterpret_cast<const uint32_t *>(packed), row_norms, centroids, groups,
+  launch_kernel(kern, dim3(blocks), dim3(256), 0, stream, reinterpret_cast<const uint32_t *>(packed), row_norms, centroids, groups,
                      per_row, last_dword, stride / per_row, stride % per_row, static_cast<uint4 *>(out));
 }
 
@@ -134,7 +134,7 @@ unsigned stream_blocks(int64_t groups) {
 int pack_lowbit_dispatch(const uint8_t *values, int bits, int64_t count, uint8_t *packed, hipStream_t stream) {
   if (count == 0) return OQ_OK;
   const int64_t nbytes = (count * bits + 7) / 8;
-  hipLaunchKernelGGL(pack_lowbit_kernel, dim3(stream_blocks((count + 7) / 8)), dim3(256), 0, stream, values, bits, count, packed, nbytes);
+  launch_kernel(pack_lowbit_kernel, dim3(stream_blocks((count + 7) / 8)), dim3(256), 0, stream, values, bits, count, packed, nbytes);
   return check_launch("pack_lowbit");
 }
 
@@ -154,11 +154,11 @@ int dequantize_dispatch(const uint8_t *packed, int bits, const uint16_t *row_nor
   }
   const dim3 grid(stream_blocks((total + 7) / 8));
   if (out_dtype == OQ_F32)
-    hipLaunchKernelGGL(dequantize_kernel<OQ_F32>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
+    launch_kernel(dequantize_kernel<OQ_F32>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
   else if (out_dtype == OQ_F16)
-    hipLaunchKernelGGL(dequantize_kernel<OQ_F16>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
+    launch_kernel(dequantize_kernel<OQ_F16>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
   else
-    hipLaunchKernelGGL(dequantize_kernel<OQ_BF16>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
+    launch_kernel(dequantize_kernel<OQ_BF16>, grid, dim3(256), 0, stream, packed, bits, row_norms, centroids, total, K, nbytes, out);
   return check_launch("dequantize_packed_weight");
 }
 

@@ -199,7 +199,7 @@ int launch_cfg(AvArgs g, hipStream_t stream) {
   auto kern = packed_gemm_av_kernel<F16, BITS, FM, FN>;
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "packed_gemm: cannot reserve %zu bytes of LDS", smem);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(total)), dim3(256), smem, stream, g);
+  launch_kernel(kern, dim3(static_cast<unsigned>(total)), dim3(256), smem, stream, g);
   return check_launch("packed_gemm_av");
 }
 

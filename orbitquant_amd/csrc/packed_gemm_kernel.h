@@ -658,7 +658,7 @@ int launch_cfg(GemmArgs g, hipStream_t stream) {
                     reserve_dynamic_lds(reinterpret_cast<const void *>(kern), kWideBytes)) ? 1 : 0;
   if (g.M > 0x7fff0000LL || g.N > 0x7fff0000LL || g.K > 0x0fffffffLL || g.a_levels > 0xffff)  // (the kernel's 32-bit row and byte counts)
     return fail(OQ_ERR_UNSUPPORTED, "packed_gemm: a dimension beyond 2^31");
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(total), splits), dim3(256), g.window_ahead ? kWideBytes : 0, stream,
+  launch_kernel(kern, dim3(static_cast<unsigned>(total), splits), dim3(256), g.window_ahead ? kWideBytes : 0, stream,
                      g.w_cents, g.act_cents, g.a, g.w, g.out_map.table, static_cast<int>(g.K), static_cast<int>(g.M),
                      static_cast<int>(g.N), g.a_levels | (g.k_splits << 16) | (g.window_ahead << 24), g);
   return check_launch("packed_gemm");

@@ -51,7 +51,7 @@ int gemm_splitk_reduce(const float *partials, int splits, int64_t M, int64_t N, 
                        hipStream_t stream) {
   const int64_t quads = M * (N / 4);
   const unsigned blocks = static_cast<unsigned>(quads / 256 + 1 < 4096 ? quads / 256 + 1 : 4096);
-#define OQ_REDUCE(DT) hipLaunchKernelGGL(splitk_reduce_kernel<DT>, dim3(blocks), dim3(256), 0, stream, partials, splits, M, N, \
+#define OQ_REDUCE(DT) launch_kernel(splitk_reduce_kernel<DT>, dim3(blocks), dim3(256), 0, stream, partials, splits, M, N, \
                                          row_scale, row_norms, bias, bias_dtype, out)
   if (out_dtype == OQ_BF16) OQ_REDUCE(OQ_BF16);
   else if (out_dtype == OQ_F16) OQ_REDUCE(OQ_F16);

@@ -90,7 +90,7 @@ int gemm_tiled_dispatch(bool f16, const void *x, const float *token_scale, const
   const int64_t row_tiles = (M + 31) / 32;
   unsigned char *tiled = static_cast<unsigned char *>(workspace);
   if (tiled == nullptr || row_tiles > 65535 || workspace_bytes < operand_order_bytes(M, K, 2) || (reinterpret_cast<uintptr_t>(tiled) & 15u) != 0) return -1;
-  hipLaunchKernelGGL(tile_activations_kernel, dim3(static_cast<unsigned>((K / 64 + 3) / 4), static_cast<unsigned>(row_tiles)), dim3(256), 0, stream,
+  launch_kernel(tile_activations_kernel, dim3(static_cast<unsigned>((K / 64 + 3) / 4), static_cast<unsigned>(row_tiles)), dim3(256), 0, stream,
                      static_cast<const uint16_t *>(x), M, K, reinterpret_cast<uint4 *>(tiled));
   if (int rc = check_launch("tile_activations")) return rc;
   const int dense_tile = tiled_choose_dense(M, N, K, bits, f16);

@@ -36,7 +36,7 @@ int launch(const GemvArgs &g, hipStream_t stream) {
   if constexpr (!BYTES) {
     if (gemv_stages_activations(g.M, g.K)) kern = packed_gemv_kernel<BYTES, BITS, R, WAVES, true>;
   }
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), 0, stream, g.w, g.a, g.w_cents, g.act_cents, g.K,
+  launch_kernel(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), 0, stream, g.w, g.a, g.w_cents, g.act_cents, g.K,
                      g.N, g.row_norms, g.M, g.a_levels, g.row_scale, g.bias, g.bias_dtype, g.out, g.out_dtype, g.out_map);
   return check_launch("packed_gemv");
 }

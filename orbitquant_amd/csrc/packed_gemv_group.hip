@@ -35,7 +35,7 @@ int launch_group(GroupArgs &ga, hipStream_t stream) {
   if constexpr (MB == 1) {
     if (gemv_stages_activations(ga.m[0].M, ga.m[0].K)) kern = packed_gemv_group_kernel<R, WAVES, true>;
   }
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(total)), dim3(64 * WAVES), 0, stream, ga);
+  launch_kernel(kern, dim3(static_cast<unsigned>(total)), dim3(64 * WAVES), 0, stream, ga);
   return check_launch("packed_linear_group");
 }
 

@@ -21,7 +21,7 @@ template <bool BYTES, int BITS, int R, int WAVES, int MB>
 int launch(const GemvArgs &g, hipStream_t stream) {
   const int64_t groups = (g.N + 16 * R - 1) / (16 * R);
   if (groups > 0x7fffffffLL) return fail(OQ_ERR_UNSUPPORTED, "packed_gemv: N too large");
-  hipLaunchKernelGGL((packed_gemv_rows_kernel<BYTES, BITS, R, WAVES, MB>), dim3(static_cast<unsigned>(groups)),
+  launch_kernel((packed_gemv_rows_kernel<BYTES, BITS, R, WAVES, MB>), dim3(static_cast<unsigned>(groups)),
                      dim3(64 * WAVES), 0, stream, g);
   return check_launch("packed_gemv_rows");
 }

@@ -80,7 +80,7 @@ int launch_generic(const GenericArgs &a, hipStream_t stream) {
   if (a.N > 0x7fffffffLL) return fail(OQ_ERR_UNSUPPORTED, "generic packed kernel: N=%lld exceeds the grid", (long long)a.N);
   const int64_t row_groups = (a.M + kWaves - 1) / kWaves;
   dim3 grid(static_cast<unsigned>(a.N), static_cast<unsigned>(row_groups < 65535 ? row_groups : 65535));
-  hipLaunchKernelGGL(packed_generic_kernel, grid, dim3(64 * kWaves), 0, stream, a);
+  launch_kernel(packed_generic_kernel, grid, dim3(64 * kWaves), 0, stream, a);
   return check_launch("packed_generic");
 }
 
@@ -115,7 +115,7 @@ int unpack_dispatch(const uint8_t *packed, int bits, int64_t count, uint8_t *out
   const int64_t nbytes = (count * bits + 7) / 8;
   const int64_t blocks = (count + 255) / 256;
   if (blocks > 0x7fffffffLL) return fail(OQ_ERR_UNSUPPORTED, "unpack: count too large");
-  hipLaunchKernelGGL(unpack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, packed, bits,
+  launch_kernel(unpack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, packed, bits,
                      count, nbytes, out);
   return check_launch("unpack_lowbit");
 }
@@ -131,7 +131,7 @@ __global__ void apply_value_map_kernel(uint16_t *out, int64_t count, const uint1
 int apply_value_map(void *out, int64_t count, const uint16_t *table, hipStream_t stream) {
   if (count <= 0) return OQ_OK;
   const int64_t blocks = (count + 255) / 256;
-  hipLaunchKernelGGL(apply_value_map_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+  launch_kernel(apply_value_map_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
                      static_cast<uint16_t *>(out), count, table);
   return check_launch("apply_value_map");
 }

@@ -31,7 +31,7 @@ int launch_for_block(const RqArgs &a, hipStream_t stream) {
     auto kern = KERN;                                                                            \
     if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))                        \
       return fail(OQ_ERR_LAUNCH, "rotate_quantize: cannot reserve %zu bytes of LDS", smem);      \
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, args);                                   \
+    launch_kernel(kern, grid, block, smem, stream, args);                                   \
   }
 #define OQ_RQ_CASE(LG)                                                                           \
   case LG:                                                                                       \

@@ -162,7 +162,7 @@ int launch_emit(const FastArgs &a, int waves, size_t smem, hipStream_t stream) {
   auto kern = rotate_quantize_fast_kernel<DT, LOG_H, EMIT, MAPPED>;
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "rotate_quantize: cannot reserve %zu bytes of LDS", smem);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.M)), dim3(64 * waves), smem, stream, a);
+  launch_kernel(kern, dim3(static_cast<unsigned>(a.M)), dim3(64 * waves), smem, stream, a);
   return check_launch("rotate_quantize (plan)");
 }
 
@@ -172,7 +172,7 @@ int launch_shared(const FastArgs &a, hipStream_t stream) {
   auto kern = a.code_format == OQ_CODES_NIBBLE ? rotate_quantize_shared_kernel<DT, LOG_H, EMIT_NIBBLE, WB> : rotate_quantize_shared_kernel<DT, LOG_H, EMIT_U8, WB>;
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "rotate_quantize: cannot reserve %zu bytes of LDS", smem);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(a.M)), dim3(static_cast<unsigned>(64 * WB * a.units)), smem, stream, a.x, a.perm, a.signs,
+  launch_kernel(kern, dim3(static_cast<unsigned>(a.M)), dim3(static_cast<unsigned>(64 * WB * a.units)), smem, stream, a.x, a.perm, a.signs,
                      a.plan, a.codes, a.norms, static_cast<int>(a.K), a.levels, a.levels_pow2, a.eps);
   return check_launch("rotate_quantize (plan, shared blocks)");
 }
@@ -252,7 +252,7 @@ int rotate_plan_build(const int32_t *perm, const int8_t *signs, const float *bou
   if (!(inv_sqrt_block > 0.0f) || !(inv_sqrt_block < 3.0e38f))
     return fail(OQ_ERR_INVALID, "rotate_plan_build: inv_sqrt_block must be positive and finite");
   if ((reinterpret_cast<uintptr_t>(plan_out) & 15u) != 0) return fail(OQ_ERR_INVALID, "rotate_plan_build: the plan must be 16-byte aligned");
-  hipLaunchKernelGGL(rotate_plan_build_kernel, dim3(static_cast<unsigned>(2 + (K + 255) / 256)), dim3(256), 0, stream, perm, signs, boundaries, levels,
+  launch_kernel(rotate_plan_build_kernel, dim3(static_cast<unsigned>(2 + (K + 255) / 256)), dim3(256), 0, stream, perm, signs, boundaries, levels,
                      static_cast<int>(K), static_cast<int>(block), inv_sqrt_block, static_cast<unsigned char *>(plan_out), perm_copy, signs_copy);
   return check_launch("rotate_plan_build");
 }

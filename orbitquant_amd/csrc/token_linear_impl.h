@@ -65,7 +65,7 @@ int launch_plan_waves(const rqf::FastArgs &q, const gemv::GemvArgs &g, hipStream
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "token_linear: cannot reserve %zu bytes of LDS", smem);
   const int64_t groups = (g.N + 16 * R - 1) / (16 * R);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), smem, stream, q, g, static_cast<int>(scratch));
+  launch_kernel(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), smem, stream, q, g, static_cast<int>(scratch));
   return check_launch("token_linear");
 }
 
@@ -96,7 +96,7 @@ int launch_token_waves(const rq::RqArgs &q, const gemv::GemvArgs &g, size_t rq_b
   if (!reserve_dynamic_lds(reinterpret_cast<const void *>(kern), smem))
     return fail(OQ_ERR_LAUNCH, "token_linear: cannot reserve %zu bytes of LDS", smem);
   const int64_t groups = (g.N + 16 * R - 1) / (16 * R);
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), smem, stream, q, g,
+  launch_kernel(kern, dim3(static_cast<unsigned>(groups)), dim3(64 * WAVES), smem, stream, q, g,
                      static_cast<int>(scratch));
   return check_launch("token_linear");
 }
