@@ -823,3 +823,43 @@ def test_streaming_tables_of_every_width(dev, wbits, abits, m, n, k):
     w = w_table.bfloat16().double()[index]
     scale = norms.double()[:, None] * row_norms.double()[None]
     assert bool(((out.cpu().double() - a @ w.T * scale).abs() <= 1e-5 * (a.abs() @ w.abs().T) * scale).all())
+
+
+@pytest.mark.parametrize("wbits", [2, 3, 4])
+@pytest.mark.parametrize(("m", "n", "k"), [(128, 192, 256), (129, 200, 320), (300, 392, 1152), (65, 184, 576), (257, 576, 64), (96, 1000, 704)])
+def test_the_128x192_tile(dev, wbits, m, n, k, library_switch):
+    """The same bits as the 128 x 128 tile with one running sum (K steps in order); with the sums of the four quarters of K kept
+    apart (codes, values staged and in operand order), an error against fp64 no larger than the four wavefronts' of
+    the 128 x 96 tile, up to a quarter of it for the order in which four numbers are added."""
+    from orbitquant_amd import ops
+
+    g = torch.Generator().manual_seed(m + n + k + wbits)
+    codes, w = torch.randint(0, 256, (m, k // 2), generator=g).to(torch.uint8).to(dev), torch.randint(0, 256, (n * k * wbits // 8,), generator=g).to(torch.uint8).to(dev)
+    norms, row_norms = torch.rand(m, generator=g).to(dev), torch.rand(n, generator=g).bfloat16().to(dev)
+    a_table, w_table = torch.randn(16, generator=g).to(dev), torch.randn(1 << wbits, generator=g).to(dev)
+    bias = torch.randn(n, generator=g).to(dev)
+
+    def linear(tile, dtype):
+        library_switch("OQ_GEMM_TILE", tile)
+        return ops.packed_linear(codes, norms, a_table, w, row_norms, w_table, code_format="nibble", activation_bits=4, weight_bits=wbits,
+                                 out_features=n, in_features=k, bias=bias.to(dtype), output_dtype=dtype)
+
+    def values(tile, dtype):
+        library_switch("OQ_GEMM_TILE", tile)
+        return ops.matmul_packed_weight_values(x.to(dtype), w, row_norms, w_table, bits=wbits, out_features=n, in_features=k, bias=bias.to(dtype))
+
+    nibbles = torch.stack((codes & 15, codes >> 4), dim=-1).view(m, k).long()
+    x = a_table[nibbles]
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+        assert torch.equal(linear("6", dtype), linear("0", dtype))
+        if dtype != torch.float32:
+            assert torch.equal(values("6", dtype), values("0", dtype))
+            assert torch.equal(values("7", dtype).isfinite(), values("0", dtype).isfinite())
+    if k % 256 == 0:
+        stream = ((w[:, None] >> torch.arange(8, device=dev, dtype=torch.uint8)) & 1).flatten()[: n * k * wbits].view(n * k, wbits).long()
+        index = (stream << torch.arange(wbits, device=dev)).sum(1).view(n, k)
+        exact = x.bfloat16().double() @ w_table.bfloat16().double()[index].T * norms.double()[:, None] * row_norms.double() + bias.double()
+        error = {tile: float((linear(tile, torch.float32).double() - exact).norm()) for tile in ("4", "6", "7")}
+        assert error["7"] <= 1.25 * error["4"]
+    else:
+        assert float((linear("7", torch.float32) - linear("6", torch.float32)).norm()) <= 1e-5 * float(linear("6", torch.float32).norm())
