@@ -68,7 +68,7 @@ def quantize_weight(
 
         device = weight.device
         # (one launch for the matrix: at 256 rows a launch, one workgroup a CU, 14336 x 4096 took 56 launches of 16 us
-        # and some 200 us of Python; one launch 84 us)
+        # and some 200 us of Python; one launch 80 us)
         if constants is None:
             constants = (rotation.permutation.to(torch.int32).to(device), rotation.signs.to(torch.int8).to(device),
                          codebook.boundaries.to(device))
