@@ -203,6 +203,20 @@ def _plan_operand(plan: torch.Tensor | None, like: torch.Tensor, dim: int, block
     return _operand(plan, "plan", like, dtype=torch.uint8, numel=expected)
 
 
+# Values of a call without a plan from which on one is built for it: the plan-based kernel takes 0.4 to 0.8 of the other's time, and
+# the plan's launch and its host work some 8 us (16-bit rows into nibbles, eager: 2048 x 5120 27.4 -> 25.2 us, 4608 x 4096
+# 42.7 -> 34.3, 4608 x 3072 40.7 -> 24.2, 4608 x 14336 204 -> 78, but 2048 x 4096 21.2 -> 23.7, 512 x 14336 23.8 -> 25.2).
+# Not for blocks beyond 4096, which that kernel does not have, nor for fp32 rows (4608 x 4096 into bytes 46 -> 54 us).
+_PLAN_FROM_VALUES = 10_000_000
+
+
+def _worth_a_plan(rows: torch.Tensor, levels: int, block_size: int, inv_sqrt_block: float) -> bool:
+    m, dim = rows.shape
+    return (m * dim >= _PLAN_FROM_VALUES and rows.dtype in (torch.float16, torch.bfloat16) and dim % 8 == 0 and dim <= 16384
+            and 8 <= block_size <= 4096 and block_size & (block_size - 1) == 0 and dim % block_size == 0
+            and 2 <= levels <= 16 and 0.0 < inv_sqrt_block < 3.0e38 and rows.data_ptr() % 16 == 0)
+
+
 def rotate_quantize(
     x: torch.Tensor,
     permutation: torch.Tensor,
@@ -222,7 +236,7 @@ def rotate_quantize(
 
     plan: None, or `rotate_plan(...)` of the same permutation, signs, boundaries, block and
     factor: more than 16 rows, and fewer where a row has several blocks or blocks of 1024 to 4096,
-    then take the plan-based kernel (same results, much faster).
+    then take the plan-based kernel (same results, much faster).  Large calls without one that write nibbles build one.
 
     input_map: None, or the table of an elementwise function f (`activation_table`): the
     result is that of rotate_quantize(f(x)), bit for bit, without f(x) ever being stored.
@@ -269,7 +283,10 @@ def rotate_quantize(
         if input_map.dtype != x.dtype or input_map.numel() != 65536 or input_map.device != x.device:
             raise ValueError("input_map must hold 65536 entries of x's dtype on x's device")
         input_map = input_map.contiguous()
-    plan = _plan_operand(plan, x, dim, block_size, levels)
+    if plan is not None:
+        plan = _plan_operand(plan, x, dim, block_size, levels)
+    elif code_format == "nibble" and mode == OQ_VALUES_NONE and input_map is None and _worth_a_plan(rows, levels, block_size, inv_sqrt_block):
+        plan = rotate_plan(permutation, signs, boundaries, block_size=block_size, inv_sqrt_block=inv_sqrt_block)
     lib = _lib.load()
     head = (m, dim, permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(), _ptr(centroids), levels,
             int(block_size), float(eps), float(inv_sqrt_block))

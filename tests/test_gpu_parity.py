@@ -863,3 +863,20 @@ def test_the_128x192_tile(dev, wbits, m, n, k, library_switch):
         assert error["7"] <= 1.25 * error["4"]
     else:
         assert float((linear("7", torch.float32) - linear("6", torch.float32)).norm()) <= 1e-5 * float(linear("6", torch.float32).norm())
+
+
+@pytest.mark.parametrize("tile", ["6", "7"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_the_128x192_tile_through_an_output_map(dev, tile, dtype, library_switch):
+    """The map is applied to what the tile stores without it, inside the matrix and at its edges."""
+    from orbitquant_amd import ops
+
+    library_switch("OQ_GEMM_TILE", tile)
+    m, n, k = 300, 392, 512
+    g = torch.Generator().manual_seed(9)
+    codes, w = torch.randint(0, 256, (m, k // 2), generator=g).to(torch.uint8).to(dev), torch.randint(0, 256, (n * k // 2,), generator=g).to(torch.uint8).to(dev)
+    args = (codes, (0.1 * torch.rand(m, generator=g)).to(dev), torch.randn(16, generator=g).to(dev), w, torch.rand(n, generator=g).bfloat16().to(dev),
+            torch.randn(16, generator=g).to(dev))
+    kw = dict(code_format="nibble", activation_bits=4, weight_bits=4, out_features=n, in_features=k, output_dtype=dtype)
+    table = ops.activation_table(torch.nn.functional.gelu, dtype, dev)
+    assert torch.equal(ops.packed_linear(*args, **kw, output_map=table), torch.nn.functional.gelu(ops.packed_linear(*args, **kw)))

@@ -376,3 +376,20 @@ def test_few_rows_with_an_unaligned_permutation(dev, which):
     want, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, signs, bounds, h, 1e-10, inv)
     assert torch.equal(codes, plain) and np.array_equal(codes.cpu().numpy(), want)
     assert np.array_equal(norms.cpu().numpy().view(np.int32), want_norms.view(np.int32))
+
+
+@pytest.mark.parametrize("k,h", [(1152, 64), (3072, 1024), (4096, 4096), (8192, 8192), (13824, 512), (104, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_a_plan_built_for_the_call_changes_nothing(dev, k, h, dtype, monkeypatch):
+    """Also where it cannot be used (a block beyond 4096, fp32 rows, rows off a 16-byte boundary), and for a gather that repeats positions."""
+    from orbitquant_amd import ops
+
+    _, _, _, inv, _, _, t = constants(dev, k, h, 4)
+    t["perm"][5] = t["perm"][9]
+    x = make_rows(40, k, dtype, seed=k).to(dev)
+    x = torch.cat([x.view(-1)[:1], x.view(-1)])[1:].view(40, k) if k == 104 else x
+    call = lambda: ops.rotate_quantize(x, t["perm"], t["signs"], t["bounds"], block_size=h, eps=1e-10, inv_sqrt_block=float(inv), code_format="nibble")
+    want, _, norms = call()
+    monkeypatch.setattr(ops, "_PLAN_FROM_VALUES", 1)
+    got, _, got_norms = call()
+    assert torch.equal(got, want) and torch.equal(got_norms, norms)
