@@ -24,7 +24,7 @@ There is no dequantized-weight or CPU fallback on this path.
 
 from __future__ import annotations
 
-from functools import lru_cache
+from functools import cached_property, lru_cache
 
 import numpy as np
 import torch
@@ -107,17 +107,22 @@ def _host_constants(rotation, activation_codebook, weight_codebook) -> dict[str,
 
 
 class _Packed(dict):
-    """Tensors on the host, and `host`, a pinned buffer that holds them one behind the other, 256 bytes apart or more."""
+    """Tensors on the host, and `host`, a pinned buffer that holds them one behind the other, 256 bytes apart or more: made
+    when it is first asked for, which a capture, in which pinned memory may not be allocated, never does."""
 
     def __init__(self, tensors: dict[str, torch.Tensor]) -> None:
         super().__init__(tensors)
         self.sizes = [(t.numel() * t.element_size() + 255) & -256 for t in tensors.values()]
-        self.host = torch.empty(sum(self.sizes), dtype=torch.uint8, device="cpu", pin_memory=True)   # (whatever the default device is)
-        raw, at = self.host.numpy(), 0   # (numpy's slices and copies, not torch's: the quantizer's launch comes 17 us sooner)
-        for t, size in zip(tensors.values(), self.sizes):
+
+    @cached_property
+    def host(self) -> torch.Tensor:
+        host = torch.empty(sum(self.sizes), dtype=torch.uint8, device="cpu", pin_memory=True)   # (whatever the default device is)
+        raw, at = host.numpy(), 0   # (numpy's slices and copies, not torch's: the quantizer's launch comes 17 us sooner)
+        for t, size in zip(self.values(), self.sizes):
             values = t.contiguous().numpy().reshape(-1).view(np.uint8)
             raw[at : at + values.size] = values
             at += size
+        return host
 
 
 @lru_cache(maxsize=16)

@@ -88,3 +88,25 @@ def test_a_capture_refuses_to_make_or_move_a_layer(source):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want) and torch.equal(made("converted", source)(x), want)
+
+
+def test_a_capture_refuses_the_first_conversion_of_a_width(source):
+    """Nothing of its constants has been made yet, and nothing may be pinned there: refused like any other, and the capture goes on."""
+    from orbitquant_amd import OrbitLinear, layers, recipe
+
+    layer, config = made("converted", source), recipe("w4a4")
+    x, weight = torch.randn(4, K, device="cuda").bfloat16(), torch.randn(40, 1352, device="cuda").bfloat16()
+    want = layer(x)
+    torch.cuda.synchronize()
+    layers._conversion_constants.cache_clear()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captur"):
+            OrbitLinear.from_weight(weight, bias=None, config=config)
+        y = layer(x)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+    assert OrbitLinear.from_weight(weight, bias=None, config=config)(torch.randn(2, 1352, device="cuda")).shape == (2, 40)

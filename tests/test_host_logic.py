@@ -303,3 +303,11 @@ def test_an_incremental_build_compiles_the_ops_only_after_a_change(monkeypatch, 
         later = out.stat().st_mtime + (5 if changed else -5)
         os.utime(header, (later, later))
         assert build.build_torch_ops() == out and len(ran) == times
+
+def test_a_conversions_constants_are_pinned_only_when_they_are_taken_to_a_gpu():
+    """Under capture they never are, and pinned memory may not be allocated there: the first conversion of a width asks for none."""
+    from orbitquant_amd import layers
+
+    made = layers._conversion_constants(136, 3, "paper", 3, 4, 2)
+    assert "host" not in vars(made) and made["_rotation_permutation"].shape == (136,)
+    assert sum(made.sizes) >= sum(t.numel() * t.element_size() for t in made.values())
