@@ -289,5 +289,10 @@ def get_codebook(dim: int, bits: int, algorithm_version: int = 2) -> LloydMaxCod
     )
 
 
+clear_with_codebooks: list = []   # what empties the caches of what is made of cached codebooks
+
+
 def clear_codebook_cache() -> None:
     get_codebook.cache_clear()
+    for clear in clear_with_codebooks:
+        clear()

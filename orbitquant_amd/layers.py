@@ -31,9 +31,9 @@ import torch
 from torch import nn
 
 from . import _lib, ops
-from .codebooks import get_codebook
+from .codebooks import clear_with_codebooks, get_codebook
 from .config import OrbitQuantConfig
-from .rotations import get_rpbh_rotation
+from .rotations import clear_with_rotations, get_rpbh_rotation
 from .weights import quantize_weight, quantized_on_gpu
 
 _LIB = torch.library.Library("orbitquant_amd", "DEF")
@@ -125,13 +125,17 @@ class _Packed(dict):
         return host
 
 
-@lru_cache(maxsize=16)
+@lru_cache(maxsize=256)
 def _conversion_constants(dim: int, seed: int, block_size, weight_bits: int, activation_bits: int, version: int) -> _Packed:
     """What a conversion takes to the GPU.  It depends on these numbers alone, like the rotation and the codebooks it is made
-    of; a model's layers have a few of them (some 70 KB each).  Packing them anew took 38 of the 82 us that lay before the
-    quantizer's launch."""
+    of, and is kept as they are: as many of them, until they are cleared (a set of a row of 14336 values is 70 KB).  Packing them
+    anew took 38 of the 82 us that lay before the quantizer's launch."""
     rotation, codebook = get_rpbh_rotation(dim, seed, block_size), get_codebook(dim, weight_bits, version)
     return _Packed({**_host_constants(rotation, get_codebook(dim, activation_bits, version), codebook), "weight_boundaries": codebook.boundaries})
+
+
+clear_with_rotations.append(_conversion_constants.cache_clear)
+clear_with_codebooks.append(_conversion_constants.cache_clear)
 
 
 def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[str, torch.Tensor]:

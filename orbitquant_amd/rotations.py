@@ -118,5 +118,10 @@ def get_rpbh_rotation(dim: int, seed: int = 0, block_size: int | str = "paper") 
     return RPBHRotation(dim=dim, seed=seed, block_size=block_size)
 
 
+clear_with_rotations: list = []   # what empties the caches of what is made of cached rotations
+
+
 def clear_rotation_cache() -> None:
     get_rpbh_rotation.cache_clear()
+    for clear in clear_with_rotations:
+        clear()

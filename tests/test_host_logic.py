@@ -304,6 +304,7 @@ def test_an_incremental_build_compiles_the_ops_only_after_a_change(monkeypatch, 
         os.utime(header, (later, later))
         assert build.build_torch_ops() == out and len(ran) == times
 
+
 def test_a_conversions_constants_are_pinned_only_when_they_are_taken_to_a_gpu():
     """Under capture they never are, and pinned memory may not be allocated there: the first conversion of a width asks for none."""
     from orbitquant_amd import layers
@@ -311,3 +312,18 @@ def test_a_conversions_constants_are_pinned_only_when_they_are_taken_to_a_gpu():
     made = layers._conversion_constants(136, 3, "paper", 3, 4, 2)
     assert "host" not in vars(made) and made["_rotation_permutation"].shape == (136,)
     assert sum(made.sizes) >= sum(t.numel() * t.element_size() for t in made.values())
+
+
+@pytest.mark.parametrize("clear", ["clear_rotation_cache", "clear_codebook_cache"])
+def test_a_conversions_constants_are_kept_as_what_they_are_made_of(clear):
+    """As many of them, and they go when the rotations or the codebooks are cleared."""
+    from orbitquant_amd import codebooks, layers, rotations
+
+    kept = layers._conversion_constants
+    kept.cache_clear()
+    for _ in range(2):   # more widths than a small cache holds, in turn
+        for seed in range(20):
+            kept(8, seed, "paper", 3, 4, 2)
+    assert kept.cache_info().misses == 20
+    getattr(rotations, clear, getattr(codebooks, clear, None))()
+    assert kept.cache_info().currsize == 0
