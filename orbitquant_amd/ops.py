@@ -203,16 +203,19 @@ def _plan_operand(plan: torch.Tensor | None, like: torch.Tensor, dim: int, block
     return _operand(plan, "plan", like, dtype=torch.uint8, numel=expected)
 
 
-# Values of a call without a plan from which on one is built for it: the plan-based kernel takes 0.4 to 0.8 of the other's time, and
-# the plan's launch and its host work some 8 us (16-bit rows into nibbles, eager: 2048 x 5120 27.4 -> 25.2 us, 4608 x 4096
-# 42.7 -> 34.3, 4608 x 3072 40.7 -> 24.2, 4608 x 14336 204 -> 78, but 2048 x 4096 21.2 -> 23.7, 512 x 14336 23.8 -> 25.2).
+# Values of a call without a plan from which on one is built for it: the plan-based kernel takes 0.25 to 0.8 of the other's time, but two
+# eager launches and the plan's host work are not done in less than some 24 us.  With blocks of 1024 and more, or rows of 512 values at most,
+# ten million 16-bit values into nibbles take the other kernel longer (1396 x 7168 31.6 -> 24.6 us, 2442 x 4096 25.4 -> 23.7, 26042 x 384 43 ->
+# 31; 4608 x 14336 204 -> 78); with smaller blocks, whose butterflies cost it least, twenty million do (4883 x 4096 in blocks of 8
+# 26.0 -> 25.1, 13021 x 1536 in blocks of 512 40 -> 34), and ten million do not (2442 x 4096 in blocks of 8 15.5 -> 22.7 us).
 # Not for blocks beyond 4096, which that kernel does not have, nor for fp32 rows (4608 x 4096 into bytes 46 -> 54 us).
 _PLAN_FROM_VALUES = 10_000_000
 
 
 def _worth_a_plan(rows: torch.Tensor, levels: int, block_size: int, inv_sqrt_block: float) -> bool:
     m, dim = rows.shape
-    return (m * dim >= _PLAN_FROM_VALUES and rows.dtype in (torch.float16, torch.bfloat16) and dim % 8 == 0 and dim <= 16384
+    from_values = _PLAN_FROM_VALUES if block_size >= 1024 or dim <= 512 else 2 * _PLAN_FROM_VALUES
+    return (m * dim >= from_values and rows.dtype in (torch.float16, torch.bfloat16) and dim % 8 == 0 and dim <= 16384
             and 8 <= block_size <= 4096 and block_size & (block_size - 1) == 0 and dim % block_size == 0
             and 2 <= levels <= 16 and 0.0 < inv_sqrt_block < 3.0e38 and rows.data_ptr() % 16 == 0)
 

@@ -116,3 +116,18 @@ def test_64x64_tiles_do_not_lessen_the_partial_sums(lib, m, n, k, wbits, parts, 
 @pytest.mark.parametrize("m,n,k", [(829, 3568, 12608), (1217, 1552, 6464), (5807, 680, 15936), (772, 4888, 2048), (299, 14224, 8000), (4668, 880, 5312)])
 def test_64x64_tiles_take_no_whole_numbers_into_fp32(lib, m, n, k):
     assert lib.oq_packed_linear_int8_workspace_bytes(m, n, k) == operand_order(m, k, 1) + operand_order(n, k, 1)
+
+
+@pytest.mark.parametrize("m,k,block,built", [
+    (2442, 4096, 4096, True), (1396, 7168, 1024, True), (26042, 384, 128, True), (19532, 512, 8, True),         # 25.4 -> 23.7, 31.6 -> 24.6, 45 -> 32, 35 -> 31 us
+    (4608, 14336, 2048, True), (4883, 4096, 8, True), (13021, 1536, 512, True), (26042, 768, 256, True),         # 204 -> 78, 26.0 -> 25.1, 40 -> 34, 49 -> 41
+    (2442, 4096, 8, False), (3907, 2560, 512, False), (698, 14336, 512, False), (13021, 768, 8, False),          # 15.5 -> 22.7, 21.0 -> 24.5, 21.7 -> 23.7, 25.1 -> 25.6
+    (9766, 1024, 128, False), (2048, 4096, 4096, False), (20000, 8192, 8192, False), (20000, 4100, 4, False)])   # 21.1 -> 24.3, 21.2 -> 23.7, no such kernel
+def test_large_quantizer_calls_build_a_plan_where_that_is_faster(m, k, block, built):
+    import torch
+
+    from orbitquant_amd import ops
+
+    for dtype, sixteen_bit in ((torch.bfloat16, True), (torch.float16, True), (torch.float32, False)):
+        rows = torch.empty(m, k, dtype=dtype, device="meta")
+        assert ops._worth_a_plan(rows, 16, block, block ** -0.5) == (built and sixteen_bit)
