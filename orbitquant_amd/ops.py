@@ -7,6 +7,7 @@ pass raw device pointers and the current HIP stream, and never synchronize.
 
 from __future__ import annotations
 
+import ctypes
 import warnings
 
 import torch
@@ -214,10 +215,13 @@ _PLAN_FROM_VALUES = 10_000_000
 
 def _worth_a_plan(rows: torch.Tensor, levels: int, block_size: int, inv_sqrt_block: float) -> bool:
     m, dim = rows.shape
-    from_values = _PLAN_FROM_VALUES if block_size >= 1024 or dim <= 512 else 2 * _PLAN_FROM_VALUES
+    if m * dim < _PLAN_FROM_VALUES:
+        return False
+    block, factor = int(block_size), ctypes.c_float(float(inv_sqrt_block)).value   # (what the library is given)
+    from_values = _PLAN_FROM_VALUES if block >= 1024 or dim <= 512 else 2 * _PLAN_FROM_VALUES
     return (m * dim >= from_values and rows.dtype in (torch.float16, torch.bfloat16) and dim % 8 == 0 and dim <= 16384
-            and 8 <= block_size <= 4096 and block_size & (block_size - 1) == 0 and dim % block_size == 0
-            and 2 <= levels <= 16 and 0.0 < inv_sqrt_block < 3.0e38 and rows.data_ptr() % 16 == 0)
+            and 8 <= block <= 4096 and block & (block - 1) == 0 and dim % block == 0
+            and 2 <= levels <= 16 and 0.0 < factor < 3.0e38 and rows.data_ptr() % 16 == 0)
 
 
 def rotate_quantize(

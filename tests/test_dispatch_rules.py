@@ -131,3 +131,14 @@ def test_large_quantizer_calls_build_a_plan_where_that_is_faster(m, k, block, bu
     for dtype, sixteen_bit in ((torch.bfloat16, True), (torch.float16, True), (torch.float32, False)):
         rows = torch.empty(m, k, dtype=dtype, device="meta")
         assert ops._worth_a_plan(rows, 16, block, block ** -0.5) == (built and sixteen_bit)
+
+
+@pytest.mark.parametrize("block,factor,built", [(4096, 1 / 64, True), (4096.0, 1 / 64, True), (64.0, 1 / 8, False), (4096, 1e-60, False),
+                                                (4096, 1e60, False), (4096, float("inf"), False), (4096, float("nan"), False), (4096, 0.0, False)])
+def test_a_plan_built_for_a_call_refuses_nothing(block, factor, built):
+    """A plan needs a factor that is positive and finite as the float it is handed over as; the kernel without one does not."""
+    import torch
+
+    from orbitquant_amd import ops
+
+    assert ops._worth_a_plan(torch.empty(2442, 4096, dtype=torch.bfloat16, device="meta"), 16, block, factor) == built
