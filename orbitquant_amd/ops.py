@@ -221,7 +221,8 @@ def _worth_a_plan(rows: torch.Tensor, levels: int, block_size: int, inv_sqrt_blo
     from_values = _PLAN_FROM_VALUES if block >= 1024 or dim <= 512 else 2 * _PLAN_FROM_VALUES
     return (m * dim >= from_values and rows.dtype in (torch.float16, torch.bfloat16) and dim % 8 == 0 and dim <= 16384
             and 8 <= block <= 4096 and block & (block - 1) == 0 and dim % block == 0
-            and 2 <= levels <= 16 and 0.0 < factor < 3.0e38 and rows.data_ptr() % 16 == 0)
+            and 2 <= levels <= 16 and 0.0 < factor < 3.0e38 and rows.data_ptr() % 16 == 0
+            and m * (64 if dim <= 512 else 512) < 1 << 32)   # (a launch's threads; the kernel without a plan has fewer a row)
 
 
 def rotate_quantize(

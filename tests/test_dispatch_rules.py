@@ -142,3 +142,13 @@ def test_a_plan_built_for_a_call_refuses_nothing(block, factor, built):
     from orbitquant_amd import ops
 
     assert ops._worth_a_plan(torch.empty(2442, 4096, dtype=torch.bfloat16, device="meta"), 16, block, factor) == built
+
+
+@pytest.mark.parametrize("m,k,block,built", [(8_388_607, 8192, 1024, True), (8_388_608, 8192, 1024, False), (16_000_000, 8192, 1024, False),
+                                             (8_388_608, 512, 8, True), (67_108_863, 8, 8, True), (67_108_864, 8, 8, False)])
+def test_a_plan_is_built_only_for_launches_of_fewer_than_2_to_the_32_threads(m, k, block, built):
+    import torch
+
+    from orbitquant_amd import ops
+
+    assert ops._worth_a_plan(torch.empty(m, k, dtype=torch.bfloat16, device="meta"), 16, block, block ** -0.5) == built
