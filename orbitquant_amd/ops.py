@@ -294,7 +294,10 @@ def rotate_quantize(
     if plan is not None:
         plan = _plan_operand(plan, x, dim, block_size, levels)
     elif code_format == "nibble" and mode == OQ_VALUES_NONE and input_map is None and _worth_a_plan(rows, levels, block_size, inv_sqrt_block):
-        plan = rotate_plan(permutation, signs, boundaries, block_size=block_size, inv_sqrt_block=inv_sqrt_block)
+        try:
+            plan = rotate_plan(permutation, signs, boundaries, block_size=block_size, inv_sqrt_block=inv_sqrt_block)
+        except torch.OutOfMemoryError:   # (the same results without one)
+            pass
     lib = _lib.load()
     head = (m, dim, permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(), _ptr(centroids), levels,
             int(block_size), float(eps), float(inv_sqrt_block))

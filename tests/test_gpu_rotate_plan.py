@@ -393,3 +393,22 @@ def test_a_plan_built_for_the_call_changes_nothing(dev, k, h, dtype, monkeypatch
     monkeypatch.setattr(ops, "_PLAN_FROM_VALUES", 1)
     got, _, got_norms = call()
     assert torch.equal(got, want) and torch.equal(got_norms, norms)
+
+
+def test_without_memory_for_a_plan_built_for_the_call(dev, monkeypatch):
+    from orbitquant_amd import ops
+
+    _, _, h, inv, _, _, t = constants(dev, 384, 128, 4)
+    x = make_rows(40, 384, torch.bfloat16, seed=7).to(dev)
+    call = lambda: ops.rotate_quantize(x, t["perm"], t["signs"], t["bounds"], block_size=128, eps=1e-10, inv_sqrt_block=float(inv), code_format="nibble")
+    want, _, norms = call()
+    asked = []
+
+    def none_left(*args, **kw):
+        asked.append(args)
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(ops, "_PLAN_FROM_VALUES", 1)
+    monkeypatch.setattr(ops, "rotate_plan", none_left)
+    got, _, got_norms = call()
+    assert len(asked) == 1 and torch.equal(got, want) and torch.equal(got_norms, norms)
