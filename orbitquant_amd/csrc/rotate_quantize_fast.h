@@ -453,13 +453,17 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   const int team = wave / WB, part = wave % WB;  // wavefronts of one block
   int4 early_a[GW], early_b[GW];
   uint2 early_signs[GW];
+  typedef int loose_i32x4 __attribute__((ext_vector_type(4), aligned(4)));        // (the permutation and the signs may lie anywhere)
+  typedef unsigned loose_u32x2 __attribute__((ext_vector_type(2), aligned(1)));
   auto request_shared = [&](int u) {
 #pragma unroll
     for (int j = 0; j < GW; ++j) {
       const uint32_t c = static_cast<uint32_t>(min(u * H + (part * GW + j) * kLaneSpan + gather_first, Ki - kChunk));
-      early_a[j] = reinterpret_cast<const int4 *>(a.perm)[c / 4u];
-      early_b[j] = reinterpret_cast<const int4 *>(a.perm)[c / 4u + 1u];
-      early_signs[j] = *reinterpret_cast<const uint2 *>(a.signs + c);
+      const loose_i32x4 lo = *reinterpret_cast<const loose_i32x4 *>(a.perm + c), hi = *reinterpret_cast<const loose_i32x4 *>(a.perm + c + 4);
+      const loose_u32x2 sg = *reinterpret_cast<const loose_u32x2 *>(a.signs + c);
+      early_a[j] = make_int4(lo.x, lo.y, lo.z, lo.w);
+      early_b[j] = make_int4(hi.x, hi.y, hi.z, hi.w);
+      early_signs[j] = make_uint2(sg.x, sg.y);
     }
   };
   Ring early;

@@ -187,7 +187,6 @@ template <int DT, int LOG_H>
 int launch_few(const FastArgs &a, hipStream_t stream) {
   if constexpr (LOG_H >= 10) {
     if (a.map != nullptr || a.packed != nullptr || a.codes == nullptr || a.values != nullptr) return -1;
-    if (((reinterpret_cast<uintptr_t>(a.perm) | reinterpret_cast<uintptr_t>(a.signs)) & 15u) != 0) return -1;
     int wb = 1;
     while (wb < (1 << (LOG_H - 9)) && a.units * wb * 2 <= 16) wb *= 2;
     if (a.M * a.units * wb > 4096 && (a.units > 2 || a.M > 1024)) return -1;

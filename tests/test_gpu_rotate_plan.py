@@ -412,3 +412,23 @@ def test_without_memory_for_a_plan_built_for_the_call(dev, monkeypatch):
     monkeypatch.setattr(ops, "rotate_plan", none_left)
     got, _, got_norms = call()
     assert len(asked) == 1 and torch.equal(got, want) and torch.equal(got_norms, norms)
+
+
+@pytest.mark.parametrize("k,h", [(4096, 4096), (3072, 1024), (14336, 2048), (16384, 4096)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("perm_off,signs_off", [(1, 0), (0, 1), (2, 4), (3, 7)])
+def test_few_rows_share_blocks_wherever_the_permutation_lies(dev, k, h, dtype, perm_off, signs_off):
+    """Elements off an aligned address do not send a call to the slower kernel.  What tells them apart: blocks are shared on the
+    signs themselves, which are here the opposite of those that the plan has, and the other kernel takes the plan's."""
+    from oracle import oracle_c
+    from orbitquant_amd import ops
+
+    perm, signs, _, inv, _, bounds, t = constants(dev, k, h, 4)
+    x = make_rows(8, k, dtype, seed=k)
+    plan = ops.rotate_plan(t["perm"], t["signs"], t["bounds"], block_size=h, inv_sqrt_block=float(inv))
+    off = lambda tensor, by: torch.cat([tensor[:by], tensor])[by:]
+    p, s = off(t["perm"], perm_off), off(-t["signs"], signs_off)
+    assert p.data_ptr() % 16 == 4 * perm_off and s.data_ptr() % 16 == signs_off
+    codes, _, norms = ops.rotate_quantize(x.to(dev), p, s, t["bounds"], block_size=h, eps=1e-10, inv_sqrt_block=float(inv), code_format="u8", plan=plan)
+    want, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, -signs, bounds, h, 1e-10, inv)
+    assert np.array_equal(codes.cpu().numpy(), want) and np.array_equal(norms.cpu().numpy().view(np.int32), want_norms.view(np.int32))
