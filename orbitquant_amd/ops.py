@@ -128,13 +128,17 @@ def rotate_plan(permutation: torch.Tensor, signs: torch.Tensor, boundaries: torc
                 inv_sqrt_block: float, copies: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:
     """The rotate plan of a layer (`oq_rotate_plan_build`): a uint8 blob on the constants' device
     that `rotate_quantize(plan=...)` and `quantized_linear(plan=...)` take to run the plan-based
-    kernel.  Built by one small launch; valid for exactly these constants.  `copies`: two tensors of the
-    permutation's and the signs' form that the launch fills with them."""
+    kernel.  Built by one small launch; valid for exactly these constants.  `copies`: two contiguous tensors of the
+    permutation's and the signs' type and size, on their device, that the launch fills with them."""
     _require_gpu(permutation, "permutation")
     dim = permutation.numel()
     permutation = _operand(permutation, "permutation", permutation, dtype=torch.int32)
     signs = _operand(signs, "signs", permutation, dtype=torch.int8, numel=dim)
     boundaries = _operand(boundaries, "boundaries", permutation, dtype=torch.float32)
+    if copies is not None:
+        for copy, of, name in zip(copies, (permutation, signs), ("permutation's copy", "signs' copy"), strict=True):
+            if _operand(copy, name, of, dtype=of.dtype, numel=dim) is not copy:
+                raise ValueError(f"the {name} must be contiguous")
     lib = _lib.load()
     plan = torch.empty(int(lib.oq_rotate_plan_bytes(dim)), dtype=torch.uint8, device=permutation.device)
     with _OnDevice(permutation):

@@ -432,3 +432,19 @@ def test_few_rows_share_blocks_wherever_the_permutation_lies(dev, k, h, dtype, p
     codes, _, norms = ops.rotate_quantize(x.to(dev), p, s, t["bounds"], block_size=h, eps=1e-10, inv_sqrt_block=float(inv), code_format="u8", plan=plan)
     want, want_norms = oracle_c.rotate_quantize(x.float().numpy(), perm, -signs, bounds, h, 1e-10, inv)
     assert np.array_equal(codes.cpu().numpy(), want) and np.array_equal(norms.cpu().numpy().view(np.int32), want_norms.view(np.int32))
+
+
+def test_copies_that_the_plans_launch_cannot_fill_are_refused(dev):
+    from orbitquant_amd import ops
+
+    _, _, _, inv, _, _, t = constants(dev, 384, 128, 4)
+    build = lambda *copies: ops.rotate_plan(t["perm"], t["signs"], t["bounds"], block_size=128, inv_sqrt_block=float(inv), copies=copies)
+    perm, signs = torch.empty_like(t["perm"]), torch.empty_like(t["signs"])
+    build(perm, signs)
+    assert torch.equal(perm, t["perm"]) and torch.equal(signs, t["signs"])
+    wide = torch.zeros(768, dtype=torch.int32, device=dev)
+    for wrong in ((perm[:383], signs), (perm, signs[1:]), (perm.long(), signs), (perm, signs.float()), (perm.cpu(), signs), (perm, signs.cpu()),
+                  (wide[::2], signs), (signs, perm), (perm,), (perm, signs, signs), (None, signs)):
+        with pytest.raises((ValueError, TypeError, AttributeError)):
+            build(*wrong)
+    assert not bool(wide.any()) and torch.equal(perm, t["perm"])
