@@ -157,8 +157,12 @@ def _on_device(tensors: dict[str, torch.Tensor], device: torch.device) -> dict[s
 
 
 def _separate(tensors: dict[str, torch.Tensor]) -> dict[str, torch.Tensor]:
-    """`_on_device`'s tensors with a storage for every type: torch saves no storage that is viewed as more than one."""
-    return {name: t.clone() if t.device.type == "cuda" and t.dtype != torch.float32 else t for name, t in tensors.items()}
+    """`_on_device`'s tensors with a storage for every type: torch saves no storage that is viewed as more than one.  (Those that
+    have one to themselves stay as they are.)"""
+    def shares(t):
+        return t.device.type == "cuda" and t.dtype != torch.float32 and t.untyped_storage().nbytes() != t.numel() * t.element_size()
+
+    return {name: t.clone() if shares(t) else t for name, t in tensors.items()}
 
 
 def _wait_for(device: torch.device) -> None:
@@ -208,9 +212,9 @@ class OrbitLinear(nn.Module):
         else:
             self.bias = nn.Parameter(bias.detach().clone(), requires_grad=False)
         device = packed_weight_indices.device
-        if constants is None:   # (`from_weight` has them on the device already, in storages of their own)
-            constants = _separate(_on_device(self._constants(), device))
-        for name, tensor in constants.items():
+        if constants is None:   # (`from_weight` has them on the device already)
+            constants = _on_device(self._constants(), device)
+        for name, tensor in _separate(constants).items():
             self.register_buffer(name, tensor, persistent=False)
         self.register_buffer("_rotation_plan", rotation_plan, persistent=False)
         if rotation_plan is None:
@@ -349,8 +353,6 @@ class OrbitLinear(nn.Module):
                                        block_size=rotation.block_size, inv_sqrt_block=rotation.normalization, copies=tuple(own.values()))
                 quantizer_constants = (constants["_rotation_permutation"], constants["_rotation_signs"], boundaries)
                 constants.update(own)
-            else:
-                constants = _separate(constants)
         packed, row_norms = quantize_weight(
             weight, rotation=rotation, codebook=codebook, bits=config.weight_bits,
             eps=config.activation_eps, row_tile=config.weight_row_tile_size, constants=quantizer_constants, plan=plan)

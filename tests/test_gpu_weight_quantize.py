@@ -287,3 +287,21 @@ def test_a_converted_layer_has_what_a_built_one_has(dev, bits):
             assert name == other and a.dtype == b.dtype and torch.equal(a, b), name
         torch.save(layer, io.BytesIO())
         layer._rotation_signs.neg_()      # (a layer's constants are its own: the next one is not made of them)
+
+
+def test_a_layer_of_constants_in_one_buffer_can_be_saved(dev):
+    import io
+
+    from orbitquant_amd import OrbitLinear, OrbitQuantConfig, layers
+
+    config = OrbitQuantConfig(weight_bits=4, activation_bits=4)
+    made = OrbitLinear.from_weight(torch.randn(136, 384).bfloat16().to(dev), bias=None, config=config)
+    constants = layers._on_device(made._constants(), made.row_norms.device)
+    layer = OrbitLinear(in_features=384, out_features=136, config=config, bias=None, packed_weight_indices=made.packed_weight_indices,
+                        row_norms=made.row_norms, constants=constants)
+    file = io.BytesIO()
+    torch.save(layer, file)
+    file.seek(0)
+    restored = torch.load(file, weights_only=False)
+    x = torch.randn(5, 384).bfloat16().to(dev)
+    assert torch.equal(restored(x), made(x)) and torch.equal(layer(x), made(x))
