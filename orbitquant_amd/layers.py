@@ -349,9 +349,8 @@ class OrbitLinear(nn.Module):
                 # (two copies behind the quantizer, 9 us, when they were cloned), and where the weights have as many bits as the
                 # activations it is the layer's plan too
                 own = {name: torch.empty_like(constants[name]) for name in ("_rotation_permutation", "_rotation_signs")}
-                plan = ops.rotate_plan(constants["_rotation_permutation"], constants["_rotation_signs"], boundaries,
-                                       block_size=rotation.block_size, inv_sqrt_block=rotation.normalization, copies=tuple(own.values()))
                 quantizer_constants = (constants["_rotation_permutation"], constants["_rotation_signs"], boundaries)
+                plan = ops._rotate_plan(*quantizer_constants, rotation.block_size, rotation.normalization, tuple(own.values()))
                 constants.update(own)
         packed, row_norms = quantize_weight(
             weight, rotation=rotation, codebook=codebook, bits=config.weight_bits,

@@ -136,20 +136,25 @@ def rotate_plan(permutation: torch.Tensor, signs: torch.Tensor, boundaries: torc
     signs = _operand(signs, "signs", permutation, dtype=torch.int8, numel=dim)
     boundaries = _operand(boundaries, "boundaries", permutation, dtype=torch.float32)
     if copies is not None:
-        for copy, of, name in zip(copies, (permutation, signs), ("permutation's copy", "signs' copy"), strict=True):
-            if _operand(copy, name, of, dtype=of.dtype, numel=dim) is not copy:
-                raise ValueError(f"the {name} must be contiguous")
+        for copy, of in zip(copies, (permutation, signs), strict=True):
+            if copy.dtype != of.dtype or copy.numel() != dim or copy.device != of.device or not copy.is_contiguous():
+                raise ValueError(f"a copy must hold {dim} contiguous {of.dtype} elements on {of.device}")
+    return _rotate_plan(permutation, signs, boundaries, block_size, inv_sqrt_block, copies)
+
+
+def _rotate_plan(permutation, signs, boundaries, block_size, inv_sqrt_block, copies) -> torch.Tensor:
+    """`rotate_plan` of operands that need no check."""
+    dim, levels = permutation.numel(), boundaries.numel() + 1
     lib = _lib.load()
     plan = torch.empty(int(lib.oq_rotate_plan_bytes(dim)), dtype=torch.uint8, device=permutation.device)
     with _OnDevice(permutation):
-        args = (permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(), boundaries.numel() + 1, dim, int(block_size),
-                float(inv_sqrt_block), plan.data_ptr())
+        args = (permutation.data_ptr(), signs.data_ptr(), boundaries.data_ptr(), levels, dim, int(block_size), float(inv_sqrt_block), plan.data_ptr())
         if copies is None:
             rc = lib.oq_rotate_plan_build(*args, _stream(permutation))
         else:
             rc = lib.oq_rotate_plan_build_copy(*args, *(t.data_ptr() for t in copies), _stream(permutation))
     _lib.check(rc, "oq_rotate_plan_build")
-    plan._oq_plan_of = (int(dim), int(block_size), int(boundaries.numel() + 1))
+    plan._oq_plan_of = (dim, int(block_size), levels)
     return plan
 
 
