@@ -18,13 +18,14 @@ int check_launch(const char *what);
 // (kernel, device) pair needs `bytes` or more than it was granted before, and answers from a
 // small table afterwards.  False if the runtime refuses.
 bool reserve_dynamic_lds(const void *kernel, size_t bytes);
-// A launch with its arguments as the kernel declares them.  (The launch syntax, which hipLaunchKernelGGL writes out, hands the
+// A launch with its arguments as the kernel declares them; one that is no value of its parameter's type without a cast, or that
+// may not fit it, does not compile.  (The launch syntax, which hipLaunchKernelGGL writes out, hands the
 // configuration to the kernel's stub through two more calls of the runtime: 0.15 us of host time a launch, sixteen tokens through the
 // linears of a decoder layer, eight launches, 69.9 -> 68.2 us.)
 template <typename... P, typename... A>
 inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, A... args) {
   static_assert(sizeof...(P) == sizeof...(A), "one argument for every parameter");
-  std::tuple<P...> values(static_cast<P>(args)...);
+  std::tuple<P...> values(P{args}...);
   std::apply(
       [&](auto &...value) {
         void *pointers[] = {const_cast<void *>(static_cast<const void *>(&value))...};

@@ -327,3 +327,21 @@ def test_a_conversions_constants_are_kept_as_what_they_are_made_of(clear):
     assert kept.cache_info().misses == 20
     getattr(rotations, clear, getattr(codebooks, clear, None))()
     assert kept.cache_info().currsize == 0
+
+
+def test_a_launch_takes_only_arguments_that_fit(tmp_path):
+    """What the launch syntax refused (a void pointer for a typed one), and whole numbers that may not fit."""
+    source = tmp_path / "launch.hip"
+    include = ROOT / "orbitquant_amd" / "csrc" / "oq_common.h"
+    source.write_text(f'#include "{include}"\n' + """
+__global__ void kernel(float *out, const float *in, int n, int64_t m) {}
+void good(float *p, int n) { oq::launch_kernel(kernel, dim3(1), dim3(64), 0, nullptr, p, p, n, n); }
+#ifdef WRONG
+void wrong(float *p, const float *q, void *v, int64_t m, unsigned u, float f, int n) { oq::launch_kernel(kernel, dim3(1), dim3(64), 0, nullptr, WRONG); }
+#endif
+""")
+    check = ["hipcc", "--offload-arch=gfx950", "--offload-host-only", "-fsyntax-only", "-std=c++17", str(source)]
+    compiles = lambda *flags: subprocess.run(check + list(flags), capture_output=True, timeout=120).returncode == 0
+    assert compiles() and compiles("-DWRONG=p,q,n,m")
+    for wrong in ("v,q,n,m", "p,v,n,m", "q,q,n,m", "p,q,m,m", "p,q,u,m", "p,q,f,m"):
+        assert not compiles("-DWRONG=" + wrong), wrong
