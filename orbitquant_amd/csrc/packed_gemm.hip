@@ -103,24 +103,27 @@ int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits) { return choose_
 // The tile that a single launch takes: the choice above, or 128 x 192 (tile 6; two codes a byte and values, weights of up to
 // four bits) where its tiles fit one round of the 256 CUs and that is the shorter launch.  It comes behind all other rules -
 // decoding first, sharing K -, which know the shapes above only.  Its price, 5 us and 0.7 us a K-step (1.4 times that
-// for two and three bits), was fitted to 420 shapes of 65 to 3000 tokens and looked at on 500 others: 27 of these take it, at 0.89
-// of the time (geometric mean), none at more than 1.01; 762 x 5720 x 2560 50 -> 37 us, 463 x 11400 x 768 18.4 -> 15.0 us, fp16 values
+// for two and three bits), was fitted to 420 shapes of 65 to 3000 tokens; 762 x 5720 x 2560 50 -> 37 us, 463 x 11400 x 768 18.4 -> 15.0 us, fp16 values
 // 512 x 12288 x 3072 47 -> 42 us.  Allowed several rounds, or the price without the 1.4, five of 40 lose 4 to 13 %.
-// Against a launch whose wavefronts share K it adds four parts of K (four_sums), so that the error of the sums
-// is that launch's; against the others, which have one running sum, it has theirs, bit for bit.
-int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *four_sums) {
+// In place of a launch whose wavefronts share K it keeps the sums of parts of K apart (separate_sums), none longer than a quarter, so that the
+// error of the sums is no larger than that launch's; such parts need twelve K-steps.  In place of the others, which have one running
+// sum, it has theirs, bit for bit.
+constexpr int kSeparateSumsFrom = 12;  // K-steps: a part of three is a quarter of K then
+
+int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *separate_sums) {
   double cost = 0.0;
-  *four_sums = 0;
+  *separate_sums = 0;
   const char *force = debug_env(ENV_GEMM_TILE);
-  if (force != nullptr && (force[0] == '6' || force[0] == '7') && bits <= 4 && !byte_codes) {  // 7: with four sums
-    *four_sums = force[0] == '7' && K >= 256;
+  if (force != nullptr && (force[0] == '6' || force[0] == '7') && bits <= 4 && !byte_codes) {  // 7: with separate sums
+    *separate_sums = force[0] == '7' && K / 64 >= kSeparateSumsFrom;
     return 6;
   }
   const int tile = choose_tile_with_cost(M, N, K, bits, &cost, byte_codes);
   if (force != nullptr || bits > 4 || byte_codes) return tile;
   const int64_t tiles = ((M + 127) / 128) * ((N + 191) / 192);
   if (tiles > 256 || 5.0 + static_cast<double>(K / 64) * 0.7 * (bits == 4 ? 1.0 : 1.4) >= cost) return tile;
-  *four_sums = tile >= 4;
+  if (tile >= 4 && K / 64 < kSeparateSumsFrom) return tile;
+  *separate_sums = tile >= 4;
   return 6;
 }
 
@@ -256,7 +259,7 @@ int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float
   g.w = w; g.row_norms = row_norms; g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype;
   g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
   g.out_map = OutMap{out_map, out_map != nullptr && out_dtype == OQ_BF16 ? kWideLoBf16 : -1};
-  int tile = gemm_launch_tile(M, N, K, bits, a_mode == A_U8, &g.four_sums);
+  int tile = gemm_launch_tile(M, N, K, bits, a_mode == A_U8, &g.separate_sums);
   g.k_splits = 1;
   if (const char *where = debug_env(ENV_GEMM_STAMPS)) g.stamps = reinterpret_cast<uint64_t *>(strtoull(where, nullptr, 0));  // builds with -DOQ_GEMM_STAMPS: a device buffer for the kernel's phase stamps
   const int splits = gemm_choose_splits(M, N, K, bits, a_mode == A_U8);
@@ -265,7 +268,7 @@ int gemm_dispatch(int a_mode, const void *a, const float *row_scale, const float
     g.k_splits = splits;
     g.partials = static_cast<float *>(workspace);
     tile = 0;  // 128x128 tiles, two workgroups per CU
-    g.four_sums = 0;
+    g.separate_sums = 0;
   }
   const int rc = a_mode == A_NIBBLE ? launch_mode<A_NIBBLE>(g, bits, tile, stream) : gemm_launch_bytes(g, bits, tile, stream);
   if (rc != OQ_OK || g.k_splits == 1) return rc;

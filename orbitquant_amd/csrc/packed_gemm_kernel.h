@@ -74,7 +74,7 @@ struct GemmArgs {
   // adds them up and applies the epilogue.
   int k_splits;
   float *partials;
-  int four_sums;             // the 128 x 192 tile adds four partial sums over K, as wavefronts that share K do (gemm_launch_tile)
+  int separate_sums;         // the 128 x 192 tile keeps the sums of parts of K apart, as wavefronts that share K do (gemm_launch_tile)
   int window_ahead;          // the launch has kWideBytes of dynamic LDS for the output map's window (set by launch_cfg)
   // Builds with -DOQ_GEMM_STAMPS only: every wavefront writes the shader-clock and real-time counter
   // values it read at its phase boundaries to stamps[(workgroup * 4 + wavefront) * 16 ...] (NULL: none).
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   g.w_cents = w_cents; g.act_cents = act_cents; g.a = a_codes; g.w = w_packed;
   g.K = K32; g.M = M32; g.N = N32;
   g.a_levels = levels_splits & 0xffff; g.k_splits = (levels_splits >> 16) & 0xff; g.window_ahead = (levels_splits >> 24) & 1;
-  g.four_sums = (levels_splits >> 25) & 1;
+  g.separate_sums = (levels_splits >> 25) & 1;
   g.out_map.table = map_table;
   {  // (tile counts from the sizes: two divisions by constants instead of two more arguments)
     constexpr int kTM = (KSPLIT == 1 ? 2 : 1) * FM * 32, kTN = (KSPLIT == 1 ? 2 : 1) * FN * 32;
@@ -489,11 +489,13 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   for (int t = 0; t < kLookups; ++t)
     lookup_read(std::integral_constant<int, 0>{}, 0, 0, t, lookup_address(std::integral_constant<int, 0>{}, 0, t));
   OQ_STAMP(2);  // first operands looked up: the loop starts
-  // The 128 x 192 tile may keep the sums of four parts of K apart, as wavefronts that share K do (whole rounds of the buffers
-  // each, about a quarter): behind each but the last the accumulators go to a second set, which the registers have room
-  // for, and start again from zero.
-  constexpr bool kMaySum = FM == 2 && FN == 3 && KSPLIT == 1;
-  const int parts = kMaySum && g.four_sums != 0 ? 4 : 1;
+  // The 128 x 192 tile may keep the sums of parts of K apart, as the four wavefronts that share K do: behind each part but the
+  // last the accumulators go to a second set, which the registers have room for, and start again from zero.  A part is whole
+  // rounds of the buffers, and no longer than a quarter of K, so that there are four to eight of them (23 K-steps are seven
+  // parts of three and one of two): the rounding errors that they leave are no larger, those of adding them up included.
+  constexpr bool kMaySum = FM == 2 && FN == 3 && KSPLIT == 1 && NBUF == 3;
+  const int part_steps = max(NBUF, steps / (4 * NBUF) * NBUF);
+  const int parts = kMaySum && g.separate_sums != 0 ? (steps + part_steps - 1) / part_steps : 1;
   f32x16 sums[kMaySum ? FM : 1][kMaySum ? FN : 1];
   if constexpr (kMaySum) {
 #pragma unroll
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   int ks = 0;
 #pragma nounroll
   for (int part = 1; part <= parts; ++part) {
-    const int part_end = kMaySum && part < parts ? steps * part / 4 / NBUF * NBUF : steps;
+    const int part_end = kMaySum && part < parts ? part * part_steps : steps;
     for (; ks + NBUF <= part_end; ks += NBUF) {
       step(std::integral_constant<int, 0>{}, ks);
       step(std::integral_constant<int, 1>{}, ks + 1);
@@ -703,7 +705,7 @@ int launch_cfg(GemmArgs g, hipStream_t stream) {
     return fail(OQ_ERR_UNSUPPORTED, "packed_gemm: a dimension beyond 2^31");
   launch_kernel(kern, dim3(static_cast<unsigned>(total), splits), dim3(256), g.window_ahead ? kWideBytes : 0, stream,
                      g.w_cents, g.act_cents, g.a, g.w, g.out_map.table, static_cast<int>(g.K), static_cast<int>(g.M),
-                     static_cast<int>(g.N), g.a_levels | (g.k_splits << 16) | (g.window_ahead << 24) | (g.four_sums << 25), g);
+                     static_cast<int>(g.N), g.a_levels | (g.k_splits << 16) | (g.window_ahead << 24) | (g.separate_sums << 25), g);
   return check_launch("packed_gemm");
 }
 

@@ -7,7 +7,7 @@
 
 namespace oq {
 
-int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *four_sums);  // packed_gemm.hip
+int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *separate_sums);  // packed_gemm.hip
 
 // x: bf16 [M, K] as it is; M * K * 2 < 4 GB, 16-byte aligned rows.  No pass, no buffer.
 int gemm_staged_dispatch(const void *x, const float *token_scale, const uint8_t *w, int bits, const uint16_t *row_norms,
@@ -18,7 +18,7 @@ int gemm_staged_dispatch(const void *x, const float *token_scale, const uint8_t 
   g.w = w; g.row_norms = row_norms; g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype;
   g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
   g.out_map = OutMap{nullptr, -1};
-  const int tile = gemm_launch_tile(M, N, K, bits, false, &g.four_sums);
+  const int tile = gemm_launch_tile(M, N, K, bits, false, &g.separate_sums);
   auto go = [&](auto bits_c) {
     constexpr int BITS = decltype(bits_c)::value;
     if constexpr (BITS <= 4) {

@@ -61,7 +61,7 @@ int launch_tiled_bits(const GemmArgs &g, int bits, int tile, hipStream_t stream)
 }  // namespace
 
 int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits);  // packed_gemm.hip
-int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *four_sums);
+int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *separate_sums);
 
 // Tile of the decode-first GEMM, -1 where looking the weights up in every tile is as fast, or where that launch takes
 // the 128 x 96 or the 64 x 64 tile, for the reasons given at gemm_choose_dense: its sums are more exact, and the same with and without
@@ -109,7 +109,7 @@ int gemm_tiled_dispatch(bool f16, const void *x, const float *token_scale, const
   g.w = w; g.row_norms = row_norms; g.w_cents = w_cents; g.bias = bias; g.bias_dtype = bias_dtype;
   g.M = M; g.N = N; g.K = K; g.out = out; g.out_dtype = out_dtype;
   g.out_map = OutMap{nullptr, -1};
-  const int tile = gemm_launch_tile(M, N, K, bits, false, &g.four_sums);
+  const int tile = gemm_launch_tile(M, N, K, bits, false, &g.separate_sums);
   return f16 ? launch_tiled_bits<A_TILED_F16>(g, bits, tile, stream) : launch_tiled_bits<A_TILED>(g, bits, tile, stream);
 }
 

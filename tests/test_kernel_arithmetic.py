@@ -82,3 +82,18 @@ def test_folded_thresholds_decide_like_multiply_then_compare(checks, block):
         assert checks.oqk_fold_mismatches(b, float(c), 4096) == 0
     t = checks.oqk_fold_threshold(float("nan"), float(c))
     assert t != t
+
+
+def test_parts_of_k_leave_no_larger_error_than_wavefronts_that_share_it():
+    """The 128 x 192 tile keeps the sums of parts of K apart, whole rounds of three K-steps and no longer than a quarter, where it takes the
+    place of four wavefronts with a quarter each.  Rounding errors as independent, of a sum's size, which grows with the root of its
+    length: one for each of a step's four products, and one for each part added to the others.  Four to eight parts."""
+    def variance(parts):
+        return 2 * sum(p * p for p in parts) + sum(sum(parts[:i]) for i in range(2, len(parts) + 1))
+
+    for steps in range(12, 1000):
+        part = steps // 12 * 3
+        parts = [min(part, steps - at) for at in range(0, steps, part)]
+        quarters = [steps * (w + 1) // 4 - steps * w // 4 for w in range(4)]
+        assert sum(parts) == sum(quarters) == steps and 4 <= len(parts) <= 8
+        assert variance(parts) <= variance(quarters), steps
