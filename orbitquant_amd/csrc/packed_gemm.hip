@@ -102,12 +102,15 @@ int gemm_choose_tile(int64_t M, int64_t N, int64_t K, int bits) { return choose_
 
 // The tile that a single launch takes: the choice above, or 128 x 192 (tile 6; two codes a byte and values, weights of up to
 // four bits) where its tiles fit one round of the 256 CUs and that is the shorter launch.  It comes behind all other rules -
-// decoding first, sharing K -, which know the shapes above only.  Its price, 5 us and 0.7 us a K-step (1.4 times that
-// for two and three bits), was fitted to 420 shapes of 65 to 3000 tokens; 762 x 5720 x 2560 50 -> 37 us, 463 x 11400 x 768 18.4 -> 15.0 us, fp16 values
-// 512 x 12288 x 3072 47 -> 42 us.  Allowed several rounds, or the price without the 1.4, five of 40 lose 4 to 13 %.
-// In place of a launch whose wavefronts share K it keeps the sums of parts of K apart (separate_sums), none longer than a quarter, so that the
-// error of the sums is no larger than that launch's; such parts need twelve K-steps.  In place of the others, which have one running
-// sum, it has theirs, bit for bit.
+// decoding first, sharing K -, which know the shapes above only.  Its price, and where it is asked, was fitted to 1350 random shapes of 65 to
+// 3000 tokens, each on both tiles; of 12000 others 544 take it, at 0.85 of the time (geometric mean): in place of 128 x 128 tiles 0.83 (none at
+// more than 1.04), of 128 x 256 0.94 (values on two of 39 at 1.07 and 1.09), of 128 x 96 0.93 and of 64 x 64 0.87 (none at more than 1.01).
+//   - in place of tiles with one running sum it has that sum, bit for bit;
+//   - in place of tiles whose wavefronts share K it keeps the sums of parts of K apart, none longer than a quarter, so that the error of the
+//     sums is no larger than that launch's.  Such parts need twelve K-steps.  128 x 96 tiles are as quick or quicker with weights of two and
+//     three bits (2035 x 2840 x 2560 40.5 us there, 42.0 here) and from K = 5888 on (2620 x 1984 x 7680 100 us, 106), and 64 x 64 ones
+//     as long as they are done in two rounds of 512 (315 x 12904 x 2048 30.5 us, 33.7).
+// Allowed several rounds, or a lower price, more shapes lose than gain.
 constexpr int kSeparateSumsFrom = 12;  // K-steps: a part of three is a quarter of K then
 
 int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes, int *separate_sums) {
@@ -119,11 +122,12 @@ int gemm_launch_tile(int64_t M, int64_t N, int64_t K, int bits, bool byte_codes,
     return 6;
   }
   const int tile = choose_tile_with_cost(M, N, K, bits, &cost, byte_codes);
-  if (force != nullptr || bits > 4 || byte_codes) return tile;
-  const int64_t tiles = ((M + 127) / 128) * ((N + 191) / 192);
-  if (tiles > 256 || 5.0 + static_cast<double>(K / 64) * 0.7 * (bits == 4 ? 1.0 : 1.4) >= cost) return tile;
-  if (tile >= 4 && K / 64 < kSeparateSumsFrom) return tile;
-  *separate_sums = tile >= 4;
+  if (force != nullptr || bits > 4 || byte_codes || ((M + 127) / 128) * ((N + 191) / 192) > 256) return tile;
+  const double steps = static_cast<double>(K / 64) * (bits == 4 ? 1.0 : 1.4);
+  if (tile < 4) return 6.5 + 0.66 * steps < cost ? 6 : tile;
+  const bool slower = tile == 4 ? bits != 4 || K > 5120 : ((M + 63) / 64) * ((N + 63) / 64) <= 1024;
+  if (slower || K / 64 < kSeparateSumsFrom || 5.0 + 0.7 * steps >= cost) return tile;
+  *separate_sums = 1;
   return 6;
 }
 

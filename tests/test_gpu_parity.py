@@ -919,6 +919,17 @@ def test_the_128x192_tile_has_the_error_of_wavefronts_that_share_k(dev, k, libra
     assert all(squared["7"] <= 1.01 ** 2 * squared[tile] for tile in squared), squared
 
 
+@pytest.mark.parametrize(("m", "n", "k", "wbits", "tile"), [
+    (333, 14336, 4096, 4, "7"), (818, 6224, 4928, 4, "7"), (389, 8200, 1472, 4, "6"),   # in place of 128 x 96, 64 x 64 and 128 x 128 tiles
+    (128, 192, 1472, 4, "5"), (389, 8200, 1472, 3, "5"), (315, 12904, 2048, 4, "5"), (2035, 2840, 2560, 2, "4"), (2371, 2264, 7936, 4, "4")])
+def test_the_rule_takes_the_128x192_tile_with_the_sums_of_the_launch_in_whose_place_it_is(dev, m, n, k, wbits, tile, library_switch):
+    o = TileOperands(dev, m, n, k, wbits)
+    taken, taken_tile = o.multiply("codes"), tile
+    for tile, same in ((t, t == taken_tile) for t in ("7", "6", "5") + (("4",) if k % 256 == 0 else ())):
+        library_switch("OQ_GEMM_TILE", tile)
+        assert torch.equal(taken, o.multiply("codes")) == same, tile
+
+
 @pytest.mark.parametrize("tile", ["6", "7"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_the_128x192_tile_through_an_output_map(dev, tile, dtype, library_switch):
