@@ -380,18 +380,30 @@ def test_few_rows_with_an_unaligned_permutation(dev, which):
 
 @pytest.mark.parametrize("k,h", [(1152, 64), (3072, 1024), (4096, 4096), (8192, 8192), (13824, 512), (104, 8)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-def test_a_plan_built_for_the_call_changes_nothing(dev, k, h, dtype, monkeypatch):
-    """Also where it cannot be used (a block beyond 4096, fp32 rows, rows off a 16-byte boundary), and for a gather that repeats positions."""
+@pytest.mark.parametrize("gather", ["bijective", "repeated"])
+@pytest.mark.parametrize("start", ["aligned", "shifted"])
+def test_a_plan_built_for_the_call_changes_nothing(dev, k, h, dtype, gather, start, monkeypatch):
+    """One is built just where it can be used: not for a block beyond 4096, fp32 rows, or rows off a 16-byte boundary.  Also for a
+    gather that repeats positions, whose signs are applied behind it."""
     from orbitquant_amd import ops
 
     _, _, _, inv, _, _, t = constants(dev, k, h, 4)
-    t["perm"][5] = t["perm"][9]
+    if gather == "repeated":
+        t["perm"][5] = t["perm"][9]
     x = make_rows(40, k, dtype, seed=k).to(dev)
-    x = torch.cat([x.view(-1)[:1], x.view(-1)])[1:].view(40, k) if k == 104 else x
+    if start == "shifted":
+        x = torch.cat([x.view(-1)[:1], x.view(-1)])[1:].view(40, k)
+    assert (x.data_ptr() % 16 == 0) == (start == "aligned")
     call = lambda: ops.rotate_quantize(x, t["perm"], t["signs"], t["bounds"], block_size=h, eps=1e-10, inv_sqrt_block=float(inv), code_format="nibble")
+    built, build = [], ops.rotate_plan
+    monkeypatch.setattr(ops, "rotate_plan", lambda *args, **kw: built.append(build(*args, **kw)) or built[-1])
     want, _, norms = call()
+    assert not built
     monkeypatch.setattr(ops, "_PLAN_FROM_VALUES", 1)
     got, _, got_norms = call()
+    assert len(built) == (dtype != torch.float32 and h <= 4096 and start == "aligned")
+    for plan in built:
+        assert plan[32:36].cpu().numpy().view(np.uint32) == (gather == "bijective")
     assert torch.equal(got, want) and torch.equal(got_norms, norms)
 
 
