@@ -271,6 +271,49 @@ def test_rows_with_thresholds_of_their_own_equal_divided_ones(dev, k, dtype, bit
     assert np.array_equal(packed.view(n, -1)[rows].cpu().numpy().reshape(-1), want)
 
 
+def cell_of(v, scale, offset):
+    """The cell of a value in a plan's table: one fused multiply-add, one rounding to 0..255."""
+    place = (v.astype(np.float64) * np.float64(scale) + np.float64(offset)).astype(np.float32)
+    return np.clip(np.rint(place), 0, 255).astype(np.int64)
+
+
+@pytest.mark.parametrize(("k", "folds"), [(4096, True), (2048, True), (3072, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_which_rows_have_thresholds_of_their_own(dev, k, dtype, folds):
+    """What tells the two ways apart: the place of a value in the table is rounded once from the rotated value, or from the divided
+    one.  In a plan whose cells without a boundary hold 0 and 15 in turn the two differ for values between two cells.  Rows of
+    few values a wavefront are divided, and so are rows whose division needs the compiler's (here: norms above 2^20)."""
+    from orbitquant_amd import ops
+
+    n, bits, levels = 2048, 4, 16
+    perm, signs, block, inv = o.rpbh_constants(k, 2, "paper")
+    bounds = (np.linspace(0.7, 1.3, levels - 1) / np.sqrt(k)).astype(np.float32)
+    w = torch.randn(n, k, generator=torch.Generator().manual_seed(k)).to(dtype)
+    w[n // 2 :] *= 2.0 ** 30
+    t = lambda a: torch.from_numpy(a).to(dev)
+    args = (w.to(dev), t(perm.astype(np.int32)), t(signs), t(bounds))
+    kw = dict(block_size=block, inv_sqrt_block=float(inv))
+    plan = ops.rotate_plan(*args[1:], **kw).clone()
+    blob = plan.cpu().numpy()
+    scale, offset = blob[40:48].view(np.float32)
+    cells = blob[-2048:].view([("bound", np.float32), ("below", np.uint32)])
+    empty = np.isinf(cells["bound"])
+    assert blob[36:40].view(np.uint32) == 256 and empty.sum() == 256 - (levels - 1)
+    cells["below"][empty] = 15 * (np.arange(256) & 1)[empty]
+    packed, _ = ops.quantize_weight(*args, bits=bits, eps=1e-10, plan=t(blob), **kw)
+    got = packed.cpu().numpy().reshape(n, -1)
+    got = np.stack([got & 15, got >> 4], axis=-1).reshape(n, k)
+
+    x32 = w.float().numpy()
+    norm = np.sqrt(o.sumsq_v1(x32)).astype(np.float32).reshape(n, 1)
+    folded = cell_of(o.rotate(x32, perm, signs, block, np.float32(1)), np.float32(scale) * (np.float32(inv) / norm), offset)
+    divided = cell_of(o.rotate(x32, perm, signs, block, inv) / norm, scale, offset)
+    differ = empty[folded] & empty[divided] & (cells["below"][folded] != cells["below"][divided])   # (the others have a boundary to compare with)
+    divides = np.arange(n)[:, None] >= (n // 2 if folds else 0)
+    assert differ[: n // 2].any() and differ[n // 2 :].any()   # (some five each)
+    assert np.array_equal(got[differ], cells["below"][np.where(divides, divided, folded)][differ])
+
+
 @pytest.mark.parametrize("bits", [(4, 4), (3, 4)])
 def test_a_converted_layer_has_what_a_built_one_has(dev, bits):
     """One plan where weights and activations share a codebook, constants in storages of their own."""
