@@ -280,7 +280,8 @@ __device__ __forceinline__ void packed_gemv_body(const GemvArgs &g, uint32_t *ld
   // workgroup reached the barrier 5.4 to 7 us after their start, when most of their weights had arrived.  Behind one
   // batch of 32 wavefront rows and more, and with several token blocks, the second one is late enough: q, k and v of
   // 4096 x 4096, 1 / 16 tokens with the quantizer 15.2 -> 14.4 / 18.3 -> 17.3 us, 33 tokens 4096 x 14336 22.0 -> 21.3 us, 64 tokens
-  // 2048 x 8192 12.5 -> 12.1 us; smaller launches lose by it (1 token 4096 x 14336 14.1 -> 14.5 us).
+  // 2048 x 8192 12.5 -> 12.1 us; smaller launches lose by it (1 token 4096 x 14336 14.1 -> 14.5 us).  (64 rows a workgroup and four
+  // blocks of tokens, four-bit weights, are one register short then: it is stored in front of the loop and read behind it.)
   constexpr int kAhead = R * WAVES >= 32 || MB > 1 ? 1 : NB;
   if constexpr (!LATE) {
 #pragma unroll

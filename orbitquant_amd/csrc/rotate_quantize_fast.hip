@@ -9,7 +9,7 @@ namespace {
 
 using namespace rqf;
 
-// ---- plan construction: once per layer, twice per converted weight ----------
+// ---- plan construction: once per layer, twice per converted weight whose activations have other bits ----------
 // Workgroup 0 makes the header and the tables, the last one checks that the permutation is one, the others write 256
 // gather entries and signs each, and copies of the two where the caller wants its own (all in one workgroup they were a chain of K / 256 memory round trips: 10.2 -> 4.9 us
 // for rows of some thousand values; 6.2 us with the second table and the check).
@@ -142,8 +142,9 @@ __global__ __launch_bounds__(512, waves_per_simd(LOG_H, MAPPED)) void rotate_qua
   rotate_quantize_row_fast<DT, LOG_H, EMIT, MAPPED>(a, smem, blockIdx.x, threadIdx.x, blockDim.x >> 6, [] {});
 }
 
-// The arguments come one by one: the first sixteen dwords are in registers when a wavefront starts
-// (-amdgpu-kernarg-preload-count), where a struct has to be fetched before the first request can be made.
+// The arguments come one by one: the first fourteen dwords, all but levels_pow2 and eps, are in registers when a wavefront
+// starts (-amdgpu-kernarg-preload-count; of sixteen such registers two hold the arguments' address), where a struct has to be
+// fetched before the first request can be made.  The other two are first used behind the row and its norm.
 template <int DT, int LOG_H, int EMIT, int WB>
 __global__ __launch_bounds__(1024) void rotate_quantize_shared_kernel(const void *x, const int32_t *perm, const int8_t *signs,
                                                                       const unsigned char *plan, uint8_t *codes, float *norms, int K,
