@@ -724,7 +724,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   } else {
     const float4 groups = *reinterpret_cast<const float4 *>(red), flags = *reinterpret_cast<const float4 *>(red + 4);
     total = (groups.x + groups.y) + (groups.z + groups.w);
-    any_tiny = flags.x != 0.0f || (waves > 1 && flags.y != 0.0f) || (waves > 2 && flags.z != 0.0f) || (waves > 3 && flags.w != 0.0f);
+    // (no short circuits: they were three dependent reads in front of the root, 17 rows of 448 values 5.42 us with them, 5.24 without)
+    any_tiny = (flags.x != 0.0f) | ((waves > 1) & (flags.y != 0.0f)) | ((waves > 2) & (flags.z != 0.0f)) | ((waves > 3) & (flags.w != 0.0f));
   }
   const float s_norm = sqrtf(total);
   Reciprocal rc;
