@@ -496,6 +496,7 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
   constexpr bool kMaySum = FM == 2 && FN == 3 && KSPLIT == 1 && NBUF == 3;
   const int part_steps = max(NBUF, steps / (4 * NBUF) * NBUF);
   const int parts = kMaySum && g.separate_sums != 0 ? (steps + part_steps - 1) / part_steps : 1;
+  int ks = 0;
   f32x16 sums[kMaySum ? FM : 1][kMaySum ? FN : 1];
   if constexpr (kMaySum) {
 #pragma unroll
@@ -504,17 +505,14 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) sums[i][j][e] = 0.0f;
-  }
-  int ks = 0;
 #pragma nounroll
-  for (int part = 1; part <= parts; ++part) {
-    const int part_end = kMaySum && part < parts ? part * part_steps : steps;
-    for (; ks + NBUF <= part_end; ks += NBUF) {
-      step(std::integral_constant<int, 0>{}, ks);
-      step(std::integral_constant<int, 1>{}, ks + 1);
-      if constexpr (NBUF == 3) step(std::integral_constant<int, 2>{}, ks + 2);
-    }
-    if constexpr (kMaySum) {
+    for (int part = 1; part <= parts; ++part) {
+      const int part_end = part < parts ? part * part_steps : steps;
+      for (; ks + NBUF <= part_end; ks += NBUF) {
+        step(std::integral_constant<int, 0>{}, ks);
+        step(std::integral_constant<int, 1>{}, ks + 1);
+        step(std::integral_constant<int, 2>{}, ks + 2);
+      }
       if (part < parts) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -526,6 +524,12 @@ __global__ __launch_bounds__(256) void packed_gemm_kernel(const float *w_cents, 
               acc[i][j][e] = 0.0f;
             }
       }
+    }
+  } else {  // (written again and not as the one part of that loop, whose code is another: bf16 values of 1467 x 7824 x 5696 138.5 us so, 135.2 here)
+    for (; ks + NBUF <= steps; ks += NBUF) {
+      step(std::integral_constant<int, 0>{}, ks);
+      step(std::integral_constant<int, 1>{}, ks + 1);
+      if constexpr (NBUF == 3) step(std::integral_constant<int, 2>{}, ks + 2);
     }
   }
   if (ks < steps) {
