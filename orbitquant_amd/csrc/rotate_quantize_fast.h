@@ -21,10 +21,10 @@
 // With few rows a wavefront alone on a block of 1024 to 4096 values is a long chain of dependent steps, so there WB
 // wavefronts share a block: each keeps 1 / WB of it in registers, and the butterflies between them go through LDS once.
 // Such a launch is one chain of memory round trips (a microsecond each, of lines that no cache near by holds) and of steps
-// that wait for each other, so everything it reads is requested when it starts: the plan's header is checked behind the
+// that wait for each other, so everything it reads is requested when it starts: the plan's header too, which is checked behind the
 // row, not in front of it, and as nothing of the plan that lies behind the header may be touched before that, the gather
 // entries and signs are made from the permutation and the signs themselves.  One row of 4096 / 14336 values, launch to
-// launch: 4.50 / 7.70 -> 4.21 / 7.05 us; 16 rows 4.78 / 8.45 -> 4.49 / 7.57 us.
+// launch: 4.44 / 7.74 -> 3.96 / 6.95 us; 17 rows of 4096 4.93 -> 4.42 us.
 //
 // The sum of squares keeps the documented order: [passes][256 lanes][8], tree over the lanes.
 // Compiled without FMA contraction.
@@ -277,6 +277,15 @@ __device__ __forceinline__ float largest_below(float b, double scale, bool &foun
 // little-endian stream; the norm is stored as bf16.
 enum EmitMode { EMIT_NIBBLE = 0, EMIT_U8 = 1, EMIT_ANY = 2, EMIT_WEIGHT = 3 };
 
+// The place where loaded values are waited for: without it that is the first use, and if this is in a loop (or behind the join of
+// two paths) that may have other loads under way, all of them are waited for, also what the caller requested in
+// `after_loads` - the whole of a one-token linear's weights.  (With that, and the plan's header in four loads that waited for
+// each other behind the row, one token through 2048 -> 4208 with two bits took 8.8 us and takes 7.7, 5120 -> 5120 with four 12.4 and
+// 11.6, cold weights; one row of 4096 / 14336 values 4.17 / 7.26 -> 3.96 / 6.95 us.)
+__device__ __forceinline__ void settle(int4 &a, int4 &b, uint2 &c) {
+  asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(a.w), "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w), "+v"(c.x), "+v"(c.y));
+}
+
 // Phase B of a row whose blocks of H values are shared by WB wavefronts each (EMIT_NIBBLE / EMIT_U8).  A wavefront
 // rotates its GW steps of 512 slots as far as its registers reach and writes them to LDS; behind one barrier a thread
 // takes CT consecutive columns of the WB parts, does the butterflies between the parts and makes their codes.
@@ -296,7 +305,11 @@ __device__ __forceinline__ void rotate_shared_blocks(const FastArgs &a, unsigned
   const bool plain = (modes & 1u) != 0u, searched = (modes & 2u) != 0u;
 #pragma nounroll
   for (int u = team; u < a.units && team < teams; u += teams) {
-    if (u != team) request(u);
+    if (u != team) {
+      request(u);
+#pragma unroll
+      for (int j = 0; j < GW; ++j) settle(ea[j], eb[j], sg[j]);
+    }
     const int first = u * H + part * SPAN;
     float y[GW][kChunk];
 #pragma unroll
@@ -415,7 +428,8 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   const int gather_first = (slot_lane ^ inverted_lanes(H)) * kChunk;               // and those whose inputs it starts from
   constexpr bool kSwapped = WB == 1 && EMIT != EMIT_ANY && H > 128;                // codes are swapped back, not values
   const int64_t K = a.K;
-  const plan::PlanHeader *hdr = reinterpret_cast<const plan::PlanHeader *>(a.plan);
+  plan::PlanHeader kept;  // WB > 1: read when everything else is requested
+  const plan::PlanHeader *hdr = WB > 1 ? &kept : reinterpret_cast<const plan::PlanHeader *>(a.plan);
   uint2 *cells = reinterpret_cast<uint2 *>(smem + kCellsAt);
   float *thr = reinterpret_cast<float *>(smem + kThrAt);
   float *cent = reinterpret_cast<float *>(smem + kCentAt);
@@ -435,11 +449,17 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   constexpr int kBatch = DT == OQ_F32 || WB > 1 ? 2 : 4;
   struct Ring { uint4 lo[kBatch], hi[kBatch], signs[kBatch]; };  // requested chunks of 512 values (fp32: both halves; 16-bit: lo only) and their signs
   auto request_row = [&](Ring &ring, int b, int i0) {  // chunks past the row: i0 >= Ki
+    if constexpr (WB > 1) {  // (none that is taken, nor one that lies partly past it: rows are whole blocks of 1024 and more)
+      const uint4 *src = reinterpret_cast<const uint4 *>(xrow + static_cast<uint32_t>(min(i0, Ki - kChunk)) * kElem);
+      ring.lo[b] = src[0];
+      if constexpr (DT == OQ_F32) ring.hi[b] = src[1];
+      return;
+    }
     ring.lo[b] = make_uint4(0u, 0u, 0u, 0u);
     ring.hi[b] = ring.lo[b];
     ring.signs[b] = ring.lo[b];
     if (i0 < Ki) {
-      if constexpr (WB == 1) ring.signs[b] = *reinterpret_cast<const uint4 *>(signs_by_position + static_cast<uint32_t>(i0));
+      ring.signs[b] = *reinterpret_cast<const uint4 *>(signs_by_position + static_cast<uint32_t>(i0));
       const uint4 *src = reinterpret_cast<const uint4 *>(xrow + static_cast<uint32_t>(i0) * kElem);
       ring.lo[b] = src[0];
       if constexpr (DT == OQ_F32) ring.hi[b] = src[1];
@@ -468,6 +488,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   };
   Ring early;
   if constexpr (WB > 1) {
+    kept = *reinterpret_cast<const plan::PlanHeader *>(a.plan);
     cell_v = reinterpret_cast<const uint2 *>(a.plan + plan::kCellsOffset)[table_idx];
     thr_v = reinterpret_cast<const float *>(a.plan + plan::kThresholdsOffset)[table_idx];
 #pragma unroll
@@ -538,7 +559,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
   auto take_chunk = [&](const Ring &ring, int b, int i0) __attribute__((always_inline)) -> float {
     float f[kChunk];
     if constexpr (DT == OQ_F32) {
-      if (i0 < Ki) {
+      if (WB > 1 || i0 < Ki) {
         uint4 lo = ring.lo[b], hi = ring.hi[b];
         if (WB == 1 && bijective) {
           const uint4 sg = ring.signs[b];
@@ -567,7 +588,7 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
         in = live ? one[0] : make_uint4(0u, 0u, 0u, 0u);
       }
       const uint32_t w[4] = {in.x, in.y, in.z, in.w};
-      if (i0 < Ki) {
+      if (WB > 1 || i0 < Ki) {
         const uint4 sg = ring.signs[b];
         *reinterpret_cast<uint4 *>(stage + 2 * i0) = WB == 1 && bijective ? make_uint4(w[0] ^ sg.x, w[1] ^ sg.y, w[2] ^ sg.z, w[3] ^ sg.w) : in;
       }
@@ -612,17 +633,21 @@ __device__ __forceinline__ void rotate_quantize_row_fast(const FastArgs &a, unsi
     // 4.6 us to stage, and takes 1.9.)
     after_loads();
     const int chunks = Ki / kLaneSpan;  // (rows are whole blocks of 1024 and more)
-#pragma nounroll
-    for (int c0 = wave; c0 < chunks; c0 += kBatch * waves) {
-      if (c0 != wave) {
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) request_row(early, b, (c0 + b * waves) * kLaneSpan + lane_first);
-      }
+    auto take_chunks = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
       for (int b = 0; b < kBatch; ++b) {
         const int c = c0 + b * waves;
         if (c < chunks) sums[((c >> 2) * 64 + lane) * 4 + (c & 3)] = take_chunk(early, b, c * kLaneSpan + lane_first);
       }
+    };
+    take_chunks(wave);
+#pragma unroll
+    for (int j = 0; j < GW; ++j) settle(early_a[j], early_b[j], early_signs[j]);
+#pragma nounroll
+    for (int c0 = wave + kBatch * waves; c0 < chunks; c0 += kBatch * waves) {
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) request_row(early, b, (c0 + b * waves) * kLaneSpan + lane_first);
+      take_chunks(c0);
     }
   } else {
     // Virtual lane t of the documented [passes][256 lanes][8] order is lane t % 64 of group t / 64; wavefront w owns the
